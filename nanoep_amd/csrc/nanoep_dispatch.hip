@@ -187,6 +187,7 @@ struct WalkArgs {
     // what only a few wavefronts need: a second turn, the prefetch workgroups, the plain list walk
     uint32_t window_vectors;        // 16-byte vectors of one window's source rows
     uint32_t source_vectors;        // ... of all source rows
+    uint32_t window_weights;        // (token, k) pairs of one window
     uint32_t rows_magic;  // fast divisor by rows_per_block
     uint32_t rows_shift;
     // gap rows
@@ -234,7 +235,26 @@ __device__ __forceinline__ void walk_gap_rows(const WalkArgs& a, uint32_t xcd, u
 // among them, and the copy wavefronts find their rows in the XCD's L2 (unless the write stream has
 // pushed a row out again before its last use: a window close to the size of the L2 re-reads part of
 // itself).  What it costs otherwise is one more L2 read per source row.
+//
+// The segment's share of the list and the window's weights come in the same way: a copy wavefront's
+// life is a chain (list entry, source row, store), and a handle that is replayed long after it was made
+// (a backward pass behind the other layers') has both in HBM only.  Handle in HBM, without -> with:
+// 32768 x 1024 top-8 129.4 -> 95.0 us, 4096 x 7168 top-8 with alignment 128 128.1 -> 97.1 us; behind a
+// layout that has just written the list 81.9 -> 78.6 us (4096 x 7168, count on the device).  One word a
+// 64-byte line is read, so 256 tokens x 8 choices are four wavefronts' loads.  Reading the next segment's
+// share too changed nothing (within 0.3 %).
 constexpr int kPrefetchLoads = 4;
+
+// Reads one word of every 64-byte line of bytes [first, end) behind `base`: `wave` of `waves`
+// wavefronts' part of them.
+__device__ __forceinline__ void touch_lines(const void* base, uint64_t first, uint64_t end, uint32_t wave, uint32_t waves) {
+    constexpr uint64_t kLine = 64;
+    for (uint64_t at = first / kLine * kLine + (wave * kWave + threadIdx.x % kWave) * kLine; at < end; at += waves * kWave * kLine) {
+        const uint64_t inside = at < first ? first : at;
+        const uint32_t word = *reinterpret_cast<const uint32_t*>(static_cast<const char*>(base) + inside);
+        asm volatile("" ::"v"(word));
+    }
+}
 
 // A uniform value as the compiler's vector value: what is computed from it runs on the vector unit.
 __device__ __forceinline__ uint32_t vector_copy(uint32_t uniform) {
@@ -374,6 +394,17 @@ __device__ __forceinline__ void walk_copy(const WalkArgs& a, uint32_t entries, u
         uint64_t window_end = window_first + a.window_vectors;
         if (window_end > a.source_vectors)
             window_end = a.source_vectors;
+        // the segment's share of the list, the window's weights (from the last wavefront on, the list's
+        // lines are the first ones'), then the window's rows
+        const uint64_t list_first = static_cast<uint64_t>(segment) * segment_entries;
+        const uint64_t list_end = list_first + segment_entries;
+        touch_lines(a.slot_order, list_first * 8, (list_end < entries ? list_end : entries) * 8, within * waves + wave, a.prefetch_blocks * waves);
+        if (a.weights != nullptr) {
+            const uint64_t weights_first = static_cast<uint64_t>(segment) * a.window_weights;
+            const uint64_t weights_end = weights_first + a.window_weights;
+            touch_lines(a.weights, weights_first * 4, (weights_end < a.source_limit ? weights_end : a.source_limit) * 4,
+                        a.prefetch_blocks * waves - 1 - (within * waves + wave), a.prefetch_blocks * waves);
+        }
         const uint64_t first = window_first + static_cast<uint64_t>(within * waves + wave) * (kPrefetchLoads * kWave);
         if (first < window_end) {
             u32x4 fetched[kPrefetchLoads];
@@ -704,6 +735,7 @@ int nanoep_dispatch(const void* x, const float* weights, const int32_t* recv_met
         a.prefetch_blocks = static_cast<uint32_t>(segment_prefetch_blocks);
         a.window_vectors = static_cast<uint32_t>(static_cast<int64_t>(window_tokens) * vectors);
         a.source_vectors = static_cast<uint32_t>(num_tokens * vectors);
+        a.window_weights = static_cast<uint32_t>(static_cast<int64_t>(window_tokens) * num_topk);
         a.segment_entries = static_cast<uint32_t>(segment_entries);
         a.windows = static_cast<uint32_t>(windows);
         a.windows_magic = windows_divisor.magic;
