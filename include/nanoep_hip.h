@@ -75,7 +75,7 @@ int nanoep_device_topology(int* out_cus, int* out_xcds, int64_t* out_l2_bytes);
  *   COMBINE_STORES (-1: by output size; 0 | 1: nontemporal / agent-scope stores for the combine's output)
  *   COMBINE_UNITS (0: by size; 1 .. 16 tokens a wavefront of the expanded combine with five or more
  *                     rows a token and the slot table; 1 = the one-token kernel)
- *   LAYOUT_LAUNCHES (0; 2 | 3: layout plan)     WINDOW_TOKENS (0; window of the slot-order list)
+ *   LAYOUT_LAUNCHES (0; 1 | 2 | 3: layout plan)  WINDOW_TOKENS (0; window of the slot-order list)
  *   RECALL_ORDER, FRESH_OUTPUTS, REBUILD_ORDER (-1; 0 | 1: host-extension policies)
  *   XCDS, L2_BYTES (0: ask the device)
  * nanoep_set_tuning / nanoep_get_tuning return NANOEP_ERR_INVALID_ARGUMENT for an unknown name;
@@ -99,8 +99,8 @@ size_t nanoep_layout_workspace_bytes(int64_t num_tokens, int num_topk, int64_t n
  * is ordered window of consecutive tokens by window, and a window's rows should fit one XCD's 4 MiB
  * L2: 512 tokens up to hidden 4096 (1024 tokens up to hidden 1024), 256 up to 8192 (and when hidden
  * is not known), then 128 and 64; fewer for batches of 257..4095 tokens so that there are eight
- * windows (sixteen before a window takes 1024 tokens), and the layout workgroup's
- * own token count when the layout needs its separate scan launch (more than 1024 workgroups). */
+ * windows (sixteen before a window takes 1024 tokens), and at most 256 for batches of more than 2^18
+ * tokens. */
 int nanoep_layout_block_tokens(int64_t num_tokens, int64_t num_local_experts, int hidden);
 
 /* Number of int64 words of the slot-order buffer for (T, K, L): T rounded up to 256, times K

@@ -9,15 +9,15 @@
 //   weights                   : fp32 [T,K] at the source, [N,K] compact, [C] expanded
 //
 // Kernels
-//   layout_count_kernel  : one workgroup per block of tokens; LDS bit matrix (expert x token) built
-//                          with LDS atomics, popcount prefixes give the in-block stable rank of
-//                          every (token,k) and the block's per-expert histogram.
-//   layout_assign_kernel<fused scan> : (few blocks) every workgroup sums the block histograms into
-//                          LDS, scans the aligned expert totals and writes its tokens' part of the
-//                          handle and of the slot-order list; workgroup 0 publishes N, C to the host.
-//   layout_single_block_kernel : (one block) count and assignment passes in a single launch.
-//   layout_scan_kernel + layout_assign_kernel<no scan> : (many blocks) the same in two launches, one
-//                          workgroup doing the scans: slot = offset[e] + block_base[b][e] + rank.
+//   layout_assign_kernel : one workgroup per block of tokens, a (token, choice) pair a lane: an LDS bit
+//                          matrix (expert x token) gives the in-block stable rank of every pair, sums over
+//                          the other blocks its expert's first slot; writes the tokens' part of the
+//                          handle and of the slot-order list.  One more workgroup publishes N, C to the
+//                          host.  Small batches: every workgroup counts the batch's ids itself, and this
+//                          is the layout's only launch.
+//   layout_histogram_kernel : ahead of it for larger batches: rows of per-expert counts, which every
+//                          assignment workgroup sums.
+//   layout_scan_kernel   : between the two for the largest: one workgroup turns the rows into prefixes.
 //   dispatch_walk_kernel : expanded layouts with the layout's slot-order list: one wavefront per
 //                          (list entry, row chunk), window of tokens by window and expert-major
 //                          inside a window, so a window's source rows stay in one XCD's L2 and every
@@ -50,7 +50,6 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
-#include <type_traits>
 
 #include "nanoep_hip.h"
 
@@ -92,7 +91,7 @@ struct Tuning {
     int combine_units = 0;          // COMBINE_UNITS: tokens a wavefront of the gather for five or more rows a token: 1 .. 16, 0 = by size
     int dispatch_pack = 0;          // DISPATCH_PACK: 1 = one list entry a wavefront of the slot-order walk whatever the row length
     int combine_stores = -1;        // COMBINE_STORES: 0 | 1 nontemporal / agent-scope stores for the combine's output, -1 = by size
-    int layout_launches = 0;        // LAYOUT_LAUNCHES: 2 | 3 forces the layout plan
+    int layout_launches = 0;        // LAYOUT_LAUNCHES: 1 | 2 | 3 forces the layout plan
     int window_tokens = 0;          // WINDOW_TOKENS: forces the window of the slot-order list
     int recall_order = -1;          // RECALL_ORDER: 0 = seven-tensor handles never get private tensors back (host extension)
     int fresh_outputs = -1;         // FRESH_OUTPUTS: 0 | 1 where a fresh dispatch's outputs are allocated (host extension)
@@ -118,19 +117,6 @@ struct Topology {
 void held_combine_residency(int out[4]);
 
 Topology current_topology(const Tuning& tuning);  // defined in nanoep_abi.hip
-
-// Calls f with the smallest compile-time bound in {4, 8, 16, 32} that covers num_topk.
-template <typename F>
-void with_topk_cap(int num_topk, F&& f) {
-    if (num_topk <= 4)
-        f(std::integral_constant<int, 4>{});
-    else if (num_topk <= 8)
-        f(std::integral_constant<int, 8>{});
-    else if (num_topk <= 16)
-        f(std::integral_constant<int, 16>{});
-    else
-        f(std::integral_constant<int, 32>{});
-}
 
 template <bool kNonTemporal>
 __device__ __forceinline__ u32x4 load_vec(const u32x4* p) {

@@ -6,8 +6,8 @@
 
 #include "nanoep_device.h"
 
-// Device memory of nanoep_layout_static: the layout kernels' workspace (block histograms, in-block
-// ranks, receive rows) for callers that cannot allocate.  Every GPU holds its own copy of the array
+// Device memory of nanoep_layout_static: the layout kernels' workspace (histogram
+// rows) for callers that cannot allocate.  Every GPU holds its own copy of the array
 // at its own address until the process ends; host code only ever uses the address that
 // hipGetSymbolAddress returns for the current device, never the array's name.
 static __device__ __align__(256) unsigned char scratch[NANOEP_STATIC_SCRATCH_BYTES];
@@ -15,8 +15,6 @@ static __device__ __align__(256) unsigned char scratch[NANOEP_STATIC_SCRATCH_BYT
 namespace nanoep {
 namespace {
 
-// Largest block of tokens a layout workgroup handles (one thread per token).
-constexpr int kMaxBlockTokens = 256;
 // What the launch plans below depend on besides the batch: the forced settings and the device's XCD
 // count and L2 size (the rows of one window should fit an XCD's L2, since the dispatch walks the
 // slot-order list window by window and wants every re-use of a source row to hit that cache).
@@ -33,10 +31,31 @@ Knobs current_knobs() {
     return {tuning.window_tokens, tuning.layout_launches, topology.xcds, topology.l2_bytes};
 }
 
-// Most blocks for which every assignment workgroup scans the block histograms itself.
-constexpr int kFusedScanMaxBlocks = 1024;
+// The slot-order buffer holds T rounded up to this many tokens' choices.
+constexpr int kOrderTokens = 256;
 // Largest window: the run of consecutive tokens the slot-order list is ordered by.
 constexpr int kMaxWindowTokens = 1024;
+// Largest batch that takes windows of more than 256 tokens.
+constexpr int64_t kMaxWideWindowBatch = int64_t{1} << 18;
+// Most threads of a layout workgroup.
+constexpr int kLayoutThreads = 1024;
+constexpr int kLayoutWaves = kLayoutThreads / kWave;
+// Most tokens of an assignment workgroup (four words of the bit matrix) and the (token, choice) pairs it aims at.
+constexpr int kMaxBlockTokens = 128;
+constexpr int kBlockPairs = 512;
+// Chunks of pairs a wavefront fetches at a time where it counts more than one.
+constexpr int kChunks = 4;
+// Pairs up to which every workgroup counts the whole batch by itself.  One launch against two, launch period:
+// 512 x 8, 128 experts 5.1 against 7.5 us, 2048 x 2, 8 experts 5.8 against 7.5, 1537 x 4, 60 experts 6.0
+// against 7.7, 1024 x 8, 128 experts 7.2 against 7.5, and 8.3 against 7.5 us at 4096 x 2 with 8 experts, where
+// the LDS additions meet on few words.
+constexpr int64_t kDirectPairs = 7168;
+// Histogram rows: the most every assignment workgroup sums by itself (a scan launch between, launch period:
+// 131072 tokens x 8, 256 experts, 512 rows 69 against 114 us; 262144 x 4, 64 experts, 1024 rows 58 against 64;
+// 524288 x 8, 2048 rows 251 against 161), and how many a wavefront fetches at a time (their number is padded
+// to a multiple of it).
+constexpr int64_t kSummedHistograms = 1024;
+constexpr int kSumRows = 16;
 
 // Tokens of one window of the slot-order list.
 //  * `hidden` (bf16 elements of a payload row, 0 = not known) sizes the window so that its rows fit an
@@ -51,7 +70,7 @@ constexpr int kMaxWindowTokens = 1024;
 //    tokens) to get there.
 // (sizes above are those of a 4 MiB L2 and 8 XCDs)
 int layout_window_tokens(int64_t tokens_total, int hidden, const Knobs& knobs) {
-    // WINDOW_TOKENS forces a window: any multiple of 32 up to 256 (one layout workgroup), or 512 / 1024
+    // WINDOW_TOKENS forces a window: any multiple of 32 up to 256, or 512 / 1024
     const int forced = knobs.window_tokens;
     if (forced >= 32 && forced % 32 == 0 && (forced <= 256 || forced == 512 || forced == 1024) && tokens_total > 256)
         return forced;
@@ -61,295 +80,311 @@ int layout_window_tokens(int64_t tokens_total, int hidden, const Knobs& knobs) {
              window > 64 && static_cast<int64_t>(window) * hidden * 2 > (window > 512 ? knobs.l2_bytes / 2 : knobs.l2_bytes - knobs.l2_bytes / 16);
              window /= 2) {
         }
-    if (tokens_total <= 256 && window > 256)
-        window = 256;  // one layout block: the whole layout is then a single launch
+    if ((tokens_total <= 256 || tokens_total > kMaxWideWindowBatch) && window > 256)
+        window = 256;
     while (tokens_total > 256 && window > 64 && (tokens_total + window - 1) / window < (window > 512 ? 2 * knobs.xcds : knobs.xcds))
         window /= 2;
     return window;
 }
 
-// Tokens handled by one layout workgroup (one thread per token): the window, at most 256, fewer when
-// the LDS bit matrix ((L+1) rows of tokens/32 words plus a 16-bit prefix per word) asks for it.  A
-// window of 512 tokens is two workgroups' worth: the assignment pass orders the list by windows from
-// the block histograms (a 512-token workgroup makes the dispatch as fast and the layout 5 us slower).
-int layout_tokens_per_block(int64_t tokens_total, int64_t local_experts, int hidden, const Knobs& knobs) {
-    if (static_cast<size_t>(local_experts + 1) * 16 > kLayoutLdsBudget)  // four int32 arrays of the assignment kernel
-        return 0;
-    const int window = layout_window_tokens(tokens_total, hidden, knobs);
-    for (int tokens = window < kMaxBlockTokens ? window : kMaxBlockTokens; tokens >= 32; tokens = tokens / 2 / 32 * 32) {
-        const size_t words = static_cast<size_t>(tokens / 32);
-        if (static_cast<size_t>(local_experts + 1) * (words * 6 + 4) <= kLayoutLdsBudget)
+// LDS of a workgroup: three counters an expert (and one row more for received tokens), then a bit
+// matrix of one bit a token.
+size_t layout_lds(int64_t local_experts, int64_t bit_words) {
+    return static_cast<size_t>(local_experts + 1) * 12 + static_cast<size_t>(local_experts) * bit_words * 4 + 16;
+}
+
+bool layout_supports(int64_t local_experts) { return local_experts > 0 && (local_experts + 1) * 16 <= static_cast<int64_t>(kLayoutLdsBudget); }
+
+// Tokens of one assignment workgroup: whole words of the bit matrix, a whole number of workgroups a window,
+// a chunk a wavefront; more once that makes two workgroups a compute unit.
+int layout_block_tokens_of(int64_t tokens_total, int window, int topk, int64_t local_experts) {
+    for (int tokens = kMaxBlockTokens; tokens > 32; tokens -= 32)
+        if (window % tokens == 0 && tokens * topk <= (tokens_total > 256 * (kBlockPairs / topk) ? 2 : 1) * kBlockPairs &&
+            layout_lds(local_experts, tokens / 32) <= kLayoutLdsBudget)
             return tokens;
+    return 32;
+}
+
+// Tokens of a histogram row: at least 64 where the window allows it, and more while an assignment wavefront
+// has more batches of rows to fetch than batches of ids between the start of its block's row and the block.
+int layout_histogram_tokens(int64_t tokens_total, int window, int block_tokens, int topk, int64_t local_experts) {
+    int tokens = block_tokens < 64 && window % 64 == 0 ? 64 : block_tokens;
+    while (window % (2 * tokens) == 0) {
+        const int64_t rows = (tokens_total + tokens - 1) / tokens;
+        const int64_t row_tasks = (rows + kSumRows - 1) / kSumRows * ((local_experts + kWave - 1) / kWave);
+        const int64_t id_batches = static_cast<int64_t>(2 * tokens - block_tokens) * topk / (kWave * kChunks);
+        if (row_tasks <= 8 || row_tasks <= id_batches)
+            break;
+        tokens *= 2;
     }
-    return 0;
+    return tokens;
 }
 
-// Layout blocks per window.  Windows of several blocks need every assignment workgroup to see the
-// block histograms (the two-launch plan); with a separate scan launch the window is the block.
-int layout_window_blocks(int64_t tokens_total, int64_t local_experts, int hidden, bool fused_scan, const Knobs& knobs) {
-    const int per_block = layout_tokens_per_block(tokens_total, local_experts, hidden, knobs);
-    const int window = layout_window_tokens(tokens_total, hidden, knobs);
-    return per_block == 0 || !fused_scan || window <= per_block ? 1 : window / per_block;
-}
-
-// Whether the layout of this batch runs as two launches (see nanoep_layout).
-bool layout_uses_fused_scan(int64_t tokens_total, int64_t local_experts, int hidden, const Knobs& knobs) {
-    const int per_block = layout_tokens_per_block(tokens_total, local_experts, hidden, knobs);
-    if (per_block == 0 || tokens_total == 0)
-        return false;
-    const int64_t blocks = (tokens_total + per_block - 1) / per_block;
-    const int forced = knobs.layout_launches;
-    if (forced == 3)
-        return false;
-    return forced == 2 || blocks <= kFusedScanMaxBlocks;
-}
-
-// Smallest block any `hidden` can lead to for this batch: what the workspace is sized for.
-int layout_smallest_block(int64_t tokens_total, int64_t local_experts, const Knobs& knobs) {
-    const int narrow = layout_tokens_per_block(tokens_total, local_experts, 1 << 20, knobs);
-    const int wide = layout_tokens_per_block(tokens_total, local_experts, 8, knobs);
-    return narrow < wide ? narrow : wide;
-}
+// What a histogram row holds besides its counts.
+struct RowInfo {
+    uint32_t received;  // tokens with any valid choice
+    uint32_t assigned;  // valid choices
+    int32_t status;     // routing status bits
+    uint32_t unused;
+};
 
 struct LayoutWorkspace {
-    int32_t* block_counts;  // [NB][L+1]; column L counts tokens with any valid choice
-    int32_t* block_status;  // [NB]
-    int32_t* packed_rank;   // [T][K]  (expert << 8) | in-block rank, or -1
-    int32_t* local_row;     // [T]
-    int64_t* totals;        // [1] total assignments, handed from the scan kernel to the assignment kernel
+    int32_t* histograms;  // [rows][L]
+    RowInfo* rows;        // [rows]
+    int64_t* totals;      // [1] total assignments, handed from the scan kernel to the assignment kernel
     size_t bytes;
 };
 
+int64_t padded_rows(int64_t rows) { return (rows + kSumRows - 1) / kSumRows * kSumRows; }
+
+// Sized for the most histogram rows a payload of any width can lead to, one every 64 tokens (32 under a
+// forced window that is no multiple of 64), padded.  The total has always had room for a word a (token, choice)
+// pair and a token as well, and callers hold buffers and one fixed array of that size: it stays.
 LayoutWorkspace carve_layout_workspace(void* base, int64_t tokens, int topk, int64_t local_experts, const Knobs& knobs) {
-    const int per_block = layout_smallest_block(tokens, local_experts, knobs);
-    const int64_t blocks = per_block == 0 ? 0 : (tokens + per_block - 1) / per_block;
+    const int row_tokens = knobs.window_tokens % 64 == 0 ? 64 : 32;
+    const int64_t rows = !layout_supports(local_experts) ? 0 : padded_rows((tokens + row_tokens - 1) / row_tokens);
     auto* cursor = static_cast<uint8_t*>(base);
     size_t offset = 0;
     LayoutWorkspace ws{};
-    ws.block_counts = reinterpret_cast<int32_t*>(cursor + offset);
-    offset = align_up(offset + static_cast<size_t>(blocks) * (local_experts + 1) * 4, 256);
-    ws.block_status = reinterpret_cast<int32_t*>(cursor + offset);
-    offset = align_up(offset + static_cast<size_t>(blocks) * 4, 256);
-    ws.packed_rank = reinterpret_cast<int32_t*>(cursor + offset);
-    offset = align_up(offset + static_cast<size_t>(tokens) * topk * 4, 256);
-    ws.local_row = reinterpret_cast<int32_t*>(cursor + offset);
-    offset = align_up(offset + static_cast<size_t>(tokens) * 4, 256);
+    ws.histograms = reinterpret_cast<int32_t*>(cursor + offset);
+    offset = align_up(offset + static_cast<size_t>(rows) * (local_experts + 1) * 4, 256);
+    ws.rows = reinterpret_cast<RowInfo*>(cursor + offset);
+    offset = align_up(offset + static_cast<size_t>(rows) * sizeof(RowInfo), 256);
     ws.totals = reinterpret_cast<int64_t*>(cursor + offset);
+    offset = align_up(offset + static_cast<size_t>(tokens) * topk * 4, 256);
+    offset = align_up(offset + static_cast<size_t>(tokens) * 4, 256);
     offset = align_up(offset + 8, 256);
     ws.bytes = offset + 256;
     return ws;
 }
 
-// A (token, k) entry of the rank table packs (expert << kRankBits) | in-block rank; -1 marks a
-// masked choice.  A layout block never holds more than 256 tokens, so the rank fits 8 bits.
-constexpr int kRankBits = 8;
-static_assert(kMaxBlockTokens <= (1 << kRankBits), "in-block ranks must fit the packed entry");
-constexpr int kRankMask = (1 << kRankBits) - 1;
-
-// One thread per token.  bits[e][w] has bit (token & 31) of word (token >> 5) set when the token
-// chose expert e; row L marks tokens with any valid choice.  Experts inside a token are distinct,
-// so the order of one expert's assignments is the token order and a popcount prefix is the rank.
-// The token's routing ids are fetched in one batch of independent loads (kCap >= K of them, the
-// surplus re-reads id 0) and stay in registers for both passes over the bit matrix.
-// What a thread of the count pass knows at its end, for a kernel that goes on to the assignment
-// pass in the same workgroup and need not read it back from memory.
-template <int kCap>
-struct CountedToken {
-    int32_t packed[kCap];  // the token's entries of the rank table
-    int32_t row;           // the token's receive row within the block, -1 when it is not sent
-    int32_t first_count;   // the block's count of histogram row threadIdx.x (0 when there is no such row)
-    int32_t bad;           // the block's routing status bits
+struct LayoutArgs {
+    const int64_t* topk_idx;  // [T][K]
+    int32_t* histograms;      // [rows][L]
+    RowInfo* rows;
+    uint32_t tokens;
+    uint32_t topk;
+    uint32_t experts;
+    uint32_t chunk_tokens;  // whole tokens a wavefront covers at a time: 64 / K
+    uint32_t chunk_pairs;   // chunk_tokens * K
+    uint32_t topk_magic;    // lane / K = (lane * topk_magic) >> 16
+    uint32_t waves;         // of a workgroup
+    uint32_t block_tokens;  // tokens of an assignment workgroup
+    uint32_t row_tokens;    // tokens of a histogram row: a multiple of block_tokens, a divisor of window_tokens
+    uint32_t row_magic;     // fast divisor by row_tokens
+    uint32_t row_shift;
+    uint32_t window_tokens;  // of the slot-order list, a multiple of block_tokens
+    uint32_t window_magic;   // fast divisor by window_tokens
+    uint32_t window_shift;
+    uint32_t row_count;    // histogram rows
+    uint32_t row_batches;  // ... in batches of kSumRows (the rows that pad the last one are zero)
+    uint32_t strips;       // experts in units of 64
+    uint32_t strips_magic;  // fast divisor by it
+    uint32_t strips_shift;
+    uint32_t per_thread;    // experts a thread takes in the scans
+    uint32_t expert_waves;  // wavefronts that have any
+    uint32_t check_tokens;  // tokens of a row whose bits fit the histogram kernel's LDS at a time
+    uint32_t expand;
+    uint32_t alignment_magic;  // fast divisor by the alignment
+    uint32_t alignment_shift;
+    int64_t alignment;
+    int64_t* totals;
+    int64_t* expert_counts;
+    int64_t* expert_offsets;
+    int64_t* send_counts;
+    int64_t* recv_rank_prefix;
+    int64_t* host_counts;
+    int64_t* snapshot;
+    int32_t* recv_metadata;
+    int64_t* dst_slots;
+    int32_t* token_slots;  // or null
+    int64_t* slot_order;   // or null
+    uint64_t list_entries;  // of the slot-order buffer, without its count word
+    uint32_t blocks;
 };
 
-template <int kCap>
-__device__ __forceinline__ void layout_count_block(const int64_t* __restrict__ topk_idx,
-                                                   int64_t num_tokens,
-                                                   int num_topk,
-                                                   int local_experts,
-                                                   int words,
-                                                   int threads,
-                                                   int64_t* __restrict__ snapshot,
-                                                   int32_t* block_counts,
-                                                   int32_t* block_status,
-                                                   int32_t* packed_rank,
-                                                   int32_t* local_row,
-                                                   CountedToken<kCap>& counted) {
-    extern __shared__ uint32_t layout_lds[];
-    const int rows = local_experts + 1;
-    // bit rows are words + 1 apart: an odd stride spreads the experts a wavefront touches over the LDS banks
-    const int stride = words + 1;
-    uint32_t* bits = layout_lds;
-    auto* prefix = reinterpret_cast<uint16_t*>(bits + static_cast<size_t>(rows) * stride);
-    __shared__ int block_bad;
+// Where an assignment workgroup gets the counts of the other workgroups' tokens from.
+enum LayoutSource {
+    kDirect,   // it counts all of the batch's ids itself: one launch, nothing passes through memory
+    kSummed,   // from the histogram rows layout_histogram_kernel left, which it sums itself
+    kScanned,  // from the prefixes layout_scan_kernel made of those rows
+};
 
-    const int tokens_per_block = words * 32;
-    const int local_token = threadIdx.x;
-    const int64_t token = static_cast<int64_t>(blockIdx.x) * tokens_per_block + local_token;
-    const bool live = local_token < tokens_per_block && token < num_tokens;
-    const int word = local_token >> 5;
-    const uint32_t bit = 1u << (local_token & 31);
+__device__ __forceinline__ int64_t round_up_to(int64_t count, const LayoutArgs& a) {
+    if (a.alignment == 1 || count == 0)
+        return count;
+    return static_cast<int64_t>(fast_divide(static_cast<uint32_t>(count) - 1u, a.alignment_magic, a.alignment_shift) + 1u) * a.alignment;
+}
 
-    typedef int64_t i64x2 __attribute__((ext_vector_type(2)));
-    typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
-    // rows of an even number of ids start 16-byte aligned when the tensor does: two ids a load and a store
-    const bool wide_ids = (num_topk & 1) == 0 && (reinterpret_cast<uintptr_t>(topk_idx) & 15) == 0;
-    const bool wide_snapshot = (num_topk & 1) == 0 && (reinterpret_cast<uintptr_t>(snapshot) & 15) == 0;
-    int64_t raw[kCap];
-    const int64_t* mine = topk_idx + (live ? token : 0) * num_topk;
-    if (wide_ids) {
-#pragma unroll
-        for (int k = 0; k < kCap; k += 2) {
-            const i64x2 pair = *reinterpret_cast<const i64x2*>(mine + (k < num_topk ? k : 0));
-            raw[k] = pair.x;
-            raw[k + 1] = pair.y;
-        }
-    } else {
-#pragma unroll
-        for (int k = 0; k < kCap; ++k)
-            raw[k] = mine[k < num_topk ? k : 0];
-    }
+// Wavefronts take (token, choice) pairs in chunks of whole tokens: pair token * K + k of the chunk on
+// that lane, the lanes left over idle.  A chunk's pairs are consecutive in every [T][K] array, so their
+// addresses are a uniform base plus the lane.  These kernels run a handful of workgroups and last a few
+// microseconds: what they cost is the instructions of a workgroup's wavefronts one after the other on
+// its compute unit (a vector instruction of 16 wavefronts is 7 ns) and the round trips between them.
+struct PairLane {
+    uint32_t lane;
+    uint32_t token;    // of the chunk
+    uint32_t k;
+    uint64_t earlier;  // the lanes of the same token's earlier choices
+};
 
-    for (int i = threadIdx.x; i < rows * stride; i += threads)
-        bits[i] = 0;
-    if (threadIdx.x == 0)
-        block_bad = 0;
-    __syncthreads();
+__device__ __forceinline__ PairLane pair_lane(const LayoutArgs& a) {
+    PairLane at;
+    at.lane = threadIdx.x % kWave;
+    at.token = (at.lane * a.topk_magic) >> 16;
+    at.k = at.lane - at.token * a.topk;
+    at.earlier = ((uint64_t{1} << at.k) - 1u) << (at.lane - at.k);
+    return at;
+}
 
-    int ids[kCap];  // expert id, -1 masked, -2 out of range
-#pragma unroll
-    for (int k = 0; k < kCap; ++k) {
-        const int64_t expert = raw[k];
-        ids[k] = (expert >= 0 && expert < local_experts) ? static_cast<int>(expert) : (expert == -1 ? -1 : -2);
-        if (!live || k >= num_topk)
-            ids[k] = -1;
-        else if (!wide_snapshot)
-            snapshot[token * num_topk + k] = expert;
-    }
-    if (live && wide_snapshot) {
-#pragma unroll
-        for (int k = 0; k < kCap; k += 2)
-            if (k < num_topk)
-                *reinterpret_cast<i64x2*>(snapshot + token * num_topk + k) = i64x2{raw[k], raw[k + 1]};
-    }
+// Pairs of the chunk that starts at token `first` of a range that ends at `end`.
+__device__ __forceinline__ uint32_t pairs_of_chunk(const LayoutArgs& a, uint32_t first, uint32_t end) {
+    if (first >= end)
+        return 0;
+    return end - first < a.chunk_tokens ? (end - first) * a.topk : a.chunk_pairs;
+}
 
+// The lane's id of that chunk, -1 when it has none.
+__device__ __forceinline__ int64_t fetch_id(const LayoutArgs& a, const PairLane& at, uint32_t first, uint32_t end) {
+    int64_t id = -1;
+    if (at.lane < pairs_of_chunk(a, first, end))
+        id = (a.topk_idx + static_cast<uint64_t>(first) * a.topk)[at.lane];
+    return id;
+}
+
+__device__ __forceinline__ bool names_expert(int64_t id, const LayoutArgs& a) { return static_cast<uint64_t>(id) < static_cast<uint64_t>(a.experts); }
+
+// (the layout goes on with what it takes for masked choices, and stays inside its bounds)
+__device__ __forceinline__ int check_id(int64_t id, const LayoutArgs& a) { return id == -1 || names_expert(id, a) ? 0 : NANOEP_ROUTING_BAD_EXPERT; }
+
+// Sets the token's bit in its expert's row of the bit matrix; true when it was set before (another
+// choice of the token names the same expert).
+__device__ __forceinline__ bool set_token_bit(uint32_t* bits, uint32_t words, int64_t id, uint32_t token) {
+    const uint32_t bit = 1u << (token % 32);
+    return (atomicOr(&bits[static_cast<uint32_t>(id) * words + token / 32], bit) & bit) != 0;
+}
+
+// Number of tokens of a chunk that open with this lane's pair: the token's first valid choice.
+__device__ __forceinline__ uint32_t count_opening(uint64_t valid_mask, bool counted, const PairLane& at) {
+    return __popcll(__ballot(counted && (valid_mask & at.earlier) == 0));
+}
+
+// The routing status bits any lane of the wavefront has.
+__device__ __forceinline__ int wave_status(int bad) {
+    return (__ballot(bad & NANOEP_ROUTING_BAD_EXPERT) ? NANOEP_ROUTING_BAD_EXPERT : 0) | (__ballot(bad & NANOEP_ROUTING_DUPLICATE) ? NANOEP_ROUTING_DUPLICATE : 0);
+}
+
+// Zeroes `words` words of LDS (16-byte aligned, room up to the next multiple of four).
+__device__ __forceinline__ void clear_lds(uint32_t* lds, uint32_t words, uint32_t threads) {
+    const u32x4 zero = {0u, 0u, 0u, 0u};
+    for (uint32_t i = threadIdx.x; i < (words + 3) / 4; i += threads)
+        reinterpret_cast<u32x4*>(lds)[i] = zero;
+}
+
+// One histogram row: the experts' counts among `row_tokens` tokens, and their RowInfo.  Rows behind the
+// batch's end come out zero.
+__global__ void __launch_bounds__(kLayoutThreads) layout_histogram_kernel(const LayoutArgs a, const uint32_t waves) {
+    extern __shared__ __align__(16) uint32_t histogram_lds[];
+    __shared__ RowInfo info;
+    const uint32_t words = a.check_tokens / 32;
+    const uint32_t counter_words = (a.experts + 3) / 4 * 4;
+    uint32_t* counts = histogram_lds;                // [L]
+    uint32_t* bits = histogram_lds + counter_words;  // [L][words]: check_tokens of the row at a time
+    const PairLane at = pair_lane(a);
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const uint32_t step = waves * a.chunk_tokens;
+    const uint32_t first = blockIdx.x * a.row_tokens;
+    const uint32_t row_end = first + a.row_tokens < a.tokens ? first + a.row_tokens : a.tokens;
     int bad = 0;
-    bool any = false;
+    uint32_t received = 0, assigned = 0;
+    uint32_t set_first = first;
+    do {
+        const uint32_t end = set_first + a.check_tokens < row_end ? set_first + a.check_tokens : row_end;
+        uint32_t chunk = set_first + wave * a.chunk_tokens;
+        int64_t id[kChunks];
 #pragma unroll
-    for (int k = 0; k < kCap; ++k) {
-        const int id = ids[k];
-        if (id >= 0) {
-            const uint32_t old = atomicOr(&bits[static_cast<size_t>(id) * stride + word], bit);
-            if (old & bit)
-                bad |= NANOEP_ROUTING_DUPLICATE;
-            any = true;
-        } else if (id == -2) {
-            bad |= NANOEP_ROUTING_BAD_EXPERT;
+        for (int j = 0; j < kChunks; ++j)
+            id[j] = fetch_id(a, at, chunk + j * step, end);
+        if (set_first == first) {
+            clear_lds(histogram_lds, counter_words + a.experts * words, waves * kWave);
+            if (threadIdx.x == 0)
+                info = RowInfo{0, 0, 0, 0};
+        } else {
+            __syncthreads();
+            clear_lds(bits, a.experts * words, waves * kWave);
         }
-    }
-    if (any)
-        atomicOr(&bits[static_cast<size_t>(local_experts) * stride + word], bit);
-    if (bad)
-        atomicOr(&block_bad, bad);
-    __syncthreads();
-
-    counted.first_count = 0;
-    for (int row = threadIdx.x; row < rows; row += threads) {
-        int running = 0;
-        for (int w = 0; w < words; ++w) {
-            prefix[static_cast<size_t>(row) * words + w] = static_cast<uint16_t>(running);
-            running += __popc(bits[static_cast<size_t>(row) * stride + w]);
-        }
-        block_counts[static_cast<int64_t>(blockIdx.x) * rows + row] = running;
-        if (row == static_cast<int>(threadIdx.x))
-            counted.first_count = running;
-    }
-    if (threadIdx.x == 0)
-        block_status[blockIdx.x] = block_bad;
-    __syncthreads();
-    counted.bad = block_bad;
-    counted.row = -1;
+        __syncthreads();
+        while (chunk < end) {
 #pragma unroll
-    for (int k = 0; k < kCap; ++k)
-        counted.packed[k] = -1;
-
-    if (live) {
-        const uint32_t below = bit - 1;
-        int32_t packed[kCap];
+            for (int j = 0; j < kChunks; ++j) {
+                const uint32_t chunk_first = chunk + j * step;
+                if (chunk_first >= end)
+                    break;  // (the same for the whole wavefront)
+                const bool valid = names_expert(id[j], a);
+                const uint64_t valid_mask = __ballot(valid);
+                if (valid) {
+                    atomicAdd(&counts[static_cast<uint32_t>(id[j])], 1u);
+                    if (set_token_bit(bits, words, id[j], chunk_first - set_first + at.token))
+                        bad |= NANOEP_ROUTING_DUPLICATE;
+                }
+                bad |= check_id(id[j], a);
+                received += count_opening(valid_mask, valid, at);
+                assigned += __popcll(valid_mask);
+            }
+            chunk += kChunks * step;
+            if (chunk < end) {
 #pragma unroll
-        for (int k = 0; k < kCap; ++k) {
-            const int id = ids[k];
-            packed[k] = -1;
-            if (id >= 0) {
-                const int rank = prefix[static_cast<size_t>(id) * words + word] +
-                                 __popc(bits[static_cast<size_t>(id) * stride + word] & below);
-                packed[k] = (id << kRankBits) | rank;
+                for (int j = 0; j < kChunks; ++j)
+                    id[j] = fetch_id(a, at, chunk + j * step, end);
             }
         }
-        if ((num_topk & 3) == 0 && (reinterpret_cast<uintptr_t>(packed_rank) & 15) == 0) {
-#pragma unroll
-            for (int k = 0; k < kCap; k += 4)
-                if (k < num_topk)
-                    *reinterpret_cast<i32x4*>(packed_rank + token * num_topk + k) = i32x4{packed[k], packed[k + 1], packed[k + 2], packed[k + 3]};
-        } else {
-#pragma unroll
-            for (int k = 0; k < kCap; ++k)
-                if (k < num_topk)
-                    packed_rank[token * num_topk + k] = packed[k];
-        }
-        const uint32_t received = bits[static_cast<size_t>(local_experts) * stride + word];
-        counted.row = (received & bit) ? prefix[static_cast<size_t>(local_experts) * words + word] + __popc(received & below) : -1;
-        local_row[token] = counted.row;
-#pragma unroll
-        for (int k = 0; k < kCap; ++k)
-            counted.packed[k] = packed[k];
+        set_first += a.check_tokens;
+    } while (set_first < row_end);
+    bad = wave_status(bad);
+    if (at.lane == 0 && (assigned != 0 || bad != 0)) {
+        atomicAdd(&info.received, received);
+        atomicAdd(&info.assigned, assigned);
+        atomicOr(&info.status, bad);
     }
+    __syncthreads();
+    int32_t* row = a.histograms + static_cast<uint64_t>(blockIdx.x) * a.experts;
+    for (uint32_t i = threadIdx.x; i < a.experts; i += waves * kWave)
+        row[i] = static_cast<int32_t>(counts[i]);
+    if (threadIdx.x == 0)
+        a.rows[blockIdx.x] = info;
 }
 
-template <int kCap>
-__global__ void __launch_bounds__(kMaxBlockTokens) layout_count_kernel(const int64_t* __restrict__ topk_idx,
-                                                           int64_t num_tokens,
-                                                           int num_topk,
-                                                           int local_experts,
-                                                           int words,
-                                                           int threads,
-                                                           int64_t* __restrict__ snapshot,
-                                                           int32_t* __restrict__ block_counts,
-                                                           int32_t* __restrict__ block_status,
-                                                           int32_t* __restrict__ packed_rank,
-                                                           int32_t* __restrict__ local_row) {
-    CountedToken<kCap> counted;
-    layout_count_block<kCap>(topk_idx, num_tokens, num_topk, local_experts, words, threads, snapshot, block_counts,
-                             block_status, packed_rank, local_row, counted);
+// The mailbox: words 1 to 3, and word 0 once they have arrived.  The stores are system-scope writes to
+// host memory and the wait between them is all the order they need: nothing else is published with
+// them, so no cache is written back (a release fence here writes back the XCD's L2, every token's part
+// of the handle included).
+__device__ __forceinline__ void publish_counts(int64_t* host_counts, int64_t received, int64_t capacity, int64_t assigned, int64_t status) {
+    __hip_atomic_store(&host_counts[1], capacity, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(&host_counts[2], assigned, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(&host_counts[3], status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __hip_atomic_store(&host_counts[0], received, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-__device__ __forceinline__ int64_t round_up_to(int64_t value, int64_t alignment) {
-    return alignment == 1 ? value : (value + alignment - 1) / alignment * alignment;
-}
-
-// Single workgroup.  Phase 1 turns every column of block_counts into its exclusive prefix over
-// blocks (threads are spread over columns x block segments so small expert counts still use the
-// whole workgroup).  Phase 2 scans the aligned expert totals.  The mailbox word 0 is stored last.
-__global__ void __launch_bounds__(kScanThreads) layout_scan_kernel(int32_t* __restrict__ block_counts,
-                                                                  const int32_t* __restrict__ block_status,
-                                                                  int num_blocks,
-                                                                  int local_experts,
-                                                                  int64_t alignment,
-                                                                  int64_t* __restrict__ expert_counts,
-                                                                  int64_t* __restrict__ expert_offsets,
-                                                                  int64_t* __restrict__ send_counts,
-                                                                  int64_t* __restrict__ recv_rank_prefix,
-                                                                  int64_t* __restrict__ totals,
-                                                                  int64_t* host_counts) {
-    extern __shared__ int32_t column_total[];  // [L+1]
+// Single workgroup.  Phase 1 turns every column of the histogram rows into its exclusive prefix
+// (threads are spread over columns x row segments so small expert counts still use the whole
+// workgroup).  Phase 2 scans the aligned expert totals.
+__global__ void __launch_bounds__(kScanThreads) layout_scan_kernel(const LayoutArgs a) {
+    extern __shared__ int32_t column_total[];  // [L+1]; column L is the received tokens
     __shared__ int32_t partial[kScanThreads];
     __shared__ int64_t scan[kScanThreads];
     __shared__ int64_t assignments[kScanThreads];
     __shared__ int status_bits;
 
     const int tid = threadIdx.x;
-    const int rows = local_experts + 1;
+    const int experts = static_cast<int>(a.experts);
+    const int rows = experts + 1;
+    const int num_blocks = static_cast<int>(a.row_count);
     if (tid == 0)
         status_bits = 0;
+    const auto word_at = [&](int b, int column) -> int32_t& {
+        return column < experts ? a.histograms[static_cast<int64_t>(b) * experts + column] : reinterpret_cast<int32_t&>(a.rows[b].received);
+    };
 
     const int columns_per_pass = rows < kScanThreads ? rows : kScanThreads;
     const int segments = kScanThreads / columns_per_pass;
@@ -364,7 +399,7 @@ __global__ void __launch_bounds__(kScanThreads) layout_scan_kernel(int32_t* __re
         int sum = 0;
         if (active)
             for (int b = begin; b < end; ++b)
-                sum += block_counts[static_cast<int64_t>(b) * rows + column];
+                sum += word_at(b, column);
         partial[tid] = active ? sum : 0;
         __syncthreads();
         if (active) {
@@ -372,9 +407,8 @@ __global__ void __launch_bounds__(kScanThreads) layout_scan_kernel(int32_t* __re
             for (int s = 0; s < segment; ++s)
                 running += partial[s * columns_per_pass + column_local];
             for (int b = begin; b < end; ++b) {
-                const int64_t at = static_cast<int64_t>(b) * rows + column;
-                const int count = block_counts[at];
-                block_counts[at] = running;
+                const int count = word_at(b, column);
+                word_at(b, column) = running;
                 running += count;
             }
             if (segment == segments - 1)
@@ -385,18 +419,18 @@ __global__ void __launch_bounds__(kScanThreads) layout_scan_kernel(int32_t* __re
 
     int bad = 0;
     for (int b = tid; b < num_blocks; b += kScanThreads)
-        bad |= block_status[b];
+        bad |= a.rows[b].status;
     if (bad)
         atomicOr(&status_bits, bad);
 
-    const int per_thread = (local_experts + kScanThreads - 1) / kScanThreads;
+    const int per_thread = (experts + kScanThreads - 1) / kScanThreads;
     const int first = tid * per_thread;
-    const int last = first + per_thread < local_experts ? first + per_thread : local_experts;
+    const int last = first + per_thread < experts ? first + per_thread : experts;
     int64_t padded_sum = 0, count_sum = 0;
     for (int e = first; e < last; ++e) {
         const int64_t count = column_total[e];
         count_sum += count;
-        padded_sum += round_up_to(count, alignment);
+        padded_sum += round_up_to(count, a);
     }
     scan[tid] = padded_sum;
     assignments[tid] = count_sum;
@@ -412,508 +446,500 @@ __global__ void __launch_bounds__(kScanThreads) layout_scan_kernel(int32_t* __re
     int64_t running = scan[tid] - padded_sum;
     for (int e = first; e < last; ++e) {
         const int64_t count = column_total[e];
-        expert_counts[e] = count;
-        expert_offsets[e] = running;
-        running += round_up_to(count, alignment);
+        a.expert_counts[e] = count;
+        a.expert_offsets[e] = running;
+        running += round_up_to(count, a);
     }
     if (tid == 0) {
-        const int64_t received = column_total[local_experts];
+        const int64_t received = column_total[experts];
         const int64_t capacity = scan[kScanThreads - 1];
-        expert_offsets[local_experts] = capacity;
-        send_counts[0] = received;
-        recv_rank_prefix[0] = received;
-        totals[0] = assignments[kScanThreads - 1];
-        host_counts[1] = capacity;
-        host_counts[2] = assignments[kScanThreads - 1];
-        host_counts[3] = status_bits;
-        __threadfence_system();
-        __hip_atomic_store(&host_counts[0], received, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        a.expert_offsets[experts] = capacity;
+        a.send_counts[0] = received;
+        a.recv_rank_prefix[0] = received;
+        a.totals[0] = assignments[kScanThreads - 1];
+        publish_counts(a.host_counts, received, capacity, assignments[kScanThreads - 1], status_bits);
     }
 }
 
-// Writes one token's part of the handle.  `packed` holds the token's entries of the rank table,
-// `slot_base[e]` is the first slot of this block's
-// assignments to expert e; `order_base[e]` is where expert e's run starts in the block's segment
-// of the slot-order list (`order` points at that segment, or is null).
-template <int kCap>
-__device__ __forceinline__ void assign_token_slots(int64_t token,
-                                                   int num_topk,
-                                                   int expand,
-                                                   int row_in_block,
-                                                   int64_t row_base,
-                                                   const int32_t* slot_base,
-                                                   const int32_t* order_base,
-                                                   const int32_t (&packed)[kCap],
-                                                   int32_t* __restrict__ recv_metadata,
-                                                   int64_t* __restrict__ dst_slots,
-                                                   int32_t* __restrict__ token_slots,
-                                                   int64_t* __restrict__ order) {
-    typedef int32_t i32x2 __attribute__((ext_vector_type(2)));
-    typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
-    // a token's row of the slot table: wide stores where the row width keeps them aligned
-    const auto store_table_row = [&](const int32_t (&values)[kCap]) {
-        if (token_slots == nullptr)
-            return;
-        int32_t* row = token_slots + token * num_topk;
-        if ((num_topk & 3) == 0 && (reinterpret_cast<uintptr_t>(token_slots) & 15) == 0) {
-#pragma unroll
-            for (int k = 0; k < kCap; k += 4)
-                if (k < num_topk)
-                    *reinterpret_cast<i32x4*>(row + k) = i32x4{values[k], values[k + 1], values[k + 2], values[k + 3]};
-        } else {
-#pragma unroll
-            for (int k = 0; k < kCap; ++k)
-                if (k < num_topk)
-                    row[k] = values[k];
-        }
-    };
-    int32_t values[kCap];
-#pragma unroll
-    for (int k = 0; k < kCap; ++k)
-        values[k] = -1;
-    if (row_in_block < 0) {
-        dst_slots[token] = -1;
-        store_table_row(values);
-        return;
-    }
-    const int64_t row = row_base + row_in_block;
-    dst_slots[token] = row;
-#pragma unroll
-    for (int k = 0; k < kCap; ++k) {
-        if (k >= num_topk)
-            break;
-        if (packed[k] >= 0) {
-            const int expert = packed[k] >> kRankBits;
-            const int rank = packed[k] & kRankMask;
-            values[k] = expand ? slot_base[expert] + rank : expert;
-            if (order != nullptr) {
-                const uint32_t source = static_cast<uint32_t>(token * num_topk + k);
-                order[order_base[expert] + rank] = (static_cast<int64_t>(values[k]) << 32) | source;
-            }
-        }
-    }
-    // the receive row [0, token, K values]: pairs of words when K is even and the table 8-byte aligned (every row then is)
-    int32_t* out = recv_metadata + row * (num_topk + 2);
-    if ((num_topk & 1) == 0 && (reinterpret_cast<uintptr_t>(recv_metadata) & 7) == 0) {
-        *reinterpret_cast<i32x2*>(out) = i32x2{0, static_cast<int32_t>(token)};
-#pragma unroll
-        for (int k = 0; k < kCap; k += 2)
-            if (k < num_topk)
-                *reinterpret_cast<i32x2*>(out + 2 + k) = i32x2{values[k], values[k + 1]};
-    } else {
-        out[0] = 0;
-        out[1] = static_cast<int32_t>(token);
-#pragma unroll
-        for (int k = 0; k < kCap; ++k)
-            if (k < num_topk)
-                out[2 + k] = values[k];
-    }
-    store_table_row(values);
+// Inclusive prefix sum over a wavefront, on the vector unit's own lane shifts (rows of 16, then the
+// rows' last lanes): a dozen instructions, against a trip to LDS and back for every step of a shuffle.
+template <int kControl, int kRowMask>
+__device__ __forceinline__ uint32_t lane_shift(uint32_t value) {
+    return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(value), kControl, kRowMask, 0xf, false));
 }
-
-__device__ __forceinline__ int64_t wave_inclusive_scan(int64_t value) {
-    const int lane = threadIdx.x & (kWave - 1);
-#pragma unroll
-    for (int distance = 1; distance < kWave; distance *= 2) {
-        const int64_t other = __shfl_up(value, distance, kWave);
-        if (lane >= distance)
-            value += other;
-    }
+template <int kControl, int kRowMask>
+__device__ __forceinline__ uint64_t lane_shift(uint64_t value) {
+    return static_cast<uint64_t>(lane_shift<kControl, kRowMask>(static_cast<uint32_t>(value))) |
+           static_cast<uint64_t>(lane_shift<kControl, kRowMask>(static_cast<uint32_t>(value >> 32))) << 32;
+}
+template <class T>
+__device__ __forceinline__ T wave_inclusive_scan(T value) {
+    value += lane_shift<0x111, 0xf>(value);  // row_shr:1
+    value += lane_shift<0x112, 0xf>(value);
+    value += lane_shift<0x114, 0xf>(value);
+    value += lane_shift<0x118, 0xf>(value);
+    value += lane_shift<0x142, 0xa>(value);  // row_bcast:15 into rows 1 and 3
+    value += lane_shift<0x143, 0xc>(value);  // row_bcast:31 into rows 2 and 3
     return value;
 }
 
-// Slot assignment, one workgroup per block of tokens (the blocks of layout_count_kernel).
-//
-// kFusedScan: `block_counts` holds the raw block histograms and every workgroup sums them itself
-// (they sit in L2): per column the total over all blocks and the part from the blocks before its
-// own, then the aligned exclusive scan over experts, all in LDS; the workgroup whose index is
-// `publisher` also writes the per-expert outputs and the host mailbox (word 0 last).  With several
-// blocks that is one more workgroup behind those of the blocks, which has no tokens of its own: the
-// store to host memory and its fence then sit on nobody's way to the token writes.  Otherwise
-// layout_scan_kernel has done that and `block_counts` holds each block's exclusive prefixes.
-//
-// Either way the workgroup also scans its own histogram over experts: that places every
-// assignment of the block in expert-major order inside the block's run of `slot_order`; the runs
-// of consecutive blocks follow each other without gaps and the unused tail of the list is -1.
-template <int kCap, bool kFusedScan, bool kOwnBlock = false>
-__device__ __forceinline__ void layout_assign_block(const int32_t* block_counts,
-                                                    const int32_t* block_status,
-                                                    int num_blocks,
-                                                    int64_t num_tokens,
-                                                    int num_topk,
-                                                    int local_experts,
-                                                    int tokens_per_block,
-                                                    int window_blocks,
-                                                    int threads,
-                                                    int expand,
-                                                    int64_t alignment,
-                                                    const int32_t* packed_rank,
-                                                    const int32_t* local_row,
-                                                    int64_t* expert_counts,
-                                                    int64_t* expert_offsets,
-                                                    int64_t* send_counts,
-                                                    int64_t* __restrict__ recv_rank_prefix,
-                                                    const int64_t* totals,
-                                                    int64_t* host_counts,
-                                                    int32_t* __restrict__ recv_metadata,
-                                                    int64_t* __restrict__ dst_slots,
-                                                    int32_t* __restrict__ token_slots,
-                                                    int64_t* __restrict__ slot_order,
-                                                    int publisher,
-                                                    const CountedToken<kCap>* own = nullptr) {
-    extern __shared__ int32_t assign_lds[];
-    __shared__ int64_t wave_padded[kMaxBlockTokens / kWave];
-    __shared__ int64_t wave_assigned[kMaxBlockTokens / kWave];
-    __shared__ int32_t wave_own[kMaxBlockTokens / kWave];
-    __shared__ int32_t wave_before[kMaxBlockTokens / kWave];
-    __shared__ int32_t wave_window_before[kMaxBlockTokens / kWave];
-    __shared__ int status_bits;
-    __shared__ int own_assignments;
-    const int rows = local_experts + 1;
-    int32_t* column_total = assign_lds;         // [L+1] totals over all blocks (fused scan only)
-    int32_t* slot_base = assign_lds + rows;     // [L+1] assignments before this block -> first slot per expert
-    // [L+1] histogram of this block's window (window_blocks consecutive blocks: the unit the slot-order
-    // list is ordered by) -> where an expert's run starts inside the window's part of the list
-    int32_t* order_base = assign_lds + 2 * rows;
-    int32_t* window_before = assign_lds + 3 * rows;  // [L+1] the window's assignments in the blocks before this one
+// One batch of histogram rows of one strip of 64 experts, a wavefront's task: task / strips is the batch,
+// task % strips the strip.
+struct RowTask {
+    uint32_t first_row;
+    uint32_t expert;  // this lane's
+    uint32_t counts[kSumRows];
+};
 
-    const int tid = threadIdx.x;
-    const int block = blockIdx.x;
-    const int64_t token = static_cast<int64_t>(block) * tokens_per_block + tid;
-    const bool live = tid < tokens_per_block && token < num_tokens;
-    // kOwnBlock: the count pass ran in this very workgroup (the batch is one block) and `own` holds
-    // what this thread found there; nothing of it is read back from memory.  With no more histogram
-    // rows than threads that goes for the histogram too: the block's counts are the totals, nothing
-    // lies before the block, and its window is the block.
-    const bool own_counts = kOwnBlock && rows <= threads;
-    int row_in_block;
-    int32_t packed[kCap];
-    if (kOwnBlock) {
-        row_in_block = own->row;
+__device__ __forceinline__ void fetch_rows(const LayoutArgs& a, const PairLane& at, uint32_t task, RowTask& out) {
+    const uint32_t batch = fast_divide(task, a.strips_magic, a.strips_shift);
+    out.first_row = batch * kSumRows;
+    out.expert = (task - batch * a.strips) * kWave + at.lane;
+    const uint32_t from = out.expert < a.experts ? out.expert : 0u;
+    const int32_t* row = a.histograms + static_cast<uint64_t>(out.first_row) * a.experts;
 #pragma unroll
-        for (int k = 0; k < kCap; ++k)
-            packed[k] = own->packed[k];
-    } else {
-        row_in_block = live ? local_row[token] : -1;
-        // fetched here, ahead of the scans, so that the round trip overlaps them
-#pragma unroll
-        for (int k = 0; k < kCap; ++k)
-            packed[k] = live ? packed_rank[token * num_topk + (k < num_topk ? k : 0)] : -1;
+    for (int j = 0; j < kSumRows; ++j) {
+        out.counts[j] = static_cast<uint32_t>(row[from]);
+        row += a.experts;
     }
+}
 
-    // the publishing workgroup gathers the blocks' routing status; the first word a thread is fetched here, used
-    // behind the histogram loads, so that its round trip is not a second one behind theirs
-    int first_status = 0;
-    if (kOwnBlock)
-        first_status = tid == 0 ? own->bad : 0;
-    else if (kFusedScan && block == publisher && tid < num_blocks)
-        first_status = block_status[tid];
-    if (own_counts) {
-        if (tid < rows) {
-            column_total[tid] = own->first_count;
-            slot_base[tid] = 0;
-            order_base[tid] = own->first_count;
-            window_before[tid] = 0;
-        }
-    } else if (kFusedScan) {
-        for (int i = tid; i < 4 * rows; i += threads)
-            assign_lds[i] = 0;
-        if (tid == 0) {
-            status_bits = 0;
-            own_assignments = 0;
-        }
-        __syncthreads();
-        const int window_first = block / window_blocks * window_blocks;
-        const int window_end = window_first + window_blocks;
+// (Sums and flags of a wavefront are reduced here before one lane adds them to LDS: an LDS addition of
+// different values by all lanes to one word is compiled into a loop over the lanes, a microsecond of it.)
+__device__ __forceinline__ uint32_t wave_sum(uint32_t value) { return __builtin_amdgcn_readlane(wave_inclusive_scan(value), kWave - 1); }
 
-        const int columns_per_pass = rows < threads ? rows : threads;
-        const int segments = threads / columns_per_pass;
-        const int blocks_per_segment = (num_blocks + segments - 1) / segments;
-        const int column_local = tid % columns_per_pass;
-        const int segment = tid / columns_per_pass;
-        const int begin = segment * blocks_per_segment;
-        const int end = begin + blocks_per_segment < num_blocks ? begin + blocks_per_segment : num_blocks;
-        // two columns a pass: with one more column than threads (L a multiple of the workgroup
-        // size, plus the received-token column) the loads of both are in flight together
-        for (int column0 = 0; column0 < rows; column0 += 2 * columns_per_pass) {
-            const int column = column0 + column_local;
-            const int second = column + columns_per_pass;
-            const bool active = segment < segments && column < rows;
-            const bool active_second = segment < segments && second < rows;
-            int total[2] = {0, 0}, before[2] = {0, 0}, own[2] = {0, 0}, window[2] = {0, 0}, earlier[2] = {0, 0};
-            // Histogram words are fetched sixteen blocks at a time, all loads of a batch in flight
-            // together whatever the number of blocks (positions past the last block re-read it and
-            // count nothing), and only a wavefront that holds a second column fetches it.
-            const bool wave_has_second = column - (tid & (kWave - 1)) + columns_per_pass < rows;
-            const int64_t second_or_first = active_second ? second : column;
-            if (active) {
-                for (int b0 = begin; b0 < end; b0 += 16) {
-                    int fetched[16], fetched_second[16];
+// What workgroup 0 of an assignment launch does: it has no tokens; it writes the per-expert outputs and the
+// host mailbox (the store to host memory and the wait for it are then on nobody's way to the token writes).
+// kDirect: it counts the batch's ids and checks them, with a bit matrix of the whole batch.
+template <int kSource>
+__device__ __forceinline__ void publish_layout(const LayoutArgs& a, uint32_t* lds) {
+    __shared__ uint64_t wave_padded[kLayoutWaves];
+    __shared__ RowInfo all;
+    const uint32_t tid = threadIdx.x;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const PairLane at = pair_lane(a);
+    uint32_t* counts = lds;  // [L]
+    uint32_t* bits = lds + (a.experts + 3) / 4 * 4;
+    const uint32_t words = kSource == kDirect ? (a.tokens + 31) / 32 : 0u;
+    const uint32_t step = a.waves * a.chunk_tokens;
+    uint32_t chunk = wave * a.chunk_tokens;
+    int64_t id[kChunks];
+    if (kSource == kDirect) {
 #pragma unroll
-                    for (int j = 0; j < 16; ++j) {
-                        const int64_t b = b0 + j < end ? b0 + j : end - 1;
-                        fetched[j] = block_counts[b * rows + column];
-                    }
-                    if (wave_has_second) {
+        for (int j = 0; j < kChunks; ++j)
+            id[j] = fetch_id(a, at, chunk + j * step, a.tokens);
+    }
+    clear_lds(lds, (a.experts + 3) / 4 * 4 + a.experts * words, a.waves * kWave);
+    if (tid == 0)
+        all = RowInfo{0, 0, 0, 0};
+    __syncthreads();
+    uint32_t received = 0, assigned = 0;
+    int bad = 0;
+    if (kSource == kDirect) {
+        while (chunk < a.tokens) {
 #pragma unroll
-                        for (int j = 0; j < 16; ++j) {
-                            const int64_t b = b0 + j < end ? b0 + j : end - 1;
-                            fetched_second[j] = block_counts[b * rows + second_or_first];
-                        }
-                    }
-#pragma unroll
-                    for (int j = 0; j < 16; ++j) {
-                        const int b = b0 + j;
-                        const int count = b < end ? fetched[j] : 0;
-                        const int count_second = wave_has_second && active_second && b < end ? fetched_second[j] : 0;
-                        const bool in_window = b >= window_first && b < window_end;
-                        total[0] += count;
-                        total[1] += count_second;
-                        before[0] += b < block ? count : 0;
-                        before[1] += b < block ? count_second : 0;
-                        own[0] = b == block ? count : own[0];
-                        own[1] = b == block ? count_second : own[1];
-                        window[0] += in_window ? count : 0;
-                        window[1] += in_window ? count_second : 0;
-                        earlier[0] += in_window && b < block ? count : 0;
-                        earlier[1] += in_window && b < block ? count_second : 0;
-                    }
+            for (int j = 0; j < kChunks; ++j) {
+                const uint32_t chunk_first = chunk + j * step;
+                if (chunk_first >= a.tokens)
+                    break;
+                const bool valid = names_expert(id[j], a);
+                const uint64_t valid_mask = __ballot(valid);
+                if (valid) {
+                    atomicAdd(&counts[static_cast<uint32_t>(id[j])], 1u);
+                    if (set_token_bit(bits, words, id[j], chunk_first + at.token))
+                        bad |= NANOEP_ROUTING_DUPLICATE;
                 }
+                bad |= check_id(id[j], a);
+                received += count_opening(valid_mask, valid, at);
+                assigned += __popcll(valid_mask);
             }
-            for (int i = 0; i < 2; ++i) {
-                const int at = i == 0 ? column : second;
-                if (!(i == 0 ? active : active_second))
-                    continue;
-                if (segments == 1) {
-                    column_total[at] = total[i];
-                    slot_base[at] = before[i];
-                    order_base[at] = window[i];
-                    window_before[at] = earlier[i];
-                } else {
-                    atomicAdd(&column_total[at], total[i]);
-                    atomicAdd(&slot_base[at], before[i]);
-                    if (window[i] != 0)
-                        atomicAdd(&order_base[at], window[i]);
-                    if (earlier[i] != 0)
-                        atomicAdd(&window_before[at], earlier[i]);
-                }
-            }
-            // this block's own assignments: one LDS atomic a wavefront (256 lanes adding to one word
-            // one after the other were most of a microsecond in front of the barrier)
-            int own_sum = (active && column < local_experts ? own[0] : 0) + (active_second && second < local_experts ? own[1] : 0);
+            chunk += kChunks * step;
+            if (chunk < a.tokens) {
 #pragma unroll
-            for (int distance = kWave / 2; distance > 0; distance /= 2)
-                own_sum += __shfl_xor(own_sum, distance, kWave);
-            if ((tid & (kWave - 1)) == 0 && own_sum != 0)
-                atomicAdd(&own_assignments, own_sum);
-        }
-        if (block == publisher) {
-            int bad = first_status;
-            for (int b = tid + threads; b < num_blocks; b += threads)
-                bad |= block_status[b];
-            if (bad)
-                atomicOr(&status_bits, bad);
+                for (int j = 0; j < kChunks; ++j)
+                    id[j] = fetch_id(a, at, chunk + j * step, a.tokens);
+            }
         }
     } else {
-        const int32_t* mine = block_counts + static_cast<int64_t>(block) * rows;
-        const bool last_block = block + 1 >= num_blocks;
-        for (int column = tid; column < rows; column += threads) {
-            const int32_t before = mine[column];
-            int32_t next;
-            if (!last_block)
-                next = mine[rows + column];
-            else
-                next = static_cast<int32_t>(column < local_experts ? expert_counts[column] : send_counts[0]);
-            order_base[column] = next - before;
-            window_before[column] = 0;  // the window is this block alone
-            slot_base[column] = before;
+        for (uint32_t task = wave; task < a.strips * a.row_batches; task += a.waves) {
+            RowTask rows;
+            fetch_rows(a, at, task, rows);
+            uint32_t total = 0;
+#pragma unroll
+            for (int j = 0; j < kSumRows; ++j)
+                total += rows.counts[j];
+            if (rows.expert < a.experts)
+                atomicAdd(&counts[rows.expert], total);
         }
+        for (uint32_t row = tid; row < a.row_count; row += a.waves * kWave) {
+            const RowInfo info = a.rows[row];
+            received += info.received;
+            assigned += info.assigned;
+            bad |= info.status;
+        }
+        received = wave_sum(received);
+        assigned = wave_sum(assigned);
+    }
+    bad = wave_status(bad);
+    if (at.lane == 0 && (assigned != 0 || bad != 0)) {
+        atomicAdd(&all.received, received);
+        atomicAdd(&all.assigned, assigned);
+        atomicOr(&all.status, bad);
     }
     __syncthreads();
-
-    const int per_thread = (local_experts + threads - 1) / threads;
-    const int first = tid * per_thread < local_experts ? tid * per_thread : local_experts;
-    const int last = first + per_thread < local_experts ? first + per_thread : local_experts;
-    int64_t padded_sum = 0, count_sum = 0;
-    int own_sum = 0, before_sum = 0, window_before_sum = 0;  // own_sum: the window's assignments (see order_base)
-    for (int e = first; e < last; ++e) {
-        if (kFusedScan) {
-            const int64_t count = column_total[e];
-            count_sum += count;
-            padded_sum += round_up_to(count, alignment);
-        }
-        own_sum += order_base[e];
-        before_sum += slot_base[e];
-        window_before_sum += window_before[e];
-    }
-    const int64_t padded_scan = kFusedScan ? wave_inclusive_scan(padded_sum) : 0;
-    const int64_t assigned_scan = kFusedScan ? wave_inclusive_scan(count_sum) : 0;
-    const int own_scan = static_cast<int>(wave_inclusive_scan(own_sum));
-    const int before_scan = static_cast<int>(wave_inclusive_scan(before_sum));
-    const int window_before_scan = static_cast<int>(wave_inclusive_scan(window_before_sum));
-    const int wave = tid / kWave;
-    const int waves = threads / kWave;
-    if ((tid & (kWave - 1)) == kWave - 1) {
-        wave_padded[wave] = padded_scan;
-        wave_assigned[wave] = assigned_scan;
-        wave_own[wave] = own_scan;
-        wave_before[wave] = before_scan;
-        wave_window_before[wave] = window_before_scan;
+    const uint32_t first = tid * a.per_thread < a.experts ? tid * a.per_thread : a.experts;
+    const uint32_t last = first + a.per_thread < a.experts ? first + a.per_thread : a.experts;
+    uint64_t padded_sum = 0, padded_scan = 0;
+    if (wave < a.expert_waves) {
+        for (uint32_t e = first; e < last; ++e)
+            padded_sum += static_cast<uint64_t>(round_up_to(counts[e], a));
+        padded_scan = wave_inclusive_scan(padded_sum);
+        if (at.lane == kWave - 1)
+            wave_padded[wave] = padded_scan;
     }
     __syncthreads();
-    int64_t running = padded_scan - padded_sum;
-    int running_own = own_scan - own_sum;
-    int64_t capacity = 0, assigned = 0;
-    // the window's assignments, those of all blocks before this one, and the window's share of the latter
-    int window_total = 0, assigned_before = 0, window_earlier = 0;
-    for (int w = 0; w < waves; ++w) {
-        running += w < wave ? wave_padded[w] : 0;
-        running_own += w < wave ? wave_own[w] : 0;
+    if (wave >= a.expert_waves)
+        return;
+    uint64_t running = padded_scan - padded_sum, capacity = 0;
+    for (uint32_t w = 0; w < a.expert_waves; ++w) {
+        running += w < wave ? wave_padded[w] : 0u;
         capacity += wave_padded[w];
-        assigned += wave_assigned[w];
-        window_total += wave_own[w];
-        assigned_before += wave_before[w];
-        window_earlier += wave_window_before[w];
     }
-    // this block's own assignments: the window's when the window is the block
-    const int own_total = kFusedScan && !own_counts ? own_assignments : window_total;
-    if (!kFusedScan)
-        assigned = totals[0];
-    for (int e = first; e < last; ++e) {
-        if (kFusedScan) {
-            const int64_t count = column_total[e];
-            if (block == publisher) {
-                expert_counts[e] = count;
-                expert_offsets[e] = running;
-            }
-            slot_base[e] += static_cast<int32_t>(running);
-            running += round_up_to(count, alignment);
-        } else {
-            slot_base[e] += static_cast<int32_t>(expert_offsets[e]);
-        }
-        const int in_window = order_base[e];
-        order_base[e] = running_own + window_before[e];  // behind the expert's entries of the window's earlier blocks
-        running_own += in_window;
+    if (tid == 0) {
+        publish_counts(a.host_counts, all.received, static_cast<int64_t>(capacity), all.assigned, all.status);
+        a.expert_offsets[a.experts] = static_cast<int64_t>(capacity);
+        a.send_counts[0] = all.received;
+        a.recv_rank_prefix[0] = all.received;
+        if (a.slot_order != nullptr)
+            a.slot_order[a.list_entries] = all.assigned;
     }
-    const int64_t received = kFusedScan ? column_total[local_experts] : 0;
+    for (uint32_t e = first; e < last; ++e) {
+        a.expert_counts[e] = counts[e];
+        a.expert_offsets[e] = static_cast<int64_t>(running);
+        running += static_cast<uint64_t>(round_up_to(counts[e], a));
+    }
+}
+
+// Slot assignment.  One workgroup per block of tokens, a chunk of (token, choice) pairs a wavefront, and,
+// unless a scan kernel has done that, one more in front of them that publishes (publish_layout).
+//
+// What a block needs of the others' tokens are sums per expert: the total (for the slots' aligned
+// offsets), the part before the block, and the window's part when a window of the slot-order list
+// holds several blocks.  kDirect: every workgroup counts the whole batch's ids into LDS by itself, an
+// LDS addition a pair, and the layout is one launch.
+//
+// Nothing here is bound by bytes (the batch's routing is under a megabyte): a launch is 2.2 us, and between
+// the first load and the last store lie 2.5 to 3.5 us of round trips and instruction issue: ids and rows
+// 0.7 us, counts 0.3, row sums 1.0, expert scan 0.4, slots 0.3, stores 0.7 (4096 x 8, 256 experts).
+// Hence a pair a lane instead of a token with all its choices a lane, all loads ahead of the first
+// wait, prefix sums by lane shifts in the wavefronts that hold experts only, and 64-token blocks (8
+// wavefronts) instead of 256-token ones.  Launch period of the whole layout, before -> after: 16 x 2 5.7 -> 4.8 us,
+// 256 x 8 with 64 experts 8.0 -> 5.0, 1537 x 6 with 60 experts 11.0 -> 7.5, 4096 x 8 with 256 experts 12.7 -> 9.0,
+// 32768 x 8 with 64 experts 16.1 -> 11.9, with 256 22.5 -> 14.8, 262144 x 4 with 64 experts 91 -> 35; from the call to the
+// counts on the host, idle device: 11.5 -> 9.0, 13.0 -> 9.9, 17.0 -> 13.5, 18.1 -> 13.9 us.
+//
+// The rank of a pair among its block's assignments to the same expert comes from a bit matrix: bit
+// (token) of row (expert) is set when the token chose it.  A token's choices are distinct, so the order
+// of an expert's assignments is the token order and the rank is the number of bits below the token's.
+template <int kSource, bool kWindow>
+__global__ void __launch_bounds__(kLayoutThreads) layout_assign_kernel(const LayoutArgs a) {
+    extern __shared__ __align__(16) uint32_t assign_lds[];
+    __shared__ uint32_t wave_padded[kLayoutWaves], wave_window[kLayoutWaves];
+    __shared__ uint32_t any_bits[kMaxBlockTokens / 32];  // the block's tokens with any valid choice
+    __shared__ struct {
+        uint32_t received_before;  // tokens with any valid choice before the block
+        uint32_t assigned;         // valid choices: all,
+        uint32_t assigned_before;  // before the block,
+        uint32_t window_start;     // before the window,
+        uint32_t own;              // in the block
+    } sums;
+    if (kSource != kScanned && blockIdx.x == 0) {
+        publish_layout<kSource>(a, assign_lds);
+        return;
+    }
+    const uint32_t tid = threadIdx.x;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const uint32_t block = kSource != kScanned ? blockIdx.x - 1 : blockIdx.x;
+    const uint32_t block_first = block * a.block_tokens;
+    const uint32_t block_end = block_first + a.block_tokens < a.tokens ? block_first + a.block_tokens : a.tokens;
+    const uint32_t window_first = kWindow ? fast_divide(block_first, a.window_magic, a.window_shift) * a.window_tokens : block_first;
+    const uint32_t own_row = kSource == kDirect ? 0u : fast_divide(block_first, a.row_magic, a.row_shift);
+    const PairLane at = pair_lane(a);
+    const uint32_t step = a.waves * a.chunk_tokens;
+    // What the workgroup reads leaves before anything waits: the wavefront's own ids, and the first of those it
+    // counts: of the whole batch, or what lies between the start of the block's histogram row and the block.
+    const uint32_t own_first = block_first + wave * a.chunk_tokens;
+    const int64_t id = fetch_id(a, at, own_first, block_end);
+    const uint32_t count_end = kSource == kDirect ? a.tokens : block_first;
+    uint32_t chunk = own_row * a.row_tokens + wave * a.chunk_tokens;
+    int64_t batch[kChunks];
+#pragma unroll
+    for (int j = 0; j < kChunks; ++j)
+        batch[j] = fetch_id(a, at, chunk + j * step, count_end);
+
+    const uint32_t tasks = kSource == kSummed ? a.strips * a.row_batches : 0u;
+    RowTask rows;
+    RowInfo info{0, 0, 0, 0};
+    if (kSource == kSummed) {
+        fetch_rows(a, at, wave < tasks ? wave : 0u, rows);
+        if (tid < a.row_count)
+            info = a.rows[tid];
+    }
+
+    const uint32_t words = a.block_tokens / 32;
+    const uint32_t counter_words = (3 * a.experts + 3) / 4 * 4;
+    uint32_t* base = assign_lds;                      // [L] counts before the block -> an expert's first slot in this block
+    uint32_t* order_base = base + a.experts;          // [L] the window's counts -> where an expert's run of the list starts
+    uint32_t* column_total = order_base + a.experts;  // [L] totals
+    uint32_t* bits = assign_lds + counter_words;      // [L][words]
+    clear_lds(assign_lds, counter_words + a.experts * words, a.waves * kWave);
+    if (tid < kMaxBlockTokens / 32)
+        any_bits[tid] = 0;
+    if (tid == 0)
+        sums = {0, 0, 0, 0, 0};
     __syncthreads();
-    if (kFusedScan && block == publisher && tid == 0) {
-        // Behind the workgroup's last barrier: the store to host memory and the wait that orders it
-        // hold up one wavefront, not the whole workgroup (in front of the barrier they were a
-        // microsecond of the kernel).
-        expert_offsets[local_experts] = capacity;
-        send_counts[0] = received;
-        recv_rank_prefix[0] = received;
-        host_counts[1] = capacity;
-        host_counts[2] = assigned;
-        host_counts[3] = kOwnBlock ? own->bad : status_bits;
-        __threadfence_system();
-        __hip_atomic_store(&host_counts[0], received, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
-    // The list is dense: a window's part starts where the assignments of the blocks before the window
-    // end.  Every block also clears as many entries of the unused tail as it has masked choices.
-    int64_t* order = nullptr;
-    if (slot_order != nullptr) {
-        order = slot_order + (assigned_before - window_earlier);
-        // every block before the last one is full; the last one holds what is left of the batch
-        const int64_t block_entries = static_cast<int64_t>(tokens_per_block) * num_topk;
-        const int64_t tokens_left = num_tokens - static_cast<int64_t>(block) * tokens_per_block;
-        const int64_t own_entries = (tokens_left < tokens_per_block ? tokens_left : tokens_per_block) * num_topk;
-        int64_t* tail = slot_order + assigned + (block * block_entries - assigned_before);
-        const int holes = static_cast<int>(own_entries) - own_total;
-        for (int i = tid; i < holes; i += threads)
-            tail[i] = -1;
-        // The buffer's size does not depend on the block size: (T rounded up to 256) * K entries, then
-        // the count word.  The last block (the one with the fewest tokens) clears what lies behind
-        // the blocks' own entries, so that everything from entry A to the count word reads -1.
-        const int64_t capacity_entries = (num_tokens + kMaxBlockTokens - 1) / kMaxBlockTokens * kMaxBlockTokens * num_topk;
-        if (block == num_blocks - 1)
-            for (int64_t i = num_tokens * num_topk + tid; i < capacity_entries; i += threads)
-                slot_order[i] = -1;
-        if (block == (kFusedScan ? publisher : 0) && tid == 0)
-            slot_order[capacity_entries] = assigned;
-    }
+    const bool own_valid = names_expert(id, a);
+    const uint64_t own_mask = __ballot(own_valid);
+    const uint32_t local = own_first - block_first + at.token;
+    const bool live = at.lane < pairs_of_chunk(a, own_first, block_end);
     if (live)
-        assign_token_slots<kCap>(token, num_topk, expand, row_in_block, slot_base[local_experts], slot_base, order_base,
-                                 packed, recv_metadata, dst_slots, token_slots, order);
-}
+        (a.snapshot + static_cast<uint64_t>(own_first) * a.topk)[at.lane] = id;
+    if (own_valid) {
+        (void)set_token_bit(bits, words, id, local);
+        if ((own_mask & at.earlier) == 0)
+            atomicOr(&any_bits[local / 32], 1u << (local % 32));
+    }
 
-template <int kCap, bool kFusedScan>
-__global__ void __launch_bounds__(kMaxBlockTokens) layout_assign_kernel(const int32_t* __restrict__ block_counts,
-                                                            const int32_t* __restrict__ block_status,
-                                                            int num_blocks,
-                                                            int64_t num_tokens,
-                                                            int num_topk,
-                                                            int local_experts,
-                                                            int tokens_per_block,
-                                                            int window_blocks,
-                                                            int threads,
-                                                            int expand,
-                                                            int64_t alignment,
-                                                            const int32_t* __restrict__ packed_rank,
-                                                            const int32_t* __restrict__ local_row,
-                                                            int64_t* expert_counts,
-                                                            int64_t* expert_offsets,
-                                                            int64_t* send_counts,
-                                                            int64_t* recv_rank_prefix,
-                                                            const int64_t* __restrict__ totals,
-                                                            int64_t* host_counts,
-                                                            int32_t* recv_metadata,
-                                                            int64_t* dst_slots,
-                                                            int32_t* token_slots,
-                                                            int64_t* slot_order,
-                                                            int publisher) {
-    layout_assign_block<kCap, kFusedScan>(block_counts, block_status, num_blocks, num_tokens, num_topk, local_experts,
-                                          tokens_per_block, window_blocks, threads, expand, alignment, packed_rank, local_row, expert_counts,
-                                          expert_offsets, send_counts, recv_rank_prefix, totals, host_counts, recv_metadata,
-                                          dst_slots, token_slots, slot_order, publisher);
-}
-
-// Whole layout in one launch when all tokens fit one block: the count pass, then (its results are
-// this workgroup's own global writes: the barrier orders them for the workgroup, and a fence of
-// wider scope in front of it would write the XCD's L2 back for nobody) the assignment pass.
-template <int kCap>
-__global__ void __launch_bounds__(kMaxBlockTokens) layout_single_block_kernel(const int64_t* topk_idx,
-                                                                  int64_t num_tokens,
-                                                                  int num_topk,
-                                                                  int local_experts,
-                                                                  int words,
-                                                                  int threads,
-                                                                  int expand,
-                                                                  int64_t alignment,
-                                                                  int64_t* snapshot,
-                                                                  int32_t* block_counts,
-                                                                  int32_t* block_status,
-                                                                  int32_t* packed_rank,
-                                                                  int32_t* local_row,
-                                                                  int64_t* expert_counts,
-                                                                  int64_t* expert_offsets,
-                                                                  int64_t* send_counts,
-                                                                  int64_t* recv_rank_prefix,
-                                                                  int64_t* host_counts,
-                                                                  int32_t* recv_metadata,
-                                                                  int64_t* dst_slots,
-                                                                  int32_t* token_slots,
-                                                                  int64_t* slot_order) {
-    CountedToken<kCap> counted;
-    layout_count_block<kCap>(topk_idx, num_tokens, num_topk, local_experts, words, threads, snapshot, block_counts,
-                             block_status, packed_rank, local_row, counted);
+    uint32_t received = 0, assigned = 0, before = 0, window_start = 0;
+    while (chunk < count_end) {
+#pragma unroll
+        for (int j = 0; j < kChunks; ++j) {
+            const uint32_t chunk_first = chunk + j * step;
+            if (chunk_first >= count_end)
+                break;  // (the same for the whole wavefront)
+            const bool valid = names_expert(batch[j], a);
+            const uint64_t valid_mask = __ballot(valid);
+            const uint32_t expert = static_cast<uint32_t>(batch[j]);
+            const uint32_t token = chunk_first + at.token;
+            const bool is_before = kSource != kDirect || token < block_first;
+            if (valid) {
+                if (kSource == kDirect)
+                    atomicAdd(&column_total[expert], is_before ? 0x10001u : 1u);
+                else
+                    atomicAdd(&base[expert], 1u);
+                if (kWindow && (kSource != kDirect || token - window_first < a.window_tokens))
+                    atomicAdd(&order_base[expert], kSource != kDirect ? 0x10000u : is_before ? 0x10001u : 1u);
+            }
+            received += count_opening(valid_mask, valid && is_before, at);
+            assigned += __popcll(valid_mask);
+            if (kSource == kDirect) {
+                before += __popcll(__ballot(valid && is_before));
+                if (kWindow)
+                    window_start += __popcll(__ballot(valid && token < window_first));
+            }
+        }
+        chunk += kChunks * step;
+        if (chunk < count_end) {
+#pragma unroll
+            for (int j = 0; j < kChunks; ++j)
+                batch[j] = fetch_id(a, at, chunk + j * step, count_end);
+        }
+    }
+    if (at.lane == 0) {
+        if (own_mask != 0)
+            atomicAdd(&sums.own, static_cast<uint32_t>(__popcll(own_mask)));
+        if (assigned != 0) {
+            atomicAdd(&sums.received_before, received);
+            atomicAdd(&sums.assigned_before, kSource == kDirect ? before : assigned);
+            if (kSource == kDirect) {
+                atomicAdd(&sums.assigned, assigned);
+                atomicAdd(&sums.window_start, kWindow ? window_start : before);
+            }
+        }
+    }
+    if (kSource == kSummed) {
+        const uint32_t window_row = kWindow ? fast_divide(window_first, a.row_magic, a.row_shift) : own_row;
+        const uint32_t window_rows = fast_divide(a.window_tokens, a.row_magic, a.row_shift);
+        for (uint32_t task = wave; task < tasks; task += a.waves) {
+            if (task != wave)
+                fetch_rows(a, at, task, rows);
+            uint32_t total = 0, earlier = 0, window = 0;
+#pragma unroll
+            for (int j = 0; j < kSumRows; ++j) {
+                const uint32_t row = rows.first_row + j;
+                total += rows.counts[j];
+                earlier += row < own_row ? rows.counts[j] : 0u;
+                if (kWindow)
+                    window += row - window_row >= window_rows ? 0u : row < own_row ? rows.counts[j] * 0x10001u : rows.counts[j];
+            }
+            if (rows.expert < a.experts) {
+                atomicAdd(&column_total[rows.expert], total);
+                atomicAdd(&base[rows.expert], earlier);
+                if (kWindow)
+                    atomicAdd(&order_base[rows.expert], window);
+            }
+        }
+        for (uint32_t row = tid; row - at.lane < a.row_count; row += a.waves * kWave) {
+            if (row != tid)
+                info = row < a.row_count ? a.rows[row] : RowInfo{0, 0, 0, 0};
+            const uint32_t all = wave_sum(info.assigned);
+            const uint32_t earlier = wave_sum(row < own_row ? info.assigned : 0u);
+            const uint32_t earlier_received = wave_sum(row < own_row ? info.received : 0u);
+            const uint32_t outside = wave_sum(row < window_row ? info.assigned : 0u);
+            if (at.lane == 0) {
+                atomicAdd(&sums.assigned, all);
+                atomicAdd(&sums.assigned_before, earlier);
+                atomicAdd(&sums.received_before, earlier_received);
+                atomicAdd(&sums.window_start, outside);
+            }
+        }
+    }
     __syncthreads();
-    layout_assign_block<kCap, true, true>(block_counts, block_status, 1, num_tokens, num_topk, local_experts, words * 32, 1, threads,
-                                          expand, alignment, packed_rank, local_row, expert_counts, expert_offsets, send_counts,
-                                          recv_rank_prefix, nullptr, host_counts, recv_metadata, dst_slots, token_slots, slot_order, 0,
-                                          &counted);
-}
+    // Experts: a thread takes a run of them (one each up to the workgroup's threads), the wavefronts
+    // without any go on to the last barrier.
+    const uint32_t first = tid * a.per_thread < a.experts ? tid * a.per_thread : a.experts;
+    const uint32_t last = first + a.per_thread < a.experts ? first + a.per_thread : a.experts;
+    // kScanned: exclusive prefixes of the block's row, of the window's first row and of the row behind the
+    // window (the totals when there is none)
+    const int32_t* prefix_row = a.histograms + static_cast<uint64_t>(own_row) * a.experts;
+    const auto padded_of = [&](uint32_t e) -> uint32_t {
+        const uint32_t total = kSource == kDirect ? column_total[e] & 0xffffu : column_total[e];
+        return kSource == kScanned ? 0u : static_cast<uint32_t>(round_up_to(total, a));
+    };
+    const auto before_of = [&](uint32_t e) -> uint32_t {
+        return kSource == kDirect ? column_total[e] >> 16 : kSource == kSummed ? base[e] : base[e] + static_cast<uint32_t>(prefix_row[e]);
+    };
+    // the window's assignments to the expert, and those of them in the blocks before this one << 16
+    const auto window_of = [&](uint32_t e) -> uint32_t {
+        if (!kWindow) {
+            uint32_t count = 0;
+            for (uint32_t w = 0; w < words; ++w)
+                count += __popc(bits[e * words + w]);
+            return count;
+        }
+        if (kSource != kScanned)
+            return order_base[e];
+        const uint32_t first_row = fast_divide(window_first, a.row_magic, a.row_shift);
+        const uint32_t end_row = first_row + fast_divide(a.window_tokens, a.row_magic, a.row_shift);
+        const uint32_t at_first = static_cast<uint32_t>(a.histograms[static_cast<uint64_t>(first_row) * a.experts + e]);
+        const uint32_t at_end = end_row < a.row_count ? static_cast<uint32_t>(a.histograms[static_cast<uint64_t>(end_row) * a.experts + e])
+                                                      : static_cast<uint32_t>(a.expert_counts[e]);
+        return order_base[e] + (at_end - at_first) + ((static_cast<uint32_t>(prefix_row[e]) - at_first) << 16);
+    };
+    uint32_t padded_sum = 0, padded_scan = 0, window_sum = 0, window_scan = 0;
+    if (wave < a.expert_waves) {
+        uint32_t before_sum = 0, window_before_sum = 0;
+        for (uint32_t e = first; e < last; ++e) {
+            const uint32_t window = window_of(e);
+            padded_sum += padded_of(e);
+            window_sum += window & 0xffffu;
+            if (kSource == kScanned) {
+                before_sum += before_of(e);
+                window_before_sum += window >> 16;
+            }
+        }
+        padded_scan = wave_inclusive_scan(padded_sum);
+        window_scan = wave_inclusive_scan(window_sum);
+        if (at.lane == kWave - 1) {
+            wave_padded[wave] = padded_scan;
+            wave_window[wave] = window_scan;
+        }
+        if (kSource == kScanned) {
+            // (the rows' sums: the partial row's are in already)
+            before_sum = wave_inclusive_scan(before_sum);
+            window_before_sum = wave_inclusive_scan(window_before_sum);
+            if (at.lane == kWave - 1) {
+                atomicAdd(&sums.assigned, before_sum);
+                atomicAdd(&sums.window_start, before_sum - window_before_sum);
+            }
+        }
+    }
+    if (a.expert_waves > 1)
+        __syncthreads();
+    else
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the sums stay within the one wavefront
+    if (wave < a.expert_waves) {
+        uint32_t running = padded_scan - padded_sum;
+        uint32_t running_window = window_scan - window_sum + sums.window_start;  // the list is dense
+        for (uint32_t w = 0; w < wave; ++w) {
+            running += wave_padded[w];
+            running_window += wave_window[w];
+        }
+        for (uint32_t e = first; e < last; ++e) {
+            const uint32_t window = window_of(e), padded = padded_of(e);
+            base[e] = (kSource == kScanned ? static_cast<uint32_t>(a.expert_offsets[e]) : running) + before_of(e);
+            order_base[e] = running_window + (window >> 16);  // behind the expert's entries of the window's earlier blocks
+            running += padded;
+            running_window += window & 0xffffu;
+        }
+    }
+    __syncthreads();
+    if (kSource == kScanned && tid == 0) {
+        sums.assigned_before = sums.assigned;
+        sums.assigned = static_cast<uint32_t>(a.totals[0]);
+        sums.received_before += a.rows[own_row].received;
+    }
+    if (kSource == kScanned)
+        __syncthreads();
 
+    if (live) {
+        const uint32_t token = own_first + at.token;
+        const uint32_t word = local / 32, below = (1u << (local % 32)) - 1u;
+        int32_t value = -1;
+        if (own_valid) {
+            const uint32_t expert = static_cast<uint32_t>(id);
+            uint32_t rank = 0;
+            for (uint32_t w = 0; w < words; ++w) {
+                const uint32_t row = bits[expert * words + w];
+                rank += __popc(w < word ? row : w == word ? row & below : 0u);
+            }
+            value = a.expand ? static_cast<int32_t>(base[expert] + rank) : static_cast<int32_t>(expert);
+            if (a.slot_order != nullptr)
+                a.slot_order[order_base[expert] + rank] =
+                    static_cast<int64_t>(static_cast<uint64_t>(static_cast<uint32_t>(value)) << 32 | (own_first * a.topk + at.lane));
+        }
+        if (a.token_slots != nullptr)
+            (a.token_slots + static_cast<uint64_t>(own_first) * a.topk)[at.lane] = value;
+        const bool is_received = (any_bits[word] >> (local % 32)) & 1u;
+        uint32_t row = sums.received_before;
+        for (uint32_t w = 0; w < words; ++w)
+            row += __popc(w < word ? any_bits[w] : w == word ? any_bits[w] & below : 0u);
+        if (at.k == 0)
+            a.dst_slots[token] = is_received ? static_cast<int64_t>(row) : -1;
+        if (is_received) {
+            // the receive row [0, token, K values]
+            int32_t* out = a.recv_metadata + static_cast<uint64_t>(row) * (a.topk + 2);
+            out[2 + at.k] = value;
+            if (at.k == 0) {
+                out[0] = 0;
+                out[1] = static_cast<int32_t>(token);
+            }
+        }
+    }
+    if (a.slot_order != nullptr) {
+        // every block clears as many entries of the list's unused tail as it has masked choices; the last one
+        // also what lies behind the batch's own entries, so that everything from entry A to the count word reads -1
+        const uint64_t entries_before = static_cast<uint64_t>(block_first) * a.topk;
+        int64_t* tail = a.slot_order + sums.assigned + (entries_before - sums.assigned_before);
+        const uint32_t holes = (block_end - block_first) * a.topk - sums.own;
+        for (uint32_t i = tid; i < holes; i += a.waves * kWave)
+            tail[i] = -1;
+        if (block == a.blocks - 1)
+            for (uint64_t i = static_cast<uint64_t>(a.tokens) * a.topk + tid; i < a.list_entries; i += a.waves * kWave)
+                a.slot_order[i] = -1;
+        if (kSource == kScanned && block == 0 && tid == 0)
+            a.slot_order[a.list_entries] = sums.assigned;
+    }
+}
 
 // Argument checks shared by the two layout entry points (everything but the workspace).
 int check_layout_arguments(const int64_t* topk_idx, int64_t num_tokens, int num_topk, int64_t num_local_experts, int64_t alignment,
                            int expand, int hidden, const int32_t* recv_metadata, const int64_t* expert_counts,
                            const int64_t* expert_offsets, const int64_t* dst_slots, const int64_t* send_counts,
                            const int64_t* topk_snapshot, const int64_t* recv_rank_prefix, const int64_t* slot_order,
-                           const int64_t* host_counts, const Knobs& knobs) {
+                           const int64_t* host_counts) {
     if (num_tokens < 0 || num_tokens > INT32_MAX || num_topk <= 0 || num_topk > kMaxTopk || num_local_experts <= 0 ||
-        num_local_experts >= (int64_t{1} << (31 - kRankBits)) || alignment <= 0 || alignment > (int64_t{1} << 31) || hidden < 0)
+        !layout_supports(num_local_experts) || alignment <= 0 || alignment > (int64_t{1} << 31) || hidden < 0)
         return NANOEP_ERR_INVALID_ARGUMENT;
     if (expert_counts == nullptr || expert_offsets == nullptr || send_counts == nullptr || recv_rank_prefix == nullptr ||
         host_counts == nullptr)
@@ -922,8 +948,6 @@ int check_layout_arguments(const int64_t* topk_idx, int64_t num_tokens, int num_
         return NANOEP_ERR_INVALID_ARGUMENT;
     // the slot-order list packs token * K + k into 32 bits and only exists for the expanded layout
     if (slot_order != nullptr && (!expand || num_tokens * num_topk >= (int64_t{1} << 31)))
-        return NANOEP_ERR_INVALID_ARGUMENT;
-    if (layout_tokens_per_block(num_tokens, num_local_experts, hidden, knobs) == 0)
         return NANOEP_ERR_INVALID_ARGUMENT;
     return NANOEP_OK;
 }
@@ -934,70 +958,125 @@ int enqueue_layout(const int64_t* topk_idx, int64_t num_tokens, int num_topk, in
                    int64_t* dst_slots, int64_t* send_counts, int64_t* topk_snapshot, int64_t* recv_rank_prefix,
                    int32_t* token_slots, int64_t* slot_order, const LayoutWorkspace& ws, int64_t* host_counts,
                    void* stream_handle, const Knobs& knobs) {
-    const int tokens_per_block = layout_tokens_per_block(num_tokens, num_local_experts, hidden, knobs);
-    const int64_t blocks64 = (num_tokens + tokens_per_block - 1) / tokens_per_block;
-    const int blocks = static_cast<int>(blocks64);
-    const int experts = static_cast<int>(num_local_experts);
-    const int words = tokens_per_block / 32;
+    const int window = layout_window_tokens(num_tokens, hidden, knobs);
+    const int block_tokens = layout_block_tokens_of(num_tokens, window, num_topk, num_local_experts);
+    const int64_t blocks = (num_tokens + block_tokens - 1) / block_tokens;
+    const int histogram_tokens = layout_histogram_tokens(num_tokens, window, block_tokens, num_topk, num_local_experts);
+    const int64_t histogram_rows = (num_tokens + histogram_tokens - 1) / histogram_tokens;
+    int check_tokens = histogram_tokens;
+    while (check_tokens > block_tokens && layout_lds(num_local_experts, check_tokens / 32) > kLayoutLdsBudget)
+        check_tokens = block_tokens;
     auto stream = static_cast<hipStream_t>(stream_handle);
 
+    const int64_t pairs = num_tokens * num_topk;
+    const int64_t batch_words = (num_tokens + 31) / 32;
+    const bool direct_fits = pairs < 65536 && layout_lds(num_local_experts, batch_words > block_tokens / 32 ? batch_words : block_tokens / 32) <= kLayoutLdsBudget;
+    int source = direct_fits && pairs <= kDirectPairs ? kDirect : histogram_rows <= kSummedHistograms ? kSummed : kScanned;
+    if (knobs.layout_launches == 1 && direct_fits)
+        source = kDirect;
+    else if (knobs.layout_launches == 2 && num_tokens > 0)
+        source = kSummed;
+    else if (knobs.layout_launches == 3)
+        source = kScanned;
+    // a chunk of the block a wavefront; in the direct plan enough wavefronts for the counting as well
+    const int chunk_tokens = kWave / num_topk;
+    int waves = (block_tokens + chunk_tokens - 1) / chunk_tokens;
+    if (source == kDirect) {
+        const int64_t counting = (pairs / kChunks + kWave - 1) / kWave;
+        if (num_tokens < block_tokens)
+            waves = static_cast<int>((num_tokens + chunk_tokens - 1) / chunk_tokens);
+        if (waves < counting)
+            waves = counting < kLayoutWaves ? static_cast<int>(counting) : kLayoutWaves;
+    }
+    if (source == kSummed) {
+        const int64_t tasks = (num_local_experts + kWave - 1) / kWave * (padded_rows(histogram_rows) / kSumRows);
+        if (waves < tasks)
+            waves = tasks < 8 ? static_cast<int>(tasks) : waves < 8 ? 8 : waves;
+    }
+    if (waves < 2)
+        waves = 2;
+    const int threads = waves * kWave;
+
+    const FastDivisor alignment_divisor = make_fast_divisor(static_cast<uint32_t>(alignment));
+    const FastDivisor row_divisor = make_fast_divisor(static_cast<uint32_t>(histogram_tokens));
+    const FastDivisor window_divisor = make_fast_divisor(static_cast<uint32_t>(window));
+    LayoutArgs a{};
+    a.topk_idx = topk_idx;
+    a.histograms = ws.histograms;
+    a.rows = ws.rows;
+    a.tokens = static_cast<uint32_t>(num_tokens);
+    a.topk = static_cast<uint32_t>(num_topk);
+    a.experts = static_cast<uint32_t>(num_local_experts);
+    a.chunk_tokens = static_cast<uint32_t>(chunk_tokens);
+    a.chunk_pairs = a.chunk_tokens * a.topk;
+    a.topk_magic = (65536u + a.topk - 1) / a.topk;
+    a.waves = static_cast<uint32_t>(waves);
+    a.block_tokens = static_cast<uint32_t>(block_tokens);
+    a.row_tokens = static_cast<uint32_t>(histogram_tokens);
+    a.row_magic = row_divisor.magic;
+    a.row_shift = row_divisor.shift;
+    a.window_tokens = static_cast<uint32_t>(window);
+    a.window_magic = window_divisor.magic;
+    a.window_shift = window_divisor.shift;
+    a.row_count = static_cast<uint32_t>(histogram_rows);
+    a.row_batches = static_cast<uint32_t>(padded_rows(histogram_rows) / kSumRows);
+    a.strips = (a.experts + kWave - 1) / kWave;
+    const FastDivisor strips_divisor = make_fast_divisor(a.strips);
+    a.strips_magic = strips_divisor.magic;
+    a.strips_shift = strips_divisor.shift;
+    a.per_thread = (a.experts + threads - 1) / threads;
+    a.expert_waves = ((a.experts + a.per_thread - 1) / a.per_thread + kWave - 1) / kWave;
+    a.check_tokens = static_cast<uint32_t>(check_tokens);
+    a.expand = expand ? 1u : 0u;
+    a.alignment = alignment;
+    a.alignment_magic = alignment_divisor.magic;
+    a.alignment_shift = alignment_divisor.shift;
+    a.totals = ws.totals;
+    a.expert_counts = expert_counts;
+    a.expert_offsets = expert_offsets;
+    a.send_counts = send_counts;
+    a.recv_rank_prefix = recv_rank_prefix;
+    a.host_counts = host_counts;
+    a.snapshot = topk_snapshot;
+    a.recv_metadata = recv_metadata;
+    a.dst_slots = dst_slots;
+    a.token_slots = token_slots;
+    a.slot_order = num_tokens > 0 ? slot_order : nullptr;
+    a.list_entries = static_cast<uint64_t>((num_tokens + kOrderTokens - 1) / kOrderTokens * kOrderTokens) * num_topk;
+    a.blocks = static_cast<uint32_t>(blocks);
+
     __atomic_store_n(&host_counts[0], int64_t{-1}, __ATOMIC_RELEASE);
-    // whole wavefronts: the kernels' scans take a wavefront's sums from its last lane (a forced window of
-    // 96, 160 or 224 tokens would otherwise leave the experts of a trailing half wavefront out)
-    const int count_threads = (tokens_per_block + kWave - 1) / kWave * kWave;
-    // Two launches while every block can afford to sum the block histograms itself (blocks x (L+1)
-    // loads from L2, spread over the workgroup): measured faster than the single-workgroup scan up to
-    // 1024 blocks whatever the expert count (8192 tokens, 256 experts: 21 against 27 us; 262144
-    // tokens: 159 against 198 us).  Beyond, the blocks^2 loads lose (2^20 tokens, 8 experts: 124
-    // against 67 us) and a third launch does the scan once.
-    const bool fused_scan = layout_uses_fused_scan(num_tokens, num_local_experts, hidden, knobs);
-    const int forced_launches = knobs.layout_launches;
-    const int window_blocks = layout_window_blocks(num_tokens, num_local_experts, hidden, fused_scan, knobs);
-    hipError_t launch_status = hipSuccess;
-    with_topk_cap(num_topk, [&](auto cap) {
-        constexpr int kCap = decltype(cap)::value;
-        if (blocks == 1 && forced_launches == 0) {
-            const size_t count_lds = static_cast<size_t>(experts + 1) * (words * 6 + 4);
-            const size_t assign_lds = static_cast<size_t>(experts + 1) * 16;
-            layout_single_block_kernel<kCap><<<1, count_threads, count_lds > assign_lds ? count_lds : assign_lds, stream>>>(
-                topk_idx, num_tokens, num_topk, experts, words, count_threads, expand, alignment, topk_snapshot,
-                ws.block_counts, ws.block_status, ws.packed_rank, ws.local_row, expert_counts, expert_offsets, send_counts,
-                recv_rank_prefix, host_counts, recv_metadata, dst_slots, token_slots, slot_order);
-            launch_status = hipGetLastError();
-            return;
-        }
-        if (blocks > 0) {
-            const size_t lds = static_cast<size_t>(experts + 1) * (words * 6 + 4);
-            layout_count_kernel<kCap><<<blocks, count_threads, lds, stream>>>(
-                topk_idx, num_tokens, num_topk, experts, words, count_threads, topk_snapshot, ws.block_counts,
-                ws.block_status, ws.packed_rank, ws.local_row);
-            if ((launch_status = hipGetLastError()) != hipSuccess)
-                return;
-        }
-        const size_t assign_lds = static_cast<size_t>(experts + 1) * 16;
-        if (fused_scan) {
-            // one workgroup more than there are blocks: the publisher
-            layout_assign_kernel<kCap, true><<<blocks + 1, count_threads, assign_lds, stream>>>(
-                ws.block_counts, ws.block_status, blocks, num_tokens, num_topk, experts, tokens_per_block, window_blocks,
-                count_threads, expand, alignment, ws.packed_rank, ws.local_row, expert_counts, expert_offsets, send_counts,
-                recv_rank_prefix, ws.totals, host_counts, recv_metadata, dst_slots, token_slots, slot_order, blocks);
-            launch_status = hipGetLastError();
-            return;
-        }
-        layout_scan_kernel<<<1, kScanThreads, static_cast<size_t>(experts + 1) * 4, stream>>>(
-            ws.block_counts, ws.block_status, blocks, experts, alignment, expert_counts, expert_offsets, send_counts,
-            recv_rank_prefix, ws.totals, host_counts);
-        if ((launch_status = hipGetLastError()) != hipSuccess)
-            return;
-        if (blocks > 0) {
-            layout_assign_kernel<kCap, false><<<blocks, count_threads, assign_lds, stream>>>(
-                ws.block_counts, ws.block_status, blocks, num_tokens, num_topk, experts, tokens_per_block, 1, count_threads,
-                expand, alignment, ws.packed_rank, ws.local_row, expert_counts, expert_offsets, send_counts,
-                recv_rank_prefix, ws.totals, host_counts, recv_metadata, dst_slots, token_slots, slot_order, 0);
-            launch_status = hipGetLastError();
-        }
-    });
-    NANOEP_HIP_TRY(launch_status);
+    if (source != kDirect && histogram_rows > 0) {
+        int64_t row_waves = (static_cast<int64_t>(histogram_tokens) + chunk_tokens - 1) / chunk_tokens;
+        row_waves = row_waves < 2 ? 2 : row_waves > kLayoutWaves ? kLayoutWaves : row_waves;
+        layout_histogram_kernel<<<a.row_batches * kSumRows, static_cast<unsigned>(row_waves * kWave),
+                                  layout_lds(num_local_experts, check_tokens / 32), stream>>>(a, static_cast<uint32_t>(row_waves));
+        NANOEP_HIP_TRY(hipGetLastError());
+    }
+    if (source == kScanned) {
+        layout_scan_kernel<<<1, kScanThreads, static_cast<size_t>(num_local_experts + 1) * 4, stream>>>(a);
+        NANOEP_HIP_TRY(hipGetLastError());
+        if (blocks == 0)
+            return NANOEP_OK;
+    }
+    const dim3 grid(static_cast<unsigned>(blocks + (source == kScanned ? 0 : 1)));
+    const size_t lds = layout_lds(num_local_experts, source == kDirect && batch_words > block_tokens / 32 ? batch_words : block_tokens / 32);
+    const bool several = window > block_tokens;
+#define NANOEP_LAUNCH_ASSIGN(SOURCE)                                                            \
+    do {                                                                                        \
+        if (several)                                                                            \
+            layout_assign_kernel<SOURCE, true><<<grid, threads, lds, stream>>>(a);       \
+        else                                                                                    \
+            layout_assign_kernel<SOURCE, false><<<grid, threads, lds, stream>>>(a);      \
+    } while (0)
+    if (source == kDirect)
+        NANOEP_LAUNCH_ASSIGN(kDirect);
+    else if (source == kSummed)
+        NANOEP_LAUNCH_ASSIGN(kSummed);
+    else
+        NANOEP_LAUNCH_ASSIGN(kScanned);
+#undef NANOEP_LAUNCH_ASSIGN
+    NANOEP_HIP_TRY(hipGetLastError());
     return NANOEP_OK;
 }
 
@@ -1201,20 +1280,15 @@ size_t nanoep_layout_workspace_bytes(int64_t num_tokens, int num_topk, int64_t n
 int nanoep_layout_block_tokens(int64_t num_tokens, int64_t num_local_experts, int hidden) {
     if (num_local_experts <= 0 || num_tokens < 0 || hidden < 0)
         return 0;
-    const Knobs knobs = current_knobs();
-    // tokens the slot-order list is ordered by: the layout workgroup's tokens times the blocks of a window
-    const int per_block = layout_tokens_per_block(num_tokens, num_local_experts, hidden, knobs);
-    const bool fused = layout_uses_fused_scan(num_tokens, num_local_experts, hidden, knobs);
-    return per_block * layout_window_blocks(num_tokens, num_local_experts, hidden, fused, knobs);
+    return layout_supports(num_local_experts) ? layout_window_tokens(num_tokens, hidden, current_knobs()) : 0;
 }
 
 int64_t nanoep_slot_order_entries(int64_t num_tokens, int num_topk, int64_t num_local_experts) {
     if (num_tokens < 0 || num_topk <= 0 || num_local_experts <= 0)
         return 0;
-    if (layout_smallest_block(num_tokens, num_local_experts, current_knobs()) == 0 || num_tokens == 0)
+    if (!layout_supports(num_local_experts) || num_tokens == 0)
         return 0;
-    // whole blocks of any size the layout may take, then the count word
-    return (num_tokens + kMaxBlockTokens - 1) / kMaxBlockTokens * kMaxBlockTokens * num_topk + 1;
+    return (num_tokens + kOrderTokens - 1) / kOrderTokens * kOrderTokens * num_topk + 1;  // the count word last
 }
 
 int nanoep_layout(const int64_t* topk_idx, int64_t num_tokens, int num_topk, int64_t num_local_experts,
@@ -1225,7 +1299,7 @@ int nanoep_layout(const int64_t* topk_idx, int64_t num_tokens, int num_topk, int
     const Knobs knobs = current_knobs();
     const int status = check_layout_arguments(topk_idx, num_tokens, num_topk, num_local_experts, alignment, expand, hidden,
                                               recv_metadata, expert_counts, expert_offsets, dst_slots, send_counts, topk_snapshot,
-                                              recv_rank_prefix, slot_order, host_counts, knobs);
+                                              recv_rank_prefix, slot_order, host_counts);
     if (status != NANOEP_OK)
         return status;
     if (workspace == nullptr)
@@ -1246,7 +1320,7 @@ int nanoep_layout_static(const int64_t* topk_idx, int64_t num_tokens, int num_to
     const Knobs knobs = current_knobs();
     const int status = check_layout_arguments(topk_idx, num_tokens, num_topk, num_local_experts, alignment, expand, hidden,
                                               recv_metadata, expert_counts, expert_offsets, dst_slots, send_counts, topk_snapshot,
-                                              recv_rank_prefix, slot_order, host_counts, knobs);
+                                              recv_rank_prefix, slot_order, host_counts);
     if (status != NANOEP_OK)
         return status;
     // the size is checked before any device is touched
@@ -1289,7 +1363,7 @@ int nanoep_rebuild_order(const int32_t* recv_metadata, const int64_t* dst_slots,
         (recv_count > 0 && recv_metadata == nullptr) || host_tag < 0 || (host_tag & 0xffffffffll) != 0)
         return NANOEP_ERR_INVALID_ARGUMENT;
     const Knobs knobs = current_knobs();
-    if (layout_smallest_block(num_tokens, num_local_experts, knobs) == 0)
+    if (!layout_supports(num_local_experts))
         return NANOEP_ERR_INVALID_ARGUMENT;  // no slot-order buffer exists for this geometry
     if (nanoep_rebuild_workspace_bytes(num_tokens, num_topk) > workspace_bytes)
         return NANOEP_ERR_WORKSPACE;
@@ -1298,7 +1372,7 @@ int nanoep_rebuild_order(const int32_t* recv_metadata, const int64_t* dst_slots,
     int sort_size = 2;
     while (sort_size < window * num_topk)
         sort_size *= 2;
-    const int64_t capacity_entries = (num_tokens + kMaxBlockTokens - 1) / kMaxBlockTokens * kMaxBlockTokens * num_topk;
+    const int64_t capacity_entries = (num_tokens + kOrderTokens - 1) / kOrderTokens * kOrderTokens * num_topk;
     auto* window_counts = static_cast<int32_t*>(workspace);
     auto stream = static_cast<hipStream_t>(stream_handle);
     if (host_count != nullptr)
