@@ -8,6 +8,7 @@
 // (csrc/bindings.cpp:11-86) with the same positional order, so a caller written against the
 // reference's backend module binds to this one unchanged.
 
+#include <ATen/hip/EmptyTensor.h>
 #include <ATen/hip/HIPContext.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
@@ -19,6 +20,7 @@
 #include <atomic>
 #include <cstdlib>
 #include <deque>
+#include <initializer_list>
 #include <limits>
 #include <memory>
 #include <mutex>
@@ -72,10 +74,128 @@ Stream external_stream(int64_t handle, c10::DeviceIndex device) {
     return c10::hip::getStreamFromExternalMasqueradingAsCUDA(reinterpret_cast<hipStream_t>(handle), device);
 }
 
+bool capturing(const Stream& stream) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    check_hip(hipStreamIsCapturing(stream.stream(), &status), "hipStreamIsCapturing");
+    return status != hipStreamCaptureStatusNone;
+}
+
+// Whether everything enqueued on the stream so far has run (never asked of a stream under capture).
+bool idle(const Stream& stream) {
+    const hipError_t state = hipStreamQuery(stream.stream());
+    if (state == hipErrorNotReady)
+        (void)hipGetLastError();  // an answer, not an error of the next call that looks for one
+    return state == hipSuccess;
+}
+
+// A point in a stream's work: a value the stream stores into a word of signal memory when it gets there.
+// Other streams wait for the word to hold at least that value, and the host can look.  Against an event
+// this is what a dependency between two streams costs here: store and wait 6 us of host time against 9 to 16
+// for hipEventRecord and hipStreamWaitEvent, and 5 us between the two streams' kernels against 11 to 13.
+struct StreamPoint {
+    uint64_t* word = nullptr;
+    uint64_t value = 0;
+
+    bool reached() const { return __atomic_load_n(word, __ATOMIC_ACQUIRE) >= value; }
+};
+
+// The words behind StreamPoints.  A word serves one store at a time and its values only grow: it is handed
+// out again when the host sees its last value there, and whoever still waits for an older one finds it
+// passed.  So nothing depends on which stream used a word before, and a word needs no owner.  There are as
+// many as stores were ever on their way at once, at most kMostWords a device; they stay for the process.
+class StreamPoints {
+   public:
+    static StreamPoints& of(c10::DeviceIndex device) {
+        static std::array<StreamPoints, kDevices> pools;
+        return pools[static_cast<size_t>(device) % kDevices];
+    }
+
+    // A point behind everything enqueued on `stream`; none when no word is free or the device has no such
+    // operations (an event serves then).
+    std::optional<StreamPoint> record(const Stream& stream) {
+        std::optional<StreamPoint> point = next_point(stream.device_index());
+        if (!point.has_value())
+            return point;
+        const hipError_t status = hipStreamWriteValue64(stream.stream(), point->word, point->value, 0);
+        if (status != hipSuccess) {
+            (void)hipGetLastError();
+            __atomic_store_n(point->word, point->value, __ATOMIC_RELEASE);  // nothing will: the word is free again
+            point.reset();
+        }
+        return point;
+    }
+
+    static void wait(const Stream& stream, const StreamPoint& point) {
+        check_hip(hipStreamWaitValue64(stream.stream(), point.word, point.value, hipStreamWaitValueGte, ~uint64_t{0}), "hipStreamWaitValue64");
+    }
+
+   private:
+    static constexpr size_t kDevices = 64;
+    static constexpr size_t kMostWords = 64;
+
+    std::optional<StreamPoint> next_point(c10::DeviceIndex device) {
+        std::lock_guard<std::mutex> lock(mutex_);
+        for (size_t tries = 0; tries < words_.size(); ++tries) {
+            StreamPoint& last = words_[next_];
+            next_ = (next_ + 1) % words_.size();
+            if (last.reached()) {
+                ++last.value;
+                return last;
+            }
+        }
+        if (supported_ < 0) {
+            int answer = 0;
+            supported_ = hipDeviceGetAttribute(&answer, hipDeviceAttributeCanUseStreamWaitValue, device) == hipSuccess && answer != 0;
+        }
+        void* memory = nullptr;
+        if (supported_ == 0 || words_.size() >= kMostWords)
+            return std::nullopt;
+        DeviceGuard guard(device);
+        if (hipExtMallocWithFlags(&memory, sizeof(uint64_t), hipMallocSignalMemory) != hipSuccess) {
+            (void)hipGetLastError();
+            return std::nullopt;
+        }
+        __atomic_store_n(static_cast<uint64_t*>(memory), uint64_t{0}, __ATOMIC_RELEASE);
+        words_.push_back(StreamPoint{static_cast<uint64_t*>(memory), 1});
+        return words_.back();
+    }
+
+    std::mutex mutex_;
+    std::vector<StreamPoint> words_;
+    size_t next_ = 0;
+    int supported_ = -1;
+};
+
+// `waiter` goes on behind what `producer` holds now.
 void wait_on(const Stream& waiter, const Stream& producer) {
+    if (!capturing(producer) && !capturing(waiter)) {
+        if (const auto point = StreamPoints::of(producer.device_index()).record(producer)) {
+            StreamPoints::wait(waiter, *point);
+            return;
+        }
+    }
     c10::Event ready(c10::DeviceType::CUDA);
     ready.record(producer.unwrap());
     waiter.unwrap().wait(ready);
+}
+
+// Tensors are made without the dispatcher (a third of its time: an allocation of torch::empty is 1.5 us of
+// a call that takes six).
+torch::Tensor new_tensor(at::IntArrayRef sizes, at::ScalarType dtype, const c10::Device& device) {
+    return torch::Tensor(at::detail::empty_cuda(sizes, dtype, device, std::nullopt));
+}
+
+// A contiguous tensor over part of another one's storage, `offset` elements of its own type from the
+// storage's start.  It shares the version counter, like a view: an edit of any part through torch shows in all.
+torch::Tensor part_of(const torch::Tensor& base, int64_t offset, at::IntArrayRef sizes, at::ScalarType dtype) {
+    auto part = at::detail::make_tensor<c10::TensorImpl>(c10::TensorImpl::VIEW, c10::Storage(base.storage()), base.key_set(),
+                                                         c10::scalarTypeToTypeMeta(dtype));
+    auto* impl = part.unsafeGetTensorImpl();
+    impl->set_storage_offset(offset);
+    impl->set_sizes_contiguous(sizes);
+    if (!base.is_inference())
+        impl->set_version_counter(base.unsafeGetTensorImpl()->version_counter());
+    return part;
 }
 
 // Compute-unit budget: 0 or the device size mean the whole device (the reference's
@@ -394,9 +514,9 @@ class PeerRuntime {
     // the scratch: the buffer is only handed out again to a call on the stream it was last used on,
     // where the launches are ordered; a call on another stream gets a buffer of its own, which is then
     // the one that is kept).  Called with the mailbox held.
-    torch::Tensor layout_workspace(size_t bytes, hipStream_t stream, const torch::TensorOptions& options) {
+    torch::Tensor layout_workspace(size_t bytes, hipStream_t stream, const c10::Device& device) {
         if (!workspace_.defined() || static_cast<size_t>(workspace_.numel()) < bytes || workspace_stream_ != stream) {
-            workspace_ = torch::empty({static_cast<int64_t>(bytes)}, options);
+            workspace_ = new_tensor({static_cast<int64_t>(bytes)}, torch::kUInt8, device);
             workspace_stream_ = stream;
         }
         return workspace_;
@@ -563,59 +683,97 @@ class PeerRuntime {
 };
 
 // What a caller gets back from an asynchronous call: a marker on the communication stream behind
-// the call's kernels, and the tensors those kernels write.  Waiting puts the consumer's stream
-// behind the marker and tells the caching allocator that the tensors are in use there, so that
-// freeing them on the consumer's side cannot hand their memory out while that stream still reads
-// it (the role of csrc/include/nano_ep/event.hpp:12-28 in the reference).
+// the call's kernels, and the tensors those kernels read and write (the role of
+// csrc/include/nano_ep/event.hpp:12-28 in the reference).  Waiting puts the consumer's stream behind the
+// marker.
+//
+// The marker holds the tensors until somebody has waited, so that none of them is freed while the
+// kernels use it on a stream its allocator does not know of; waiting tells the allocator of the
+// consumer's stream instead, which costs nothing for tensors that were allocated there (telling it of the
+// communication stream makes it record an event for every block when it is freed).  A marker that goes
+// away with nobody having waited tells it of the communication stream after all.
 class CompletionEvent {
    public:
-    static std::shared_ptr<CompletionEvent> record_behind(const Stream& producer, std::vector<torch::Tensor> written) {
+    static std::shared_ptr<CompletionEvent> record_behind(const Stream& producer, std::vector<torch::Tensor> written,
+                                                          std::vector<torch::Tensor> read) {
         auto marker = std::make_shared<CompletionEvent>();
         marker->written_ = std::move(written);
-        marker->done_.record(producer.unwrap());
+        marker->read_ = std::move(read);
+        marker->producer_ = producer;
+        if (!capturing(producer))
+            marker->point_ = StreamPoints::of(producer.device_index()).record(producer);
+        if (!marker->point_.has_value())
+            marker->done_.record(producer.unwrap());
         return marker;
     }
 
-    void order_after(const Stream& consumer) const {
-        consumer.unwrap().wait(done_);
-        for (const auto& tensor : written_)
-            if (tensor.defined() && tensor.numel() > 0)
-                tensor.record_stream(consumer.unwrap());
+    void order_after(const Stream& consumer) {
+        if (!point_.has_value()) {
+            consumer.unwrap().wait(done_);
+        } else if (!point_->reached()) {
+            TORCH_CHECK(!capturing(consumer), "a completion event of work outside a HIP graph cannot be waited on inside its capture");
+            StreamPoints::wait(consumer, *point_);
+        }
+        std::lock_guard<std::mutex> lock(mutex_);
+        note_use(written_, consumer);
+        note_use(read_, consumer);
+        read_.clear();
+        waited_ = true;
     }
 
-    void current_stream_wait() const { order_after(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA()); }
+    void current_stream_wait() { order_after(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA()); }
 
     CompletionEvent() : done_(c10::DeviceType::CUDA) {}
+    CompletionEvent(const CompletionEvent&) = delete;
+    CompletionEvent& operator=(const CompletionEvent&) = delete;
+    ~CompletionEvent() {
+        if (waited_ || !producer_.has_value())
+            return;
+        try {
+            note_use(written_, *producer_);
+            note_use(read_, *producer_);
+        } catch (...) {
+        }
+    }
 
    private:
-    c10::Event done_;
-    std::vector<torch::Tensor> written_;
+    static void note_use(const std::vector<torch::Tensor>& tensors, const Stream& stream) {
+        for (const auto& tensor : tensors)
+            if (tensor.defined() && tensor.numel() > 0)
+                tensor.record_stream(stream.unwrap());
+    }
+
+    std::mutex mutex_;
+    std::optional<StreamPoint> point_;
+    c10::Event done_;  // where there is no point
+    std::optional<Stream> producer_;
+    bool waited_ = false;
+    std::vector<torch::Tensor> written_, read_;
 };
 
 namespace {
 
 // What a tensor argument has to look like: where it lives, its element type and its extents
 // (-1 leaves an extent open).  Every tensor check of dispatch, combine and the cached handle is one
-// `require` against such a description; the message is the caller-visible part.
-struct TensorSpec {
-    c10::Device device;
-    at::ScalarType dtype;
-    std::vector<int64_t> extents;
-
-    bool describes(const torch::Tensor& tensor) const {
-        if (!tensor.defined() || tensor.device() != device || tensor.scalar_type() != dtype || !tensor.is_contiguous() ||
-            tensor.dim() != static_cast<int64_t>(extents.size()))
+// `require`; the message is the caller-visible part.
+bool describes(const torch::Tensor& tensor, const c10::Device& device, at::ScalarType dtype, std::initializer_list<int64_t> extents) {
+    if (!tensor.defined() || tensor.device() != device || tensor.scalar_type() != dtype || !tensor.is_contiguous() ||
+        tensor.dim() != static_cast<int64_t>(extents.size()))
+        return false;
+    const auto sizes = tensor.sizes();
+    size_t axis = 0;
+    for (const int64_t extent : extents) {
+        if (extent >= 0 && sizes[axis] != extent)
             return false;
-        for (size_t axis = 0; axis < extents.size(); ++axis)
-            if (extents[axis] >= 0 && tensor.size(static_cast<int64_t>(axis)) != extents[axis])
-                return false;
-        return true;
+        ++axis;
     }
-};
+    return true;
+}
 
 template <class... Message>
-void require(const torch::Tensor& tensor, const TensorSpec& spec, const Message&... message) {
-    TORCH_CHECK(spec.describes(tensor), message...);
+void require(const torch::Tensor& tensor, const c10::Device& device, at::ScalarType dtype, std::initializer_list<int64_t> extents,
+             const Message&... message) {
+    TORCH_CHECK(describes(tensor, device, dtype, extents), message...);
 }
 
 bool vector_aligned(const torch::Tensor& tensor) {
@@ -629,39 +787,33 @@ void require_dispatch_inputs(const torch::Tensor& x, const torch::Tensor& routin
     const c10::Device here(c10::DeviceType::CUDA, static_cast<c10::DeviceIndex>(device));
     TORCH_CHECK(x.defined() && x.is_cuda() && x.device() == here && x.dim() == 2 && x.is_contiguous(),
                 "x must be contiguous CUDA [T,H] on the runtime device");
-    require(x, {here, torch::kBFloat16, {-1, -1}}, "dispatch x must be bfloat16");
+    require(x, here, torch::kBFloat16, {-1, -1}, "dispatch x must be bfloat16");
     const int64_t tokens = x.size(0), hidden = x.size(1);
     TORCH_CHECK(hidden > 0 && hidden % kHiddenAlignment == 0, "dispatch hidden must be a positive multiple of 256");
     TORCH_CHECK(vector_aligned(x), "dispatch x data pointer must be 16-byte aligned");
-    require(routing, {here, torch::kInt64, {tokens, -1}}, "indices must be contiguous CUDA int64 [T,K] on the x device");
+    require(routing, here, torch::kInt64, {tokens, -1}, "indices must be contiguous CUDA int64 [T,K] on the x device");
     const int64_t topk = routing.size(1);
     TORCH_CHECK(topk >= 1 && topk <= 32, "num_topk must be in [1, 32]");
     TORCH_CHECK(num_experts > 0, "num_experts must be positive and divisible by world_size");
     TORCH_CHECK(max_tokens <= std::numeric_limits<int32_t>::max(), "max_tokens exceeds int32 metadata range");
     TORCH_CHECK(max_tokens > 0 && tokens <= max_tokens, "source token count exceeds max_tokens");
     if (weights.has_value())
-        require(*weights, {here, torch::kFloat32, {tokens, topk}}, "weights must be contiguous CUDA float32 [T,K] on the x device");
+        require(*weights, here, torch::kFloat32, {tokens, topk}, "weights must be contiguous CUDA float32 [T,K] on the x device");
 }
 
 // The seven handle tensors of a cached call against the geometry they must describe.
 void require_handle_tensors(const std::vector<torch::Tensor>& metadata, const c10::Device& here, int64_t source_tokens, int64_t topk,
                             int64_t local_experts) {
-    struct Field {
-        const char* name;
-        at::ScalarType dtype;
-        std::vector<int64_t> extents;
+    const auto field = [&](int index, const char* name, at::ScalarType dtype, std::initializer_list<int64_t> extents) {
+        require(metadata[index], here, dtype, extents, "cached ", name, " has invalid CUDA storage or shape");
     };
-    const Field fields[7] = {
-        {"recv_metadata", torch::kInt32, {-1, topk + 2}},
-        {"expert_counts", torch::kInt64, {local_experts}},
-        {"expert_offsets", torch::kInt64, {local_experts + 1}},
-        {"dst_slots", torch::kInt64, {source_tokens, 1}},
-        {"send_counts", torch::kInt64, {1}},
-        {"source_topk_snapshot", torch::kInt64, {source_tokens, topk}},
-        {"recv_rank_prefix", torch::kInt64, {1}},
-    };
-    for (int i = 0; i < 7; ++i)
-        require(metadata[i], {here, fields[i].dtype, fields[i].extents}, "cached ", fields[i].name, " has invalid CUDA storage or shape");
+    field(0, "recv_metadata", torch::kInt32, {-1, topk + 2});
+    field(1, "expert_counts", torch::kInt64, {local_experts});
+    field(2, "expert_offsets", torch::kInt64, {local_experts + 1});
+    field(3, "dst_slots", torch::kInt64, {source_tokens, 1});
+    field(4, "send_counts", torch::kInt64, {1});
+    field(5, "source_topk_snapshot", torch::kInt64, {source_tokens, topk});
+    field(6, "recv_rank_prefix", torch::kInt64, {1});
 }
 
 // The optional eighth handle tensor: int32 [T,K] slot table written by the layout kernels.
@@ -708,12 +860,22 @@ Stream work_stream(int64_t comm_handle, const Stream& compute, c10::DeviceIndex 
         return comm;
     // While the caller's stream is being captured into a graph no other stream may be queried;
     // a captured call is ordered by the graph alone.
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    check_hip(hipStreamIsCapturing(compute.stream(), &capture), "hipStreamIsCapturing");
-    if (capture == hipStreamCaptureStatusNone && hipStreamQuery(comm.stream()) == hipErrorNotReady)
+    if (!capturing(compute) && !idle(comm))
         wait_on(compute, comm);
     return compute;
 }
+
+// Makes `stream` the current one of its device while it lives, if it is another one than `current`.
+class StreamSwitch {
+   public:
+    StreamSwitch(const Stream& stream, const Stream& current) {
+        if (!same_queue(stream, current))
+            guard_.reset_stream(stream.unwrap());
+    }
+
+   private:
+    OptionalStreamGuard guard_;
+};
 
 void order_comm_after_inputs(const Stream& comm, const Stream& compute, int64_t previous_event, bool async_op) {
     if (previous_event != -1) {
@@ -801,29 +963,23 @@ DispatchResult dispatch(PeerRuntime& runtime,
     const auto comm = work_stream(comm_stream, compute, device, async_op, cu_budget != 0);
     order_comm_after_inputs(comm, compute, previous_event, async_op);
 
-    StreamGuard comm_guard(comm.unwrap());
-    // Sync results belong to the caller's stream, async results to the communication stream
-    // (protected by record_stream when the consumer waits on the completion event).
-    const auto allocate_for_consumer = [&](auto&& make) {
-        OptionalStreamGuard allocation_guard;
-        if (!async_op)
-            allocation_guard.reset_stream(compute.unwrap());
-        return make();
-    };
-
-    const auto float_options = x.options().dtype(torch::kFloat32);
+    const StreamSwitch on_comm(comm, compute);
+    // Results are allocated on the caller's stream: the work is ordered behind what that stream held
+    // when the call was made, and what it does with the results comes behind the call (a synchronous one) or
+    // behind the completion event, which holds them until somebody has waited.  An asynchronous call with
+    // an event of its own is ordered behind that event only: its results come from the communication
+    // stream's pool.
+    const bool callers_pool = !async_op || previous_event == -1;
+    const c10::Device here = x.device();
     torch::Tensor out_x, out_indices, out_weights;
     // x_rows rows of payload (and expanded weights), n_rows rows of compact indices / weights
     const auto allocate_outputs = [&](int64_t x_rows, int64_t n_rows) {
-        allocate_for_consumer([&] {
-            out_x = torch::empty({x_rows, hidden}, x.options());
-            if (!expand)
-                out_indices = torch::empty({n_rows, topk}, routing.options());
-            out_weights = !weights.has_value() ? torch::empty({0}, float_options)
-                          : expand            ? torch::empty({x_rows}, float_options)
-                                              : torch::empty({n_rows, topk}, float_options);
-            return 0;
-        });
+        const StreamSwitch pool(callers_pool ? compute : comm, comm);
+        out_x = new_tensor({x_rows, hidden}, torch::kBFloat16, here);
+        if (!expand)
+            out_indices = new_tensor({n_rows, topk}, torch::kInt64, here);
+        if (weights.has_value())
+            out_weights = expand ? new_tensor({x_rows}, torch::kFloat32, here) : new_tensor({n_rows, topk}, torch::kFloat32, here);
     };
     // What the permute reads of a handle, as plain pointers.  order_entries: A, or -1 for "the whole
     // slot-order buffer is there and the kernel finds A in its last word".
@@ -892,14 +1048,12 @@ DispatchResult dispatch(PeerRuntime& runtime,
             // replays, where the payload is large enough for the slot-order walk to pay for that
             // (the REBUILD_ORDER switch: 0 never, 1 always).  Not under stream capture: a captured
             // replay must not depend on when the rebuilt tensors are dropped.
-            const int rebuild_switch = tuning_switch("REBUILD_ORDER");
+            const int rebuild_switch = expand && !has_private ? tuning_switch("REBUILD_ORDER") : 0;
             const bool worth_it = rebuild_switch >= 0 ? rebuild_switch != 0 : expanded_capacity * hidden * 2 >= kRebuildPayloadBytes;
             std::shared_ptr<PeerRuntime::RebuiltHandle> rebuilt;
             if (expand && !has_private && worth_it && tokens * topk < (int64_t{1} << 31) &&
                 nanoep_slot_order_entries(tokens, static_cast<int>(topk), local_experts) > 0) {
-                hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-                check_hip(hipStreamIsCapturing(comm.stream(), &capture), "hipStreamIsCapturing");
-                if (capture == hipStreamCaptureStatusNone)
+                if (!capturing(comm))
                     rebuilt = private_tensors_of(runtime, metadata, expanded_capacity, tokens, topk, local_experts, hidden, comm);
             }
             if (rebuilt) {
@@ -911,12 +1065,8 @@ DispatchResult dispatch(PeerRuntime& runtime,
             launch_permute(view, recv_count, expanded_capacity, /*count_on_device=*/rebuilt && view.order_entries < 0);
         }
     } else {
-        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-        check_hip(hipStreamIsCapturing(comm.stream(), &capture), "hipStreamIsCapturing");
-        TORCH_CHECK(capture == hipStreamCaptureStatusNone, "Fresh dispatch with host count polling cannot be captured in a HIP graph");
+        TORCH_CHECK(!capturing(comm), "Fresh dispatch with host count polling cannot be captured in a HIP graph");
 
-        const auto int64_options = routing.options();
-        torch::Tensor recv_metadata, expert_counts, expert_offsets, dst_slots, send_counts, snapshot, prefix, token_slots, slot_order;
         // the slot-order list packs token * K + k into 32 bits
         const bool ordered = expand && tokens * topk < (int64_t{1} << 31);
         // The handle tensors of one call are views of one allocation (the int64 ones, then the int32 ones), and the
@@ -937,20 +1087,20 @@ DispatchResult dispatch(PeerRuntime& runtime,
         TORCH_CHECK(nanoep_layout_block_tokens(tokens, local_experts, static_cast<int>(hidden)) > 0,
                     "the layout kernels take at most 3839 local experts, got ", local_experts);
         // one allocation: the int64 tensors first, the int32 ones behind them as a view of the same storage
-        torch::Tensor arena64, arena32;
-        allocate_for_consumer([&] {
-            arena64 = torch::empty({count64 + (count32 + 1) / 2}, int64_options);
-            return 0;
-        });
-        // arena64: expert_counts [L] | expert_offsets [L+1] | send_counts [1] | recv_rank_prefix [1] |
-        //          dst_slots [T] | topk snapshot [T*K] | slot_order;   arena32: recv_metadata [T*(K+2)] | token_slots [T*K]
-        int64_t* base64 = arena64.data_ptr<int64_t>();
+        torch::Tensor arena;
+        {
+            const StreamSwitch pool(callers_pool ? compute : comm, comm);
+            arena = new_tensor({count64 + (count32 + 1) / 2}, torch::kInt64, here);
+        }
+        // int64: expert_counts [L] | expert_offsets [L+1] | send_counts [1] | recv_rank_prefix [1] |
+        //        dst_slots [T] | topk snapshot [T*K] | slot_order;   int32: recv_metadata [T*(K+2)] | token_slots [T*K]
+        int64_t* base64 = arena.data_ptr<int64_t>();
         int32_t* base32 = reinterpret_cast<int32_t*>(base64 + count64);
 
         // From here until the counts have been read this call owns the runtime's mailbox; a fresh
         // dispatch of another thread on the same runtime waits here for its turn.
         PeerRuntime::CountsTurn turn(runtime);
-        const auto workspace = runtime.layout_workspace(workspace_bytes, comm.stream(), int64_options.dtype(torch::kUInt8));
+        const auto workspace = runtime.layout_workspace(workspace_bytes, comm.stream(), here);
         const int layout_status =
             nanoep_layout(routing.data_ptr<int64_t>(), tokens, static_cast<int>(topk), local_experts, alignment, expand ? 1 : 0,
                           static_cast<int>(hidden), base32, base64, base64 + at_offsets, base64 + at_dst, base64 + at_send, base64 + at_snapshot,
@@ -1014,23 +1164,16 @@ DispatchResult dispatch(PeerRuntime& runtime,
             }
         }
 
-        arena32 = arena64.narrow(0, count64, (count32 + 1) / 2).view(torch::kInt32);
-        expert_counts = arena64.narrow(0, 0, local_experts);
-        expert_offsets = arena64.narrow(0, at_offsets, local_experts + 1);
-        send_counts = arena64.narrow(0, at_send, 1);
-        prefix = arena64.narrow(0, at_prefix, 1);
-        dst_slots = arena64.narrow(0, at_dst, tokens).view({tokens, 1});
-        snapshot = arena64.narrow(0, at_snapshot, tokens * topk).view({tokens, topk});
-        recv_metadata = arena32.narrow(0, 0, tokens * (topk + 2)).view({tokens, topk + 2});
-        metadata = {recv_metadata, expert_counts, expert_offsets, dst_slots, send_counts, snapshot, prefix};
-        if (expand) {
-            token_slots = arena32.narrow(0, at_table, tokens * topk).view({tokens, topk});
-            metadata.push_back(token_slots);  // private eighth entry: slot[t,k] in one lookup
-        }
-        if (ordered) {
-            slot_order = arena64.narrow(0, at_order, order_entries);
-            metadata.push_back(slot_order);  // private ninth entry: assignments in block-wise slot order
-        }
+        metadata.reserve(9);
+        metadata.resize(7);
+        metadata[1] = part_of(arena, 0, {local_experts}, torch::kInt64);
+        metadata[2] = part_of(arena, at_offsets, {local_experts + 1}, torch::kInt64);
+        metadata[3] = part_of(arena, at_dst, {tokens, 1}, torch::kInt64);
+        metadata[4] = part_of(arena, at_send, {1}, torch::kInt64);
+        metadata[5] = part_of(arena, at_snapshot, {tokens, topk}, torch::kInt64);
+        metadata[6] = part_of(arena, at_prefix, {1}, torch::kInt64);
+        if (expand)  // private eighth entry: slot[t,k] in one lookup
+            metadata.push_back(part_of(arena, 2 * count64 + at_table, {tokens, topk}, torch::kInt32));
 
         int64_t counts[NANOEP_HOST_COUNT_WORDS] = {0, 0, 0, 0};
         const int status = turn.wait(comm.stream(), kCountTimeoutSeconds, counts);
@@ -1044,10 +1187,11 @@ DispatchResult dispatch(PeerRuntime& runtime,
         TORCH_CHECK(recv_count >= 0 && recv_count <= tokens, "dispatch receive count exceeds the source token count");
         TORCH_CHECK(!expand || expanded_capacity <= std::numeric_limits<int32_t>::max(),
                     "expanded capacity exceeds int32 metadata range");
-        metadata[0] = recv_metadata.narrow(0, 0, recv_count);
+        metadata[0] = part_of(arena, 2 * count64, {recv_count, topk + 2}, torch::kInt32);
         if (ordered) {
-            TORCH_CHECK(counts[2] >= 0 && counts[2] <= slot_order.size(0), "assignment count exceeds the slot-order list");
-            metadata[8] = slot_order.narrow(0, 0, counts[2]);  // replays walk the A assignments only
+            // private ninth entry: assignments in window-wise slot order (replays walk the A assignments only)
+            TORCH_CHECK(counts[2] >= 0 && counts[2] <= order_entries, "assignment count exceeds the slot-order list");
+            metadata.push_back(part_of(arena, at_order, {counts[2]}, torch::kInt64));
             runtime.note_valid_share(counts[2], tokens * topk);
         }
         const int64_t used_rows = expand ? expanded_capacity : recv_count;
@@ -1057,11 +1201,11 @@ DispatchResult dispatch(PeerRuntime& runtime,
         const bool early_outputs_fit = speculative && used_rows <= early_rows && used_rows * 5 >= early_rows * 4;
         runtime.note_used_rows(geometry, used_rows);
         if (early_outputs_fit) {
-            out_x = out_x.narrow(0, 0, used_rows);
+            out_x = part_of(out_x, 0, {used_rows, hidden}, torch::kBFloat16);
             if (!expand)
-                out_indices = out_indices.narrow(0, 0, recv_count);
+                out_indices = part_of(out_indices, 0, {recv_count, topk}, torch::kInt64);
             if (weights.has_value())
-                out_weights = out_weights.narrow(0, 0, used_rows);
+                out_weights = expand ? part_of(out_weights, 0, {used_rows}, torch::kFloat32) : part_of(out_weights, 0, {recv_count, topk}, torch::kFloat32);
         } else {
             allocate_outputs(used_rows, recv_count);
             if (recv_count > 0)
@@ -1073,23 +1217,25 @@ DispatchResult dispatch(PeerRuntime& runtime,
             runtime.remember_private(metadata, alignment);
     }
 
+    // absent ones at this boundary, made off the path to the launch
     if (expand)
-        out_indices = torch::empty({0}, routing.options());  // absent at this boundary; made off the path to the launch
+        out_indices = new_tensor({0}, torch::kInt64, here);
+    if (!weights.has_value())
+        out_weights = new_tensor({0}, torch::kFloat32, here);
     std::vector<torch::Tensor> outputs{out_x, out_indices, out_weights};
     std::shared_ptr<CompletionEvent> event;
     if (async_op) {
-        if (x.numel() > 0)
-            x.record_stream(comm.unwrap());
-        if (!cached && indices.numel() > 0)
-            indices.record_stream(comm.unwrap());
-        if (weights.has_value() && weights->numel() > 0)
-            weights->record_stream(comm.unwrap());
-        for (const auto& tensor : cached_metadata)
-            if (tensor.numel() > 0)
-                tensor.record_stream(comm.unwrap());
-        auto protected_tensors = outputs;
-        protected_tensors.insert(protected_tensors.end(), metadata.begin(), metadata.end());
-        event = CompletionEvent::record_behind(comm, std::move(protected_tensors));
+        std::vector<torch::Tensor> read{x};
+        if (cached)
+            read.insert(read.end(), cached_metadata.begin(), cached_metadata.end());
+        else
+            read.push_back(indices);
+        if (weights.has_value())
+            read.push_back(*weights);
+        std::vector<torch::Tensor> written{out_x, out_indices, out_weights};
+        if (!cached)
+            written.push_back(metadata[1]);  // the handle's tensors share one allocation
+        event = CompletionEvent::record_behind(comm, std::move(written), std::move(read));
     } else if (!same_queue(comm, compute)) {
         wait_on(compute, comm);
     }
@@ -1118,7 +1264,7 @@ CombineResult combine(PeerRuntime& runtime,
     const c10::Device here(c10::DeviceType::CUDA, device);
     TORCH_CHECK(x.is_cuda() && x.device() == here && x.is_contiguous() && x.size(1) > 0,
                 "combine x must be contiguous CUDA [N,H] or [C,H] on the runtime device");
-    require(x, {here, torch::kBFloat16, {-1, -1}}, "combine x must be bfloat16");
+    require(x, here, torch::kBFloat16, {-1, -1}, "combine x must be bfloat16");
     TORCH_CHECK(reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0, "combine x data pointer must be 16-byte aligned");
     TORCH_CHECK(x.size(1) % kHiddenAlignment == 0, "combine hidden must be a positive multiple of 256");
     TORCH_CHECK(metadata[1].dim() == 1 && metadata[1].numel() > 0,
@@ -1135,26 +1281,25 @@ CombineResult combine(PeerRuntime& runtime,
     TORCH_CHECK(expand ? (x.size(0) >= recv_count && (recv_count != 0 || x.size(0) == 0)) : x.size(0) == recv_count,
                 "combine x rows do not match the receive layout");
     if (weights.has_value())
-        require(*weights, {here, torch::kFloat32, expand ? std::vector<int64_t>{x.size(0)} : std::vector<int64_t>{recv_count, topk}},
-                "combine weights must be contiguous CUDA float32 [N,K] or expanded [C] on the x device");
+        TORCH_CHECK(expand ? describes(*weights, here, torch::kFloat32, {x.size(0)}) : describes(*weights, here, torch::kFloat32, {recv_count, topk}),
+                    "combine weights must be contiguous CUDA float32 [N,K] or expanded [C] on the x device");
     if (bias.has_value())
-        require(*bias, {here, torch::kBFloat16, {source_tokens, hidden}},
+        require(*bias, here, torch::kBFloat16, {source_tokens, hidden},
                 "combine bias must be contiguous [T,H], with the output dtype on the x device");
     const int cu_budget = resolve_cu_budget(num_sms, device);
 
     const auto compute = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(device);
     const auto comm = work_stream(comm_stream, compute, device, async_op, cu_budget != 0);
     order_comm_after_inputs(comm, compute, previous_event, async_op);
-    StreamGuard comm_guard(comm.unwrap());
+    const StreamSwitch on_comm(comm, compute);
 
     torch::Tensor combined_x, combined_weights;
     {
-        OptionalStreamGuard allocation_guard;
-        if (!async_op)
-            allocation_guard.reset_stream(compute.unwrap());
-        combined_x = torch::empty({source_tokens, hidden}, x.options());
-        combined_weights = torch::empty(weights.has_value() ? std::vector<int64_t>{source_tokens, topk} : std::vector<int64_t>{0},
-                                        x.options().dtype(torch::kFloat32));
+        // (as in dispatch: the caller's pool, unless the call is ordered behind an event of its own only)
+        const StreamSwitch pool(!async_op || previous_event == -1 ? compute : comm, comm);
+        combined_x = new_tensor({source_tokens, hidden}, torch::kBFloat16, here);
+        if (weights.has_value())
+            combined_weights = new_tensor({source_tokens, topk}, torch::kFloat32, here);
     }
     if (source_tokens > 0) {
         // a seven-tensor handle of the latest fresh dispatch gets its slot table back from the runtime
@@ -1168,9 +1313,7 @@ CombineResult combine(PeerRuntime& runtime,
         // ... or the table a replayed dispatch of this handle had rebuilt
         std::shared_ptr<PeerRuntime::RebuiltHandle> rebuilt;
         if (table == nullptr && expand && metadata.size() == 7 && recv_count > 0 && tuning_switch("REBUILD_ORDER") != 0) {
-            hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-            check_hip(hipStreamIsCapturing(comm.stream(), &capture), "hipStreamIsCapturing");
-            if (capture == hipStreamCaptureStatusNone && (rebuilt = runtime.find_rebuilt(metadata, x.size(0)))) {
+            if (!capturing(comm) && (rebuilt = runtime.find_rebuilt(metadata, x.size(0)))) {
                 if (rebuilt->made_on != comm.stream()) {
                     if (!rebuilt->ready.query())
                         comm.unwrap().wait(rebuilt->ready);
@@ -1188,19 +1331,18 @@ CombineResult combine(PeerRuntime& runtime,
                      "combine");
     }
 
+    if (!weights.has_value())
+        combined_weights = new_tensor({0}, torch::kFloat32, here);
     std::vector<torch::Tensor> outputs{combined_x, combined_weights};
     std::shared_ptr<CompletionEvent> event;
     if (async_op) {
-        if (x.numel() > 0)
-            x.record_stream(comm.unwrap());
-        if (weights.has_value() && weights->numel() > 0)
-            weights->record_stream(comm.unwrap());
-        if (bias.has_value() && bias->numel() > 0)
-            bias->record_stream(comm.unwrap());
-        for (const auto& tensor : metadata)
-            if (tensor.numel() > 0)
-                tensor.record_stream(comm.unwrap());
-        event = CompletionEvent::record_behind(comm, outputs);
+        std::vector<torch::Tensor> read(metadata);
+        read.push_back(x);
+        if (weights.has_value())
+            read.push_back(*weights);
+        if (bias.has_value())
+            read.push_back(*bias);
+        event = CompletionEvent::record_behind(comm, outputs, std::move(read));
     } else if (!same_queue(comm, compute)) {
         wait_on(compute, comm);
     }

@@ -55,3 +55,91 @@ def test_every_layout_plan_reports_bad_routing(device, tuning, launches, token, 
     idx[token, 4] = idx[token, 0] if bad is None else bad
     _, counts = cabi.layout(idx.to(device), 24, 1, True, raise_on_routing=False)
     assert counts[3] == status
+
+
+def small_case(device, seed, tokens=96, hidden=512, experts=12, topk=4):
+    idx = cases.routing("dropout", tokens, experts, topk, seed=seed)
+    x, w = cases.payload(tokens, hidden, seed=seed), cases.gate_weights(tokens, topk, seed=seed)
+    want_x, _, want_w, lay = oracle.dispatch(x, idx, experts, w, do_expand=True)
+    want, _ = oracle.combine(want_x, lay.recv_metadata(True), lay.dst_slots, do_expand=True)
+    return EPConfig(experts, topk, hidden, tokens), x.to(device), idx.to(device), w.to(device), want_x, want_w, want
+
+
+# More asynchronous calls on their way than there are words for their completion points (64): the rest of
+# them are ordered by events, and all of them behind the caller's stream, which is busy when they are made.
+@pytest.mark.parametrize("calls", [1, 63, 64, 65, 150])
+def test_asynchronous_calls_beyond_the_words_for_their_completion(device, calls):
+    config, x, idx, w, want_x, _, want = small_case(device, 5)
+    with Buffer(None, config) as buffer:
+        handle = buffer.dispatch(x, topk_idx=idx, weights=w, do_expand=True).handle
+        late_x = torch.zeros_like(x)
+        torch.cuda.synchronize()
+        torch.cuda._sleep(20_000_000)
+        late_x.copy_(x)
+        kept = [buffer.dispatch(late_x, handle=handle, async_op=True) for _ in range(calls)]
+        for received in kept:
+            received.event.current_stream_wait()
+        combined = buffer.combine(kept[-1].x, handle, async_op=True)
+        combined.event.current_stream_wait()
+        got = combined.x.clone()
+        assert_same_bits(got, want, "combine")
+        for received in kept[:: max(1, calls // 8)]:
+            assert_same_bits(received.x, want_x, "dispatch")
+
+
+# Callers on more streams than the device has hardware queues, each with a chain of asynchronous calls, made
+# round-robin: every chain is ordered, whatever the streams share.
+@pytest.mark.parametrize("streams", [2, 9])
+def test_asynchronous_chains_on_many_streams(device, streams):
+    lanes = []
+    for lane in range(streams):
+        config, x, idx, w, want_x, want_w, want = small_case(device, 20 + lane, tokens=40 + lane)
+        lanes.append((Buffer(None, config), torch.cuda.Stream(), x, idx, w, want))
+    torch.cuda.synchronize()
+    results = [None] * streams
+    for step in range(6):
+        for lane, (buffer, stream, x, idx, w, _) in enumerate(lanes):
+            with torch.cuda.stream(stream):
+                received = buffer.dispatch(x if step == 0 else results[lane].x, topk_idx=idx, weights=w, do_expand=True, async_op=True)
+                received.event.current_stream_wait()
+                y = received.x * 1  # the caller's own work between the calls
+                # (the next step dispatches what this one combined: the sums are fed back once, then the source again)
+                results[lane] = buffer.combine(y, received.handle, async_op=True)
+                results[lane].event.current_stream_wait()
+                if step % 2:
+                    results[lane].x.copy_(x)
+    torch.cuda.synchronize()
+    for lane, (buffer, stream, x, idx, w, want) in enumerate(lanes):
+        with torch.cuda.stream(stream):
+            received = buffer.dispatch(results[lane].x, topk_idx=idx, do_expand=True, async_op=True)
+            received.event.current_stream_wait()
+            combined = buffer.combine(received.x, received.handle, async_op=True)
+            combined.event.current_stream_wait()
+        torch.cuda.synchronize()
+        assert_same_bits(combined.x, want, f"lane {lane}")
+        buffer.close()
+
+
+# A completion event that goes away unwaited keeps the call's tensors safe from the allocator: what the call
+# reads and writes is freed and its memory asked for again while the call still waits for its stream.
+@pytest.mark.parametrize("explicit_event", [False, True])
+def test_a_dropped_completion_event_protects_the_calls_memory(device, explicit_event):
+    config, x, idx, w, want_x, want_w, _ = small_case(device, 8, tokens=200, hidden=1024)
+    with Buffer(None, config) as buffer:
+        handle = buffer.dispatch(x, topk_idx=idx, weights=w, do_expand=True).handle
+        torch.cuda.synchronize()
+        source = x.clone()
+        ready = None
+        if explicit_event:
+            ready = torch.cuda.Event()
+            ready.record()
+        with torch.cuda.stream(buffer.comm_stream):
+            torch.cuda._sleep(20_000_000)
+        received = buffer.dispatch(source, handle=handle, weights=w, async_op=True, previous_event=ready)
+        payload, gates = received.x, received.topk_weights
+        del received, source
+        poison = [torch.full_like(x, -77.0) for _ in range(4)] + [torch.full_like(want_x, -77.0, device=device) for _ in range(4)]
+        torch.cuda.synchronize()
+        assert_same_bits(payload, want_x, "payload")
+        assert_same_bits(gates, want_w, "weights")
+        del poison
