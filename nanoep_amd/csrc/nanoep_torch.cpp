@@ -230,11 +230,6 @@ class PeerRuntime {
         host_counts_ = static_cast<int64_t*>(mailbox);
         for (int i = 0; i < NANOEP_HOST_COUNT_WORDS; ++i)
             host_counts_[i] = -1;
-        void* words = nullptr;
-        check_hip(hipHostMalloc(&words, kRebuiltHandles * sizeof(int64_t), hipHostMallocMapped | hipHostMallocCoherent), "hipHostMalloc");
-        rebuilt_counts_ = static_cast<int64_t*>(words);
-        for (size_t i = 0; i < kRebuiltHandles; ++i)
-            rebuilt_counts_[i] = -1;
     }
 
     ~PeerRuntime() {
@@ -481,6 +476,13 @@ class PeerRuntime {
         entry->capacity = capacity;
         std::shared_ptr<RebuiltHandle> retired;  // released after the lock
         std::lock_guard<std::mutex> lock(private_mutex_);
+        if (rebuilt_counts_ == nullptr) {  // (most runtimes never rebuild a handle, and pinned memory takes 40 us)
+            void* words = nullptr;
+            check_hip(hipHostMalloc(&words, kRebuiltHandles * sizeof(int64_t), hipHostMallocMapped | hipHostMallocCoherent), "hipHostMalloc");
+            rebuilt_counts_ = static_cast<int64_t*>(words);
+            for (size_t i = 0; i < kRebuiltHandles; ++i)
+                rebuilt_counts_[i] = -1;
+        }
         size_t at = kRebuiltHandles;
         for (size_t i = 0; i < kRebuiltHandles && at == kRebuiltHandles; ++i)
             if (!rebuilt_[i] || rebuilt_[i]->snapshot.expired())
@@ -853,7 +855,17 @@ bool same_queue(const Stream& a, const Stream& b) { return a.stream() == b.strea
 // A synchronous call must leave its results ordered on the caller's stream, so it runs there
 // directly instead of bouncing through the communication stream with two cross-stream events; it
 // still comes after everything enqueued earlier on the communication stream.
+//
+// kNoStream in place of that stream says that nothing has ever been put on it: a synchronous call then has
+// nothing there to come behind, and a stream that nobody uses is never set up (the handle alone takes
+// the runtime 80 us, the first question how it is doing 120 to 200 us, of a new buffer's first call).
+constexpr int64_t kNoStream = -1;
+
 Stream work_stream(int64_t comm_handle, const Stream& compute, c10::DeviceIndex device, bool async_op, bool budgeted) {
+    if (comm_handle == kNoStream) {
+        TORCH_CHECK(!async_op && !budgeted, "an asynchronous call, or one with a compute-unit budget, needs its stream");
+        return compute;
+    }
     const auto comm = external_stream(comm_handle, device);
     // (a call with a compute-unit budget runs on the stream it was handed: that stream carries the CU mask)
     if (async_op || budgeted || same_queue(comm, compute))

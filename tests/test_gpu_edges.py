@@ -143,3 +143,32 @@ def test_a_dropped_completion_event_protects_the_calls_memory(device, explicit_e
         assert_same_bits(payload, want_x, "payload")
         assert_same_bits(gates, want_w, "weights")
         del poison
+
+
+# A synchronous call passes over a communication stream nothing was ever put on, and comes behind what the
+# caller, an asynchronous call or a call with a compute-unit budget put there.
+@pytest.mark.parametrize("through", ["comm_stream", "budget_stream", "async"])
+def test_synchronous_calls_come_behind_the_communication_stream(device, through):
+    config, x, idx, w, want_x, _, _ = small_case(device, 31)
+    with Buffer(None, config) as buffer:
+        handle = buffer.dispatch(x, topk_idx=idx, do_expand=True).handle
+        late_x = torch.zeros_like(x)
+        torch.cuda.synchronize()
+        stream = {"comm_stream": lambda: buffer.comm_stream, "budget_stream": lambda: buffer.budget_stream(128),
+                  "async": lambda: None}[through]()
+        if stream is None:
+            torch.cuda._sleep(20_000_000)
+            late_x.copy_(x)
+            first = buffer.dispatch(late_x, handle=handle, async_op=True)
+            side = torch.cuda.Stream()
+            with torch.cuda.stream(side):  # not ordered behind the copy but through the communication stream
+                got = buffer.dispatch(late_x, handle=handle)
+                got_x = got.x
+            first.event.current_stream_wait()
+        else:
+            with torch.cuda.stream(stream):
+                torch.cuda._sleep(20_000_000)
+                late_x.copy_(x)
+            got_x = buffer.dispatch(late_x, handle=handle).x
+        torch.cuda.synchronize()
+        assert_same_bits(got_x, want_x, through)
