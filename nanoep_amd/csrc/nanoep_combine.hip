@@ -144,11 +144,12 @@ __global__ void __launch_bounds__(1024) combine_rows_kernel(const u32x4* __restr
         out_weights[static_cast<int64_t>(token) * num_topk + lane] = valid ? weights[slot] : 0.0f;
 }
 
-// Expanded layout with at most kTopk <= 4 rows per token and the slot table at hand: the same
-// gather-sum as combine_rows_kernel, carrying only what that case needs (the token's slots come as
-// scalars straight from the table).  With so few rows per token the kernel is short and close to a
-// copy, and the general kernel's bookkeeping showed (Mixtral-shaped batch: 19.3 us against 17.3 us
-// for the bare access pattern).
+// Expanded layout with kTopk <= 8 rows per token and the slot table at hand: the same gather-sum as
+// combine_rows_kernel, carrying only what that case needs.  The token's slots come as scalars straight from
+// the table, so a masked choice's load is branched around by the whole wavefront, and as many rows are
+// fetched as there are choices (Mixtral-shaped batch, two rows: 17.3 us as the bare access pattern, 19.3 with the
+// general kernel's bookkeeping).  One token's chunk a wavefront: short launches are bound by
+// the chain slots -> rows -> store, not by bytes, and a second token a wavefront is a second chain.
 template <int kTopk>
 __global__ void __launch_bounds__(1024) combine_few_rows_kernel(const u32x4* __restrict__ y,              // [C][vectors]
                                                                 const float* __restrict__ weights,       // [C] or null
@@ -195,18 +196,19 @@ __global__ void __launch_bounds__(1024) combine_few_rows_kernel(const u32x4* __r
     const uint32_t vector = chunk * kWave + threadIdx.x;
     const bool in_row = vector < vectors;
     const uint32_t load_vector = in_row ? vector : 0u;
-    const int32_t* slots = token_slots + static_cast<uint64_t>(token) * topk;
+    const int32_t* slots = token_slots + static_cast<uint64_t>(token) * kTopk;
     int32_t slot[kTopk];
-    bool valid[kTopk];
 #pragma unroll
-    for (int k = 0; k < kTopk; ++k) {
-        slot[k] = uniform_load(slots + (static_cast<uint32_t>(k) < topk ? k : 0));
-        valid[k] = static_cast<uint32_t>(k) < topk && slot[k] >= 0 && static_cast<uint32_t>(slot[k]) < y_rows;
-    }
+    for (int k = 0; k < kTopk; ++k)
+        slot[k] = uniform_load(slots + k);
+    bool valid[kTopk];
     u32x4 data[kTopk];
 #pragma unroll
-    for (int k = 0; k < kTopk; ++k)  // a masked k re-reads row 0 and drops it: the loads stay unconditional
-        data[k] = load_vec<true>(y + static_cast<uint64_t>(valid[k] ? slot[k] : 0) * vectors + load_vector);
+    for (int k = 0; k < kTopk; ++k) {
+        valid[k] = static_cast<uint32_t>(slot[k]) < y_rows;
+        if (valid[k])  // (the same for the whole wavefront)
+            data[k] = load_vec<true>(y + static_cast<uint64_t>(static_cast<uint32_t>(slot[k])) * vectors + load_vector);
+    }
     u32x4 bias_data = {0u, 0u, 0u, 0u};
     if (bias != nullptr)
         bias_data = load_vec<true>(bias + static_cast<uint64_t>(token) * vectors + load_vector);
@@ -239,14 +241,17 @@ __global__ void __launch_bounds__(1024) combine_few_rows_kernel(const u32x4* __r
     }
 }
 
-// Expanded layout with the slot table at hand and five or more rows a token: one wavefront (a
+// Expanded layout with the slot table at hand and seven or more rows a token, batches of more wavefronts than
+// the device holds with a token each: one wavefront (a
 // workgroup of its own) produces the same 1 KiB chunk of the output rows of up to kUnits tokens
 // and holds the packed sums back in registers until the last one is done.  The units are
 // sized so that all wavefronts of the launch are resident at once wherever the batch allows it: the
 // whole device then reads first and writes last, and HBM sees the output as one burst behind the
-// gather instead of a write among every eight reads.  A token's rows are fetched eight at a time (a
-// masked k re-reads row 0 so that the loads stay unconditional).
-template <int kUnits>
+// gather instead of a write among every eight reads.  A token's rows are fetched all at once (kTopk of
+// them) or eight at a time (kTopk 0; a masked k re-reads row 0 so that the loads stay unconditional).  The
+// slots go through a vector load and lane reads here: as scalar loads, with masked rows branched around, a
+// wavefront's tokens wait for each other longer (4096 x 7168 top-8 80 -> 93 us).
+template <int kUnits, int kTopk>
 __global__ void __launch_bounds__(kWave) combine_held_kernel(const u32x4* __restrict__ y,              // [C][vectors]
                                                              const float* __restrict__ weights,       // [C] or null
                                                              const u32x4* __restrict__ bias,          // [T][vectors] or null
@@ -318,18 +323,19 @@ __global__ void __launch_bounds__(kWave) combine_held_kernel(const u32x4* __rest
         if (bias != nullptr)
             bias_data = load_vec<true>(bias + static_cast<uint64_t>(token) * vectors + load_vector);
         float acc[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-        // eight rows a pass, in ascending k
-        for (uint32_t base = 0; base < (valid_mask != 0 ? topk : 0u); base += kHeldRows) {
-            u32x4 data[kHeldRows];
+        // in ascending k, all rows at once or eight a pass
+        constexpr int kRows = kTopk != 0 ? kTopk : kHeldRows;
+        for (uint32_t base = 0; base < (valid_mask == 0 ? 0u : kTopk != 0 ? 1u : topk); base += kRows) {
+            u32x4 data[kRows];
 #pragma unroll
-            for (int k = 0; k < kHeldRows; ++k) {
+            for (int k = 0; k < kRows; ++k) {
                 uint64_t source_row = 0;
                 if ((valid_mask >> (base + k)) & 1)
                     source_row = static_cast<uint32_t>(__builtin_amdgcn_readlane(slot, (base + k) & (kWave - 1)));
                 data[k] = load_vec<true>(y + source_row * vectors + load_vector);
             }
 #pragma unroll
-            for (int k = 0; k < kHeldRows; ++k)
+            for (int k = 0; k < kRows; ++k)
                 if ((valid_mask >> (base + k)) & 1)
                     accumulate(acc, data[k]);
         }
@@ -442,15 +448,22 @@ __global__ void __launch_bounds__(1024) combine_compact_kernel(const u32x4* __re
 // was written against) is the answer when the runtime gives none.
 template <int kUnits>
 int held_wavefronts_per_cu(int fallback) {
-    hipFuncAttributes attributes{};
-    if (hipFuncGetAttributes(&attributes, reinterpret_cast<const void*>(&combine_held_kernel<kUnits>)) != hipSuccess ||
-        attributes.numRegs <= 0) {
-        (void)hipGetLastError();
-        return fallback;
+    // (the variants for other numbers of rows need no more registers than one of these two)
+    const void* kernels[] = {reinterpret_cast<const void*>(&combine_held_kernel<kUnits, 8>),
+                             reinterpret_cast<const void*>(&combine_held_kernel<kUnits, 0>)};
+    int fewest = 32;
+    for (const void* kernel : kernels) {
+        hipFuncAttributes attributes{};
+        if (hipFuncGetAttributes(&attributes, kernel) != hipSuccess || attributes.numRegs <= 0) {
+            (void)hipGetLastError();
+            return fallback;
+        }
+        const int granules = (attributes.numRegs + 7) / 8 * 8;
+        const int per_simd = 512 / granules;
+        const int held = 4 * (per_simd > 8 ? 8 : per_simd < 1 ? 1 : per_simd);
+        fewest = held < fewest ? held : fewest;
     }
-    const int granules = (attributes.numRegs + 7) / 8 * 8;
-    const int per_simd = 512 / granules;
-    return 4 * (per_simd > 8 ? 8 : per_simd < 1 ? 1 : per_simd);
+    return fewest;
 }
 
 }  // namespace
@@ -533,8 +546,13 @@ int nanoep_combine(const void* y, const float* weights, const void* bias, const 
         NANOEP_HIP_TRY(hipGetLastError());
         return NANOEP_OK;
     }
-    // Five or more rows a token with the slot table at hand: wavefronts that hold the sums of 2 to 16
-    // tokens back and write them at their end; as many tokens a wavefront as it takes for the launch to
+    // With the slot table at hand, a wavefront takes one token's chunk (combine_few_rows_kernel up to eight rows a
+    // token) or holds the sums of 2 to 16 tokens back and writes them at its end (combine_held_kernel).
+    //  * One: up to 6 rows a token, and launches whose wavefronts are all resident with one token each (32 a
+    //    compute unit).  Held -> one token, rows in the caches: 128 x 4096 top-8 4.0 -> 3.0 us, 1024 x 1024 5.0 -> 4.0,
+    //    768 x 4096 10.1 -> 9.5, 1024 x 4096 (8192 wavefronts) 12.3 -> 12.4, 1024 x 7168 20.4 -> 21.0; top-6: 1537 x 2816 11.3 ->
+    //    10.2, 2048 x 2816 14.4 -> 12.9, 4096 x 2816 25.9 -> 26.1, 8192 x 2816 52.7 -> 51.4.
+    //  * Held: as many tokens a wavefront as it takes for the launch to
     // fit what the device holds at once with the registers of sixteen held rows (16 wavefronts a
     // compute unit), or a whole multiple of that when sixteen tokens a wavefront are not enough: a
     // launch a little larger than what is resident waits for its last few wavefronts with the device
@@ -543,15 +561,15 @@ int nanoep_combine(const void* y, const float* weights, const void* bias, const 
     // (token, chunk) a wavefront, sources from HBM: 4096 x 7168 top-8 78.2 -> 73.7 us, 8192 x 2048
     // 49.1 -> 47.6, 2048 x 7168 39.9 -> 37.8, 32768 x 1024 89.0 -> 83.4, 32768 x 512 46.1 -> 44.7,
     // 8192 x 7168 159.2 -> 155.4; 4096 x 4096 top-16 82.9 -> 79.7, 2048 x 7168 top-12 57.8 -> 55.3.  With
-    // two to four rows a token the held sums lose to
-    // combine_few_rows_kernel (4096 x 4096 top-2: 17.3 us against 18.1 to 30.5).
+    // two to four rows a token the held sums lose (4096 x 4096 top-2: 17.3 us against 18.1 to 30.5).
     // NANOEP_COMBINE_UNITS=1 keeps one token a wavefront, 2..16 asks for that many.
     int held_units = 0;
     int64_t held_resident = 0, held_side = 0;
-    if (direct && num_topk > 4 && num_topk <= 32 && tuning.combine_units != 1) {
+    const Topology topology = current_topology(tuning);
+    const int64_t cus = num_cus > 0 ? num_cus : topology.cus;
+    const bool one_token = tuning.combine_units == 1 || (tuning.combine_units == 0 && (num_topk <= 6 || num_tokens * chunks <= cus * 32));
+    if (direct && num_topk > 4 && !one_token) {
         // (the wavefronts of sixteen held rows a compute unit holds, on the compute units this call may use)
-        const Topology topology = current_topology(tuning);
-        const int64_t cus = num_cus > 0 ? num_cus : topology.cus;
         const int64_t resident = cus * topology.held_wavefronts[3];
         held_resident = resident;
         // (the side wavefronts that restore the weights are in the launch too)
@@ -583,26 +601,34 @@ int nanoep_combine(const void* y, const float* weights, const void* bias, const 
         const bool strided = held_groups * chunks <= held_resident;
         if (held_blocks >= (int64_t{1} << 31))
             return NANOEP_ERR_INVALID_ARGUMENT;
-#define NANOEP_LAUNCH_HELD(UNITS)                                                                                      \
-    combine_held_kernel<UNITS><<<dim3(static_cast<unsigned>(held_blocks)), dim3(kWave), 0, stream>>>(                 \
+#define NANOEP_LAUNCH_HELD(UNITS, TOPK)                                                                                \
+    combine_held_kernel<UNITS, TOPK><<<dim3(static_cast<unsigned>(held_blocks)), dim3(kWave), 0, stream>>>(            \
         static_cast<const u32x4*>(y), weights, static_cast<const u32x4*>(bias), token_slots, static_cast<u32x4*>(out_x), \
         out_weights, static_cast<uint32_t>(num_tokens), static_cast<uint32_t>(y_rows), static_cast<uint32_t>(chunks),   \
         chunks_divisor.magic, chunks_divisor.shift, static_cast<uint32_t>(vectors), static_cast<uint32_t>(num_topk), flags, \
         static_cast<uint32_t>(held_side_blocks), static_cast<uint32_t>(held_units),                                      \
         strided ? 1u : static_cast<uint32_t>(held_units), strided ? static_cast<uint32_t>(held_groups) : 1u)
-        if (held_units > 8)
-            NANOEP_LAUNCH_HELD(16);
-        else if (held_units > 4)
-            NANOEP_LAUNCH_HELD(8);
-        else if (held_units > 2)
-            NANOEP_LAUNCH_HELD(4);
-        else
-            NANOEP_LAUNCH_HELD(2);
+#define NANOEP_LAUNCH_HELD_ROWS(UNITS)                     \
+    switch (num_topk) {                                    \
+        case 7: NANOEP_LAUNCH_HELD(UNITS, 7); break;       \
+        case 8: NANOEP_LAUNCH_HELD(UNITS, 8); break;       \
+        default: NANOEP_LAUNCH_HELD(UNITS, 0); break;      \
+    }
+        if (held_units > 8) {
+            NANOEP_LAUNCH_HELD_ROWS(16)
+        } else if (held_units > 4) {
+            NANOEP_LAUNCH_HELD_ROWS(8)
+        } else if (held_units > 2) {
+            NANOEP_LAUNCH_HELD_ROWS(4)
+        } else {
+            NANOEP_LAUNCH_HELD_ROWS(2)
+        }
+#undef NANOEP_LAUNCH_HELD_ROWS
 #undef NANOEP_LAUNCH_HELD
         NANOEP_HIP_TRY(hipGetLastError());
         return NANOEP_OK;
     }
-    if (direct && num_topk <= 4) {
+    if (direct && num_topk <= 8) {
 #define NANOEP_LAUNCH_FEW(TOPK)                                                                                       \
     combine_few_rows_kernel<TOPK><<<grid_with_side, block, 0, stream>>>(                                             \
         static_cast<const u32x4*>(y), weights, static_cast<const u32x4*>(bias), token_slots,                         \
@@ -610,12 +636,16 @@ int nanoep_combine(const void* y, const float* weights, const void* bias, const 
         blocking.parts, parts_divisor.magic, parts_divisor.shift, blocking.chunks_per_block, blocking.rows_per_block, \
         static_cast<uint32_t>(vectors), static_cast<uint32_t>(chunks), static_cast<uint32_t>(num_topk),              \
         flags, topk_divisor.magic, topk_divisor.shift, static_cast<uint32_t>(side_blocks))
-        if (num_topk == 1)
-            NANOEP_LAUNCH_FEW(1);
-        else if (num_topk == 2)
-            NANOEP_LAUNCH_FEW(2);
-        else
-            NANOEP_LAUNCH_FEW(4);
+        switch (num_topk) {
+            case 1: NANOEP_LAUNCH_FEW(1); break;
+            case 2: NANOEP_LAUNCH_FEW(2); break;
+            case 3: NANOEP_LAUNCH_FEW(3); break;
+            case 4: NANOEP_LAUNCH_FEW(4); break;
+            case 5: NANOEP_LAUNCH_FEW(5); break;
+            case 6: NANOEP_LAUNCH_FEW(6); break;
+            case 7: NANOEP_LAUNCH_FEW(7); break;
+            default: NANOEP_LAUNCH_FEW(8); break;
+        }
 #undef NANOEP_LAUNCH_FEW
         NANOEP_HIP_TRY(hipGetLastError());
         return NANOEP_OK;
@@ -626,25 +656,19 @@ int nanoep_combine(const void* y, const float* weights, const void* bias, const 
         token_slots, static_cast<u32x4*>(out_x), out_weights, recv_count, y_rows, static_cast<uint32_t>(num_tokens), \
         blocking.parts, parts_divisor.magic, parts_divisor.shift, blocking.chunks_per_block, blocking.rows_per_block,  \
         vectors, chunks, num_topk, flags)
-#define NANOEP_LAUNCH_COMBINE_GROUP(GROUP)    \
-    do {                                     \
-        if (direct)                          \
-            NANOEP_LAUNCH_COMBINE(GROUP, true);  \
-        else                                 \
-            NANOEP_LAUNCH_COMBINE(GROUP, false); \
-    } while (0)
     // the group size is the number of rows fetched per pass: the smallest of 1, 2, 4, 8, 16 covering K
-    if (num_topk <= 1)
-        NANOEP_LAUNCH_COMBINE_GROUP(1);
+    if (direct)
+        NANOEP_LAUNCH_COMBINE(16, true);
+    else if (num_topk <= 1)
+        NANOEP_LAUNCH_COMBINE(1, false);
     else if (num_topk <= 2)
-        NANOEP_LAUNCH_COMBINE_GROUP(2);
+        NANOEP_LAUNCH_COMBINE(2, false);
     else if (num_topk <= 4)
-        NANOEP_LAUNCH_COMBINE_GROUP(4);
+        NANOEP_LAUNCH_COMBINE(4, false);
     else if (num_topk <= 8)
-        NANOEP_LAUNCH_COMBINE_GROUP(8);
+        NANOEP_LAUNCH_COMBINE(8, false);
     else
-        NANOEP_LAUNCH_COMBINE_GROUP(16);
-#undef NANOEP_LAUNCH_COMBINE_GROUP
+        NANOEP_LAUNCH_COMBINE(16, false);
 #undef NANOEP_LAUNCH_COMBINE
     NANOEP_HIP_TRY(hipGetLastError());
     return NANOEP_OK;

@@ -172,3 +172,33 @@ def test_synchronous_calls_come_behind_the_communication_stream(device, through)
             got_x = buffer.dispatch(late_x, handle=handle).x
         torch.cuda.synchronize()
         assert_same_bits(got_x, want_x, through)
+
+
+# The one-token combine for every number of rows it is made for, at rows that end inside a chunk, with all of
+# bias, weights and the extra rounding, and around the batch size from which sums are held back (8192 wavefronts).
+@pytest.mark.parametrize("topk", range(1, 9))
+@pytest.mark.parametrize("tokens,hidden", [(3, 256), (70, 2816)])
+def test_one_token_combine_for_every_row_count(device, topk, tokens, hidden):
+    idx = cases.routing("sparse", tokens, 12, topk, seed=topk)
+    metadata, counts = cabi.layout(idx.to(device), 12, 1, True, hidden=hidden)
+    lay = oracle.layout(idx, 12, 1)
+    y, bias = cases.payload(counts[1], hidden, seed=topk), cases.payload(tokens, hidden, seed=99)
+    w = cases.gate_weights(counts[1], 1, seed=3).flatten()
+    for multiple in (False, True):
+        out, out_w = cabi.combine(y.to(device), w.to(device), bias.to(device), metadata, counts, True, multiple_reduction=multiple, poison=0xA5)
+        want, want_w = oracle.combine(y, lay.recv_metadata(True), lay.dst_slots, do_expand=True, weights=w, bias=bias,
+                                      multiple_reduction=multiple)
+        assert_same_bits(out, want, "combine")
+        assert_same_bits(out_w, want_w, "weights")
+
+
+@pytest.mark.parametrize("topk", [7, 8, 9])
+@pytest.mark.parametrize("tokens", [1024, 1025])
+def test_combine_around_the_batch_that_holds_sums_back(device, topk, tokens):
+    idx = cases.routing("dropout", tokens, 16, topk, seed=topk)
+    metadata, counts = cabi.layout(idx.to(device), 16, 1, True, hidden=4096)
+    lay = oracle.layout(idx, 16, 1)
+    y = cases.payload(counts[1], 4096, seed=topk)
+    out, _ = cabi.combine(y.to(device), None, None, metadata, counts, True, poison=0xA5)
+    want, _ = oracle.combine(y, lay.recv_metadata(True), lay.dst_slots, do_expand=True)
+    assert_same_bits(out, want, "combine")
