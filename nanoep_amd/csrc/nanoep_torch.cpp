@@ -710,13 +710,16 @@ class CompletionEvent {
     }
 
     void order_after(const Stream& consumer) {
-        if (!point_.has_value()) {
-            consumer.unwrap().wait(done_);
-        } else if (!point_->reached()) {
-            TORCH_CHECK(!capturing(consumer), "a completion event of work outside a HIP graph cannot be waited on inside its capture");
-            StreamPoints::wait(consumer, *point_);
-        }
         std::lock_guard<std::mutex> lock(mutex_);
+        if (point_.has_value() && !capturing(consumer)) {
+            if (!point_->reached())
+                StreamPoints::wait(consumer, *point_);
+        } else {
+            // A consumer under capture is told of an event, and the runtime says what it makes of that.
+            if (point_.has_value())
+                done_.record(producer_->unwrap());
+            consumer.unwrap().wait(done_);
+        }
         note_use(written_, consumer);
         note_use(read_, consumer);
         read_.clear();
@@ -747,7 +750,7 @@ class CompletionEvent {
 
     std::mutex mutex_;
     std::optional<StreamPoint> point_;
-    c10::Event done_;  // where there is no point
+    c10::Event done_;  // where there is no point, or a consumer under capture
     std::optional<Stream> producer_;
     bool waited_ = false;
     std::vector<torch::Tensor> written_, read_;

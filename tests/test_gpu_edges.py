@@ -145,6 +145,46 @@ def test_a_dropped_completion_event_protects_the_calls_memory(device, explicit_e
         del poison
 
 
+# Waiting inside a graph's capture for a call made outside it comes to what the runtime makes of a plain event
+# behind the same work, and does not depend on how the call's completion is kept.
+@pytest.mark.parametrize("finished", [False, True])
+def test_a_wait_inside_a_capture_is_an_events(device, finished):
+    config, x, idx, w, want_x, _, _ = small_case(device, 12)
+
+    def captures(wait):
+        scratch = torch.zeros(8, device=device)
+        graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+        torch.cuda.current_stream().synchronize()
+        refused = False
+        with torch.cuda.stream(stream):
+            graph.capture_begin(capture_error_mode="thread_local")
+            try:
+                scratch.add_(1)
+                wait()
+            except RuntimeError:
+                refused = True
+            try:
+                graph.capture_end()
+            except RuntimeError:
+                refused = True
+        return refused
+
+    with Buffer(None, config) as buffer:
+        handle = buffer.dispatch(x, topk_idx=idx, do_expand=True).handle
+        if not finished:
+            with torch.cuda.stream(buffer.comm_stream):
+                torch.cuda._sleep(20_000_000)
+        received = buffer.dispatch(x, handle=handle, async_op=True)
+        plain = torch.cuda.Event()
+        plain.record(buffer.comm_stream)
+        if finished:
+            torch.cuda.synchronize()
+        assert captures(received.event.current_stream_wait) == captures(lambda: plain.wait())
+        received.event.current_stream_wait()
+        torch.cuda.synchronize()
+        assert_same_bits(received.x, want_x, "payload")
+
+
 # A synchronous call passes over a communication stream nothing was ever put on, and comes behind what the
 # caller, an asynchronous call or a call with a compute-unit budget put there.
 @pytest.mark.parametrize("through", ["comm_stream", "budget_stream", "async"])
