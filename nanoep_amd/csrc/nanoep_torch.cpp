@@ -694,15 +694,19 @@ class PeerRuntime {
 // consumer's stream instead, which costs nothing for tensors that were allocated there (telling it of the
 // communication stream makes it record an event for every block when it is freed).  A marker that goes
 // away with nobody having waited tells it of the communication stream after all.
+//
+// A caller that is on the communication stream itself most likely waits there, and gets an event: on one
+// queue that is no work for the GPU, where the store of a StreamPoint stands between the kernels (8192 x 2048
+// top-8, alignment 128, launch period: event 52.9 us a dispatch and 50.3 a combine, store 59.4 and 55.2).
 class CompletionEvent {
    public:
-    static std::shared_ptr<CompletionEvent> record_behind(const Stream& producer, std::vector<torch::Tensor> written,
-                                                          std::vector<torch::Tensor> read) {
+    static std::shared_ptr<CompletionEvent> record_behind(const Stream& producer, const Stream& caller,
+                                                          std::vector<torch::Tensor> written, std::vector<torch::Tensor> read) {
         auto marker = std::make_shared<CompletionEvent>();
         marker->written_ = std::move(written);
         marker->read_ = std::move(read);
         marker->producer_ = producer;
-        if (!capturing(producer))
+        if (producer.stream() != caller.stream() && !capturing(producer))
             marker->point_ = StreamPoints::of(producer.device_index()).record(producer);
         if (!marker->point_.has_value())
             marker->done_.record(producer.unwrap());
@@ -1250,7 +1254,7 @@ DispatchResult dispatch(PeerRuntime& runtime,
         std::vector<torch::Tensor> written{out_x, out_indices, out_weights};
         if (!cached)
             written.push_back(metadata[1]);  // the handle's tensors share one allocation
-        event = CompletionEvent::record_behind(comm, std::move(written), std::move(read));
+        event = CompletionEvent::record_behind(comm, compute, std::move(written), std::move(read));
     } else if (!same_queue(comm, compute)) {
         wait_on(compute, comm);
     }
@@ -1357,7 +1361,7 @@ CombineResult combine(PeerRuntime& runtime,
             read.push_back(*weights);
         if (bias.has_value())
             read.push_back(*bias);
-        event = CompletionEvent::record_behind(comm, outputs, std::move(read));
+        event = CompletionEvent::record_behind(comm, compute, outputs, std::move(read));
     } else if (!same_queue(comm, compute)) {
         wait_on(compute, comm);
     }

@@ -120,6 +120,28 @@ def test_asynchronous_chains_on_many_streams(device, streams):
         buffer.close()
 
 
+# Asynchronous calls of a caller that is on the communication stream itself, waited for there and from another
+# stream, behind work that keeps the communication stream busy.
+@pytest.mark.parametrize("consumer", ["there", "elsewhere"])
+def test_asynchronous_calls_made_on_the_communication_stream(device, consumer):
+    config, x, idx, w, want_x, _, want = small_case(device, 31)
+    with Buffer(None, config) as buffer:
+        handle = buffer.dispatch(x, topk_idx=idx, weights=w, do_expand=True).handle
+        elsewhere = torch.cuda.Stream()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(buffer.comm_stream):
+            torch.cuda._sleep(20_000_000)
+            received = buffer.dispatch(x, handle=handle, async_op=True)
+            combined = buffer.combine(received.x, handle, async_op=True)
+        with torch.cuda.stream(buffer.comm_stream if consumer == "there" else elsewhere):
+            received.event.current_stream_wait()
+            combined.event.current_stream_wait()
+            got_x, got = received.x.clone(), combined.x.clone()
+        torch.cuda.synchronize()
+        assert_same_bits(got_x, want_x, "dispatch")
+        assert_same_bits(got, want, "combine")
+
+
 # A completion event that goes away unwaited keeps the call's tensors safe from the allocator: what the call
 # reads and writes is freed and its memory asked for again while the call still waits for its stream.
 @pytest.mark.parametrize("explicit_event", [False, True])
