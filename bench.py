@@ -627,7 +627,8 @@ def measure(workload, args, device, detailed):
     if not workload.expand:
         combine_kernel = "combine_compact_kernel"
     else:
-        combine_kernel = "combine_few_rows_kernel" if workload.topk <= 4 else "combine_held_kernel" if workload.topk <= 8 else "combine_rows_kernel"
+        one_token = workload.topk <= 6 or workload.tokens * -(-workload.hidden // 512) <= 32 * torch.cuda.get_device_properties(0).multi_processor_count
+        combine_kernel = "combine_held_kernel" if not one_token else "combine_few_rows_kernel" if workload.topk <= 8 else "combine_rows_kernel"
     result.update(
         {
             "value": round(value, 1),

@@ -1330,8 +1330,8 @@ int nanoep_layout_static(const int64_t* topk_idx, int64_t num_tokens, int num_to
     const int scratch_status = static_scratch_of_current_device(&base);
     if (scratch_status != NANOEP_OK)
         return scratch_status;
-    // Nothing in the workspace has to start at zero: the count pass writes every histogram row, status
-    // word, rank entry and receive row that the later passes of the same call read.
+    // Nothing in the workspace has to start at zero: the histogram kernel writes every row (counts
+    // and status) that the later kernels of the same call read.
     const LayoutWorkspace ws = carve_layout_workspace(base, num_tokens, num_topk, num_local_experts, knobs);
     return enqueue_layout(topk_idx, num_tokens, num_topk, num_local_experts, alignment, expand, hidden, recv_metadata, expert_counts,
                           expert_offsets, dst_slots, send_counts, topk_snapshot, recv_rank_prefix, token_slots, slot_order, ws,
