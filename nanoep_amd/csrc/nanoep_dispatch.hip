@@ -188,6 +188,7 @@ struct WalkArgs {
     uint32_t window_vectors;        // 16-byte vectors of one window's source rows
     uint32_t source_vectors;        // ... of all source rows
     uint32_t window_weights;        // (token, k) pairs of one window
+    uint32_t touch_waves;           // wavefronts of a segment that bring in its list share and weights
     uint32_t rows_magic;  // fast divisor by rows_per_block
     uint32_t rows_shift;
     // gap rows
@@ -241,8 +242,10 @@ __device__ __forceinline__ void walk_gap_rows(const WalkArgs& a, uint32_t xcd, u
 // (a backward pass behind the other layers') has both in HBM only.  Handle in HBM, without -> with:
 // 32768 x 1024 top-8 129.4 -> 95.0 us, 4096 x 7168 top-8 with alignment 128 128.1 -> 97.1 us; behind a
 // layout that has just written the list 81.9 -> 78.6 us (4096 x 7168, count on the device).  One word a
-// 64-byte line is read, so 256 tokens x 8 choices are four wavefronts' loads.  Reading the next segment's
-// share too changed nothing (within 0.3 %).
+// 64-byte line is read, so 256 tokens x 8 choices are four wavefronts' loads for the list and two for the
+// weights, and the other prefetch wavefronts leave that aside with one comparison (with all of them taking
+// part 4096 x 7168 top-8 through a handle still in the caches took 75.5 us instead of 74.6; with the
+// rows' loads ahead of these 76.1).  Reading the next segment's share too changed nothing (within 0.3 %).
 constexpr int kPrefetchLoads = 4;
 
 // Reads one word of every 64-byte line of bytes [first, end) behind `base`: `wave` of `waves`
@@ -396,16 +399,19 @@ __device__ __forceinline__ void walk_copy(const WalkArgs& a, uint32_t entries, u
             window_end = a.source_vectors;
         // the segment's share of the list, the window's weights (from the last wavefront on, the list's
         // lines are the first ones'), then the window's rows
-        const uint64_t list_first = static_cast<uint64_t>(segment) * segment_entries;
-        const uint64_t list_end = list_first + segment_entries;
-        touch_lines(a.slot_order, list_first * 8, (list_end < entries ? list_end : entries) * 8, within * waves + wave, a.prefetch_blocks * waves);
-        if (a.weights != nullptr) {
-            const uint64_t weights_first = static_cast<uint64_t>(segment) * a.window_weights;
-            const uint64_t weights_end = weights_first + a.window_weights;
-            touch_lines(a.weights, weights_first * 4, (weights_end < a.source_limit ? weights_end : a.source_limit) * 4,
-                        a.prefetch_blocks * waves - 1 - (within * waves + wave), a.prefetch_blocks * waves);
+        const uint32_t nth = within * waves + wave;
+        if (nth < a.touch_waves) {
+            const uint64_t list_first = static_cast<uint64_t>(segment) * segment_entries;
+            const uint64_t list_end = list_first + segment_entries;
+            touch_lines(a.slot_order, list_first * 8, (list_end < entries ? list_end : entries) * 8, nth, a.touch_waves);
+            if (a.weights != nullptr) {
+                const uint64_t weights_first = static_cast<uint64_t>(segment) * a.window_weights;
+                const uint64_t weights_end = weights_first + a.window_weights;
+                touch_lines(a.weights, weights_first * 4, (weights_end < a.source_limit ? weights_end : a.source_limit) * 4,
+                            a.touch_waves - 1 - nth, a.touch_waves);
+            }
         }
-        const uint64_t first = window_first + static_cast<uint64_t>(within * waves + wave) * (kPrefetchLoads * kWave);
+        const uint64_t first = window_first + static_cast<uint64_t>(nth) * (kPrefetchLoads * kWave);
         if (first < window_end) {
             u32x4 fetched[kPrefetchLoads];
 #pragma unroll
@@ -736,6 +742,11 @@ int nanoep_dispatch(const void* x, const float* weights, const int32_t* recv_met
         a.window_vectors = static_cast<uint32_t>(static_cast<int64_t>(window_tokens) * vectors);
         a.source_vectors = static_cast<uint32_t>(num_tokens * vectors);
         a.window_weights = static_cast<uint32_t>(static_cast<int64_t>(window_tokens) * num_topk);
+        // (a 64-byte line a lane: 8 list entries or 16 weights)
+        const int64_t touch_waves = (segment_entries + 8 * kWave - 1) / (8 * kWave) + 1 +
+                                    (weights == nullptr ? 0 : (a.window_weights + 16 * kWave - 1) / (16 * kWave));
+        const int64_t prefetch_waves = segment_prefetch_blocks * waves;
+        a.touch_waves = static_cast<uint32_t>(touch_waves < prefetch_waves ? touch_waves : prefetch_waves);
         a.segment_entries = static_cast<uint32_t>(segment_entries);
         a.windows = static_cast<uint32_t>(windows);
         a.windows_magic = windows_divisor.magic;

@@ -697,7 +697,7 @@ class PeerRuntime {
 //
 // A caller that is on the communication stream itself most likely waits there, and gets an event: on one
 // queue that is no work for the GPU, where the store of a StreamPoint stands between the kernels (8192 x 2048
-// top-8, alignment 128, launch period: event 52.9 us a dispatch and 50.3 a combine, store 59.4 and 55.2).
+// top-8, alignment 128, launch period: event 55.2 us a dispatch and 50.5 a combine, store 59.4 and 55.2).
 class CompletionEvent {
    public:
     static std::shared_ptr<CompletionEvent> record_behind(const Stream& producer, const Stream& caller,
