@@ -991,6 +991,8 @@ DispatchResult dispatch(PeerRuntime& runtime,
     const bool callers_pool = !async_op || previous_event == -1;
     const c10::Device here = x.device();
     torch::Tensor out_x, out_indices, out_weights;
+    // early outputs that gave way to exact ones: the kernel that writes them may still be running
+    std::vector<torch::Tensor> replaced;
     // x_rows rows of payload (and expanded weights), n_rows rows of compact indices / weights
     const auto allocate_outputs = [&](int64_t x_rows, int64_t n_rows) {
         const StreamSwitch pool(callers_pool ? compute : comm, comm);
@@ -1226,6 +1228,8 @@ DispatchResult dispatch(PeerRuntime& runtime,
             if (weights.has_value())
                 out_weights = expand ? part_of(out_weights, 0, {used_rows}, torch::kFloat32) : part_of(out_weights, 0, {recv_count, topk}, torch::kFloat32);
         } else {
+            if (speculative)
+                replaced = {out_x, out_indices, out_weights};
             allocate_outputs(used_rows, recv_count);
             if (recv_count > 0)
                 launch_permute(view_of(metadata), recv_count, expanded_capacity);
@@ -1251,6 +1255,7 @@ DispatchResult dispatch(PeerRuntime& runtime,
             read.push_back(indices);
         if (weights.has_value())
             read.push_back(*weights);
+        read.insert(read.end(), replaced.begin(), replaced.end());  // (in use for as long as what is read)
         std::vector<torch::Tensor> written{out_x, out_indices, out_weights};
         if (!cached)
             written.push_back(metadata[1]);  // the handle's tensors share one allocation

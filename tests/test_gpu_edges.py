@@ -167,6 +167,38 @@ def test_a_dropped_completion_event_protects_the_calls_memory(device, explicit_e
         del poison
 
 
+# Early outputs that do not fit what routing filled are replaced by exact ones while the kernel that writes them may
+# still be running: an asynchronous call holds them until it has been waited for, and what the caller
+# allocates and fills before that stays as it was filled.  `first` makes the forecast that the second batch misses.
+@pytest.mark.parametrize(
+    "tokens,hidden,experts,topk,expand,alignment,first",
+    [(4096, 4096, 16, 4, True, 1, None), (8192, 4096, 16, 1, False, 1, None), (2048, 4096, 64, 4, True, 128, "random")],
+)
+def test_replaced_early_outputs_stay_the_calls_until_it_is_waited_for(device, tokens, hidden, experts, topk, expand, alignment, first):
+    x, w = cases.payload(tokens, hidden, seed=3), cases.gate_weights(tokens, topk, seed=3)
+    idx = cases.routing("sparse", tokens, experts, topk, seed=3)
+    x_dev, idx_dev, w_dev = x.to(device), idx.to(device), w.to(device)
+    with Buffer(None, EPConfig(experts, topk, hidden, tokens)) as buffer:
+        early_rows = tokens * topk if expand else tokens
+        if first is not None:
+            seen = buffer.dispatch(x_dev, topk_idx=cases.routing(first, tokens, experts, topk, seed=4).to(device), weights=w_dev,
+                                   do_expand=expand, alignment=alignment).handle.layout.expanded_capacity
+            early_rows = seen + (seen + 7) // 8
+        torch.cuda.synchronize()
+        before = torch.cuda.memory_allocated()
+        received = buffer.dispatch(x_dev, topk_idx=idx_dev, weights=w_dev, do_expand=expand, alignment=alignment, async_op=True)
+        held = torch.cuda.memory_allocated() - before
+        mine = [torch.full((early_rows, hidden), -77.0, dtype=torch.bfloat16, device=device) for _ in range(2)]
+        assert received.x.shape[0] * 5 < early_rows * 4
+        early_bytes = early_rows * hidden * 2
+        assert held >= early_bytes + received.x.numel() * 2
+        received.event.current_stream_wait()
+        assert torch.cuda.memory_allocated() - before < held + early_bytes * 2  # given back: `mine` is the two besides
+        assert_dispatch_result(received, x, idx, w, experts, expand, alignment, False)
+        for tensor in mine:
+            assert bool((tensor == -77.0).all())
+
+
 # Waiting inside a graph's capture for a call made outside it comes to what the runtime makes of a plain event
 # behind the same work, and does not depend on how the call's completion is kept.
 @pytest.mark.parametrize("finished", [False, True])
