@@ -693,25 +693,50 @@ class PeerRuntime {
 // kernels use it on a stream its allocator does not know of; waiting tells the allocator of the
 // consumer's stream instead, which costs nothing for tensors that were allocated there (telling it of the
 // communication stream makes it record an event for every block when it is freed).  A marker that goes
-// away with nobody having waited tells it of the communication stream after all.
+// away with nobody having waited tells it of the communication stream after all.  It is made before
+// the call enqueues anything, so that this also covers a call that ends in an error half way: bad routing
+// ids are known while the layout and the permute behind it are still at work.  A synchronous call with a
+// compute-unit budget has a marker for that alone.
 //
 // A caller that is on the communication stream itself most likely waits there, and gets an event: on one
 // queue that is no work for the GPU, where the store of a StreamPoint stands between the kernels (8192 x 2048
 // top-8, alignment 128, launch period: event 55.2 us a dispatch and 50.5 a combine, store 59.4 and 55.2).
 class CompletionEvent {
    public:
-    static std::shared_ptr<CompletionEvent> record_behind(const Stream& producer, const Stream& caller,
-                                                          std::vector<torch::Tensor> written, std::vector<torch::Tensor> read) {
-        auto marker = std::make_shared<CompletionEvent>();
-        marker->written_ = std::move(written);
-        marker->read_ = std::move(read);
-        marker->producer_ = producer;
-        if (producer.stream() != caller.stream() && !capturing(producer))
-            marker->point_ = StreamPoints::of(producer.device_index()).record(producer);
-        if (!marker->point_.has_value())
-            marker->done_.record(producer.unwrap());
-        return marker;
+    explicit CompletionEvent(const Stream& producer) : done_(c10::DeviceType::CUDA), producer_(producer) {}
+    CompletionEvent(const CompletionEvent&) = delete;
+    CompletionEvent& operator=(const CompletionEvent&) = delete;
+    ~CompletionEvent() {
+        if (settled_)
+            return;
+        try {
+            note_use(written_, producer_);
+            note_use(read_, producer_);
+        } catch (...) {
+        }
     }
+
+    // What the call's kernels read, and what they write: held from before they are enqueued.
+    void reads(const torch::Tensor& tensor) { read_.push_back(tensor); }
+    void reads(const std::vector<torch::Tensor>& tensors) { read_.insert(read_.end(), tensors.begin(), tensors.end()); }
+    void writes(const torch::Tensor& tensor) { written_.push_back(tensor); }
+
+    // What was written so far is no result after all: in use for as long as what is read.
+    void discard_written() {
+        reads(written_);
+        written_.clear();
+    }
+
+    // The call is complete: the marker goes behind all that its stream holds now.
+    void record(const Stream& caller) {
+        if (producer_.stream() != caller.stream() && !capturing(producer_))
+            point_ = StreamPoints::of(producer_.device_index()).record(producer_);
+        if (!point_.has_value())
+            done_.record(producer_.unwrap());
+    }
+
+    // The caller's stream has come behind the work without this marker: the tensors need nobody any more.
+    void settle() { settled_ = true; }
 
     void order_after(const Stream& consumer) {
         std::lock_guard<std::mutex> lock(mutex_);
@@ -721,29 +746,16 @@ class CompletionEvent {
         } else {
             // A consumer under capture is told of an event, and the runtime says what it makes of that.
             if (point_.has_value())
-                done_.record(producer_->unwrap());
+                done_.record(producer_.unwrap());
             consumer.unwrap().wait(done_);
         }
         note_use(written_, consumer);
         note_use(read_, consumer);
         read_.clear();
-        waited_ = true;
+        settled_ = true;
     }
 
     void current_stream_wait() { order_after(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA()); }
-
-    CompletionEvent() : done_(c10::DeviceType::CUDA) {}
-    CompletionEvent(const CompletionEvent&) = delete;
-    CompletionEvent& operator=(const CompletionEvent&) = delete;
-    ~CompletionEvent() {
-        if (waited_ || !producer_.has_value())
-            return;
-        try {
-            note_use(written_, *producer_);
-            note_use(read_, *producer_);
-        } catch (...) {
-        }
-    }
 
    private:
     static void note_use(const std::vector<torch::Tensor>& tensors, const Stream& stream) {
@@ -755,8 +767,8 @@ class CompletionEvent {
     std::mutex mutex_;
     std::optional<StreamPoint> point_;
     c10::Event done_;  // where there is no point, or a consumer under capture
-    std::optional<Stream> producer_;
-    bool waited_ = false;
+    Stream producer_;
+    bool settled_ = false;  // somebody has waited, or nobody needs to
     std::vector<torch::Tensor> written_, read_;
 };
 
@@ -983,6 +995,17 @@ DispatchResult dispatch(PeerRuntime& runtime,
     order_comm_after_inputs(comm, compute, previous_event, async_op);
 
     const StreamSwitch on_comm(comm, compute);
+    // Answers for what the call uses on a stream that the memory's owner may not know of.
+    const auto marker = async_op || !same_queue(comm, compute) ? std::make_shared<CompletionEvent>(comm) : nullptr;
+    if (marker) {
+        marker->reads(x);
+        if (cached)
+            marker->reads(cached_metadata);
+        else
+            marker->reads(indices);
+        if (weights.has_value())
+            marker->reads(*weights);
+    }
     // Results are allocated on the caller's stream: the work is ordered behind what that stream held
     // when the call was made, and what it does with the results comes behind the call (a synchronous one) or
     // behind the completion event, which holds them until somebody has waited.  An asynchronous call with
@@ -991,8 +1014,6 @@ DispatchResult dispatch(PeerRuntime& runtime,
     const bool callers_pool = !async_op || previous_event == -1;
     const c10::Device here = x.device();
     torch::Tensor out_x, out_indices, out_weights;
-    // early outputs that gave way to exact ones: the kernel that writes them may still be running
-    std::vector<torch::Tensor> replaced;
     // x_rows rows of payload (and expanded weights), n_rows rows of compact indices / weights
     const auto allocate_outputs = [&](int64_t x_rows, int64_t n_rows) {
         const StreamSwitch pool(callers_pool ? compute : comm, comm);
@@ -1001,6 +1022,9 @@ DispatchResult dispatch(PeerRuntime& runtime,
             out_indices = new_tensor({n_rows, topk}, torch::kInt64, here);
         if (weights.has_value())
             out_weights = expand ? new_tensor({x_rows}, torch::kFloat32, here) : new_tensor({n_rows, topk}, torch::kFloat32, here);
+        if (marker)
+            for (const auto* tensor : {&out_x, &out_indices, &out_weights})
+                marker->writes(*tensor);
     };
     // What the permute reads of a handle, as plain pointers.  order_entries: A, or -1 for "the whole
     // slot-order buffer is there and the kernel finds A in its last word".
@@ -1113,6 +1137,8 @@ DispatchResult dispatch(PeerRuntime& runtime,
             const StreamSwitch pool(callers_pool ? compute : comm, comm);
             arena = new_tensor({count64 + (count32 + 1) / 2}, torch::kInt64, here);
         }
+        if (marker)
+            marker->writes(arena);
         // int64: expert_counts [L] | expert_offsets [L+1] | send_counts [1] | recv_rank_prefix [1] |
         //        dst_slots [T] | topk snapshot [T*K] | slot_order;   int32: recv_metadata [T*(K+2)] | token_slots [T*K]
         int64_t* base64 = arena.data_ptr<int64_t>();
@@ -1228,8 +1254,11 @@ DispatchResult dispatch(PeerRuntime& runtime,
             if (weights.has_value())
                 out_weights = expand ? part_of(out_weights, 0, {used_rows}, torch::kFloat32) : part_of(out_weights, 0, {recv_count, topk}, torch::kFloat32);
         } else {
-            if (speculative)
-                replaced = {out_x, out_indices, out_weights};
+            // the kernel that writes early outputs that gave way to exact ones may still be running
+            if (speculative && marker) {
+                marker->discard_written();
+                marker->writes(arena);
+            }
             allocate_outputs(used_rows, recv_count);
             if (recv_count > 0)
                 launch_permute(view_of(metadata), recv_count, expanded_capacity);
@@ -1246,24 +1275,14 @@ DispatchResult dispatch(PeerRuntime& runtime,
     if (!weights.has_value())
         out_weights = new_tensor({0}, torch::kFloat32, here);
     std::vector<torch::Tensor> outputs{out_x, out_indices, out_weights};
-    std::shared_ptr<CompletionEvent> event;
     if (async_op) {
-        std::vector<torch::Tensor> read{x};
-        if (cached)
-            read.insert(read.end(), cached_metadata.begin(), cached_metadata.end());
-        else
-            read.push_back(indices);
-        if (weights.has_value())
-            read.push_back(*weights);
-        read.insert(read.end(), replaced.begin(), replaced.end());  // (in use for as long as what is read)
-        std::vector<torch::Tensor> written{out_x, out_indices, out_weights};
-        if (!cached)
-            written.push_back(metadata[1]);  // the handle's tensors share one allocation
-        event = CompletionEvent::record_behind(comm, compute, std::move(written), std::move(read));
-    } else if (!same_queue(comm, compute)) {
+        marker->record(compute);
+    } else if (marker) {
         wait_on(compute, comm);
+        marker->settle();
     }
-    return std::make_tuple(std::move(outputs), std::move(metadata), std::array<int64_t, 2>{recv_count, expanded_capacity}, std::move(event));
+    return std::make_tuple(std::move(outputs), std::move(metadata), std::array<int64_t, 2>{recv_count, expanded_capacity},
+                           async_op ? marker : nullptr);
 }
 
 using CombineResult = std::tuple<std::vector<torch::Tensor>, std::shared_ptr<CompletionEvent>>;
@@ -1316,6 +1335,16 @@ CombineResult combine(PeerRuntime& runtime,
     const auto comm = work_stream(comm_stream, compute, device, async_op, cu_budget != 0);
     order_comm_after_inputs(comm, compute, previous_event, async_op);
     const StreamSwitch on_comm(comm, compute);
+    // (as in dispatch)
+    const auto marker = async_op || !same_queue(comm, compute) ? std::make_shared<CompletionEvent>(comm) : nullptr;
+    if (marker) {
+        marker->reads(metadata);
+        marker->reads(x);
+        if (weights.has_value())
+            marker->reads(*weights);
+        if (bias.has_value())
+            marker->reads(*bias);
+    }
 
     torch::Tensor combined_x, combined_weights;
     {
@@ -1324,6 +1353,10 @@ CombineResult combine(PeerRuntime& runtime,
         combined_x = new_tensor({source_tokens, hidden}, torch::kBFloat16, here);
         if (weights.has_value())
             combined_weights = new_tensor({source_tokens, topk}, torch::kFloat32, here);
+        if (marker) {
+            marker->writes(combined_x);
+            marker->writes(combined_weights);
+        }
     }
     if (source_tokens > 0) {
         // a seven-tensor handle of the latest fresh dispatch gets its slot table back from the runtime
@@ -1358,19 +1391,13 @@ CombineResult combine(PeerRuntime& runtime,
     if (!weights.has_value())
         combined_weights = new_tensor({0}, torch::kFloat32, here);
     std::vector<torch::Tensor> outputs{combined_x, combined_weights};
-    std::shared_ptr<CompletionEvent> event;
     if (async_op) {
-        std::vector<torch::Tensor> read(metadata);
-        read.push_back(x);
-        if (weights.has_value())
-            read.push_back(*weights);
-        if (bias.has_value())
-            read.push_back(*bias);
-        event = CompletionEvent::record_behind(comm, compute, outputs, std::move(read));
-    } else if (!same_queue(comm, compute)) {
+        marker->record(compute);
+    } else if (marker) {
         wait_on(compute, comm);
+        marker->settle();
     }
-    return std::make_tuple(std::move(outputs), std::move(event));
+    return std::make_tuple(std::move(outputs), async_op ? marker : nullptr);
 }
 
 std::vector<int64_t> window_layout(int ranks, int64_t tokens, int hidden, int topk, int64_t num_experts, bool allow_multiple_reduction) {

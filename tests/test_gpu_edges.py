@@ -199,6 +199,41 @@ def test_replaced_early_outputs_stay_the_calls_until_it_is_waited_for(device, to
             assert bool((tensor == -77.0).all())
 
 
+def active_bytes():
+    """Memory the allocator gives to nobody: in use, or freed while a stream it was told of may still use it."""
+    return torch.cuda.memory_stats()["active_bytes.all.current"]
+
+
+# A fresh dispatch learns of bad routing ids while its layout and the permute behind it are at work on a stream that is
+# not the caller's: what they write goes back to the caller's allocator, but to nobody before they are done.
+@pytest.mark.parametrize("how", [{"async_op": True}, {"num_sms": 128}], ids=["asynchronous", "budget"])
+@pytest.mark.parametrize("expand", [True, False])
+def test_a_call_that_fails_leaves_its_memory_to_its_kernels(device, how, expand):
+    tokens, hidden, experts, topk = 4096, 4096, 16, 4
+    x, idx = cases.payload(tokens, hidden, seed=6), cases.routing("random", tokens, experts, topk, seed=6)
+    x_dev, idx_dev, bad_dev = x.to(device), idx.to(device), idx.to(device)
+    bad_dev[tokens // 2, 1] = experts
+    early_rows = tokens * topk if expand else tokens
+    with Buffer(None, EPConfig(experts, topk, hidden, tokens)) as buffer:
+        torch.cuda.synchronize()
+        before = active_bytes()
+        with pytest.raises(RuntimeError, match="out of range"):
+            buffer.dispatch(x_dev, topk_idx=bad_dev, do_expand=expand, **how)
+        assert active_bytes() - before >= early_rows * hidden * 2
+        mine = [torch.full((early_rows, hidden), -77.0, dtype=torch.bfloat16, device=device) for _ in range(2)]
+        torch.cuda.synchronize()
+        for tensor in mine:
+            assert bool((tensor == -77.0).all())
+        del mine, tensor
+        kept = torch.empty(1, device=device)  # (the allocator looks for what is done when it is asked for memory)
+        assert active_bytes() - before < early_rows * hidden * 2
+        received = buffer.dispatch(x_dev, topk_idx=idx_dev, do_expand=expand, **how)
+        if received.event is not None:
+            received.event.current_stream_wait()
+        assert_dispatch_result(received, x, idx, None, experts, expand, 1, False)
+        del kept
+
+
 # Waiting inside a graph's capture for a call made outside it comes to what the runtime makes of a plain event
 # behind the same work, and does not depend on how the call's completion is kept.
 @pytest.mark.parametrize("finished", [False, True])
