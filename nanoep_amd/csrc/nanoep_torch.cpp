@@ -256,8 +256,8 @@ class PeerRuntime {
     // One fresh dispatch's use of the mailbox, from before its layout is enqueued until the host has
     // read N and C (the reference's prepare_dispatch_counts / wait_dispatch_counts /
     // fail_dispatch_counts, csrc/peer.cu:187-232).  Fresh dispatches of other threads wait their
-    // turn at the constructor.  A turn that ends without `wait` having delivered the counts (a
-    // timeout, a HIP error, an exception in between) leaves the runtime failed for good: a word the
+    // turn at the constructor.  A turn that has begun and ends without `wait` having delivered the counts
+    // (a timeout, a HIP error, an exception in between) leaves the runtime failed for good: a word the
     // device stores late must never answer a later call.
     class CountsTurn {
        public:
@@ -275,6 +275,9 @@ class PeerRuntime {
         }
 
         int64_t* mailbox() const { return runtime_.host_counts_; }
+
+        // The layout is enqueued next: from here on the turn needs its counts.
+        void begin() { settled_ = false; }
 
         // Nothing was enqueued that could still write the mailbox: the turn ends without a verdict.
         void abandon() { settled_ = true; }
@@ -295,14 +298,17 @@ class PeerRuntime {
        private:
         PeerRuntime& runtime_;
         std::unique_lock<std::mutex> lock_;
-        bool settled_ = false;
+        bool settled_ = true;
     };
 
     bool counts_failed() const { return counts_failed_.load(); }
 
     // What a fresh dispatch whose counts never arrive leaves behind, without making a GPU misbehave:
     // a turn at the mailbox that ends with no verdict.  For tests of the failure latch.
-    void lose_counts_for_test() { CountsTurn lost(*this); }
+    void lose_counts_for_test() {
+        CountsTurn lost(*this);
+        lost.begin();
+    }
 
     // Whether fresh dispatches should allocate their outputs after the counts are known: set when a
     // call that allocated at the upper bound turned out to hold over 1.25 times what it used (many
@@ -992,8 +998,6 @@ DispatchResult dispatch(PeerRuntime& runtime,
 
     const auto compute = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(device);
     const auto comm = work_stream(comm_stream, compute, device, async_op, cu_budget != 0);
-    order_comm_after_inputs(comm, compute, previous_event, async_op);
-
     const StreamSwitch on_comm(comm, compute);
     // Answers for what the call uses on a stream that the memory's owner may not know of.
     const auto marker = async_op || !same_queue(comm, compute) ? std::make_shared<CompletionEvent>(comm) : nullptr;
@@ -1006,12 +1010,17 @@ DispatchResult dispatch(PeerRuntime& runtime,
         if (weights.has_value())
             marker->reads(*weights);
     }
-    // Results are allocated on the caller's stream: the work is ordered behind what that stream held
-    // when the call was made, and what it does with the results comes behind the call (a synchronous one) or
+    // Results are allocated on the caller's stream: the work is ordered behind what that stream holds
+    // then, and what it does with the results comes behind the call (a synchronous one) or
     // behind the completion event, which holds them until somebody has waited.  An asynchronous call with
     // an event of its own is ordered behind that event only: its results come from the communication
     // stream's pool.
+    //
+    // The caller's stream may be other threads' as well: a block of its pool may have been freed a moment ago, with the
+    // kernels that used it still to run.  So the communication stream comes behind the caller's
+    // after the allocation, never before it; one that has to be made later is followed by a wait of its own.
     const bool callers_pool = !async_op || previous_event == -1;
+    const bool borrows = callers_pool && !same_queue(comm, compute);
     const c10::Device here = x.device();
     torch::Tensor out_x, out_indices, out_weights;
     // x_rows rows of payload (and expanded weights), n_rows rows of compact indices / weights
@@ -1077,6 +1086,7 @@ DispatchResult dispatch(PeerRuntime& runtime,
         TORCH_CHECK(!expand || expanded_capacity <= std::numeric_limits<int32_t>::max(),
                     "expanded capacity exceeds int32 metadata range");
         allocate_outputs(expand ? expanded_capacity : recv_count, recv_count);
+        order_comm_after_inputs(comm, compute, previous_event, async_op);
         // A handle that went through the reference's Python class carries the seven tensors of the
         // reference only.  If it is one of this runtime's latest fresh dispatches, the runtime still
         // has its private tensors and the payload takes the slot-order walk
@@ -1110,8 +1120,6 @@ DispatchResult dispatch(PeerRuntime& runtime,
             launch_permute(view, recv_count, expanded_capacity, /*count_on_device=*/rebuilt && view.order_entries < 0);
         }
     } else {
-        TORCH_CHECK(!capturing(comm), "Fresh dispatch with host count polling cannot be captured in a HIP graph");
-
         // the slot-order list packs token * K + k into 32 bits
         const bool ordered = expand && tokens * topk < (int64_t{1} << 31);
         // The handle tensors of one call are views of one allocation (the int64 ones, then the int32 ones), and the
@@ -1147,15 +1155,6 @@ DispatchResult dispatch(PeerRuntime& runtime,
         // From here until the counts have been read this call owns the runtime's mailbox; a fresh
         // dispatch of another thread on the same runtime waits here for its turn.
         PeerRuntime::CountsTurn turn(runtime);
-        const auto workspace = runtime.layout_workspace(workspace_bytes, comm.stream(), here);
-        const int layout_status =
-            nanoep_layout(routing.data_ptr<int64_t>(), tokens, static_cast<int>(topk), local_experts, alignment, expand ? 1 : 0,
-                          static_cast<int>(hidden), base32, base64, base64 + at_offsets, base64 + at_dst, base64 + at_send, base64 + at_snapshot,
-                          base64 + at_prefix, expand ? base32 + at_table : nullptr, order_entries > 0 ? base64 + at_order : nullptr,
-                          workspace.data_ptr(), workspace_bytes, turn.mailbox(), comm.stream());
-        if (layout_status != NANOEP_OK && layout_status != NANOEP_ERR_HIP)
-            turn.abandon();  // refused before anything was enqueued
-        check_status(layout_status, "layout");
 
         // The exact shapes (N, C) are only known once the layout kernels have run.  Waiting for
         // them before launching the permute leaves the GPU idle for a host round trip, so where the
@@ -1184,6 +1183,22 @@ DispatchResult dispatch(PeerRuntime& runtime,
                 early_rows = std::min(row_bound, runtime.forecast_rows(geometry));
         }
         const bool speculative = early_rows > 0;
+        if (speculative && borrows)
+            allocate_outputs(early_rows, tokens);
+        order_comm_after_inputs(comm, compute, previous_event, async_op);
+        TORCH_CHECK(!capturing(comm), "Fresh dispatch with host count polling cannot be captured in a HIP graph");
+
+        const auto workspace = runtime.layout_workspace(workspace_bytes, comm.stream(), here);
+        turn.begin();
+        const int layout_status =
+            nanoep_layout(routing.data_ptr<int64_t>(), tokens, static_cast<int>(topk), local_experts, alignment, expand ? 1 : 0,
+                          static_cast<int>(hidden), base32, base64, base64 + at_offsets, base64 + at_dst, base64 + at_send, base64 + at_snapshot,
+                          base64 + at_prefix, expand ? base32 + at_table : nullptr, order_entries > 0 ? base64 + at_order : nullptr,
+                          workspace.data_ptr(), workspace_bytes, turn.mailbox(), comm.stream());
+        if (layout_status != NANOEP_OK && layout_status != NANOEP_ERR_HIP)
+            turn.abandon();  // refused before anything was enqueued
+        check_status(layout_status, "layout");
+
         if (speculative) {
             // enqueued straight from the arena's pointers: the tensors of the handle are made below,
             // while the GPU works
@@ -1196,7 +1211,8 @@ DispatchResult dispatch(PeerRuntime& runtime,
             fresh.expert_counts = base64;
             fresh.expert_offsets = base64 + at_offsets;
             try {
-                allocate_outputs(early_rows, tokens);
+                if (!borrows)
+                    allocate_outputs(early_rows, tokens);
                 launch_permute(fresh, tokens, early_rows, /*count_on_device=*/true);
             } catch (...) {
                 // The layout is under way and will publish its counts whatever went wrong here (most
@@ -1260,8 +1276,11 @@ DispatchResult dispatch(PeerRuntime& runtime,
                 marker->writes(arena);
             }
             allocate_outputs(used_rows, recv_count);
-            if (recv_count > 0)
+            if (recv_count > 0) {
+                if (borrows)
+                    wait_on(comm, compute);
                 launch_permute(view_of(metadata), recv_count, expanded_capacity);
+            }
         }
         if (tokens > 0 && bound_rule)
             runtime.note_output_fill(bound_is_close);
@@ -1333,7 +1352,6 @@ CombineResult combine(PeerRuntime& runtime,
 
     const auto compute = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(device);
     const auto comm = work_stream(comm_stream, compute, device, async_op, cu_budget != 0);
-    order_comm_after_inputs(comm, compute, previous_event, async_op);
     const StreamSwitch on_comm(comm, compute);
     // (as in dispatch)
     const auto marker = async_op || !same_queue(comm, compute) ? std::make_shared<CompletionEvent>(comm) : nullptr;
@@ -1348,7 +1366,8 @@ CombineResult combine(PeerRuntime& runtime,
 
     torch::Tensor combined_x, combined_weights;
     {
-        // (as in dispatch: the caller's pool, unless the call is ordered behind an event of its own only)
+        // (as in dispatch: the caller's pool, unless the call is ordered behind an event of its own only, and
+        // the order made behind the allocation)
         const StreamSwitch pool(!async_op || previous_event == -1 ? compute : comm, comm);
         combined_x = new_tensor({source_tokens, hidden}, torch::kBFloat16, here);
         if (weights.has_value())
@@ -1358,6 +1377,7 @@ CombineResult combine(PeerRuntime& runtime,
             marker->writes(combined_weights);
         }
     }
+    order_comm_after_inputs(comm, compute, previous_event, async_op);
     if (source_tokens > 0) {
         // a seven-tensor handle of the latest fresh dispatch gets its slot table back from the runtime
         std::vector<torch::Tensor> handle;

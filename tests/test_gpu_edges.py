@@ -1,5 +1,8 @@
 """GPU tests at the edges of single kernel paths, against the CPU oracle (bit for bit)."""
 
+import time
+from concurrent.futures import ThreadPoolExecutor
+
 import pytest
 import torch
 
@@ -232,6 +235,63 @@ def test_a_call_that_fails_leaves_its_memory_to_its_kernels(device, how, expand)
             received.event.current_stream_wait()
         assert_dispatch_result(received, x, idx, None, experts, expand, 1, False)
         del kept
+
+
+@pytest.fixture(scope="module")
+def spin(device):
+    """spin(milliseconds): keeps the current stream busy for about that long."""
+    start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    torch.cuda._sleep(100_000)
+    start.record()
+    torch.cuda._sleep(1_000_000)
+    end.record()
+    end.synchronize()
+    cycles = 1_000_000 / start.elapsed_time(end)
+    return lambda milliseconds: torch.cuda._sleep(int(cycles * milliseconds))
+
+
+# A block of the caller's pool that another thread on the caller's stream has freed, with its kernels still to run, becomes an
+# asynchronous call's result while that call is on its way: waiting for its turn behind another fresh dispatch
+# (outputs made ahead of the counts), or for its counts (outputs made behind them).
+@pytest.mark.parametrize("outputs", ["early", "exact"])
+def test_results_come_behind_whoever_had_their_memory_last(device, spin, outputs):
+    tokens, hidden, experts, topk = 2048, 4096, 16, 4
+    idx = cases.routing("random" if outputs == "early" else "sparse", tokens, experts, topk, seed=14)
+    x = cases.payload(tokens, hidden, seed=14)
+    x_dev, idx_dev = x.to(device), idx.to(device)
+    rows = tokens * topk if outputs == "early" else oracle.layout(idx, experts, 1).expanded_capacity
+    mine, others = torch.cuda.Stream(), torch.cuda.Stream()
+
+    def dispatch(stream, busy, **how):
+        with torch.cuda.stream(stream):
+            spin(busy)
+            return buffer.dispatch(x_dev, topk_idx=idx_dev, do_expand=True, **how)
+
+    with Buffer(None, EPConfig(experts, topk, hidden, tokens)) as buffer, ThreadPoolExecutor(2) as threads:
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+        if outputs == "early":
+            first = threads.submit(dispatch, others, 600)  # has the runtime's mailbox until its counts are there
+            time.sleep(0.1)
+        else:
+            with torch.cuda.stream(buffer.comm_stream):
+                spin(600)
+        call = threads.submit(dispatch, mine, 0, async_op=True)
+        time.sleep(0.2)
+        with torch.cuda.stream(mine):
+            had = torch.empty((rows, hidden), dtype=torch.bfloat16, device=device)
+            where = had.data_ptr()
+            spin(1000)
+            had.fill_(-77.0)
+            del had
+        received = call.result(timeout=60)
+        assert received.x.data_ptr() == where  # (else this looks at nothing)
+        with torch.cuda.stream(mine):
+            received.event.current_stream_wait()
+        torch.cuda.synchronize()
+        assert_dispatch_result(received, x, idx, None, experts, True, 1, False)
+        if outputs == "early":
+            assert_dispatch_result(first.result(timeout=60), x, idx, None, experts, True, 1, False)
 
 
 # Waiting inside a graph's capture for a call made outside it comes to what the runtime makes of a plain event
