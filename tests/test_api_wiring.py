@@ -194,6 +194,19 @@ def test_a_compute_unit_budget_picks_the_stream_and_keeps_the_calls_in_order(con
     assert buffer.budget_stream(64) is buffer._budget_streams[64]
 
 
+@pytest.mark.parametrize("asynchronous", [False, True])
+def test_only_a_whole_device_call_goes_without_the_communication_stream(context, asynchronous):
+    """A buffer's first call: a synchronous one on the whole device has nothing to come behind and is handed no
+    stream; one with a compute-unit budget runs on the communication stream where the runtime has none for it."""
+    buffer, x = context.buffer, FakeTensor("x", torch.zeros((2, 256), dtype=torch.bfloat16))
+    buffer._comm_quiet = True
+    buffer.dispatch(x, topk_idx=context.indices, async_op=asynchronous)
+    assert context.calls[-1].args[13] == (11 if asynchronous else -1)
+    buffer._comm_quiet = True
+    buffer.dispatch(x, topk_idx=context.indices, num_sms=24, async_op=asynchronous)
+    assert context.calls[-1].args[13] == 11 and not buffer._comm_quiet
+
+
 def test_dispatch_argument_rules(context):
     buffer = context.buffer
     x = context.tensor("x", torch.zeros((2, 256), dtype=torch.bfloat16))
