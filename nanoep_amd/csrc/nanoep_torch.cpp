@@ -546,6 +546,7 @@ class PeerRuntime {
     // That confines the budget to steps of P (32 of 256 on an MI355X), rounded down, at least one step.
     int64_t budget_stream(int cus) {
         TORCH_CHECK(!closed_.load(), "PeerRuntime is closed");
+        DeviceGuard guard(static_cast<c10::DeviceIndex>(device_));  // (the topology is the current device's)
         int device_cus = 0, xcds = 0;
         check_status(nanoep_device_topology(&device_cus, &xcds, nullptr), "device_topology");
         if (cus <= 0 || cus >= device_cus || xcds <= 1 || device_cus % xcds != 0 || (device_cus / xcds) % xcds != 0)
@@ -566,7 +567,6 @@ class PeerRuntime {
             if ((a + c) % xcds < steps)
                 mask[bit / 32] |= 1u << (bit % 32);
         }
-        DeviceGuard guard(static_cast<c10::DeviceIndex>(device_));
         hipStream_t stream = nullptr;
         check_hip(hipExtStreamCreateWithCUMask(&stream, static_cast<uint32_t>(mask.size()), mask.data()), "hipExtStreamCreateWithCUMask");
         streams.emplace_back(device_, steps, stream);
@@ -575,6 +575,7 @@ class PeerRuntime {
 
     // compute units a budget stream's kernels can run on (what budget_stream rounds `cus` to)
     int budget_stream_cus(int cus) const {
+        DeviceGuard guard(static_cast<c10::DeviceIndex>(device_));
         int device_cus = 0, xcds = 0;
         check_status(nanoep_device_topology(&device_cus, &xcds, nullptr), "device_topology");
         if (cus <= 0 || cus >= device_cus || xcds <= 1 || device_cus % xcds != 0 || (device_cus / xcds) % xcds != 0)
