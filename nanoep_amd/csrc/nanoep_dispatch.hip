@@ -188,7 +188,8 @@ struct WalkArgs {
     uint32_t window_vectors;        // 16-byte vectors of one window's source rows
     uint32_t source_vectors;        // ... of all source rows
     uint32_t window_weights;        // (token, k) pairs of one window
-    uint32_t touch_waves;           // wavefronts of a segment that bring in its list share and weights
+    uint32_t touch_waves;           // wavefronts of a segment that bring in a list share and the window's weights
+    uint32_t touch_distance;        // segments from this one to the one whose list share that is (less than windows)
     uint32_t rows_magic;  // fast divisor by rows_per_block
     uint32_t rows_shift;
     // gap rows
@@ -237,15 +238,24 @@ __device__ __forceinline__ void walk_gap_rows(const WalkArgs& a, uint32_t xcd, u
 // pushed a row out again before its last use: a window close to the size of the L2 re-reads part of
 // itself).  What it costs otherwise is one more L2 read per source row.
 //
-// The segment's share of the list and the window's weights come in the same way: a copy wavefront's
+// A share of the list and the window's weights come in the same way: a copy wavefront's
 // life is a chain (list entry, source row, store), and a handle that is replayed long after it was made
 // (a backward pass behind the other layers') has both in HBM only.  Handle in HBM, without -> with:
-// 32768 x 1024 top-8 129.4 -> 95.0 us, 4096 x 7168 top-8 with alignment 128 128.1 -> 97.1 us; behind a
-// layout that has just written the list 81.9 -> 78.6 us (4096 x 7168, count on the device).  One word a
+// 32768 x 1024 top-8 128.2 -> 93.5 us, 4096 x 7168 top-8 with alignment 128 122.9 -> 90.6 us.  One word a
 // 64-byte line is read, so 256 tokens x 8 choices are four wavefronts' loads for the list and two for the
-// weights, and the other prefetch wavefronts leave that aside with one comparison (with all of them taking
-// part 4096 x 7168 top-8 through a handle still in the caches took 75.5 us instead of 74.6; with the
-// rows' loads ahead of these 76.1).  Reading the next segment's share too changed nothing (within 0.3 %).
+// weights, and the other prefetch wavefronts leave that aside with one comparison.  Reading the next
+// segment's share too changed nothing (within 0.3 %).
+//
+// Whose share: with its list in the XCD's own L2 a copy wavefront asks for its source row sooner than
+// the prefetch has brought it, and where the handle comes from the last-level cache anyway (a replay
+// right behind the layout, the fresh dispatch itself) the walk loses by that what it never had to gain.  Rows of 1024 to 4096
+// elements with five and more of them a token lose most; there the share is that of the segment half a
+// walk away: the list comes from HBM to the last-level cache just the same, and into an L2 that does not use it.
+// Cold sources, handle in the caches (in HBM), no list at all / own share / that share: 8192 x 2048 top-8 with
+// alignment 128 47.3 / 48.9 / 46.7 us (60.2 / 49.2 / 47.2), 4096 x 2048 top-8 20.6 / 22.2 / 20.5 (22.1 / 22.1 / 20.5),
+// 8192 x 2816 top-6 46.1 / 49.3 / 45.8 (66.1 / 49.2 / 45.9), 4096 x 4096 top-8 44.8 / 45.4 / 44.5 (55.9 / 45.5 / 44.7).  Elsewhere the own
+// share is level or better: 65536 x 512 top-8 100.3 / 97.5 / 100.3 (141.6 / 98.9 / 101.7), 32768 x 1024 top-2 36.9 / 36.1 /
+// 36.7, 4096 x 7168 top-8 74.6 / 74.0 / 74.4, and with windows that XCDs share 3000 x 2816 top-8 27.5 / 26.8 / 27.8.
 constexpr int kPrefetchLoads = 4;
 
 // Reads one word of every 64-byte line of bytes [first, end) behind `base`: `wave` of `waves`
@@ -397,11 +407,14 @@ __device__ __forceinline__ void walk_copy(const WalkArgs& a, uint32_t entries, u
         uint64_t window_end = window_first + a.window_vectors;
         if (window_end > a.source_vectors)
             window_end = a.source_vectors;
-        // the segment's share of the list, the window's weights (from the last wavefront on, the list's
+        // a segment's share of the list, the window's weights (from the last wavefront on, the list's
         // lines are the first ones'), then the window's rows
         const uint32_t nth = within * waves + wave;
         if (nth < a.touch_waves) {
-            const uint64_t list_first = static_cast<uint64_t>(segment) * segment_entries;
+            uint32_t list_segment = segment + a.touch_distance;
+            if (list_segment >= a.windows)
+                list_segment -= a.windows;
+            const uint64_t list_first = static_cast<uint64_t>(list_segment) * segment_entries;
             const uint64_t list_end = list_first + segment_entries;
             touch_lines(a.slot_order, list_first * 8, (list_end < entries ? list_end : entries) * 8, nth, a.touch_waves);
             if (a.weights != nullptr) {
@@ -747,6 +760,10 @@ int nanoep_dispatch(const void* x, const float* weights, const int32_t* recv_met
                                     (weights == nullptr ? 0 : (a.window_weights + 16 * kWave - 1) / (16 * kWave));
         const int64_t prefetch_waves = segment_prefetch_blocks * waves;
         a.touch_waves = static_cast<uint32_t>(touch_waves < prefetch_waves ? touch_waves : prefetch_waves);
+        // Five choices a token and more, rows of 1024 to 4096 elements, whole windows an XCD: the list share of the
+        // segment half a walk away, which another XCD copies at the same time.
+        const bool touch_ahead_of_others = windows % xcds.count == 0 && num_topk > 4 && vectors >= 2 * kWave && vectors <= 8 * kWave;
+        a.touch_distance = touch_ahead_of_others ? static_cast<uint32_t>(windows / 2) : 0u;
         a.segment_entries = static_cast<uint32_t>(segment_entries);
         a.windows = static_cast<uint32_t>(windows);
         a.windows_magic = windows_divisor.magic;

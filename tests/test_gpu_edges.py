@@ -28,6 +28,18 @@ def test_list_and_weight_lines_of_ragged_windows(device, tokens, hidden, experts
     run_dispatch_combine(device, cases.routing(kind, tokens, experts, topk, seed=tokens), hidden, experts, 1, True, True, True)
 
 
+# Five choices a token and more, rows of 1024 to 4096 elements and whole windows an XCD: the prefetch workgroups touch the
+# list share of a segment half the walk away.  Shares that start inside a line, a last window cut short, lists far shorter
+# than their segments; one choice, one element step and one window beside the rule.
+@pytest.mark.parametrize(
+    "tokens,hidden,experts,topk,kind",
+    [(512, 1024, 9, 5, "dropout"), (511, 4096, 40, 8, "random"), (1000, 2816, 16, 6, "sparse"), (2048, 2048, 64, 32, "dropout"),
+     (512, 1024, 9, 4, "dropout"), (512, 768, 9, 5, "dropout"), (511, 4352, 9, 5, "dropout"), (513, 1024, 9, 5, "dropout")],
+)
+def test_list_lines_of_a_segment_half_the_walk_away(device, tokens, hidden, experts, topk, kind):
+    run_dispatch_combine(device, cases.routing(kind, tokens, experts, topk, seed=hidden), hidden, experts, 1, True, True, True)
+
+
 # The layout's three plans (1: every workgroup counts the batch, 2: histogram rows summed by every
 # workgroup, 3: histogram rows scanned by one) at the edges of its blocks, rows and wavefront chunks: batches one
 # token around a block, choices whose chunks leave lanes idle, experts around a strip of 64 and beyond the
