@@ -627,7 +627,10 @@ def measure(workload, args, device, detailed):
     if not workload.expand:
         combine_kernel = "combine_compact_kernel"
     else:
-        one_token = workload.topk <= 6 or workload.tokens * -(-workload.hidden // 512) <= 32 * torch.cuda.get_device_properties(0).multi_processor_count
+        # (nanoep_combine's rule)
+        chunks, topk = -(-workload.hidden // 512), workload.topk
+        waves = workload.tokens * chunks / torch.cuda.get_device_properties(0).multi_processor_count
+        one_token = topk <= 5 or (topk == 6 and (chunks > 4 or waves < 128)) or waves <= (32 if topk <= 12 else 20 if topk <= 16 else 12)
         combine_kernel = "combine_held_kernel" if not one_token else "combine_few_rows_kernel" if workload.topk <= 8 else "combine_rows_kernel"
     result.update(
         {

@@ -241,8 +241,8 @@ __global__ void __launch_bounds__(1024) combine_few_rows_kernel(const u32x4* __r
     }
 }
 
-// Expanded layout with the slot table at hand and seven or more rows a token, batches of more wavefronts than
-// the device holds with a token each: one wavefront (a
+// Expanded layout with the slot table at hand, six or more rows a token and more wavefronts than are better off with
+// a token each (the rule stands at the launch): one wavefront (a
 // workgroup of its own) produces the same 1 KiB chunk of the output rows of up to kUnits tokens
 // and holds the packed sums back in registers until the last one is done.  The units are
 // sized so that all wavefronts of the launch are resident at once wherever the batch allows it: the
@@ -547,11 +547,21 @@ int nanoep_combine(const void* y, const float* weights, const void* bias, const 
         return NANOEP_OK;
     }
     // With the slot table at hand, a wavefront takes one token's chunk (combine_few_rows_kernel up to eight rows a
-    // token) or holds the sums of 2 to 16 tokens back and writes them at its end (combine_held_kernel).
-    //  * One: up to 6 rows a token, and launches whose wavefronts are all resident with one token each (32 a
-    //    compute unit).  Held -> one token, rows in the caches: 128 x 4096 top-8 4.0 -> 3.0 us, 1024 x 1024 5.0 -> 4.0,
-    //    768 x 4096 10.1 -> 9.5, 1024 x 4096 (8192 wavefronts) 12.3 -> 12.4, 1024 x 7168 20.4 -> 21.0; top-6: 1537 x 2816 11.3 ->
-    //    10.2, 2048 x 2816 14.4 -> 12.9, 4096 x 2816 25.9 -> 26.1, 8192 x 2816 52.7 -> 51.4.
+    // token, combine_rows_kernel beyond) or holds the sums of 2 to 16 tokens back and writes them at its end
+    // (combine_held_kernel).  Held -> one token, rows from HBM (in the caches):
+    //  * One: up to 5 rows a token (16384 x 512 18.5 -> 16.4 us (17.2 -> 13.6), 4096 x 4096 36.9 -> 31.6 (36.1 -> 30.4),
+    //    4681 x 7168 66.5 -> 57.9), and 6, except the long launches of short rows below (2730 x 2816 18.4 -> 17.5 (16.9 -> 14.5), 10922 x
+    //    2816 69.0 -> 63.8, 4096 x 4096 34.6 -> 34.8, 8192 x 4096 66.4 -> 67.8, 4681 x 7168 71.1 -> 67.6).
+    //  * One: launches whose wavefronts are all resident with one token each (32 a compute unit), up to 12 rows:
+    //    128 x 4096 top-8 4.4 -> 4.1, 512 x 4096 8.1 -> 7.8 (5.3 -> 5.2), 2048 x 1024 8.1 -> 7.7 (6.0 -> 5.3), 1024 x 4096 12.7 -> 13.0
+    //    (10.4 -> 10.2), 1170 x 7168 13.2 -> 12.9 (11.1 -> 10.0); top-10 512 x 4096 10.6 -> 9.6 (8.4 -> 7.3), 1024 x 4096 17.2 -> 17.4
+    //    (15.5 -> 15.0); top-12 512 x 4096 11.0 -> 10.4 (8.9 -> 8.0), 1024 x 4096 18.1 -> 18.5 (16.5 -> 16.2).  So small a batch's rows
+    //    are in the last-level cache when their producer has just written them.  With more rows less than that
+    //    pays: 20 a compute unit up to 16 (640 x 4096 top-16 14.7 -> 14.8 (12.7 -> 11.8), 1024 x 4096 22.3 -> 23.2 (19.9 -> 20.4)), 12 beyond (384
+    //    x 4096 top-24 13.9 -> 14.0 (12.0 -> 11.8), 512 x 4096 16.7 -> 17.8 (14.9 -> 15.9); top-32 384 x 4096 17.2 -> 16.5 (15.3 -> 14.2),
+    //    640 x 4096 26.4 -> 26.5 (24.7 -> 23.8), 768 x 4096 30.5 -> 31.6 (28.2 -> 28.9)).
+    //  * Held: 6 rows of up to 2048 elements from 128 wavefronts a compute unit on: 16384 x 1024 35.8 -> 34.6 (35.2 -> 33.4), 65536 x 512
+    //    69.4 -> 66.4, 65536 x 1024 147.8 -> 138.5, 16384 x 2048 68.4 -> 67.1 (one -> held).
     //  * Held: as many tokens a wavefront as it takes for the launch to
     // fit what the device holds at once with the registers of sixteen held rows (16 wavefronts a
     // compute unit), or a whole multiple of that when sixteen tokens a wavefront are not enough: a
@@ -567,7 +577,9 @@ int nanoep_combine(const void* y, const float* weights, const void* bias, const 
     int64_t held_resident = 0, held_side = 0;
     const Topology topology = current_topology(tuning);
     const int64_t cus = num_cus > 0 ? num_cus : topology.cus;
-    const bool one_token = tuning.combine_units == 1 || (tuning.combine_units == 0 && (num_topk <= 6 || num_tokens * chunks <= cus * 32));
+    const int resident_with_one = num_topk <= 12 ? 32 : num_topk <= 16 ? 20 : 12;  // wavefronts a compute unit
+    const bool few_rows = num_topk <= 5 || (num_topk == 6 && (chunks > 4 || num_tokens * chunks < cus * 128));
+    const bool one_token = tuning.combine_units == 1 || (tuning.combine_units == 0 && (few_rows || num_tokens * chunks <= cus * resident_with_one));
     if (direct && num_topk > 4 && !one_token) {
         // (the wavefronts of sixteen held rows a compute unit holds, on the compute units this call may use)
         const int64_t resident = cus * topology.held_wavefronts[3];
@@ -610,6 +622,7 @@ int nanoep_combine(const void* y, const float* weights, const void* bias, const 
         strided ? 1u : static_cast<uint32_t>(held_units), strided ? static_cast<uint32_t>(held_groups) : 1u)
 #define NANOEP_LAUNCH_HELD_ROWS(UNITS)                     \
     switch (num_topk) {                                    \
+        case 6: NANOEP_LAUNCH_HELD(UNITS, 6); break;       \
         case 7: NANOEP_LAUNCH_HELD(UNITS, 7); break;       \
         case 8: NANOEP_LAUNCH_HELD(UNITS, 8); break;       \
         default: NANOEP_LAUNCH_HELD(UNITS, 0); break;      \

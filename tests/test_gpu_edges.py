@@ -403,3 +403,16 @@ def test_combine_around_the_batch_that_holds_sums_back(device, topk, tokens):
     out, _ = cabi.combine(y.to(device), None, None, metadata, counts, True, poison=0xA5)
     want, _ = oracle.combine(y, lay.recv_metadata(True), lay.dst_slots, do_expand=True)
     assert_same_bits(out, want, "combine")
+
+
+# The same for the other lines of that rule: six rows of up to 2048 elements, and more than eight rows a token.
+@pytest.mark.parametrize("tokens,hidden,topk", [(8191, 2048, 6), (8192, 2048, 6), (640, 4096, 16), (641, 4096, 16), (384, 4096, 17), (385, 4096, 17)])
+def test_combine_around_other_batches_that_hold_sums_back(device, tokens, hidden, topk):
+    idx = cases.routing("dropout", tokens, 32, topk, seed=topk)
+    metadata, counts = cabi.layout(idx.to(device), 32, 1, True, hidden=hidden)
+    lay = oracle.layout(idx, 32, 1)
+    y, w = cases.payload(counts[1], hidden, seed=topk), cases.gate_weights(counts[1], 1, seed=3).flatten()
+    out, out_w = cabi.combine(y.to(device), w.to(device), None, metadata, counts, True, poison=0xA5)
+    want, want_w = oracle.combine(y, lay.recv_metadata(True), lay.dst_slots, do_expand=True, weights=w)
+    assert_same_bits(out, want, "combine")
+    assert_same_bits(out_w, want_w, "weights")
