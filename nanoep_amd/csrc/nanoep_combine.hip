@@ -166,21 +166,18 @@ __global__ void __launch_bounds__(1024) combine_few_rows_kernel(const u32x4* __r
                                                                 uint32_t rows_per_block,    // == blockDim.z
                                                                 uint32_t vectors,
                                                                 uint32_t chunks,
-                                                                uint32_t topk,
                                                                 int flags,  // kCombineMultipleReduction | kCombineAgentStores
-                                                                uint32_t topk_magic,  // fast divisor by K
-                                                                uint32_t topk_shift,
                                                                 uint32_t side_blocks) {
     NANOEP_FETCH_ARGS_4(y, token_slots, out_x, bias);
     NANOEP_FETCH_ARGS_4(tokens, y_rows, parts, parts_magic);
     NANOEP_FETCH_ARGS_4(parts_shift, chunks_per_block, rows_per_block, vectors);
-    NANOEP_FETCH_ARGS_4(chunks, topk, flags, out_weights);
+    NANOEP_FETCH_ARGS_4(chunks, flags, side_blocks, out_weights);
     if (blockIdx.x < side_blocks) {
         // weights back to their (token, k): one lane each, in workgroups of their own at the front
         // of the grid (on the first payload wavefront of a row they are a second round trip)
         const uint32_t wave = threadIdx.z * chunks_per_block + threadIdx.y;
         const uint32_t flat = (blockIdx.x * (chunks_per_block * rows_per_block) + wave) * kWave + threadIdx.x;
-        if (fast_divide(flat, topk_magic, topk_shift) >= tokens)
+        if (flat / kTopk >= tokens)
             return;
         const int32_t slot = token_slots[flat];
         out_weights[flat] = slot >= 0 && static_cast<uint32_t>(slot) < y_rows ? weights[slot] : 0.0f;
@@ -647,8 +644,7 @@ int nanoep_combine(const void* y, const float* weights, const void* bias, const 
         static_cast<const u32x4*>(y), weights, static_cast<const u32x4*>(bias), token_slots,                         \
         static_cast<u32x4*>(out_x), out_weights, static_cast<uint32_t>(num_tokens), static_cast<uint32_t>(y_rows),   \
         blocking.parts, parts_divisor.magic, parts_divisor.shift, blocking.chunks_per_block, blocking.rows_per_block, \
-        static_cast<uint32_t>(vectors), static_cast<uint32_t>(chunks), static_cast<uint32_t>(num_topk),              \
-        flags, topk_divisor.magic, topk_divisor.shift, static_cast<uint32_t>(side_blocks))
+        static_cast<uint32_t>(vectors), static_cast<uint32_t>(chunks), flags, static_cast<uint32_t>(side_blocks))
         switch (num_topk) {
             case 1: NANOEP_LAUNCH_FEW(1); break;
             case 2: NANOEP_LAUNCH_FEW(2); break;

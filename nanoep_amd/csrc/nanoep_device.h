@@ -31,9 +31,10 @@
 //                          plain launch order, single-wavefront workgroups, nothing but the copy.
 //   combine_rows_kernel  : one wavefront per (source token, row chunk): gathers the token's rows in
 //                          ascending k, fp32 accumulate, one round-to-nearest-even bf16 store.
-//   combine_few_rows_kernel : the same for K <= 4 with the slot table, without the bookkeeping.
-//   combine_held_kernel  : the same for K > 4 with the slot table: a wavefront sums its chunk of 2
-//                          to 16 consecutive tokens' rows and writes them all at its end, so that a
+//   combine_few_rows_kernel : the same for K <= 8 with the slot table, without the bookkeeping: all
+//                          launches with K <= 5, most with K = 6 and the small ones with K = 7, 8.
+//   combine_held_kernel  : the same for K >= 6 with the slot table in larger launches: a wavefront sums
+//                          its chunk of 2 to 16 tokens' rows and writes them all at its end, so that a
 //                          launch whose wavefronts are all resident reads first and writes last.
 //   rebuild_table_kernel + rebuild_order_kernel : the slot table and the slot-order list of a handle
 //                          rebuilt from its recv_metadata and dst_slots alone (an LDS bitonic sort

@@ -1128,8 +1128,7 @@ DispatchResult dispatch(PeerRuntime& runtime,
         // host latency, the GPU starts three allocator round trips after the call instead of ten
         // and works while the rest of the bookkeeping is done.
         const int64_t order_entries = ordered ? nanoep_slot_order_entries(tokens, static_cast<int>(topk), local_experts) : 0;
-        // offsets of the int64 tensors in the arena; the per-token ones start 16-byte aligned (even
-        // offsets), which lets the layout kernels move two ids a lane at a time
+        // offsets of the int64 tensors in the arena; the per-token ones start 16-byte aligned (even offsets)
         const auto even = [](int64_t words) { return (words + 1) / 2 * 2; };
         const int64_t at_offsets = local_experts, at_send = 2 * local_experts + 1, at_prefix = at_send + 1;
         const int64_t at_dst = even(at_prefix + 1), at_snapshot = even(at_dst + tokens), at_order = even(at_snapshot + tokens * topk);
