@@ -158,7 +158,7 @@ def test_asynchronous_calls_made_on_the_communication_stream(device, consumer):
 
 
 # A completion event that goes away unwaited keeps the call's tensors safe from the allocator: what the call
-# reads and writes is freed and its memory asked for again while the call still waits for its stream.
+# reads is freed and its memory asked for again while the call still waits for its stream.
 @pytest.mark.parametrize("explicit_event", [False, True])
 def test_a_dropped_completion_event_protects_the_calls_memory(device, explicit_event):
     config, x, idx, w, want_x, want_w, _ = small_case(device, 8, tokens=200, hidden=1024)
@@ -180,6 +180,42 @@ def test_a_dropped_completion_event_protects_the_calls_memory(device, explicit_e
         assert_same_bits(payload, want_x, "payload")
         assert_same_bits(gates, want_w, "weights")
         del poison
+
+
+def active_bytes():
+    """Memory the allocator gives to nobody: in use, or freed while a stream it was told of may still use it."""
+    return torch.cuda.memory_stats()["active_bytes.all.current"]
+
+
+# The same for what the call writes: results, and a fresh dispatch's handle, dropped with the event while the kernels
+# that write them are to run.  (A fresh dispatch returns behind its layout: its permute may have run when the memory is asked
+# for again, but the allocator has been told of it.)
+@pytest.mark.parametrize("call", ["replay", "fresh", "combine"])
+def test_a_dropped_completion_event_protects_the_calls_results(device, call):
+    tokens, hidden, experts, topk = 2048, 4096, 16, 4
+    x, idx = cases.payload(tokens, hidden, seed=8).to(device), cases.routing("random", tokens, experts, topk, seed=8).to(device)
+    with Buffer(None, EPConfig(experts, topk, hidden, tokens)) as buffer:
+        first = buffer.dispatch(x, topk_idx=idx, do_expand=True)
+        if call != "fresh":
+            with torch.cuda.stream(buffer.comm_stream):
+                torch.cuda._sleep(20_000_000)
+        before = active_bytes()
+        if call == "combine":
+            shape, handle_bytes = (tokens, hidden), 0
+            result = buffer.combine(first.x, first.handle, async_op=True)
+        else:
+            shape, handle_bytes = (tokens * topk, hidden), 0 if call == "replay" else tokens * topk * 24
+            result = buffer.dispatch(x, async_op=True, **({"handle": first.handle} if call == "replay" else {"topk_idx": idx, "do_expand": True}))
+        assert result.x.shape == shape
+        del result
+        assert active_bytes() - before >= shape[0] * hidden * 2 + handle_bytes
+        mine = [torch.full(shape, -77.0, dtype=torch.bfloat16, device=device) for _ in range(3)]
+        small = [torch.full((1 << 20,), 77, dtype=torch.int64, device=device) for _ in range(3)]
+        torch.cuda.synchronize()
+        for tensor in mine:
+            assert bool((tensor == -77.0).all())
+        for tensor in small:
+            assert bool((tensor == 77).all())
 
 
 # Early outputs that do not fit what routing filled are replaced by exact ones while the kernel that writes them may
@@ -212,11 +248,6 @@ def test_replaced_early_outputs_stay_the_calls_until_it_is_waited_for(device, to
         assert_dispatch_result(received, x, idx, w, experts, expand, alignment, False)
         for tensor in mine:
             assert bool((tensor == -77.0).all())
-
-
-def active_bytes():
-    """Memory the allocator gives to nobody: in use, or freed while a stream it was told of may still use it."""
-    return torch.cuda.memory_stats()["active_bytes.all.current"]
 
 
 # A fresh dispatch learns of bad routing ids while its layout and the permute behind it are at work on a stream that is
