@@ -18,7 +18,7 @@ per-launch times, with the fastest region beside it (`*_min`).  Plain streams of
 (`stream_ceiling`: nanoep_stream_probe launches in the shape of the kernels) are timed in the same
 run and every roofline entry carries `frac_of_stream_ceiling` beside `frac`.  The other benchmark
 shapes follow under `roofline_by_workload` (same protocol, shorter CPU samples; `--workload
-deepseek-v3` leaves them out).
+deepseek-v3` leaves them out), a row of figures each; `--record FILE` keeps everything that was measured.
 """
 
 from __future__ import annotations
@@ -66,6 +66,9 @@ def parse_args():
                              "every launch of a kernel name is then the same work); `streams`: only the plain streams")
     parser.add_argument("--no-calibration", dest="calibration", action="store_false",
                         help="skip the plain streams (nanoep_stream_probe) that give every roofline entry its frac_of_stream_ceiling")
+    parser.add_argument("--record", metavar="FILE", default="",
+                        help="also write everything that was measured there, as JSON (the printed line leaves out the plain streams, the switches, "
+                             "the graph and side-stream series and the other workloads' details)")
     parser.add_argument("--calibration-copy-mib", type=int, default=0,
                         help="also launch the plain copy kernel on this many MiB (known-size reference for profiler byte counters)")
     return parser.parse_args()
@@ -711,6 +714,33 @@ def measure(workload, args, device, detailed):
     return result
 
 
+def brief(result):
+    """What the printed line holds of the record: the headline with its rooflines and CPU baseline, one row of figures for
+    every other workload.  It stays below 8000 characters, so that whoever keeps the end of the output keeps all of it."""
+    line = {key: value for key, value in result.items()
+            if key not in ("stream_ceiling", "dispatch_prefetch_switch", "hip_graph_step", "side_stream_consumer", "roofline_by_workload")}
+    rows = {}
+    for name, entry in result.get("roofline_by_workload", {}).items():
+        row = {"step_GBps": entry["value"]}
+        for call, roofline in (("dispatch", entry["roofline"]), ("combine", entry["roofline_combine"])):
+            row[call] = {"us": entry[f"{call}_us"], "frac": roofline["frac"]}
+            if "frac_of_stream_ceiling" in roofline:
+                row[call]["frac_of_stream_ceiling"] = roofline["frac_of_stream_ceiling"]
+            if roofline["traffic"] is not None:
+                row[call]["traffic_over_algorithmic"] = round(roofline["traffic"] / roofline["algorithmic_bytes"], 3)
+        for key in ("dispatch_us_cache_resident_source", "fresh_dispatch_us_host", "bit_exact_vs_oracle"):
+            if key in entry:
+                row[key] = entry[key]
+        if "side_stream_consumer" in entry:
+            row["side_stream_us"] = [entry["side_stream_consumer"][key] for key in ("dispatch_us", "combine_us")]
+        if "cpu_baseline" in entry:
+            row["cpu_us_per_step"] = entry["cpu_baseline"]["us_per_step"]
+        rows[name] = row
+    if rows:
+        line["roofline_by_workload"] = rows
+    return line
+
+
 # (the largest batch first: it takes the longest and sits furthest above its target, see main())
 OTHER_WORKLOADS = ["ep8-share", "deepseek-v3-a128", "short-rows-1024", "short-rows-512", "qwen3-moe", "mixtral", "latency-256", "readme-toy"]
 
@@ -801,7 +831,9 @@ def main():
         del source, target
     if failed:
         log("ERROR: GPU results of a timed configuration differ from the oracle")
-    print(json.dumps(result), flush=True)
+    if args.record:
+        Path(args.record).write_text(json.dumps(result, indent=1) + "\n")
+    print(json.dumps(brief(result)), flush=True)
     return 1 if failed else 0
 
 

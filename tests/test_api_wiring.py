@@ -3,6 +3,7 @@ native module, handle packaging and event keep-alives.  The fake backend's signa
 boundary, in the order the reference's unit tests pin (tests/unit/test_cuda_dispatch.py:77-94,
 tests/unit/test_cuda_combine.py:141-154)."""
 
+import json
 from types import SimpleNamespace
 
 import pytest
@@ -379,3 +380,28 @@ def test_the_benchmark_refuses_more_than_one_gpu():
     assert done.returncode != 0
     assert "ONE GPU" in done.stderr + done.stdout
     assert not any(line.startswith("{") for line in done.stdout.splitlines())
+
+
+def test_the_benchmarks_line_stays_short_whatever_the_record_holds():
+    """The printed line has the headline, its rooflines and one row for every other workload, in under 8000 characters."""
+    import bench
+    from nanoep_amd import workloads
+
+    ceiling = {"GBps": 6333.912, "kind": "fan-out 1:7", "window": 128, "waves_per_workgroup": 4}
+    record = {"metric": "m" * 120, "stream_ceiling": {str(i): "x" * 50 for i in range(200)}, "hip_graph_step": {"step": "y" * 500},
+              "dispatch_prefetch_switch": {}, "roofline_by_workload": {}}
+    names = [name for name in workloads.WORKLOADS if name != bench.HEADLINE]
+    for name in names:
+        entry = {"value": 6431.0, "dispatch_us": 142.671, "combine_us": 143.352, "dispatch_us_cache_resident_source": 142.031,
+                 "fresh_dispatch_us_host": 168.4, "bit_exact_vs_oracle": True, "stream_ceiling": record["stream_ceiling"],
+                 "side_stream_consumer": {"dispatch_us": 64.2, "combine_us": 59.4, "timed": "z" * 400}, "cpu_baseline": {"us_per_step": 164594.6}}
+        for key, kernel in (("roofline", "dispatch_walk_kernel"), ("roofline_combine", "combine_held_kernel")):
+            entry[key] = bench.roofline_entry(kernel, name, 940000000, 142.67, 141.3, ceiling)
+        record["roofline_by_workload"][name] = entry
+    line = bench.brief(record)
+    assert line["metric"] == record["metric"] and set(line["roofline_by_workload"]) == set(names)
+    row = line["roofline_by_workload"][names[0]]
+    assert row["dispatch"]["us"] == 142.671 and row["side_stream_us"] == [64.2, 59.4]
+    assert row["combine"]["frac_of_stream_ceiling"] == entry["roofline_combine"]["frac_of_stream_ceiling"]
+    # (what is besides them in a line is the headline's own figures: 4000 characters)
+    assert len(json.dumps(line)) < 4000 and len(json.dumps(record)) > 8000
