@@ -180,8 +180,11 @@ void wait_on(const Stream& waiter, const Stream& producer) {
 }
 
 // Tensors are made without the dispatcher (a third of its time: an allocation of torch::empty is 1.5 us of
-// a call that takes six).
+// a call that takes six), unless torch is to fill what is left uninitialized.
 torch::Tensor new_tensor(at::IntArrayRef sizes, at::ScalarType dtype, const c10::Device& device) {
+    const auto& context = at::globalContext();
+    if (C10_UNLIKELY(context.deterministicAlgorithms() && context.deterministicFillUninitializedMemory()))
+        return torch::empty(sizes, torch::TensorOptions().dtype(dtype).device(device));
     return torch::Tensor(at::detail::empty_cuda(sizes, dtype, device, std::nullopt));
 }
 

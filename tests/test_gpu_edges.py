@@ -5,10 +5,12 @@ from concurrent.futures import ThreadPoolExecutor
 
 import pytest
 import torch
+from torch.utils import deterministic
 
 import cabi
 import cases
 from nanoep_amd import Buffer, EPConfig
+from nanoep_amd._native import load_extension
 from oracle import nanoep_oracle as oracle
 from test_gpu_buffer_api import assert_dispatch_result, assert_same_bits
 from test_gpu_cabi_parity import assert_layout, run_dispatch_combine
@@ -447,3 +449,38 @@ def test_combine_around_other_batches_that_hold_sums_back(device, tokens, hidden
     want, want_w = oracle.combine(y, lay.recv_metadata(True), lay.dst_slots, do_expand=True, weights=w)
     assert_same_bits(out, want, "combine")
     assert_same_bits(out_w, want_w, "weights")
+
+
+# Where torch is to fill uninitialized memory, a result's rows that no call writes (alignment gaps without zero padding)
+# hold torch's fill value and not what their memory held before, through the native module, which accepts that mode.
+@pytest.mark.parametrize("asynchronous", [False, True])
+def test_deterministic_fill_reaches_the_rows_nobody_writes(device, asynchronous):
+    native = load_extension()
+    config, x, idx, w, _, _, _ = small_case(device, 8, tokens=200, hidden=1024)
+    lay = oracle.layout(idx.cpu(), config.num_experts, 16)
+    gaps = torch.ones(lay.expanded_capacity, dtype=torch.bool)
+    for count, offset in zip(lay.expert_counts.tolist(), lay.expert_offsets.tolist()):
+        gaps[offset : offset + count] = False
+    assert bool(gaps.any())
+    enabled, fill = torch.are_deterministic_algorithms_enabled(), deterministic.fill_uninitialized_memory
+    warn_only = torch.is_deterministic_algorithms_warn_only_enabled()
+    with Buffer(None, config) as buffer:
+        torch.use_deterministic_algorithms(True)
+        deterministic.fill_uninitialized_memory = True
+        try:
+            metadata, capacity = [], 0
+            for _ in ("fresh", "cached"):
+                used = [torch.full((lay.expanded_capacity, 1024), 5.0, dtype=torch.bfloat16, device=device) for _ in range(4)]
+                del used
+                outputs, handle, counts, event = native.dispatch(
+                    buffer._runtime, x, idx, w, config.num_experts, config.num_max_tokens_per_rank, 16, metadata, capacity, False,
+                    expand=True, zero_padding=False, num_sms=0, comm_stream=buffer.comm_stream.cuda_stream, async_op=asynchronous,
+                )
+                if event is not None:
+                    event.current_stream_wait()
+                assert bool(outputs[0].cpu()[gaps].isnan().all()) and not bool(outputs[0].cpu()[~gaps].isnan().any())
+                assert bool(outputs[2].cpu()[gaps].isnan().all())
+                metadata, capacity = (metadata or list(handle)), counts[1]
+        finally:
+            deterministic.fill_uninitialized_memory = fill
+            torch.use_deterministic_algorithms(enabled, warn_only=warn_only)
