@@ -80,12 +80,12 @@ bool capturing(const Stream& stream) {
     return status != hipStreamCaptureStatusNone;
 }
 
-// Whether everything enqueued on the stream so far has run (never asked of a stream under capture).
-bool idle(const Stream& stream) {
+// Whether something enqueued on the stream has yet to run (never asked of a stream under capture).
+bool busy(const Stream& stream) {
     const hipError_t state = hipStreamQuery(stream.stream());
     if (state == hipErrorNotReady)
         (void)hipGetLastError();  // an answer, not an error of the next call that looks for one
-    return state == hipSuccess;
+    return state == hipErrorNotReady;
 }
 
 // A point in a stream's work: a value the stream stores into a word of signal memory when it gets there.
@@ -900,8 +900,9 @@ Stream work_stream(int64_t comm_handle, const Stream& compute, c10::DeviceIndex 
     if (async_op || budgeted || same_queue(comm, compute))
         return comm;
     // While the caller's stream is being captured into a graph no other stream may be queried;
-    // a captured call is ordered by the graph alone.
-    if (!capturing(compute) && !idle(comm))
+    // a captured call is ordered by the graph alone.  A communication stream under capture holds nothing that runs
+    // before its graph does: waiting for it would make the call part of that graph.
+    if (!capturing(compute) && !capturing(comm) && busy(comm))
         wait_on(compute, comm);
     return compute;
 }

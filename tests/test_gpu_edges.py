@@ -484,3 +484,31 @@ def test_deterministic_fill_reaches_the_rows_nobody_writes(device, asynchronous)
         finally:
             deterministic.fill_uninitialized_memory = fill
             torch.use_deterministic_algorithms(enabled, warn_only=warn_only)
+
+
+# A synchronous call on another stream while somebody captures the communication stream: it runs, now, and the capture
+# has nothing of it.
+def test_synchronous_calls_beside_a_capture_of_the_communication_stream(device):
+    config, x, idx, w, want_x, _, _ = small_case(device, 12)
+    with Buffer(None, config) as buffer:
+        handle = buffer.dispatch(x, topk_idx=idx, do_expand=True).handle
+        side, stream = torch.cuda.Stream(), buffer.comm_stream
+        scratch = torch.zeros(8, device=device)
+        with torch.cuda.stream(side):
+            buffer.dispatch(x, handle=handle)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.stream(stream):
+            graph.capture_begin(capture_error_mode="relaxed")
+            try:
+                scratch.add_(1)
+                with torch.cuda.stream(side):
+                    received = buffer.dispatch(x, handle=handle).x
+                    side.synchronize()
+            finally:
+                graph.capture_end()
+        assert_same_bits(received, want_x, "dispatch")
+        for _ in range(3):
+            graph.replay()
+        torch.cuda.synchronize()
+        assert scratch.tolist() == [3.0] * 8
