@@ -749,6 +749,7 @@ class CompletionEvent {
     void settle() { settled_ = true; }
 
     void order_after(const Stream& consumer) {
+        std::vector<torch::Tensor> let_go;  // behind the lock: a tensor's end may run Python, and that other waiters of this marker
         std::lock_guard<std::mutex> lock(mutex_);
         if (point_.has_value() && !capturing(consumer)) {
             if (!point_->reached())
@@ -761,7 +762,7 @@ class CompletionEvent {
         }
         note_use(written_, consumer);
         note_use(read_, consumer);
-        read_.clear();
+        let_go.swap(read_);
         settled_ = true;
     }
 

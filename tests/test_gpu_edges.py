@@ -1,6 +1,8 @@
 """GPU tests at the edges of single kernel paths, against the CPU oracle (bit for bit)."""
 
+import threading
 import time
+import weakref
 from concurrent.futures import ThreadPoolExecutor
 
 import pytest
@@ -512,3 +514,32 @@ def test_synchronous_calls_beside_a_capture_of_the_communication_stream(device):
             graph.replay()
         torch.cuda.synchronize()
         assert scratch.tolist() == [3.0] * 8
+
+
+# What a waited-for call has read is let go of by the wait, and its end may run Python (here: a weak reference's callback)
+# while another thread waits for the same call.
+def test_two_threads_wait_for_a_call_whose_inputs_end_there(device):
+    native = load_extension()
+    config, x, idx, w, want_x, _, _ = small_case(device, 8)
+    with Buffer(None, config) as buffer, ThreadPoolExecutor(2) as threads:
+        handle = buffer.dispatch(x, topk_idx=idx, do_expand=True).handle
+        source, ended = x.clone(), threading.Event()
+
+        def on_end(_):
+            ended.set()
+            time.sleep(0.3)
+
+        watch = weakref.ref(source, on_end)
+        outputs, _, _, event = native.dispatch(
+            buffer._runtime, source, idx, None, config.num_experts, config.num_max_tokens_per_rank, 1, list(handle.tensors()),
+            handle.layout.expanded_capacity, False, expand=True, zero_padding=False, num_sms=0, comm_stream=buffer.comm_stream.cuda_stream,
+        )
+        del source
+        first = threads.submit(event.current_stream_wait)
+        assert ended.wait(timeout=10)
+        second = threads.submit(event.current_stream_wait)
+        first.result(timeout=10)
+        second.result(timeout=10)
+        torch.cuda.synchronize()
+        assert_same_bits(outputs[0], want_x, "dispatch")
+        del watch
