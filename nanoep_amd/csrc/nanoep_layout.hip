@@ -45,6 +45,15 @@ constexpr int kMaxBlockTokens = 128;
 constexpr int kBlockPairs = 512;
 // Chunks of pairs a wavefront fetches at a time where it counts more than one.
 constexpr int kChunks = 4;
+// Chunks of its block an assignment wavefront takes: one, so that a workgroup is done soon, until the launch has more
+// wavefronts than half the device holds.  From there on it is the rounds of workgroups that cost, each the whole chain of round
+// trips, and fewer wavefronts with more chunks are fewer rounds: two behind histogram rows, where a workgroup's
+// wavefronts also share the summing of the rows, four behind a scan.  Launch period of the layout, one chunk -> two (four):
+// 32768 x 16, 64 experts 17.8 -> 15.0 (15.4) us, 65536 x 8, 64 18.5 -> 15.7 (15.9), 65536 x 32, 256 89 -> 70 (71), 131072 x 8, 64
+// 31 -> 25.5 (25.8); behind a scan 400000 x 8, 64 129 -> 97 (96), 400000 x 10, 64 139 -> 117 (107).
+constexpr int kSummedChunks = 2;
+constexpr int kScannedChunks = 4;
+constexpr int64_t kOneChunkWaves = 4096;
 // Pairs up to which every workgroup counts the whole batch by itself.  One launch against two, launch period:
 // 512 x 8, 128 experts 5.1 against 7.5 us, 2048 x 2, 8 experts 5.8 against 7.5, 1537 x 4, 60 experts 6.0
 // against 7.7, 1024 x 8, 128 experts 7.2 against 7.5, and 8.3 against 7.5 us at 4096 x 2 with 8 experts, where
@@ -382,10 +391,6 @@ __global__ void __launch_bounds__(kScanThreads) layout_scan_kernel(const LayoutA
     const int num_blocks = static_cast<int>(a.row_count);
     if (tid == 0)
         status_bits = 0;
-    const auto word_at = [&](int b, int column) -> int32_t& {
-        return column < experts ? a.histograms[static_cast<int64_t>(b) * experts + column] : reinterpret_cast<int32_t&>(a.rows[b].received);
-    };
-
     const int columns_per_pass = rows < kScanThreads ? rows : kScanThreads;
     const int segments = kScanThreads / columns_per_pass;
     const int blocks_per_segment = (num_blocks + segments - 1) / segments;
@@ -394,12 +399,14 @@ __global__ void __launch_bounds__(kScanThreads) layout_scan_kernel(const LayoutA
         const int segment = tid / columns_per_pass;
         const int column = column0 + column_local;
         const bool active = segment < segments && column < rows;
+        int32_t* const words = column < experts ? a.histograms + column : reinterpret_cast<int32_t*>(&a.rows->received);
+        const int64_t stride = column < experts ? experts : static_cast<int>(sizeof(RowInfo) / sizeof(int32_t));
         const int begin = segment * blocks_per_segment;
         const int end = begin + blocks_per_segment < num_blocks ? begin + blocks_per_segment : num_blocks;
         int sum = 0;
         if (active)
             for (int b = begin; b < end; ++b)
-                sum += word_at(b, column);
+                sum += words[b * stride];
         partial[tid] = active ? sum : 0;
         __syncthreads();
         if (active) {
@@ -407,8 +414,8 @@ __global__ void __launch_bounds__(kScanThreads) layout_scan_kernel(const LayoutA
             for (int s = 0; s < segment; ++s)
                 running += partial[s * columns_per_pass + column_local];
             for (int b = begin; b < end; ++b) {
-                const int count = word_at(b, column);
-                word_at(b, column) = running;
+                const int count = words[b * stride];
+                words[b * stride] = running;
                 running += count;
             }
             if (segment == segments - 1)
@@ -641,7 +648,9 @@ __device__ __forceinline__ void publish_layout(const LayoutArgs& a, uint32_t* ld
 // The rank of a pair among its block's assignments to the same expert comes from a bit matrix: bit
 // (token) of row (expert) is set when the token chose it.  A token's choices are distinct, so the order
 // of an expert's assignments is the token order and the rank is the number of bits below the token's.
-template <int kSource, bool kWindow>
+//
+// kOwn: chunks of the block a wavefront takes.
+template <int kSource, bool kWindow, int kOwn>
 __global__ void __launch_bounds__(kLayoutThreads) layout_assign_kernel(const LayoutArgs a) {
     extern __shared__ __align__(16) uint32_t assign_lds[];
     __shared__ uint32_t wave_padded[kLayoutWaves], wave_window[kLayoutWaves];
@@ -669,7 +678,10 @@ __global__ void __launch_bounds__(kLayoutThreads) layout_assign_kernel(const Lay
     // What the workgroup reads leaves before anything waits: the wavefront's own ids, and the first of those it
     // counts: of the whole batch, or what lies between the start of the block's histogram row and the block.
     const uint32_t own_first = block_first + wave * a.chunk_tokens;
-    const int64_t id = fetch_id(a, at, own_first, block_end);
+    int64_t id[kOwn];
+#pragma unroll
+    for (int o = 0; o < kOwn; ++o)
+        id[o] = fetch_id(a, at, own_first + o * step, block_end);
     const uint32_t count_end = kSource == kDirect ? a.tokens : block_first;
     uint32_t chunk = own_row * a.row_tokens + wave * a.chunk_tokens;
     int64_t batch[kChunks];
@@ -698,16 +710,21 @@ __global__ void __launch_bounds__(kLayoutThreads) layout_assign_kernel(const Lay
     if (tid == 0)
         sums = {0, 0, 0, 0, 0};
     __syncthreads();
-    const bool own_valid = names_expert(id, a);
-    const uint64_t own_mask = __ballot(own_valid);
-    const uint32_t local = own_first - block_first + at.token;
-    const bool live = at.lane < pairs_of_chunk(a, own_first, block_end);
-    if (live)
-        (a.snapshot + static_cast<uint64_t>(own_first) * a.topk)[at.lane] = id;
-    if (own_valid) {
-        (void)set_token_bit(bits, words, id, local);
-        if ((own_mask & at.earlier) == 0)
-            atomicOr(&any_bits[local / 32], 1u << (local % 32));
+    uint32_t own = 0;
+#pragma unroll
+    for (int o = 0; o < kOwn; ++o) {
+        const uint32_t own_chunk = own_first + o * step;
+        const bool own_valid = names_expert(id[o], a);
+        const uint64_t own_mask = __ballot(own_valid);
+        const uint32_t local = own_chunk - block_first + at.token;
+        if (at.lane < pairs_of_chunk(a, own_chunk, block_end))
+            (a.snapshot + static_cast<uint64_t>(own_chunk) * a.topk)[at.lane] = id[o];
+        if (own_valid) {
+            (void)set_token_bit(bits, words, id[o], local);
+            if ((own_mask & at.earlier) == 0)
+                atomicOr(&any_bits[local / 32], 1u << (local % 32));
+        }
+        own += __popcll(own_mask);
     }
 
     uint32_t received = 0, assigned = 0, before = 0, window_start = 0;
@@ -746,8 +763,8 @@ __global__ void __launch_bounds__(kLayoutThreads) layout_assign_kernel(const Lay
         }
     }
     if (at.lane == 0) {
-        if (own_mask != 0)
-            atomicAdd(&sums.own, static_cast<uint32_t>(__popcll(own_mask)));
+        if (own != 0)
+            atomicAdd(&sums.own, own);
         if (assigned != 0) {
             atomicAdd(&sums.received_before, received);
             atomicAdd(&sums.assigned_before, kSource == kDirect ? before : assigned);
@@ -882,12 +899,17 @@ __global__ void __launch_bounds__(kLayoutThreads) layout_assign_kernel(const Lay
     if (kSource == kScanned)
         __syncthreads();
 
-    if (live) {
-        const uint32_t token = own_first + at.token;
+#pragma unroll
+    for (int o = 0; o < kOwn; ++o) {
+        const uint32_t own_chunk = own_first + o * step;
+        if (at.lane >= pairs_of_chunk(a, own_chunk, block_end))
+            continue;
+        const uint32_t local = own_chunk - block_first + at.token;
+        const uint32_t token = own_chunk + at.token;
         const uint32_t word = local / 32, below = (1u << (local % 32)) - 1u;
         int32_t value = -1;
-        if (own_valid) {
-            const uint32_t expert = static_cast<uint32_t>(id);
+        if (names_expert(id[o], a)) {
+            const uint32_t expert = static_cast<uint32_t>(id[o]);
             uint32_t rank = 0;
             for (uint32_t w = 0; w < words; ++w) {
                 const uint32_t row = bits[expert * words + w];
@@ -896,10 +918,10 @@ __global__ void __launch_bounds__(kLayoutThreads) layout_assign_kernel(const Lay
             value = a.expand ? static_cast<int32_t>(base[expert] + rank) : static_cast<int32_t>(expert);
             if (a.slot_order != nullptr)
                 a.slot_order[order_base[expert] + rank] =
-                    static_cast<int64_t>(static_cast<uint64_t>(static_cast<uint32_t>(value)) << 32 | (own_first * a.topk + at.lane));
+                    static_cast<int64_t>(static_cast<uint64_t>(static_cast<uint32_t>(value)) << 32 | (own_chunk * a.topk + at.lane));
         }
         if (a.token_slots != nullptr)
-            (a.token_slots + static_cast<uint64_t>(own_first) * a.topk)[at.lane] = value;
+            (a.token_slots + static_cast<uint64_t>(own_chunk) * a.topk)[at.lane] = value;
         const bool is_received = (any_bits[word] >> (local % 32)) & 1u;
         uint32_t row = sums.received_before;
         for (uint32_t w = 0; w < words; ++w)
@@ -978,7 +1000,7 @@ int enqueue_layout(const int64_t* topk_idx, int64_t num_tokens, int num_topk, in
         source = kSummed;
     else if (knobs.layout_launches == 3)
         source = kScanned;
-    // a chunk of the block a wavefront; in the direct plan enough wavefronts for the counting as well
+    // one or more chunks of the block a wavefront; in the direct plan enough wavefronts for the counting as well
     const int chunk_tokens = kWave / num_topk;
     int waves = (block_tokens + chunk_tokens - 1) / chunk_tokens;
     if (source == kDirect) {
@@ -988,6 +1010,8 @@ int enqueue_layout(const int64_t* topk_idx, int64_t num_tokens, int num_topk, in
         if (waves < counting)
             waves = counting < kLayoutWaves ? static_cast<int>(counting) : kLayoutWaves;
     }
+    const int own = source == kScanned ? kScannedChunks : source == kSummed && blocks * waves > kOneChunkWaves ? kSummedChunks : 1;
+    waves = (waves + own - 1) / own;
     if (source == kSummed) {
         const int64_t tasks = (num_local_experts + kWave - 1) / kWave * (padded_rows(histogram_rows) / kSumRows);
         if (waves < tasks)
@@ -1062,19 +1086,21 @@ int enqueue_layout(const int64_t* topk_idx, int64_t num_tokens, int num_topk, in
     const dim3 grid(static_cast<unsigned>(blocks + (source == kScanned ? 0 : 1)));
     const size_t lds = layout_lds(num_local_experts, source == kDirect && batch_words > block_tokens / 32 ? batch_words : block_tokens / 32);
     const bool several = window > block_tokens;
-#define NANOEP_LAUNCH_ASSIGN(SOURCE)                                                            \
+#define NANOEP_LAUNCH_ASSIGN(SOURCE, OWN)                                                       \
     do {                                                                                        \
         if (several)                                                                            \
-            layout_assign_kernel<SOURCE, true><<<grid, threads, lds, stream>>>(a);       \
+            layout_assign_kernel<SOURCE, true, OWN><<<grid, threads, lds, stream>>>(a);         \
         else                                                                                    \
-            layout_assign_kernel<SOURCE, false><<<grid, threads, lds, stream>>>(a);      \
+            layout_assign_kernel<SOURCE, false, OWN><<<grid, threads, lds, stream>>>(a);        \
     } while (0)
     if (source == kDirect)
-        NANOEP_LAUNCH_ASSIGN(kDirect);
+        NANOEP_LAUNCH_ASSIGN(kDirect, 1);
+    else if (source == kSummed && own == 1)
+        NANOEP_LAUNCH_ASSIGN(kSummed, 1);
     else if (source == kSummed)
-        NANOEP_LAUNCH_ASSIGN(kSummed);
+        NANOEP_LAUNCH_ASSIGN(kSummed, kSummedChunks);
     else
-        NANOEP_LAUNCH_ASSIGN(kScanned);
+        NANOEP_LAUNCH_ASSIGN(kScanned, kScannedChunks);
 #undef NANOEP_LAUNCH_ASSIGN
     NANOEP_HIP_TRY(hipGetLastError());
     return NANOEP_OK;

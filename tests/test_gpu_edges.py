@@ -63,6 +63,19 @@ def test_layout_plans_at_their_edges(device, tuning, launches, tokens, experts, 
         assert_layout(metadata, counts, oracle.layout(idx, experts, alignment), expand, hidden)
 
 
+# Batches whose assignment wavefronts take two chunks of a block each (more than 4096 wavefronts with one): the last block
+# cut short inside a wavefront's first or second chunk, an odd number of chunks a block; and one token less than it takes.
+@pytest.mark.parametrize(
+    "tokens,experts,topk,hidden",
+    [(16385, 40, 32, 2048), (8192, 40, 32, 2048), (8193, 33, 32, 512), (65570, 24, 5, 2048), (32801, 300, 9, 4096), (140001, 5, 3, 1024)],
+)
+def test_layout_with_two_chunks_a_wavefront(device, tokens, experts, topk, hidden):
+    idx = cases.routing("dropout", tokens, experts, topk, seed=topk)
+    for expand in (True, False):
+        metadata, counts = cabi.layout(idx.to(device), experts, 16, expand, hidden=hidden)
+        assert_layout(metadata, counts, oracle.layout(idx, experts, 16), expand, hidden)
+
+
 # One bad token anywhere in the batch is found by every plan: an id in another half of its 64 bits, a
 # duplicate in the token's first and last choice, in the first and last block.
 @pytest.mark.parametrize("launches", [1, 2, 3])
