@@ -1173,22 +1173,22 @@ DispatchResult dispatch(PeerRuntime& runtime,
         const int64_t choice_bound = expand ? tokens * topk : tokens;
         const int64_t gap_bound = expand ? local_experts * (alignment - 1) : 0;
         const int64_t row_bound = choice_bound + gap_bound;
-        const int order_switch = tuning_switch("FRESH_OUTPUTS");  // 0: always exact, 1: at the bound whenever the rule allows it
         const bool bound_rule = gap_bound * 8 <= choice_bound;
         PeerRuntime::OutputForecast geometry;
         geometry.tokens = tokens, geometry.topk = topk, geometry.experts = local_experts, geometry.alignment = alignment;
         geometry.hidden = hidden, geometry.expand = expand;
         // rows the outputs are allocated for ahead of the counts: the bound where it is close, else what
         // the latest call of this geometry used plus an eighth, else nothing (the exact order)
+        const auto rows_ahead = [&]() -> int64_t {
+            const int order_switch = tuning_switch("FRESH_OUTPUTS");  // 0: always exact, 1: at the bound whenever the rule allows it
+            if (tokens == 0 || order_switch == 0 || row_bound > std::numeric_limits<int32_t>::max())
+                return 0;
+            if (!bound_rule)
+                return std::min(row_bound, runtime.forecast_rows(geometry));
+            return order_switch == 1 || !runtime.prefers_exact_outputs() ? row_bound : 0;
+        };
         int64_t early_rows = 0;
-        if (tokens > 0 && order_switch != 0 && row_bound <= std::numeric_limits<int32_t>::max()) {
-            if (bound_rule && (order_switch == 1 || !runtime.prefers_exact_outputs()))
-                early_rows = row_bound;
-            else if (!bound_rule)
-                early_rows = std::min(row_bound, runtime.forecast_rows(geometry));
-        }
-        const bool speculative = early_rows > 0;
-        if (speculative && borrows)
+        if (borrows && (early_rows = rows_ahead()) > 0)
             allocate_outputs(early_rows, tokens);
         order_comm_after_inputs(comm, compute, previous_event, async_op);
         TORCH_CHECK(!capturing(comm), "Fresh dispatch with host count polling cannot be captured in a HIP graph");
@@ -1204,6 +1204,9 @@ DispatchResult dispatch(PeerRuntime& runtime,
             turn.abandon();  // refused before anything was enqueued
         check_status(layout_status, "layout");
 
+        if (!borrows)  // (off the path to the layout)
+            early_rows = rows_ahead();
+        const bool speculative = early_rows > 0;
         if (speculative) {
             // enqueued straight from the arena's pointers: the tensors of the handle are made below,
             // while the GPU works
