@@ -627,7 +627,7 @@ __device__ __forceinline__ void publish_layout(const LayoutArgs& a, uint32_t* ld
     }
 }
 
-// Slot assignment.  One workgroup per block of tokens, a chunk of (token, choice) pairs a wavefront, and,
+// Slot assignment.  One workgroup per block of tokens, kOwn chunks of (token, choice) pairs a wavefront, and,
 // unless a scan kernel has done that, one more in front of them that publishes (publish_layout).
 //
 // What a block needs of the others' tokens are sums per expert: the total (for the slots' aligned
@@ -648,8 +648,6 @@ __device__ __forceinline__ void publish_layout(const LayoutArgs& a, uint32_t* ld
 // The rank of a pair among its block's assignments to the same expert comes from a bit matrix: bit
 // (token) of row (expert) is set when the token chose it.  A token's choices are distinct, so the order
 // of an expert's assignments is the token order and the rank is the number of bits below the token's.
-//
-// kOwn: chunks of the block a wavefront takes.
 template <int kSource, bool kWindow, int kOwn>
 __global__ void __launch_bounds__(kLayoutThreads) layout_assign_kernel(const LayoutArgs a) {
     extern __shared__ __align__(16) uint32_t assign_lds[];
