@@ -290,11 +290,30 @@ __device__ __forceinline__ void clear_lds(uint32_t* lds, uint32_t words, uint32_
         reinterpret_cast<u32x4*>(lds)[i] = zero;
 }
 
+// A workgroup barrier for what passes through LDS alone: loads from and stores to global memory stay on their way
+// across it.  Nothing in these kernels passes between threads through global memory; a __syncthreads() here waits for
+// the ids' and rows' loads at the first barrier and for the snapshot's stores at the next one.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// Names a word of every cache line of the arguments: they arrive with the first batch of scalar loads, and what is
+// asked for later is in the scalar cache.  Left where it is first used, a line is a round trip to memory of its own on the
+// way of every wavefront, 0.2 to 0.4 us each.
+__device__ __forceinline__ void fetch_layout_arguments(const LayoutArgs& a) {
+    static_assert(sizeof(LayoutArgs) <= 4 * 64, "one word of every line");
+    NANOEP_FETCH_ARGS_4(a.topk_idx, a.per_thread, a.alignment, a.dst_slots);
+    NANOEP_FETCH_ARGS_2(a.blocks, a.blocks);
+}
+
 // One histogram row: the experts' counts among `row_tokens` tokens, and their RowInfo.  Rows behind the
 // batch's end come out zero.
 __global__ void __launch_bounds__(kLayoutThreads) layout_histogram_kernel(const LayoutArgs a, const uint32_t waves) {
     extern __shared__ __align__(16) uint32_t histogram_lds[];
     __shared__ RowInfo info;
+    NANOEP_FETCH_ARGS_4(a.topk_idx, a.experts, a.check_tokens, waves);
     const uint32_t words = a.check_tokens / 32;
     const uint32_t counter_words = (a.experts + 3) / 4 * 4;
     uint32_t* counts = histogram_lds;                // [L]
@@ -319,10 +338,10 @@ __global__ void __launch_bounds__(kLayoutThreads) layout_histogram_kernel(const 
             if (threadIdx.x == 0)
                 info = RowInfo{0, 0, 0, 0};
         } else {
-            __syncthreads();
+            lds_barrier();
             clear_lds(bits, a.experts * words, waves * kWave);
         }
-        __syncthreads();
+        lds_barrier();
         while (chunk < end) {
 #pragma unroll
             for (int j = 0; j < kChunks; ++j) {
@@ -355,7 +374,7 @@ __global__ void __launch_bounds__(kLayoutThreads) layout_histogram_kernel(const 
         atomicAdd(&info.assigned, assigned);
         atomicOr(&info.status, bad);
     }
-    __syncthreads();
+    lds_barrier();
     int32_t* row = a.histograms + static_cast<uint64_t>(blockIdx.x) * a.experts;
     for (uint32_t i = threadIdx.x; i < a.experts; i += waves * kWave)
         row[i] = static_cast<int32_t>(counts[i]);
@@ -539,7 +558,7 @@ __device__ __forceinline__ void publish_layout(const LayoutArgs& a, uint32_t* ld
     clear_lds(lds, (a.experts + 3) / 4 * 4 + a.experts * words, a.waves * kWave);
     if (tid == 0)
         all = RowInfo{0, 0, 0, 0};
-    __syncthreads();
+    lds_barrier();
     uint32_t received = 0, assigned = 0;
     int bad = 0;
     if (kSource == kDirect) {
@@ -593,7 +612,7 @@ __device__ __forceinline__ void publish_layout(const LayoutArgs& a, uint32_t* ld
         atomicAdd(&all.assigned, assigned);
         atomicOr(&all.status, bad);
     }
-    __syncthreads();
+    lds_barrier();
     const uint32_t first = tid * a.per_thread < a.experts ? tid * a.per_thread : a.experts;
     const uint32_t last = first + a.per_thread < a.experts ? first + a.per_thread : a.experts;
     uint64_t padded_sum = 0, padded_scan = 0;
@@ -604,7 +623,7 @@ __device__ __forceinline__ void publish_layout(const LayoutArgs& a, uint32_t* ld
         if (at.lane == kWave - 1)
             wave_padded[wave] = padded_scan;
     }
-    __syncthreads();
+    lds_barrier();
     if (wave >= a.expert_waves)
         return;
     uint64_t running = padded_scan - padded_sum, capacity = 0;
@@ -651,6 +670,7 @@ __device__ __forceinline__ void publish_layout(const LayoutArgs& a, uint32_t* ld
 template <int kSource, bool kWindow, int kOwn>
 __global__ void __launch_bounds__(kLayoutThreads) layout_assign_kernel(const LayoutArgs a) {
     extern __shared__ __align__(16) uint32_t assign_lds[];
+    fetch_layout_arguments(a);
     __shared__ uint32_t wave_padded[kLayoutWaves], wave_window[kLayoutWaves];
     __shared__ uint32_t any_bits[kMaxBlockTokens / 32];  // the block's tokens with any valid choice
     __shared__ struct {
@@ -707,7 +727,7 @@ __global__ void __launch_bounds__(kLayoutThreads) layout_assign_kernel(const Lay
         any_bits[tid] = 0;
     if (tid == 0)
         sums = {0, 0, 0, 0, 0};
-    __syncthreads();
+    lds_barrier();
     uint32_t own = 0;
 #pragma unroll
     for (int o = 0; o < kOwn; ++o) {
@@ -809,7 +829,7 @@ __global__ void __launch_bounds__(kLayoutThreads) layout_assign_kernel(const Lay
             }
         }
     }
-    __syncthreads();
+    lds_barrier();
     // Experts: a thread takes a run of them (one each up to the workgroup's threads), the wavefronts
     // without any go on to the last barrier.
     const uint32_t first = tid * a.per_thread < a.experts ? tid * a.per_thread : a.experts;
@@ -870,7 +890,7 @@ __global__ void __launch_bounds__(kLayoutThreads) layout_assign_kernel(const Lay
         }
     }
     if (a.expert_waves > 1)
-        __syncthreads();
+        lds_barrier();
     else
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the sums stay within the one wavefront
     if (wave < a.expert_waves) {
@@ -888,14 +908,14 @@ __global__ void __launch_bounds__(kLayoutThreads) layout_assign_kernel(const Lay
             running_window += window & 0xffffu;
         }
     }
-    __syncthreads();
+    lds_barrier();
     if (kSource == kScanned && tid == 0) {
         sums.assigned_before = sums.assigned;
         sums.assigned = static_cast<uint32_t>(a.totals[0]);
         sums.received_before += a.rows[own_row].received;
     }
     if (kSource == kScanned)
-        __syncthreads();
+        lds_barrier();
 
 #pragma unroll
     for (int o = 0; o < kOwn; ++o) {
