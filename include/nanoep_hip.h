@@ -70,8 +70,8 @@ int nanoep_device_topology(int* out_cus, int* out_xcds, int64_t* out_l2_bytes);
  *   DISPATCH_SPAN (0: by size; 1 | 2 | 4 chunks a wavefront of the slot-order walk)
  *   DISPATCH_PACK (0: rows of at most 512 / 256 bytes go four / eight list entries a wavefront in
  *                     that walk; 1: one entry a wavefront whatever the row length)
- *   DISPATCH_PREFETCH (-1: on; 0: no window-wise source prefetch in that walk, for sources that are
- *                     known to sit in the last-level cache)
+ *   DISPATCH_PREFETCH (-1: on; 0: no window-wise source prefetch in that walk, and none beside the
+ *                     layout, for sources that are known to sit in the last-level cache)
  *   COMBINE_STORES (-1: by output size; 0 | 1: nontemporal / agent-scope stores for the combine's output)
  *   COMBINE_UNITS (0: by size; 1 .. 16 tokens a wavefront of the expanded combine with five or more
  *                     rows a token and the slot table; 1 = the one-token kernel)
@@ -136,6 +136,19 @@ int nanoep_layout(const int64_t* topk_idx, int64_t num_tokens, int num_topk, int
                   int64_t* expert_offsets, int64_t* dst_slots, int64_t* send_counts, int64_t* topk_snapshot,
                   int64_t* recv_rank_prefix, int32_t* token_slots, int64_t* slot_order, void* workspace,
                   size_t workspace_bytes, int64_t* host_counts, void* stream);
+
+/*
+ * nanoep_layout for a caller that dispatches x (bf16 [T, hidden], 16-byte aligned, hidden % 8 == 0) right behind it on the
+ * same stream: the layout's launches leave most of the device idle, and workgroups of their own read the first rows of x
+ * there, which the dispatch then finds in the caches.  Results are nanoep_layout's.  x is only read, and only ahead of a
+ * slot-order walk with its prefetch (slot_order given, DISPATCH_PREFETCH not 0).  NULL for x is nanoep_layout.
+ * It has no counterpart in the reference.
+ */
+int nanoep_layout_ahead(const int64_t* topk_idx, int64_t num_tokens, int num_topk, int64_t num_local_experts,
+                        int64_t alignment, int expand, int hidden, int32_t* recv_metadata, int64_t* expert_counts,
+                        int64_t* expert_offsets, int64_t* dst_slots, int64_t* send_counts, int64_t* topk_snapshot,
+                        int64_t* recv_rank_prefix, int32_t* token_slots, int64_t* slot_order, void* workspace,
+                        size_t workspace_bytes, int64_t* host_counts, const void* x, void* stream);
 
 /* Size of the device array behind nanoep_layout_static (4 MiB on every GPU the library runs on). */
 #define NANOEP_STATIC_SCRATCH_BYTES (4u << 20)

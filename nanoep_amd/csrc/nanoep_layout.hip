@@ -21,6 +21,7 @@ namespace {
 struct Knobs {
     int window_tokens;
     int layout_launches;
+    int dispatch_prefetch;
     int xcds;
     int64_t l2_bytes;
 };
@@ -28,7 +29,7 @@ struct Knobs {
 Knobs current_knobs() {
     const Tuning tuning = current_tuning();
     const Topology topology = current_topology(tuning);
-    return {tuning.window_tokens, tuning.layout_launches, topology.xcds, topology.l2_bytes};
+    return {tuning.window_tokens, tuning.layout_launches, tuning.dispatch_prefetch, topology.xcds, topology.l2_bytes};
 }
 
 // The slot-order buffer holds T rounded up to this many tokens' choices.
@@ -129,6 +130,18 @@ int layout_histogram_tokens(int64_t tokens_total, int window, int block_tokens, 
     return tokens;
 }
 
+// Source rows that a layout which knows of them reads ahead for the dispatch behind it (read_source_ahead): bytes read beside
+// the histogram rows and beside the assignment.  Both launches leave most of the device idle and wait for round trips,
+// not for bytes, until the reads go on longer than they do: a pass with nothing / 4 + 0 / 8 + 0 / 16 + 0 / 4 + 4 / 8 + 4 / 8 + 8 MiB,
+// 1537 x 2816 top-6 32.85 / 32.34 / 31.98 / 31.96 / 31.70 / 31.90 / 31.88 us, 4096 x 4096 top-2 40.89 / 40.79 / 41.12 / 41.16 / 40.69 /
+// 40.46 / 41.09, 4096 x 7168 top-8 158.9 / 158.3 / 157.8 / 157.8 / 157.8 / 157.6 / 157.8, 8192 x 2048 top-8 123.4 / 122.7 / 122.6 / 122.4 /
+// 122.6 / 122.1 / 122.5, 32768 x 512 top-8 99.4 / 99.2 / 98.9 / 99.2 / 99.1 / 98.4 / 98.5; with one launch, 0 / 4 / 8 MiB beside it, 800 x 7168
+// top-8 39.2 / 38.6 / 38.7, 512 x 4096 top-8 24.0 / 23.8 / 24.1.
+constexpr int64_t kHistogramAheadBytes = int64_t{8} << 20;
+constexpr int64_t kAssignAheadBytes = int64_t{4} << 20;
+// Vectors a lane of the workgroups that read ahead has in flight.
+constexpr int kAheadLoads = 8;
+
 // What a histogram row holds besides its counts.
 struct RowInfo {
     uint32_t received;  // tokens with any valid choice
@@ -211,6 +224,38 @@ struct LayoutArgs {
     uint64_t list_entries;  // of the slot-order buffer, without its count word
     uint32_t blocks;
 };
+
+// Workgroups behind a layout launch's own: they read the rows that the dispatch of this batch starts with.  The dispatch
+// gives every XCD a contiguous share of the windows, so workgroup b (on XCD b % count) reads on from the start of that
+// XCD's share: its L2 then holds the first rows of the XCD's first window before the dispatch is launched, and the last-level cache
+// what does not fit.  Nothing depends on these reads.
+struct SourceAhead {
+    const u32x4* x;        // [T][row vectors], or null
+    uint32_t work_blocks;  // workgroups of the launch's own
+    uint32_t vectors;      // of all source rows
+    uint32_t share;        // of an XCD's part of them
+    uint32_t first;        // of a share that this launch begins with
+    XcdMap xcds;
+};
+
+__device__ __forceinline__ void read_source_ahead(const SourceAhead& s, uint32_t waves) {
+    const uint32_t ordinal = fast_divide(blockIdx.x - s.work_blocks, s.xcds.magic, s.xcds.shift);
+    const uint32_t xcd = blockIdx.x - fast_divide(blockIdx.x, s.xcds.magic, s.xcds.shift) * s.xcds.count;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const uint64_t in_share = s.first + (static_cast<uint64_t>(ordinal) * waves + wave) * (kAheadLoads * kWave);
+    const uint64_t first = static_cast<uint64_t>(xcd) * s.share + in_share;
+    if (in_share >= s.share || first >= s.vectors)
+        return;
+    u32x4 fetched[kAheadLoads];
+#pragma unroll
+    for (int u = 0; u < kAheadLoads; ++u) {
+        const uint64_t from = first + u * kWave + threadIdx.x % kWave;
+        fetched[u] = s.x[from < s.vectors ? from : first];
+    }
+#pragma unroll
+    for (int u = 0; u < kAheadLoads; ++u)
+        asm volatile("" ::"v"(fetched[u].x), "v"(fetched[u].y), "v"(fetched[u].z), "v"(fetched[u].w));
+}
 
 // Where an assignment workgroup gets the counts of the other workgroups' tokens from.
 enum LayoutSource {
@@ -310,10 +355,15 @@ __device__ __forceinline__ void fetch_layout_arguments(const LayoutArgs& a) {
 
 // One histogram row: the experts' counts among `row_tokens` tokens, and their RowInfo.  Rows behind the
 // batch's end come out zero.
-__global__ void __launch_bounds__(kLayoutThreads) layout_histogram_kernel(const LayoutArgs a, const uint32_t waves) {
+__global__ void __launch_bounds__(kLayoutThreads) layout_histogram_kernel(const LayoutArgs a, const uint32_t waves, const SourceAhead ahead) {
     extern __shared__ __align__(16) uint32_t histogram_lds[];
     __shared__ RowInfo info;
     NANOEP_FETCH_ARGS_4(a.topk_idx, a.experts, a.check_tokens, waves);
+    NANOEP_FETCH_ARGS_2(ahead.x, ahead.work_blocks);
+    if (blockIdx.x >= ahead.work_blocks) {
+        read_source_ahead(ahead, waves);
+        return;
+    }
     const uint32_t words = a.check_tokens / 32;
     const uint32_t counter_words = (a.experts + 3) / 4 * 4;
     uint32_t* counts = histogram_lds;                // [L]
@@ -668,9 +718,14 @@ __device__ __forceinline__ void publish_layout(const LayoutArgs& a, uint32_t* ld
 // (token) of row (expert) is set when the token chose it.  A token's choices are distinct, so the order
 // of an expert's assignments is the token order and the rank is the number of bits below the token's.
 template <int kSource, bool kWindow, int kOwn>
-__global__ void __launch_bounds__(kLayoutThreads) layout_assign_kernel(const LayoutArgs a) {
+__global__ void __launch_bounds__(kLayoutThreads) layout_assign_kernel(const LayoutArgs a, const SourceAhead ahead) {
     extern __shared__ __align__(16) uint32_t assign_lds[];
     fetch_layout_arguments(a);
+    NANOEP_FETCH_ARGS_2(ahead.x, ahead.work_blocks);
+    if (blockIdx.x >= ahead.work_blocks) {
+        read_source_ahead(ahead, a.waves);
+        return;
+    }
     __shared__ uint32_t wave_padded[kLayoutWaves], wave_window[kLayoutWaves];
     __shared__ uint32_t any_bits[kMaxBlockTokens / 32];  // the block's tokens with any valid choice
     __shared__ struct {
@@ -992,12 +1047,13 @@ int check_layout_arguments(const int64_t* topk_idx, int64_t num_tokens, int num_
     return NANOEP_OK;
 }
 
-// Enqueues the layout launches over a carved workspace; the arguments have been checked.
+// Enqueues the layout launches over a carved workspace; the arguments have been checked.  x: the rows that will be
+// dispatched right behind the layout, or null.
 int enqueue_layout(const int64_t* topk_idx, int64_t num_tokens, int num_topk, int64_t num_local_experts, int64_t alignment,
                    int expand, int hidden, int32_t* recv_metadata, int64_t* expert_counts, int64_t* expert_offsets,
                    int64_t* dst_slots, int64_t* send_counts, int64_t* topk_snapshot, int64_t* recv_rank_prefix,
                    int32_t* token_slots, int64_t* slot_order, const LayoutWorkspace& ws, int64_t* host_counts,
-                   void* stream_handle, const Knobs& knobs) {
+                   const void* x, void* stream_handle, const Knobs& knobs) {
     const int window = layout_window_tokens(num_tokens, hidden, knobs);
     const int block_tokens = layout_block_tokens_of(num_tokens, window, num_topk, num_local_experts);
     const int64_t blocks = (num_tokens + block_tokens - 1) / block_tokens;
@@ -1087,13 +1143,35 @@ int enqueue_layout(const int64_t* topk_idx, int64_t num_tokens, int num_topk, in
     a.list_entries = static_cast<uint64_t>((num_tokens + kOrderTokens - 1) / kOrderTokens * kOrderTokens) * num_topk;
     a.blocks = static_cast<uint32_t>(blocks);
 
+    SourceAhead ahead{};
+    ahead.xcds = make_xcd_map(knobs.xcds);
+    const int64_t row_vectors = hidden / 8;
+    const int64_t window_rows = (num_tokens + window - 1) / window * window;
+    if (x != nullptr && window_rows * row_vectors < (int64_t{1} << 31)) {
+        ahead.x = static_cast<const u32x4*>(x);
+        ahead.vectors = static_cast<uint32_t>(num_tokens * row_vectors);
+        ahead.share = static_cast<uint32_t>((window_rows + ahead.xcds.count - 1) / ahead.xcds.count * row_vectors);
+    }
+    // Workgroups that read up to `bytes` more of the rows behind a launch's own, as many on every XCD.
+    const auto blocks_ahead = [&](unsigned work_blocks, int block_waves, int64_t bytes) {
+        ahead.work_blocks = work_blocks;
+        const int64_t left = ahead.share > ahead.first ? ahead.share - ahead.first : 0;
+        const int64_t most = (left + kAheadLoads * kWave - 1) / (kAheadLoads * kWave);  // (wavefronts a share)
+        const int64_t waves_an_xcd = bytes / (int64_t{kAheadLoads * kWave} * 16) / ahead.xcds.count;
+        const int64_t blocks_an_xcd = ((most < waves_an_xcd ? most : waves_an_xcd) + block_waves - 1) / block_waves;
+        return ahead.x == nullptr ? 0u : static_cast<unsigned>(blocks_an_xcd * ahead.xcds.count);
+    };
+
     __atomic_store_n(&host_counts[0], int64_t{-1}, __ATOMIC_RELEASE);
     if (source != kDirect && histogram_rows > 0) {
         int64_t row_waves = (static_cast<int64_t>(histogram_tokens) + chunk_tokens - 1) / chunk_tokens;
         row_waves = row_waves < 2 ? 2 : row_waves > kLayoutWaves ? kLayoutWaves : row_waves;
-        layout_histogram_kernel<<<a.row_batches * kSumRows, static_cast<unsigned>(row_waves * kWave),
-                                  layout_lds(num_local_experts, check_tokens / 32), stream>>>(a, static_cast<uint32_t>(row_waves));
+        const unsigned row_blocks = a.row_batches * kSumRows;
+        const unsigned more = blocks_ahead(row_blocks, static_cast<int>(row_waves), kHistogramAheadBytes);
+        layout_histogram_kernel<<<row_blocks + more, static_cast<unsigned>(row_waves * kWave),
+                                  layout_lds(num_local_experts, check_tokens / 32), stream>>>(a, static_cast<uint32_t>(row_waves), ahead);
         NANOEP_HIP_TRY(hipGetLastError());
+        ahead.first = static_cast<uint32_t>(more / ahead.xcds.count * row_waves * (kAheadLoads * kWave));
     }
     if (source == kScanned) {
         layout_scan_kernel<<<1, kScanThreads, static_cast<size_t>(num_local_experts + 1) * 4, stream>>>(a);
@@ -1101,15 +1179,16 @@ int enqueue_layout(const int64_t* topk_idx, int64_t num_tokens, int num_topk, in
         if (blocks == 0)
             return NANOEP_OK;
     }
-    const dim3 grid(static_cast<unsigned>(blocks + (source == kScanned ? 0 : 1)));
+    const unsigned assign_blocks = static_cast<unsigned>(blocks + (source == kScanned ? 0 : 1));
+    const dim3 grid(assign_blocks + blocks_ahead(assign_blocks, waves, kAssignAheadBytes));
     const size_t lds = layout_lds(num_local_experts, source == kDirect && batch_words > block_tokens / 32 ? batch_words : block_tokens / 32);
     const bool several = window > block_tokens;
 #define NANOEP_LAUNCH_ASSIGN(SOURCE, OWN)                                                       \
     do {                                                                                        \
         if (several)                                                                            \
-            layout_assign_kernel<SOURCE, true, OWN><<<grid, threads, lds, stream>>>(a);         \
+            layout_assign_kernel<SOURCE, true, OWN><<<grid, threads, lds, stream>>>(a, ahead);         \
         else                                                                                    \
-            layout_assign_kernel<SOURCE, false, OWN><<<grid, threads, lds, stream>>>(a);        \
+            layout_assign_kernel<SOURCE, false, OWN><<<grid, threads, lds, stream>>>(a, ahead);        \
     } while (0)
     if (source == kDirect)
         NANOEP_LAUNCH_ASSIGN(kDirect, 1);
@@ -1340,20 +1419,32 @@ int nanoep_layout(const int64_t* topk_idx, int64_t num_tokens, int num_topk, int
                   int64_t* expert_offsets, int64_t* dst_slots, int64_t* send_counts, int64_t* topk_snapshot,
                   int64_t* recv_rank_prefix, int32_t* token_slots, int64_t* slot_order, void* workspace,
                   size_t workspace_bytes, int64_t* host_counts, void* stream_handle) {
+    return nanoep_layout_ahead(topk_idx, num_tokens, num_topk, num_local_experts, alignment, expand, hidden, recv_metadata,
+                               expert_counts, expert_offsets, dst_slots, send_counts, topk_snapshot, recv_rank_prefix, token_slots,
+                               slot_order, workspace, workspace_bytes, host_counts, nullptr, stream_handle);
+}
+
+int nanoep_layout_ahead(const int64_t* topk_idx, int64_t num_tokens, int num_topk, int64_t num_local_experts,
+                        int64_t alignment, int expand, int hidden, int32_t* recv_metadata, int64_t* expert_counts,
+                        int64_t* expert_offsets, int64_t* dst_slots, int64_t* send_counts, int64_t* topk_snapshot,
+                        int64_t* recv_rank_prefix, int32_t* token_slots, int64_t* slot_order, void* workspace,
+                        size_t workspace_bytes, int64_t* host_counts, const void* x, void* stream_handle) {
     const Knobs knobs = current_knobs();
     const int status = check_layout_arguments(topk_idx, num_tokens, num_topk, num_local_experts, alignment, expand, hidden,
                                               recv_metadata, expert_counts, expert_offsets, dst_slots, send_counts, topk_snapshot,
                                               recv_rank_prefix, slot_order, host_counts);
     if (status != NANOEP_OK)
         return status;
-    if (workspace == nullptr)
+    if (workspace == nullptr || (x != nullptr && (hidden % 8 != 0 || !aligned16(x))))
         return NANOEP_ERR_INVALID_ARGUMENT;
     const LayoutWorkspace ws = carve_layout_workspace(workspace, num_tokens, num_topk, num_local_experts, knobs);
     if (ws.bytes > workspace_bytes)
         return NANOEP_ERR_WORKSPACE;
+    // only the slot-order walk takes the rows window by window
+    const bool reads_ahead = slot_order != nullptr && knobs.dispatch_prefetch != 0;
     return enqueue_layout(topk_idx, num_tokens, num_topk, num_local_experts, alignment, expand, hidden, recv_metadata, expert_counts,
                           expert_offsets, dst_slots, send_counts, topk_snapshot, recv_rank_prefix, token_slots, slot_order, ws,
-                          host_counts, stream_handle, knobs);
+                          host_counts, reads_ahead ? x : nullptr, stream_handle, knobs);
 }
 
 int nanoep_layout_static(const int64_t* topk_idx, int64_t num_tokens, int num_topk, int64_t num_local_experts,
@@ -1379,7 +1470,7 @@ int nanoep_layout_static(const int64_t* topk_idx, int64_t num_tokens, int num_to
     const LayoutWorkspace ws = carve_layout_workspace(base, num_tokens, num_topk, num_local_experts, knobs);
     return enqueue_layout(topk_idx, num_tokens, num_topk, num_local_experts, alignment, expand, hidden, recv_metadata, expert_counts,
                           expert_offsets, dst_slots, send_counts, topk_snapshot, recv_rank_prefix, token_slots, slot_order, ws,
-                          host_counts, stream_handle, knobs);
+                          host_counts, nullptr, stream_handle, knobs);
 }
 
 size_t nanoep_rebuild_workspace_bytes(int64_t num_tokens, int num_topk) {

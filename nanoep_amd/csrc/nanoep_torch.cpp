@@ -1196,10 +1196,11 @@ DispatchResult dispatch(PeerRuntime& runtime,
         const auto workspace = runtime.layout_workspace(workspace_bytes, comm.stream(), here);
         turn.begin();
         const int layout_status =
-            nanoep_layout(routing.data_ptr<int64_t>(), tokens, static_cast<int>(topk), local_experts, alignment, expand ? 1 : 0,
-                          static_cast<int>(hidden), base32, base64, base64 + at_offsets, base64 + at_dst, base64 + at_send, base64 + at_snapshot,
-                          base64 + at_prefix, expand ? base32 + at_table : nullptr, order_entries > 0 ? base64 + at_order : nullptr,
-                          workspace.data_ptr(), workspace_bytes, turn.mailbox(), comm.stream());
+            nanoep_layout_ahead(routing.data_ptr<int64_t>(), tokens, static_cast<int>(topk), local_experts, alignment, expand ? 1 : 0,
+                                static_cast<int>(hidden), base32, base64, base64 + at_offsets, base64 + at_dst, base64 + at_send,
+                                base64 + at_snapshot, base64 + at_prefix, expand ? base32 + at_table : nullptr,
+                                order_entries > 0 ? base64 + at_order : nullptr, workspace.data_ptr(), workspace_bytes, turn.mailbox(),
+                                tokens > 0 ? x.data_ptr() : nullptr, comm.stream());
         if (layout_status != NANOEP_OK && layout_status != NANOEP_ERR_HIP)
             turn.abandon();  // refused before anything was enqueued
         check_status(layout_status, "layout");

@@ -93,6 +93,18 @@ def test_argument_checks_come_before_any_device_work():
     assert library.nanoep_wait_counts(null, null, 0.0, out) == 1
 
 
+def test_layout_with_source_rows_checks_them_before_any_device_work():
+    library = cabi.lib()
+    ahead = library.nanoep_layout_ahead
+    ahead.argtypes = [*library.nanoep_layout.argtypes[:-1], ctypes.c_void_p, ctypes.c_void_p]
+    null = None
+    # what nanoep_layout refuses; no workspace; rows that are not 16-byte aligned; a row width that is no multiple of 8
+    assert ahead(null, -1, 2, 4, 1, 0, 256, null, null, null, null, null, null, null, null, null, null, 0, null, 64, null) == 1
+    assert ahead(8, 4, 2, 4, 1, 1, 256, 8, 8, 8, 8, 8, 8, 8, 8, 8, null, 0, 8, 64, null) == 1
+    assert ahead(8, 4, 2, 4, 1, 1, 256, 8, 8, 8, 8, 8, 8, 8, 8, 8, 8, 1 << 20, 8, 72, null) == 1
+    assert ahead(8, 4, 2, 4, 1, 1, 252, 8, 8, 8, 8, 8, 8, 8, 8, 8, 8, 1 << 20, 8, 64, null) == 1
+
+
 def test_tuning_switches_are_set_through_the_abi_and_read_from_the_environment_once(monkeypatch):
     """The switches are parsed from NANOEP_<NAME> once; afterwards only nanoep_set_tuning changes
     them (an environment variable set later is not seen until nanoep_reset_tuning reads it)."""

@@ -1,5 +1,6 @@
 """GPU tests at the edges of single kernel paths, against the CPU oracle (bit for bit)."""
 
+import ctypes
 import threading
 import time
 import weakref
@@ -87,6 +88,30 @@ def test_every_layout_plan_reports_bad_routing(device, tuning, launches, token, 
     idx[token, 4] = idx[token, 0] if bad is None else bad
     _, counts = cabi.layout(idx.to(device), 24, 1, True, raise_on_routing=False)
     assert counts[3] == status
+
+
+# A layout that is told of the rows reads the first of them beside its own work: rows fewer than a wavefront reads, XCD shares
+# that end inside one, as many rows as are read beside the first launch and one more, more than both launches read, one
+# launch and three.  The layout is the same, and so are the rows.
+@pytest.mark.parametrize("xcds", [0, 3, 16])
+@pytest.mark.parametrize(
+    "tokens,hidden,topk,launches",
+    [(1, 8, 2, 0), (33, 256, 5, 0), (257, 1032, 3, 2), (2048, 2048, 8, 2), (2049, 2048, 4, 3), (4100, 2816, 6, 0), (700, 7168, 8, 1)],
+)
+def test_layout_that_reads_source_rows_ahead(device, tuning, monkeypatch, tokens, hidden, topk, launches, xcds):
+    tuning("XCDS", xcds)
+    tuning("LAYOUT_LAUNCHES", launches)
+    library = cabi.lib()
+    ahead = library.nanoep_layout_ahead
+    ahead.argtypes = [*library.nanoep_layout.argtypes[:-1], ctypes.c_void_p, ctypes.c_void_p]
+    x = cases.payload(tokens, hidden, seed=tokens)
+    rows = x.to(device)
+    monkeypatch.setattr(library, "nanoep_layout", lambda *args: ahead(*args[:-1], rows.data_ptr(), args[-1]))
+    idx = cases.routing("dropout", tokens, 24, topk, seed=tokens)
+    for expand in (True, False):
+        metadata, counts = cabi.layout(idx.to(device), 24, 16, expand, hidden=hidden)
+        assert_layout(metadata, counts, oracle.layout(idx, 24, 16), expand, hidden)
+    assert_same_bits(rows, x)
 
 
 def small_case(device, seed, tokens=96, hidden=512, experts=12, topk=4):
