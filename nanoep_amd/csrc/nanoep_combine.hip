@@ -266,11 +266,14 @@ __global__ void __launch_bounds__(kWave) combine_held_kernel(const u32x4* __rest
                                                              uint32_t side_blocks,
                                                              uint32_t units,        // tokens a wavefront, at most kUnits
                                                              uint32_t first_scale,  // first token of a wavefront = group * first_scale
-                                                             uint32_t stride) {     // distance between a wavefront's tokens
+                                                             uint32_t stride,       // distance between a wavefront's tokens
+                                                             uint32_t per_xcd,      // payload workgroups an XCD takes in a row, 0: dealt one by one
+                                                             XcdMap xcds) {
     NANOEP_FETCH_ARGS_4(y, token_slots, out_x, bias);
     NANOEP_FETCH_ARGS_4(tokens, y_rows, chunks, chunks_magic);
     NANOEP_FETCH_ARGS_4(chunks_shift, vectors, topk, flags);
     NANOEP_FETCH_ARGS_4(side_blocks, units, first_scale, stride);
+    NANOEP_FETCH_ARGS_4(per_xcd, xcds.count, xcds.magic, xcds.shift);
     const uint32_t lane = threadIdx.x;
     if (blockIdx.x < side_blocks) {
         // weights back to their (token, k): kHeldSideEntries consecutive ones a lane, in workgroups
@@ -292,8 +295,14 @@ __global__ void __launch_bounds__(kWave) combine_held_kernel(const u32x4* __rest
                 out_weights[flat + j] = restored[j];
         return;
     }
-    const uint32_t payload_block = blockIdx.x - side_blocks;
+    uint32_t payload_block = blockIdx.x - side_blocks;
+    if (per_xcd != 0) {
+        const uint32_t turn = fast_divide(payload_block, xcds.magic, xcds.shift);
+        payload_block = (payload_block - turn * xcds.count) * per_xcd + turn;
+    }
     const uint32_t group = fast_divide(payload_block, chunks_magic, chunks_shift);
+    if (per_xcd != 0 && group >= stride)
+        return;  // (the last XCD's share is cut short; there are as many groups as the stride says)
     const uint32_t chunk = payload_block - group * chunks;
     const uint32_t vector = chunk * kWave + lane;
     const bool in_row = vector < vectors;
@@ -602,12 +611,22 @@ int nanoep_combine(const void* y, const float* weights, const void* bias, const 
         const FastDivisor chunks_divisor = make_fast_divisor(static_cast<uint32_t>(chunks));
         const int64_t held_side_blocks = held_side;
         const int64_t held_groups = (num_tokens + held_units - 1) / held_units;
-        const int64_t held_blocks = held_groups * chunks + held_side_blocks;
         // A launch that is resident as a whole gives a wavefront every held_groups-th token instead of
         // consecutive ones (4096 x 7168 top-8 74.8 -> 73.6 us, 8192 x 2048 47.4 -> 46.9, 32768 x 512
         // 44.7 -> 43.5, 32768 x 1024 84.2 -> 83.7; within half a percent at 2048 x 7168, 3000 x 7168,
         // 4096 x 4096 top-16).  Launches of several rounds lose with it (16384 x 7168: 311 -> 323 us).
         const bool strided = held_groups * chunks <= held_resident;
+        // ... and, with the rows of a token fetched at once and all sixteen tokens a wavefront, every XCD a run of neighbouring
+        // groups: the rows its wavefronts read in an expert's segment at any moment are neighbours too.  Dealt one by one -> in
+        // runs, top-8: 4600 x 7168 83.7 -> 80.9 us, 8192 x 4096 84.1 -> 82.4, 16384 x 2048 83.3 -> 82.2, 32768 x 1024 83.4 -> 82.0, 60000 x
+        // 512 78.4 -> 76.5; top-7 8192 x 4096 78.0 -> 74.5, 32768 x 1024 76.7 -> 76.0.  Nine to fifteen tokens a wavefront are within a
+        // percent of level either way (4096 x 7168 72.9 -> 72.4, with segments padded to 128 level; 3600 x 7168 68.2 -> 67.9, 2800 x 7168 53.4 ->
+        // 53.9, 3300 x 7168 61.8 -> 62.2).  Fewer tokens, more rows a token, several rounds or one token a wavefront: level or
+        // slower (8192 x 2048 45.1 -> 45.4, 4000 x 5120 top-10 70.1 -> 71.0, 12000 x 2816 top-7 80.7 -> 81.4, 16384 x 2048 top-4 47.5 -> 50.0).
+        const XcdMap xcds = make_xcd_map(topology.xcds);
+        const bool in_runs = strided && held_units == 16 && num_topk <= kHeldRows;
+        const int64_t per_xcd = in_runs ? (held_groups * chunks + xcds.count - 1) / xcds.count : 0;
+        const int64_t held_blocks = held_side_blocks + (in_runs ? per_xcd * xcds.count : held_groups * chunks);
         if (held_blocks >= (int64_t{1} << 31))
             return NANOEP_ERR_INVALID_ARGUMENT;
 #define NANOEP_LAUNCH_HELD(UNITS, TOPK)                                                                                \
@@ -616,7 +635,8 @@ int nanoep_combine(const void* y, const float* weights, const void* bias, const 
         out_weights, static_cast<uint32_t>(num_tokens), static_cast<uint32_t>(y_rows), static_cast<uint32_t>(chunks),   \
         chunks_divisor.magic, chunks_divisor.shift, static_cast<uint32_t>(vectors), static_cast<uint32_t>(num_topk), flags, \
         static_cast<uint32_t>(held_side_blocks), static_cast<uint32_t>(held_units),                                      \
-        strided ? 1u : static_cast<uint32_t>(held_units), strided ? static_cast<uint32_t>(held_groups) : 1u)
+        strided ? 1u : static_cast<uint32_t>(held_units), strided ? static_cast<uint32_t>(held_groups) : 1u,                \
+        static_cast<uint32_t>(per_xcd), xcds)
 #define NANOEP_LAUNCH_HELD_ROWS(UNITS)                     \
     switch (num_topk) {                                    \
         case 6: NANOEP_LAUNCH_HELD(UNITS, 6); break;       \

@@ -114,6 +114,23 @@ def test_layout_that_reads_source_rows_ahead(device, tuning, monkeypatch, tokens
     assert_same_bits(rows, x)
 
 
+# Sixteen held tokens a wavefront of the combine: every XCD takes a run of the groups.  Fewer workgroups than XCDs, shares that
+# come out even, a last share cut short and an empty one, a last group of one token, and side workgroups in front.
+@pytest.mark.parametrize("xcds", [0, 1, 3, 16])
+@pytest.mark.parametrize("tokens,hidden,topk", [(1, 256, 8), (16, 4096, 7), (17, 1536, 6), (129, 520, 8), (400, 2816, 8), (1009, 512, 7)])
+def test_sixteen_held_tokens_in_runs_of_groups(device, tuning, tokens, hidden, topk, xcds):
+    tuning("XCDS", xcds)
+    idx = cases.routing("dropout", tokens, 24, topk, seed=hidden)
+    lay = oracle.layout(idx, 24, 16)
+    y = cases.payload(lay.expanded_capacity, hidden, seed=tokens)
+    w = cases.gate_weights(lay.expanded_capacity, 1, seed=tokens).reshape(-1)
+    want, want_w = oracle.combine(y, lay.recv_metadata(True), lay.dst_slots, weights=w, do_expand=True)
+    metadata, counts = cabi.layout(idx.to(device), 24, 16, True, hidden=hidden)
+    got, got_w = cabi.combine(y.to(device), w.to(device), None, metadata, counts, True, poison=0xA5, units=16)
+    assert_same_bits(got, want)
+    assert_same_bits(got_w, want_w)
+
+
 def small_case(device, seed, tokens=96, hidden=512, experts=12, topk=4):
     idx = cases.routing("dropout", tokens, experts, topk, seed=seed)
     x, w = cases.payload(tokens, hidden, seed=seed), cases.gate_weights(tokens, topk, seed=seed)
