@@ -70,8 +70,9 @@ int nanoep_device_topology(int* out_cus, int* out_xcds, int64_t* out_l2_bytes);
  *   DISPATCH_SPAN (0: by size; 1 | 2 | 4 chunks a wavefront of the slot-order walk)
  *   DISPATCH_PACK (0: rows of at most 512 / 256 bytes go four / eight list entries a wavefront in
  *                     that walk; 1: one entry a wavefront whatever the row length)
- *   DISPATCH_PREFETCH (-1: on; 0: no window-wise source prefetch in that walk, and none beside the
- *                     layout, for sources that are known to sit in the last-level cache)
+ *   DISPATCH_PREFETCH (-1: window-wise source prefetch in that walk but for batches of one window; 1: there
+ *                     too; 0: none, and none beside the layout, for sources that are known to sit in the
+ *                     last-level cache)
  *   COMBINE_STORES (-1: by output size; 0 | 1: nontemporal / agent-scope stores for the combine's output)
  *   COMBINE_UNITS (0: by size; 1 .. 16 tokens a wavefront of the expanded combine with five or more
  *                     rows a token and the slot table; 1 = the one-token kernel)
@@ -226,8 +227,8 @@ int nanoep_wait_counts(int64_t* host_counts, void* stream, double timeout_second
  * -g (g > 1) for about g entries, which is cheaper when many choices are masked and correct whatever
  * A turns out to be (workgroups then take several turns).
  * The slot-order walk reads every window's source rows front to back just ahead of the window's
- * copies (unless the DISPATCH_PREFETCH switch is 0): the same bytes from HBM, as one sequential burst
- * per window instead of one row at a time among the stores.  It serves lists of fewer than 2^29
+ * copies (unless the DISPATCH_PREFETCH switch is 0, or all of the batch is one window and the device
+ * has several XCDs): the same bytes from HBM, as one sequential burst per window instead of one row at a time among the stores.  It serves lists of fewer than 2^29
  * entries and rows of up to 64 KiB; beyond either the work is walked in source-token order.
  * x / recv_x are bf16, 16-byte aligned, H % 8 == 0.  weights / recv_weights / recv_topk_idx may be
  * NULL (recv_topk_idx must be NULL when expanded).  num_cus is the reference's SM budget

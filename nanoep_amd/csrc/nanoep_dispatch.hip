@@ -707,9 +707,14 @@ int nanoep_dispatch(const void* x, const float* weights, const int32_t* recv_met
         // nearly the same number of entries each, so equal shares of the list follow them closely.
         // With sources that come from HBM it gains 5 to 22 % (rows of 512 elements most, 7168 least),
         // with sources that sit in the last-level cache it costs 0 to 4 %: on unless
-        // NANOEP_DISPATCH_PREFETCH=0.
+        // NANOEP_DISPATCH_PREFETCH=0.  A batch of one window (up to 256 tokens) goes without on a device of several XCDs: every XCD
+        // copies a part of that window, and the prefetch would bring its rows to the first one only, ahead of that XCD's copies.
+        // On -> off, sources from HBM (in the caches): 256 x 4096 top-8 5.4 -> 4.9 us (level), 256 x 7168 8.0 -> 7.6 (5.6 -> 5.3), 200 x 5120
+        // top-6 6.3 -> 5.9 (5.1 -> 4.8), 256 x 7168 top-2 5.1 -> 4.4; count on the device 256 x 7168 8.7 -> 7.7; handle in HBM 8.3 -> 7.9.
+        // (NANOEP_DISPATCH_PREFETCH=1 asks for it there too.)  With five to seven windows it depends: 257 x 7168 6.9 -> 6.3, but 384 x 4096 top-6 5.6 -> 5.8 (5.1 -> 5.5).
         const int window_tokens = nanoep_layout_block_tokens(num_tokens, num_local_experts, hidden);
-        const bool prefetch = window_tokens > 0 && copy_blocks > 0 && tuning.dispatch_prefetch != 0;
+        const bool prefetch = window_tokens > 0 && copy_blocks > 0 &&
+                              (tuning.dispatch_prefetch > 0 || (tuning.dispatch_prefetch != 0 && (num_tokens > window_tokens || xcds.count == 1)));
         // Segments are the windows of the batch; each takes the workgroups that copy its share of the
         // entries the host expects, behind the ones that read the window's rows.
         int64_t segment_entries = 0, segment_copy_blocks = 0, segment_prefetch_blocks = 0, windows = 1;

@@ -114,6 +114,15 @@ def test_layout_that_reads_source_rows_ahead(device, tuning, monkeypatch, tokens
     assert_same_bits(rows, x)
 
 
+# A batch of one window goes without the walk's prefetch on several XCDs, with it on one: the largest such batch and one token
+# more, one token, and rows that share workgroups or wavefronts, with the count on the host and on the device.
+@pytest.mark.parametrize("xcds", [0, 1])
+@pytest.mark.parametrize("tokens,hidden,topk,alignment", [(1, 512, 8, 4), (256, 4096, 3, 16), (257, 4096, 3, 16), (255, 256, 8, 1), (256, 1536, 6, 128)])
+def test_walk_of_a_batch_of_one_window(device, tuning, tokens, hidden, topk, alignment, xcds):
+    tuning("XCDS", xcds)
+    run_dispatch_combine(device, cases.routing("dropout", tokens, 24, topk, seed=hidden), hidden, 24, alignment, True, True, True)
+
+
 # Sixteen held tokens a wavefront of the combine: every XCD takes a run of the groups.  Fewer workgroups than XCDs, shares that
 # come out even, a last share cut short and an empty one, a last group of one token, and side workgroups in front.
 @pytest.mark.parametrize("xcds", [0, 1, 3, 16])
