@@ -281,3 +281,49 @@ def test_native_argument_checks_keep_the_reference_wording(device):
                 buffer.combine(torch.zeros((counts[1], hidden), dtype=torch.bfloat16, device=device), broken, None, None, expand=True)
     finally:
         buffer.close()
+
+
+# The operators' other call forms: a call with all arguments by position and of plain types is unpacked by hand, any other is
+# bound; both give the same results and refuse the same things.
+def test_operator_call_forms_agree(device):
+    native = load_extension()
+    tokens, experts, topk, hidden = 33, 8, 3, 512
+    idx = cases.routing("dropout", tokens, experts, topk, seed=4)
+    x, w = cases.payload(tokens, hidden, seed=4), cases.gate_weights(tokens, topk, seed=4)
+    buffer = ReferenceShapedBuffer(native, device, experts, topk, hidden, tokens)
+    try:
+        x_gpu, idx_gpu, w_gpu = x.to(device), idx.to(device), w.to(device)
+        stream = buffer.comm_stream.cuda_stream
+        plain = [buffer.runtime, x_gpu, idx_gpu, w_gpu, experts, tokens, 4, [], 0, False, True, True, 0, stream, -1, False]
+        names = ("runtime", "x", "indices", "weights", "num_experts", "max_tokens", "alignment", "cached_metadata", "cached_expanded_capacity",
+                 "allow_multiple_reduction", "expand", "zero_padding", "num_sms", "comm_stream", "previous_event", "async_op")
+        want_x, _, want_w, lay = oracle.dispatch(x, idx, experts, w, do_expand=True, alignment=4)
+        forms = [
+            native.dispatch(*plain),
+            native.dispatch(**dict(zip(names, plain))),
+            native.dispatch(*plain[:10], expand=True, zero_padding=True, num_sms=0, comm_stream=stream, async_op=False),
+            native.dispatch(*plain[:7], (), *plain[8:]),  # a tuple of no tensors
+        ]
+        for outputs, metadata, counts, completed in forms:
+            assert type(outputs) is list and type(metadata) is list and type(counts) is list and completed is None
+            assert counts == [lay.recv_count, lay.expanded_capacity] and len(metadata) == 9
+            assert same_bits(outputs[0], want_x) and outputs[1].numel() == 0 and same_bits(outputs[2], want_w)
+        metadata = forms[0][1]
+        want, _ = oracle.combine(want_x, lay.recv_metadata(True), lay.dst_slots, do_expand=True)
+        arguments = [buffer.runtime, forms[0][0][0], metadata, None, None, tokens, True, False, 0, stream, -1, False]
+        for call in (lambda: native.combine(*arguments), lambda: native.combine(*arguments[:2], tuple(metadata), *arguments[3:]),
+                     lambda: native.combine(*arguments[:10], async_op=False)):
+            outputs, completed = call()
+            assert type(outputs) is list and completed is None and same_bits(outputs[0], want) and outputs[1].numel() == 0
+        for position, wrong in ((0, None), (1, None), (1, [1]), (3, 1.0), (4, "8"), (4, 1 << 70), (7, [None]), (7, None), (10, "yes"), (12, 1 << 40)):
+            with pytest.raises(TypeError, match="incompatible function arguments"):
+                native.dispatch(*plain[:position], wrong, *plain[position + 1 :])
+        for position, wrong in ((0, 1), (1, None), (2, [1]), (3, "w"), (8, None)):
+            with pytest.raises(TypeError, match="incompatible function arguments"):
+                native.combine(*arguments[:position], wrong, *arguments[position + 1 :])
+        with pytest.raises(RuntimeError, match="dispatch x must be bfloat16"):
+            native.dispatch(*plain[:1], x_gpu.float(), *plain[2:])
+        with pytest.raises(RuntimeError, match="num_sms must be between 0"):
+            native.combine(*arguments[:8], -1, *arguments[9:])
+    finally:
+        buffer.close()
