@@ -22,6 +22,7 @@ struct Knobs {
     int window_tokens;
     int layout_launches;
     int dispatch_prefetch;
+    int cus;
     int xcds;
     int64_t l2_bytes;
 };
@@ -29,7 +30,7 @@ struct Knobs {
 Knobs current_knobs() {
     const Tuning tuning = current_tuning();
     const Topology topology = current_topology(tuning);
-    return {tuning.window_tokens, tuning.layout_launches, tuning.dispatch_prefetch, topology.xcds, topology.l2_bytes};
+    return {tuning.window_tokens, tuning.layout_launches, tuning.dispatch_prefetch, topology.cus, topology.xcds, topology.l2_bytes};
 }
 
 // The slot-order buffer holds T rounded up to this many tokens' choices.
@@ -130,13 +131,15 @@ int layout_histogram_tokens(int64_t tokens_total, int window, int block_tokens, 
     return tokens;
 }
 
-// Source rows that a layout which knows of them reads ahead for the dispatch behind it (read_source_ahead): bytes read beside
-// the histogram rows and beside the assignment.  Both launches leave most of the device idle and wait for round trips,
-// not for bytes, until the reads go on longer than they do: a pass with nothing / 4 + 0 / 8 + 0 / 16 + 0 / 4 + 4 / 8 + 4 / 8 + 8 MiB,
-// 1537 x 2816 top-6 32.85 / 32.34 / 31.98 / 31.96 / 31.70 / 31.90 / 31.88 us, 4096 x 4096 top-2 40.89 / 40.79 / 41.12 / 41.16 / 40.69 /
-// 40.46 / 41.09, 4096 x 7168 top-8 158.9 / 158.3 / 157.8 / 157.8 / 157.8 / 157.6 / 157.8, 8192 x 2048 top-8 123.4 / 122.7 / 122.6 / 122.4 /
-// 122.6 / 122.1 / 122.5, 32768 x 512 top-8 99.4 / 99.2 / 98.9 / 99.2 / 99.1 / 98.4 / 98.5; with one launch, 0 / 4 / 8 MiB beside it, 800 x 7168
-// top-8 39.2 / 38.6 / 38.7, 512 x 4096 top-8 24.0 / 23.8 / 24.1.
+// Source rows that a layout which knows of them reads ahead for the dispatch behind it (read_source_ahead): 4 MiB beside the
+// assignment, 8 MiB beside the histogram rows where the assignment has more than two workgroups a compute unit (there any more of
+// them wait for a place: + 2 us with as little as 2 MiB), nothing in between (16384 x 1024 top-8 55.8 -> 56.6 (level)).  Both launches wait for round trips, not for bytes, until the reads
+// go on longer than they do.  Layout and dispatch, launch period, sources from HBM (in the last-level cache), nothing -> 4 MiB
+// beside the assignment: 1537 x 2816 top-6 19.4 -> 18.8 us (18.1 -> 18.1), 2048 x 5120 top-8 34.0 -> 33.5 (31.3 -> 31.4), 4096 x 4096 top-2
+// 25.4 -> 25.2 (20.3 -> 20.2), 4096 x 7168 top-8 85.2 -> 85.1 (81.8 -> 81.4), 8192 x 2048 61.6 -> 61.4 (57.5 -> 57.1), 16384 x 2048 top-4 66.7 ->
+// 67.2 (57.7 -> 57.4); nothing -> 8 MiB beside the histogram rows: 32768 x 512 top-8 61.1 -> 61.0 (55.1 -> 54.6), 32768 x 1024 105.8 -> 105.9
+// (95.9 -> 94.9), 65536 x 512 top-4 77.8 -> 77.5 (63.3 -> 62.6).  Both, 8 + 4 MiB, gains another percent with resident sources and loses up
+// to 3 with sources from HBM (4096 x 4096 top-2 26.1, 16384 x 2048 68.4, 32768 x 1024 108.2).
 constexpr int64_t kHistogramAheadBytes = int64_t{8} << 20;
 constexpr int64_t kAssignAheadBytes = int64_t{4} << 20;
 // Vectors a lane of the workgroups that read ahead has in flight.
@@ -234,7 +237,6 @@ struct SourceAhead {
     uint32_t work_blocks;  // workgroups of the launch's own
     uint32_t vectors;      // of all source rows
     uint32_t share;        // of an XCD's part of them
-    uint32_t first;        // of a share that this launch begins with
     XcdMap xcds;
 };
 
@@ -242,7 +244,7 @@ __device__ __forceinline__ void read_source_ahead(const SourceAhead& s, uint32_t
     const uint32_t ordinal = fast_divide(blockIdx.x - s.work_blocks, s.xcds.magic, s.xcds.shift);
     const uint32_t xcd = blockIdx.x - fast_divide(blockIdx.x, s.xcds.magic, s.xcds.shift) * s.xcds.count;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const uint64_t in_share = s.first + (static_cast<uint64_t>(ordinal) * waves + wave) * (kAheadLoads * kWave);
+    const uint64_t in_share = (static_cast<uint64_t>(ordinal) * waves + wave) * (kAheadLoads * kWave);
     const uint64_t first = static_cast<uint64_t>(xcd) * s.share + in_share;
     if (in_share >= s.share || first >= s.vectors)
         return;
@@ -1143,6 +1145,8 @@ int enqueue_layout(const int64_t* topk_idx, int64_t num_tokens, int num_topk, in
     a.list_entries = static_cast<uint64_t>((num_tokens + kOrderTokens - 1) / kOrderTokens * kOrderTokens) * num_topk;
     a.blocks = static_cast<uint32_t>(blocks);
 
+    const unsigned assign_blocks = static_cast<unsigned>(blocks + (source == kScanned ? 0 : 1));
+    const unsigned rounds = source == kDirect ? 1u : (assign_blocks + static_cast<unsigned>(knobs.cus) - 1u) / static_cast<unsigned>(knobs.cus);
     SourceAhead ahead{};
     ahead.xcds = make_xcd_map(knobs.xcds);
     const int64_t row_vectors = hidden / 8;
@@ -1152,11 +1156,10 @@ int enqueue_layout(const int64_t* topk_idx, int64_t num_tokens, int num_topk, in
         ahead.vectors = static_cast<uint32_t>(num_tokens * row_vectors);
         ahead.share = static_cast<uint32_t>((window_rows + ahead.xcds.count - 1) / ahead.xcds.count * row_vectors);
     }
-    // Workgroups that read up to `bytes` more of the rows behind a launch's own, as many on every XCD.
+    // Workgroups that read up to `bytes` of the rows behind a launch's own, as many on every XCD.
     const auto blocks_ahead = [&](unsigned work_blocks, int block_waves, int64_t bytes) {
         ahead.work_blocks = work_blocks;
-        const int64_t left = ahead.share > ahead.first ? ahead.share - ahead.first : 0;
-        const int64_t most = (left + kAheadLoads * kWave - 1) / (kAheadLoads * kWave);  // (wavefronts a share)
+        const int64_t most = (int64_t{ahead.share} + kAheadLoads * kWave - 1) / (kAheadLoads * kWave);  // (wavefronts a share)
         const int64_t waves_an_xcd = bytes / (int64_t{kAheadLoads * kWave} * 16) / ahead.xcds.count;
         const int64_t blocks_an_xcd = ((most < waves_an_xcd ? most : waves_an_xcd) + block_waves - 1) / block_waves;
         return ahead.x == nullptr ? 0u : static_cast<unsigned>(blocks_an_xcd * ahead.xcds.count);
@@ -1167,11 +1170,10 @@ int enqueue_layout(const int64_t* topk_idx, int64_t num_tokens, int num_topk, in
         int64_t row_waves = (static_cast<int64_t>(histogram_tokens) + chunk_tokens - 1) / chunk_tokens;
         row_waves = row_waves < 2 ? 2 : row_waves > kLayoutWaves ? kLayoutWaves : row_waves;
         const unsigned row_blocks = a.row_batches * kSumRows;
-        const unsigned more = blocks_ahead(row_blocks, static_cast<int>(row_waves), kHistogramAheadBytes);
+        const unsigned more = blocks_ahead(row_blocks, static_cast<int>(row_waves), rounds > 2 ? kHistogramAheadBytes : 0);
         layout_histogram_kernel<<<row_blocks + more, static_cast<unsigned>(row_waves * kWave),
                                   layout_lds(num_local_experts, check_tokens / 32), stream>>>(a, static_cast<uint32_t>(row_waves), ahead);
         NANOEP_HIP_TRY(hipGetLastError());
-        ahead.first = static_cast<uint32_t>(more / ahead.xcds.count * row_waves * (kAheadLoads * kWave));
     }
     if (source == kScanned) {
         layout_scan_kernel<<<1, kScanThreads, static_cast<size_t>(num_local_experts + 1) * 4, stream>>>(a);
@@ -1179,8 +1181,7 @@ int enqueue_layout(const int64_t* topk_idx, int64_t num_tokens, int num_topk, in
         if (blocks == 0)
             return NANOEP_OK;
     }
-    const unsigned assign_blocks = static_cast<unsigned>(blocks + (source == kScanned ? 0 : 1));
-    const dim3 grid(assign_blocks + blocks_ahead(assign_blocks, waves, kAssignAheadBytes));
+    const dim3 grid(assign_blocks + blocks_ahead(assign_blocks, waves, rounds > 1 ? 0 : kAssignAheadBytes));
     const size_t lds = layout_lds(num_local_experts, source == kDirect && batch_words > block_tokens / 32 ? batch_words : block_tokens / 32);
     const bool several = window > block_tokens;
 #define NANOEP_LAUNCH_ASSIGN(SOURCE, OWN)                                                       \
