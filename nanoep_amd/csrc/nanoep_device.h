@@ -14,7 +14,8 @@
 //                          the other blocks its expert's first slot; writes the tokens' part of the
 //                          handle and of the slot-order list.  One more workgroup publishes N, C to the
 //                          host.  Small batches: every workgroup counts the batch's ids itself, and this
-//                          is the layout's only launch.
+//                          is the layout's only launch.  Told of the rows that will be dispatched, this launch or the
+//                          histogram's has workgroups that read the first of them into the caches.
 //   layout_histogram_kernel : ahead of it for larger batches: rows of per-expert counts, which every
 //                          assignment workgroup sums.
 //   layout_scan_kernel   : between the two for the largest: one workgroup turns the rows into prefixes.
@@ -88,7 +89,7 @@ struct Tuning {
     int rows_per_block = 0;         // ROWS_PER_BLOCK: rows a workgroup, 0 = by shape
     int dispatch_order = -1;        // DISPATCH_ORDER: 0 forces the token-order walk
     int dispatch_span = 0;          // DISPATCH_SPAN: 1 | 2 | 4 chunks a wavefront of the slot-order walk, 0 = by size
-    int dispatch_prefetch = -1;     // DISPATCH_PREFETCH: 0 = no window-wise source prefetch in the slot-order walk
+    int dispatch_prefetch = -1;     // DISPATCH_PREFETCH: 0 = no window-wise source prefetch in the slot-order walk, 1 = also for batches of one window
     int combine_units = 0;          // COMBINE_UNITS: tokens a wavefront of the gather for five or more rows a token: 1 .. 16, 0 = by size
     int dispatch_pack = 0;          // DISPATCH_PACK: 1 = one list entry a wavefront of the slot-order walk whatever the row length
     int combine_stores = -1;        // COMBINE_STORES: 0 | 1 nontemporal / agent-scope stores for the combine's output, -1 = by size

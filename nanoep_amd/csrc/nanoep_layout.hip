@@ -132,8 +132,9 @@ int layout_histogram_tokens(int64_t tokens_total, int window, int block_tokens, 
 }
 
 // Source rows that a layout which knows of them reads ahead for the dispatch behind it (read_source_ahead): 4 MiB beside the
-// assignment, 8 MiB beside the histogram rows where the assignment has more than two workgroups a compute unit (there any more of
-// them wait for a place: + 2 us with as little as 2 MiB), nothing in between (16384 x 1024 top-8 55.8 -> 56.6 (level)).  Both launches wait for round trips, not for bytes, until the reads
+// assignment while that has no more workgroups than the device compute units (any more of them wait for a place: + 2 us with as
+// little as 2 MiB), 8 MiB beside the histogram rows of batches whose pairs are 4096 wavefronts' (2^18) and more, nothing in between
+// (16384 x 1024 top-8 55.8 -> 56.6 (level) with 8 MiB beside the rows).  Both launches wait for round trips, not for bytes, until the reads
 // go on longer than they do.  Layout and dispatch, launch period, sources from HBM (in the last-level cache), nothing -> 4 MiB
 // beside the assignment: 1537 x 2816 top-6 19.4 -> 18.8 us (18.1 -> 18.1), 2048 x 5120 top-8 34.0 -> 33.5 (31.3 -> 31.4), 4096 x 4096 top-2
 // 25.4 -> 25.2 (20.3 -> 20.2), 4096 x 7168 top-8 85.2 -> 85.1 (81.8 -> 81.4), 8192 x 2048 61.6 -> 61.4 (57.5 -> 57.1), 16384 x 2048 top-4 66.7 ->
@@ -1146,7 +1147,8 @@ int enqueue_layout(const int64_t* topk_idx, int64_t num_tokens, int num_topk, in
     a.blocks = static_cast<uint32_t>(blocks);
 
     const unsigned assign_blocks = static_cast<unsigned>(blocks + (source == kScanned ? 0 : 1));
-    const unsigned rounds = source == kDirect ? 1u : (assign_blocks + static_cast<unsigned>(knobs.cus) - 1u) / static_cast<unsigned>(knobs.cus);
+    const bool beside_histogram = source != kDirect && pairs >= kOneChunkWaves * kWave;
+    const bool beside_assignment = !beside_histogram && (source == kDirect || assign_blocks <= static_cast<unsigned>(knobs.cus));
     SourceAhead ahead{};
     ahead.xcds = make_xcd_map(knobs.xcds);
     const int64_t row_vectors = hidden / 8;
@@ -1170,7 +1172,7 @@ int enqueue_layout(const int64_t* topk_idx, int64_t num_tokens, int num_topk, in
         int64_t row_waves = (static_cast<int64_t>(histogram_tokens) + chunk_tokens - 1) / chunk_tokens;
         row_waves = row_waves < 2 ? 2 : row_waves > kLayoutWaves ? kLayoutWaves : row_waves;
         const unsigned row_blocks = a.row_batches * kSumRows;
-        const unsigned more = blocks_ahead(row_blocks, static_cast<int>(row_waves), rounds > 2 ? kHistogramAheadBytes : 0);
+        const unsigned more = blocks_ahead(row_blocks, static_cast<int>(row_waves), beside_histogram ? kHistogramAheadBytes : 0);
         layout_histogram_kernel<<<row_blocks + more, static_cast<unsigned>(row_waves * kWave),
                                   layout_lds(num_local_experts, check_tokens / 32), stream>>>(a, static_cast<uint32_t>(row_waves), ahead);
         NANOEP_HIP_TRY(hipGetLastError());
@@ -1181,7 +1183,7 @@ int enqueue_layout(const int64_t* topk_idx, int64_t num_tokens, int num_topk, in
         if (blocks == 0)
             return NANOEP_OK;
     }
-    const dim3 grid(assign_blocks + blocks_ahead(assign_blocks, waves, rounds > 1 ? 0 : kAssignAheadBytes));
+    const dim3 grid(assign_blocks + blocks_ahead(assign_blocks, waves, beside_assignment ? kAssignAheadBytes : 0));
     const size_t lds = layout_lds(num_local_experts, source == kDirect && batch_words > block_tokens / 32 ? batch_words : block_tokens / 32);
     const bool several = window > block_tokens;
 #define NANOEP_LAUNCH_ASSIGN(SOURCE, OWN)                                                       \

@@ -91,13 +91,13 @@ def test_every_layout_plan_reports_bad_routing(device, tuning, launches, token, 
 
 
 # A layout that is told of the rows reads the first of them beside its own work: rows fewer than a wavefront reads, XCD shares
-# that end inside one, as many rows as are read and one more, one launch and three, and more assignment workgroups than the
-# device has compute units.  The layout is the same, and so are the rows.
+# that end inside one, as many rows as are read and one more, one launch and three, 2^18 pairs and a few
+# less.  The layout is the same, and so are the rows.
 @pytest.mark.parametrize("xcds", [0, 3, 16])
 @pytest.mark.parametrize(
     "tokens,hidden,topk,launches",
     [(1, 8, 2, 0), (33, 256, 5, 0), (257, 1032, 3, 2), (2048, 2048, 8, 2), (2049, 2048, 4, 3), (4100, 2816, 6, 0), (700, 7168, 8, 1),
-     (1024, 2048, 2, 0), (16500, 256, 8, 0)],
+     (1024, 2048, 2, 0), (32768, 256, 8, 0), (32767, 256, 8, 0)],
 )
 def test_layout_that_reads_source_rows_ahead(device, tuning, monkeypatch, tokens, hidden, topk, launches, xcds):
     tuning("XCDS", xcds)
