@@ -151,6 +151,9 @@ int nanoep_layout_ahead(const int64_t* topk_idx, int64_t num_tokens, int num_top
                         int64_t* recv_rank_prefix, int32_t* token_slots, int64_t* slot_order, void* workspace,
                         size_t workspace_bytes, int64_t* host_counts, const void* x, void* stream);
 
+/* Bytes of x that nanoep_layout_ahead reads for such a batch, as the device and the switches are now; 0: none.  A host function. */
+int64_t nanoep_layout_ahead_bytes(int64_t num_tokens, int num_topk, int64_t num_local_experts, int hidden);
+
 /* Size of the device array behind nanoep_layout_static (4 MiB on every GPU the library runs on). */
 #define NANOEP_STATIC_SCRATCH_BYTES (4u << 20)
 

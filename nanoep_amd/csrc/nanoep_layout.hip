@@ -4,6 +4,7 @@
 
 #include <mutex>
 
+#include "nanoep_ahead.h"
 #include "nanoep_device.h"
 
 // Device memory of nanoep_layout_static: the layout kernels' workspace (histogram
@@ -143,8 +144,6 @@ int layout_histogram_tokens(int64_t tokens_total, int window, int block_tokens, 
 // to 3 with sources from HBM (4096 x 4096 top-2 26.1, 16384 x 2048 68.4, 32768 x 1024 108.2).
 constexpr int64_t kHistogramAheadBytes = int64_t{8} << 20;
 constexpr int64_t kAssignAheadBytes = int64_t{4} << 20;
-// Vectors a lane of the workgroups that read ahead has in flight.
-constexpr int kAheadLoads = 8;
 
 // What a histogram row holds besides its counts.
 struct RowInfo {
@@ -245,16 +244,13 @@ __device__ __forceinline__ void read_source_ahead(const SourceAhead& s, uint32_t
     const uint32_t ordinal = fast_divide(blockIdx.x - s.work_blocks, s.xcds.magic, s.xcds.shift);
     const uint32_t xcd = blockIdx.x - fast_divide(blockIdx.x, s.xcds.magic, s.xcds.shift) * s.xcds.count;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const uint64_t in_share = (static_cast<uint64_t>(ordinal) * waves + wave) * (kAheadLoads * kWave);
-    const uint64_t first = static_cast<uint64_t>(xcd) * s.share + in_share;
-    if (in_share >= s.share || first >= s.vectors)
+    const AheadRange range = ahead_range(s.vectors, s.share, xcd, ordinal, waves, wave);
+    if (range.first >= range.end)
         return;
     u32x4 fetched[kAheadLoads];
 #pragma unroll
-    for (int u = 0; u < kAheadLoads; ++u) {
-        const uint64_t from = first + u * kWave + threadIdx.x % kWave;
-        fetched[u] = s.x[from < s.vectors ? from : first];
-    }
+    for (int u = 0; u < kAheadLoads; ++u)
+        fetched[u] = s.x[ahead_vector(range, u, threadIdx.x % kWave)];
 #pragma unroll
     for (int u = 0; u < kAheadLoads; ++u)
         asm volatile("" ::"v"(fetched[u].x), "v"(fetched[u].y), "v"(fetched[u].z), "v"(fetched[u].w));
@@ -1050,6 +1046,84 @@ int check_layout_arguments(const int64_t* topk_idx, int64_t num_tokens, int num_
     return NANOEP_OK;
 }
 
+// Whether a layout of this batch, told of the rows and given the slot-order list, reads any ahead.
+bool reads_ahead(int64_t num_tokens, int num_topk, int /*hidden*/, const Knobs& knobs) {
+    return num_tokens * num_topk < (int64_t{1} << 31) && knobs.dispatch_prefetch != 0;
+}
+
+// The launches of one layout, from the batch's geometry.
+struct LayoutPlan {
+    int window;
+    int block_tokens;
+    int64_t blocks;
+    int histogram_tokens;
+    int64_t histogram_rows;
+    int source;
+    int chunk_tokens;
+    int own;            // chunks of its block an assignment wavefront takes
+    int waves;          // of an assignment workgroup
+    int row_waves;      // of a histogram workgroup
+    size_t assign_lds;
+    // workgroups of the two launches, without those that read ahead
+    uint32_t row_blocks;
+    uint32_t assign_blocks;
+    // ... and those that do where the rows are known
+    AheadPlan beside_rows;
+    AheadPlan beside_assignment;
+};
+
+LayoutPlan plan_layout(int64_t num_tokens, int num_topk, int64_t num_local_experts, int hidden, const Knobs& knobs) {
+    LayoutPlan plan{};
+    plan.window = layout_window_tokens(num_tokens, hidden, knobs);
+    plan.block_tokens = layout_block_tokens_of(num_tokens, plan.window, num_topk, num_local_experts);
+    plan.blocks = (num_tokens + plan.block_tokens - 1) / plan.block_tokens;
+    plan.histogram_tokens = layout_histogram_tokens(num_tokens, plan.window, plan.block_tokens, num_topk, num_local_experts);
+    plan.histogram_rows = (num_tokens + plan.histogram_tokens - 1) / plan.histogram_tokens;
+
+    const int64_t pairs = num_tokens * num_topk;
+    const int64_t batch_words = (num_tokens + 31) / 32;
+    const int64_t block_words = plan.block_tokens / 32;
+    const size_t direct_lds = layout_lds(num_local_experts, batch_words > block_words ? batch_words : block_words);
+    const bool direct_fits = pairs < 65536 && direct_lds <= kLayoutLdsBudget;
+    plan.source = direct_fits && pairs <= kDirectPairs ? kDirect : plan.histogram_rows <= kSummedHistograms ? kSummed : kScanned;
+    if (knobs.layout_launches == 1 && direct_fits)
+        plan.source = kDirect;
+    else if (knobs.layout_launches == 2 && num_tokens > 0)
+        plan.source = kSummed;
+    else if (knobs.layout_launches == 3)
+        plan.source = kScanned;
+    plan.assign_lds = plan.source == kDirect ? direct_lds : layout_lds(num_local_experts, block_words);
+    // one or more chunks of the block a wavefront; in the direct plan enough wavefronts for the counting as well
+    plan.chunk_tokens = kWave / num_topk;
+    int waves = (plan.block_tokens + plan.chunk_tokens - 1) / plan.chunk_tokens;
+    if (plan.source == kDirect) {
+        const int64_t counting = (pairs / kChunks + kWave - 1) / kWave;
+        if (num_tokens < plan.block_tokens)
+            waves = static_cast<int>((num_tokens + plan.chunk_tokens - 1) / plan.chunk_tokens);
+        if (waves < counting)
+            waves = counting < kLayoutWaves ? static_cast<int>(counting) : kLayoutWaves;
+    }
+    plan.own = plan.source == kScanned ? kScannedChunks : plan.source == kSummed && plan.blocks * waves > kOneChunkWaves ? kSummedChunks : 1;
+    waves = (waves + plan.own - 1) / plan.own;
+    if (plan.source == kSummed) {
+        const int64_t tasks = (num_local_experts + kWave - 1) / kWave * (padded_rows(plan.histogram_rows) / kSumRows);
+        if (waves < tasks)
+            waves = tasks < 8 ? static_cast<int>(tasks) : waves < 8 ? 8 : waves;
+    }
+    plan.waves = waves < 2 ? 2 : waves;
+    const int row_waves = (plan.histogram_tokens + plan.chunk_tokens - 1) / plan.chunk_tokens;
+    plan.row_waves = row_waves < 2 ? 2 : row_waves > kLayoutWaves ? kLayoutWaves : row_waves;
+    plan.row_blocks = static_cast<uint32_t>(padded_rows(plan.histogram_rows));
+    plan.assign_blocks = static_cast<uint32_t>(plan.blocks + (plan.source == kScanned ? 0 : 1));
+
+    const int64_t row_vectors = hidden / 8, xcds = make_xcd_map(knobs.xcds).count;
+    if (plan.source != kDirect && pairs >= kOneChunkWaves * kWave)
+        plan.beside_rows = plan_ahead(num_tokens, row_vectors, plan.window, xcds, plan.row_waves, kHistogramAheadBytes);
+    else if (plan.source == kDirect || plan.assign_blocks <= static_cast<unsigned>(knobs.cus))
+        plan.beside_assignment = plan_ahead(num_tokens, row_vectors, plan.window, xcds, plan.waves, kAssignAheadBytes);
+    return plan;
+}
+
 // Enqueues the layout launches over a carved workspace; the arguments have been checked.  x: the rows that will be
 // dispatched right behind the layout, or null.
 int enqueue_layout(const int64_t* topk_idx, int64_t num_tokens, int num_topk, int64_t num_local_experts, int64_t alignment,
@@ -1057,50 +1131,16 @@ int enqueue_layout(const int64_t* topk_idx, int64_t num_tokens, int num_topk, in
                    int64_t* dst_slots, int64_t* send_counts, int64_t* topk_snapshot, int64_t* recv_rank_prefix,
                    int32_t* token_slots, int64_t* slot_order, const LayoutWorkspace& ws, int64_t* host_counts,
                    const void* x, void* stream_handle, const Knobs& knobs) {
-    const int window = layout_window_tokens(num_tokens, hidden, knobs);
-    const int block_tokens = layout_block_tokens_of(num_tokens, window, num_topk, num_local_experts);
-    const int64_t blocks = (num_tokens + block_tokens - 1) / block_tokens;
-    const int histogram_tokens = layout_histogram_tokens(num_tokens, window, block_tokens, num_topk, num_local_experts);
-    const int64_t histogram_rows = (num_tokens + histogram_tokens - 1) / histogram_tokens;
-    int check_tokens = histogram_tokens;
-    while (check_tokens > block_tokens && layout_lds(num_local_experts, check_tokens / 32) > kLayoutLdsBudget)
-        check_tokens = block_tokens;
+    const LayoutPlan plan = plan_layout(num_tokens, num_topk, num_local_experts, hidden, knobs);
+    int check_tokens = plan.histogram_tokens;
+    while (check_tokens > plan.block_tokens && layout_lds(num_local_experts, check_tokens / 32) > kLayoutLdsBudget)
+        check_tokens = plan.block_tokens;
     auto stream = static_cast<hipStream_t>(stream_handle);
-
-    const int64_t pairs = num_tokens * num_topk;
-    const int64_t batch_words = (num_tokens + 31) / 32;
-    const bool direct_fits = pairs < 65536 && layout_lds(num_local_experts, batch_words > block_tokens / 32 ? batch_words : block_tokens / 32) <= kLayoutLdsBudget;
-    int source = direct_fits && pairs <= kDirectPairs ? kDirect : histogram_rows <= kSummedHistograms ? kSummed : kScanned;
-    if (knobs.layout_launches == 1 && direct_fits)
-        source = kDirect;
-    else if (knobs.layout_launches == 2 && num_tokens > 0)
-        source = kSummed;
-    else if (knobs.layout_launches == 3)
-        source = kScanned;
-    // one or more chunks of the block a wavefront; in the direct plan enough wavefronts for the counting as well
-    const int chunk_tokens = kWave / num_topk;
-    int waves = (block_tokens + chunk_tokens - 1) / chunk_tokens;
-    if (source == kDirect) {
-        const int64_t counting = (pairs / kChunks + kWave - 1) / kWave;
-        if (num_tokens < block_tokens)
-            waves = static_cast<int>((num_tokens + chunk_tokens - 1) / chunk_tokens);
-        if (waves < counting)
-            waves = counting < kLayoutWaves ? static_cast<int>(counting) : kLayoutWaves;
-    }
-    const int own = source == kScanned ? kScannedChunks : source == kSummed && blocks * waves > kOneChunkWaves ? kSummedChunks : 1;
-    waves = (waves + own - 1) / own;
-    if (source == kSummed) {
-        const int64_t tasks = (num_local_experts + kWave - 1) / kWave * (padded_rows(histogram_rows) / kSumRows);
-        if (waves < tasks)
-            waves = tasks < 8 ? static_cast<int>(tasks) : waves < 8 ? 8 : waves;
-    }
-    if (waves < 2)
-        waves = 2;
-    const int threads = waves * kWave;
+    const int threads = plan.waves * kWave;
 
     const FastDivisor alignment_divisor = make_fast_divisor(static_cast<uint32_t>(alignment));
-    const FastDivisor row_divisor = make_fast_divisor(static_cast<uint32_t>(histogram_tokens));
-    const FastDivisor window_divisor = make_fast_divisor(static_cast<uint32_t>(window));
+    const FastDivisor row_divisor = make_fast_divisor(static_cast<uint32_t>(plan.histogram_tokens));
+    const FastDivisor window_divisor = make_fast_divisor(static_cast<uint32_t>(plan.window));
     LayoutArgs a{};
     a.topk_idx = topk_idx;
     a.histograms = ws.histograms;
@@ -1108,19 +1148,19 @@ int enqueue_layout(const int64_t* topk_idx, int64_t num_tokens, int num_topk, in
     a.tokens = static_cast<uint32_t>(num_tokens);
     a.topk = static_cast<uint32_t>(num_topk);
     a.experts = static_cast<uint32_t>(num_local_experts);
-    a.chunk_tokens = static_cast<uint32_t>(chunk_tokens);
+    a.chunk_tokens = static_cast<uint32_t>(plan.chunk_tokens);
     a.chunk_pairs = a.chunk_tokens * a.topk;
     a.topk_magic = (65536u + a.topk - 1) / a.topk;
-    a.waves = static_cast<uint32_t>(waves);
-    a.block_tokens = static_cast<uint32_t>(block_tokens);
-    a.row_tokens = static_cast<uint32_t>(histogram_tokens);
+    a.waves = static_cast<uint32_t>(plan.waves);
+    a.block_tokens = static_cast<uint32_t>(plan.block_tokens);
+    a.row_tokens = static_cast<uint32_t>(plan.histogram_tokens);
     a.row_magic = row_divisor.magic;
     a.row_shift = row_divisor.shift;
-    a.window_tokens = static_cast<uint32_t>(window);
+    a.window_tokens = static_cast<uint32_t>(plan.window);
     a.window_magic = window_divisor.magic;
     a.window_shift = window_divisor.shift;
-    a.row_count = static_cast<uint32_t>(histogram_rows);
-    a.row_batches = static_cast<uint32_t>(padded_rows(histogram_rows) / kSumRows);
+    a.row_count = static_cast<uint32_t>(plan.histogram_rows);
+    a.row_batches = plan.row_blocks / kSumRows;
     a.strips = (a.experts + kWave - 1) / kWave;
     const FastDivisor strips_divisor = make_fast_divisor(a.strips);
     a.strips_magic = strips_divisor.magic;
@@ -1144,60 +1184,46 @@ int enqueue_layout(const int64_t* topk_idx, int64_t num_tokens, int num_topk, in
     a.token_slots = token_slots;
     a.slot_order = num_tokens > 0 ? slot_order : nullptr;
     a.list_entries = static_cast<uint64_t>((num_tokens + kOrderTokens - 1) / kOrderTokens * kOrderTokens) * num_topk;
-    a.blocks = static_cast<uint32_t>(blocks);
+    a.blocks = static_cast<uint32_t>(plan.blocks);
 
-    const unsigned assign_blocks = static_cast<unsigned>(blocks + (source == kScanned ? 0 : 1));
-    const bool beside_histogram = source != kDirect && pairs >= kOneChunkWaves * kWave;
-    const bool beside_assignment = !beside_histogram && (source == kDirect || assign_blocks <= static_cast<unsigned>(knobs.cus));
     SourceAhead ahead{};
+    ahead.x = static_cast<const u32x4*>(x);
     ahead.xcds = make_xcd_map(knobs.xcds);
-    const int64_t row_vectors = hidden / 8;
-    const int64_t window_rows = (num_tokens + window - 1) / window * window;
-    if (x != nullptr && window_rows * row_vectors < (int64_t{1} << 31)) {
-        ahead.x = static_cast<const u32x4*>(x);
-        ahead.vectors = static_cast<uint32_t>(num_tokens * row_vectors);
-        ahead.share = static_cast<uint32_t>((window_rows + ahead.xcds.count - 1) / ahead.xcds.count * row_vectors);
-    }
-    // Workgroups that read up to `bytes` of the rows behind a launch's own, as many on every XCD.
-    const auto blocks_ahead = [&](unsigned work_blocks, int block_waves, int64_t bytes) {
+    // Workgroups of a launch with those that read ahead.
+    const auto with_ahead = [&](uint32_t work_blocks, const AheadPlan& beside) {
         ahead.work_blocks = work_blocks;
-        const int64_t most = (int64_t{ahead.share} + kAheadLoads * kWave - 1) / (kAheadLoads * kWave);  // (wavefronts a share)
-        const int64_t waves_an_xcd = bytes / (int64_t{kAheadLoads * kWave} * 16) / ahead.xcds.count;
-        const int64_t blocks_an_xcd = ((most < waves_an_xcd ? most : waves_an_xcd) + block_waves - 1) / block_waves;
-        return ahead.x == nullptr ? 0u : static_cast<unsigned>(blocks_an_xcd * ahead.xcds.count);
+        ahead.vectors = beside.vectors;
+        ahead.share = beside.share;
+        return work_blocks + (x == nullptr ? 0u : beside.blocks);
     };
 
     __atomic_store_n(&host_counts[0], int64_t{-1}, __ATOMIC_RELEASE);
-    if (source != kDirect && histogram_rows > 0) {
-        int64_t row_waves = (static_cast<int64_t>(histogram_tokens) + chunk_tokens - 1) / chunk_tokens;
-        row_waves = row_waves < 2 ? 2 : row_waves > kLayoutWaves ? kLayoutWaves : row_waves;
-        const unsigned row_blocks = a.row_batches * kSumRows;
-        const unsigned more = blocks_ahead(row_blocks, static_cast<int>(row_waves), beside_histogram ? kHistogramAheadBytes : 0);
-        layout_histogram_kernel<<<row_blocks + more, static_cast<unsigned>(row_waves * kWave),
-                                  layout_lds(num_local_experts, check_tokens / 32), stream>>>(a, static_cast<uint32_t>(row_waves), ahead);
+    if (plan.source != kDirect && plan.histogram_rows > 0) {
+        const uint32_t grid = with_ahead(plan.row_blocks, plan.beside_rows);
+        layout_histogram_kernel<<<grid, plan.row_waves * kWave, layout_lds(num_local_experts, check_tokens / 32), stream>>>(
+            a, static_cast<uint32_t>(plan.row_waves), ahead);
         NANOEP_HIP_TRY(hipGetLastError());
     }
-    if (source == kScanned) {
+    if (plan.source == kScanned) {
         layout_scan_kernel<<<1, kScanThreads, static_cast<size_t>(num_local_experts + 1) * 4, stream>>>(a);
         NANOEP_HIP_TRY(hipGetLastError());
-        if (blocks == 0)
+        if (plan.blocks == 0)
             return NANOEP_OK;
     }
-    const dim3 grid(assign_blocks + blocks_ahead(assign_blocks, waves, beside_assignment ? kAssignAheadBytes : 0));
-    const size_t lds = layout_lds(num_local_experts, source == kDirect && batch_words > block_tokens / 32 ? batch_words : block_tokens / 32);
-    const bool several = window > block_tokens;
+    const dim3 grid(with_ahead(plan.assign_blocks, plan.beside_assignment));
+    const bool several = plan.window > plan.block_tokens;
 #define NANOEP_LAUNCH_ASSIGN(SOURCE, OWN)                                                       \
     do {                                                                                        \
         if (several)                                                                            \
-            layout_assign_kernel<SOURCE, true, OWN><<<grid, threads, lds, stream>>>(a, ahead);         \
+            layout_assign_kernel<SOURCE, true, OWN><<<grid, threads, plan.assign_lds, stream>>>(a, ahead);  \
         else                                                                                    \
-            layout_assign_kernel<SOURCE, false, OWN><<<grid, threads, lds, stream>>>(a, ahead);        \
+            layout_assign_kernel<SOURCE, false, OWN><<<grid, threads, plan.assign_lds, stream>>>(a, ahead); \
     } while (0)
-    if (source == kDirect)
+    if (plan.source == kDirect)
         NANOEP_LAUNCH_ASSIGN(kDirect, 1);
-    else if (source == kSummed && own == 1)
+    else if (plan.source == kSummed && plan.own == 1)
         NANOEP_LAUNCH_ASSIGN(kSummed, 1);
-    else if (source == kSummed)
+    else if (plan.source == kSummed)
         NANOEP_LAUNCH_ASSIGN(kSummed, kSummedChunks);
     else
         NANOEP_LAUNCH_ASSIGN(kScanned, kScannedChunks);
@@ -1409,6 +1435,19 @@ int nanoep_layout_block_tokens(int64_t num_tokens, int64_t num_local_experts, in
     return layout_supports(num_local_experts) ? layout_window_tokens(num_tokens, hidden, current_knobs()) : 0;
 }
 
+int64_t nanoep_layout_ahead_bytes(int64_t num_tokens, int num_topk, int64_t num_local_experts, int hidden) {
+    if (num_tokens <= 0 || num_tokens > INT32_MAX || num_topk <= 0 || num_topk > kMaxTopk || !layout_supports(num_local_experts) || hidden <= 0 ||
+        hidden % 8 != 0)
+        return 0;
+    const Knobs knobs = current_knobs();
+    if (!reads_ahead(num_tokens, num_topk, hidden, knobs))
+        return 0;
+    const LayoutPlan plan = plan_layout(num_tokens, num_topk, num_local_experts, hidden, knobs);
+    const uint32_t xcds = make_xcd_map(knobs.xcds).count;
+    return ahead_bytes(plan.beside_rows, plan.row_blocks, xcds, plan.row_waves) +
+           ahead_bytes(plan.beside_assignment, plan.assign_blocks, xcds, plan.waves);
+}
+
 int64_t nanoep_slot_order_entries(int64_t num_tokens, int num_topk, int64_t num_local_experts) {
     if (num_tokens < 0 || num_topk <= 0 || num_local_experts <= 0)
         return 0;
@@ -1443,11 +1482,10 @@ int nanoep_layout_ahead(const int64_t* topk_idx, int64_t num_tokens, int num_top
     const LayoutWorkspace ws = carve_layout_workspace(workspace, num_tokens, num_topk, num_local_experts, knobs);
     if (ws.bytes > workspace_bytes)
         return NANOEP_ERR_WORKSPACE;
-    // only the slot-order walk takes the rows window by window
-    const bool reads_ahead = slot_order != nullptr && knobs.dispatch_prefetch != 0;
+    const bool ahead = x != nullptr && slot_order != nullptr && reads_ahead(num_tokens, num_topk, hidden, knobs);
     return enqueue_layout(topk_idx, num_tokens, num_topk, num_local_experts, alignment, expand, hidden, recv_metadata, expert_counts,
                           expert_offsets, dst_slots, send_counts, topk_snapshot, recv_rank_prefix, token_slots, slot_order, ws,
-                          host_counts, reads_ahead ? x : nullptr, stream_handle, knobs);
+                          host_counts, ahead ? x : nullptr, stream_handle, knobs);
 }
 
 int nanoep_layout_static(const int64_t* topk_idx, int64_t num_tokens, int num_topk, int64_t num_local_experts,

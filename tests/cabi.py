@@ -45,6 +45,8 @@ def lib() -> ctypes.CDLL:
         handle.nanoep_layout_block_tokens.argtypes = [i64, i64, i]
         handle.nanoep_slot_order_entries.restype = i64
         handle.nanoep_slot_order_entries.argtypes = [i64, i, i64]
+        handle.nanoep_layout_ahead_bytes.restype = i64
+        handle.nanoep_layout_ahead_bytes.argtypes = [i64, i, i64, i]
         handle.nanoep_layout.argtypes = [p, i64, i, i64, i64, i, i, p, p, p, p, p, p, p, p, p, p, sz, p, p]
         handle.nanoep_layout_static.argtypes = [p, i64, i, i64, i64, i, i, p, p, p, p, p, p, p, p, p, p, p]
         handle.nanoep_wait_counts.argtypes = [p, p, dbl, ctypes.POINTER(i64)]
