@@ -141,8 +141,10 @@ int nanoep_layout(const int64_t* topk_idx, int64_t num_tokens, int num_topk, int
 /*
  * nanoep_layout for a caller that dispatches x (bf16 [T, hidden], 16-byte aligned, hidden % 8 == 0) right behind it on the
  * same stream: the layout's launches leave most of the device idle, and workgroups of their own read the first rows of x
- * there, which the dispatch then finds in the caches.  Results are nanoep_layout's.  x is only read, and only ahead of a
- * slot-order walk with its prefetch (slot_order given, DISPATCH_PREFETCH not 0).  NULL for x is nanoep_layout.
+ * there, which the dispatch then finds in the caches.  Results are nanoep_layout's.  x is only read, and only where the
+ * dispatch will walk the slot-order list (slot_order given; not DISPATCH_ORDER 0, nor rows and lists that nanoep_dispatch walks in
+ * source-token order), DISPATCH_PREFETCH is not 0 and the launches have room: nanoep_layout_ahead_bytes says how much.  Batches of one window, whose
+ * walk goes without a prefetch of its own, are read ahead too.  NULL for x is nanoep_layout.
  * It has no counterpart in the reference.
  */
 int nanoep_layout_ahead(const int64_t* topk_idx, int64_t num_tokens, int num_topk, int64_t num_local_experts,

@@ -643,21 +643,10 @@ int nanoep_dispatch(const void* x, const float* weights, const int32_t* recv_met
     const int64_t order_bound = nanoep_slot_order_entries(num_tokens, num_topk, num_local_experts) - 1;
     const int vectors = hidden / 8;
     const int row_chunks = (vectors + kWave - 1) / kWave;
-    // The slot-order walk is used whenever the handle carries the list.  With cache-resident sources and
-    // fewer than eight token blocks the token-order walk is up to 15 % faster, but with cold sources
-    // it is 25-60 % slower at every size, so the list decides.  A wavefront moves one 1 KiB chunk; two
-    // once the source outgrows the last-level cache (the single-chunk walk then loses a quarter of
-    // its rate) and as many as it takes for a row to fit the 16 wavefronts of a workgroup
-    // (NANOEP_DISPATCH_SPAN=1|2|4 asks for a number).  The walk addresses the list with 32-bit byte
-    // offsets: list buffers of 2^29 entries and more, and rows beyond 64 KiB, take the token-order walk.
-    int span = static_cast<int64_t>(num_tokens) * hidden * 2 > kLastLevelCacheBytes ? 2 : 1;
-    if (tuning.dispatch_span == 1 || tuning.dispatch_span == 2 || tuning.dispatch_span == 4)
-        span = tuning.dispatch_span;
-    while (span < 4 && (row_chunks + span - 1) / span > kMaxWavesPerBlock)
-        span *= 2;
-    const int pieces = (row_chunks + span - 1) / span;
-    const bool ordered = expand && slot_order != nullptr && order_bound > 0 && tuning.dispatch_order != 0 &&
-                         pieces <= kMaxWavesPerBlock && order_bound < (int64_t{1} << 29);
+    // The slot-order walk is used whenever the handle carries the list and plan_list_walk takes it.
+    const ListWalk walk = plan_list_walk(num_tokens, order_bound, hidden, tuning);
+    const int span = walk.span, pieces = walk.pieces;
+    const bool ordered = expand && slot_order != nullptr && walk.taken;
     if (ordered && slot_order_entries > order_bound)
         return NANOEP_ERR_INVALID_ARGUMENT;
     if (num_tokens * num_topk >= (int64_t{1} << 31) || static_cast<int64_t>(num_tokens) * vectors >= (int64_t{1} << 32))

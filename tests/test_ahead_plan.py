@@ -80,5 +80,15 @@ def test_how_much_a_layout_reads_ahead():
         assert 4 * MIB < bytes_ahead(32768, 8, 64, 512) <= 8 * MIB
         for refused in ((0, 2, 2, 256), (16, 0, 2, 256), (16, 33, 64, 256), (16, 2, 0, 256), (16, 2, 3840, 256), (16, 2, 2, 0), (16, 2, 2, 252)):
             assert bytes_ahead(*refused) == 0
-        with cabi.forced_tuning({"DISPATCH_PREFETCH": 0}):
-            assert bytes_ahead(1537, 6, 60, 2816) == 0
+
+
+def test_nothing_is_read_ahead_where_no_list_is_walked():
+    with cabi.forced_tuning({"XCDS": 8}):
+        assert bytes_ahead(300, 8, 64, 32768) > 0 and bytes_ahead(300, 8, 64, 32776) == 0  # rows beyond 64 KiB
+        assert bytes_ahead(1 << 26, 8, 64, 8) == 0  # lists of 2^29 entries
+        for switch in ("DISPATCH_PREFETCH", "DISPATCH_ORDER"):
+            with cabi.forced_tuning({switch: 0}):
+                for batch in ((16, 2, 2, 256), (256, 8, 64, 4096), (1537, 6, 60, 2816), (32768, 8, 64, 512)):
+                    assert bytes_ahead(*batch) == 0
+        with cabi.forced_tuning({"DISPATCH_PREFETCH": 1}):
+            assert bytes_ahead(256, 8, 64, 4096) > 0
