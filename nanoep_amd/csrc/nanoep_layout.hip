@@ -131,14 +131,18 @@ int layout_histogram_tokens(int64_t tokens_total, int window, int block_tokens, 
     return tokens;
 }
 
-// Source rows that a layout which knows of them reads ahead for the dispatch behind it (read_source_ahead): 4 MiB beside the
-// assignment while that has no more workgroups than the device compute units (any more of them wait for a place: + 2 us with as
-// little as 2 MiB), 8 MiB beside the histogram rows of batches whose pairs are 4096 wavefronts' (2^18) and more, nothing in between
-// (16384 x 1024 top-8 55.8 -> 56.6 (level) with 8 MiB beside the rows).  Both launches wait for round trips, not for bytes, until the reads
-// go on longer than they do.  Layout and dispatch, launch period, sources from HBM (in the last-level cache), nothing -> 4 MiB
-// beside the assignment: 1537 x 2816 top-6 19.4 -> 18.8 us (18.1 -> 18.1), 2048 x 5120 top-8 34.0 -> 33.5 (31.3 -> 31.4), 4096 x 4096 top-2
-// 25.4 -> 25.2 (20.3 -> 20.2), 4096 x 7168 top-8 85.2 -> 85.1 (81.8 -> 81.4), 8192 x 2048 61.6 -> 61.4 (57.5 -> 57.1), 16384 x 2048 top-4 66.7 ->
-// 67.2 (57.7 -> 57.4); nothing -> 8 MiB beside the histogram rows: 32768 x 512 top-8 61.1 -> 61.0 (55.1 -> 54.6), 32768 x 1024 105.8 -> 105.9
+// Source rows that a layout which knows of them reads ahead for the dispatch behind it (read_source_ahead): up to 4 MiB beside the
+// assignment while that launch then has a workgroup for no more than three quarters of the compute units, up to 2 MiB until it has one for
+// each, nothing beyond (what waits for a place holds the launch up); 8 MiB beside the histogram rows of batches whose pairs are 4096
+// wavefronts' (2^18) and more.  Both launches wait for round trips, not for bytes, until the reads go on longer than they do.
+// Layout and dispatch, launch period, no row used again within 768 MiB (one x, in the caches), nothing -> this rule:
+// 4 MiB: 800 x 7168 top-8 25.0 -> 24.1 us (21.9 -> 22.0), 1024 x 2048 top-4 11.6 -> 10.4 (10.6 -> 10.6), 1537 x 2816 top-6 22.9 -> 21.4
+// (17.9 -> 17.9), 2048 x 5120 top-8 34.4 -> 34.0 (31.6 -> 31.6), 3000 x 4096 43.9 -> 43.0 (38.5 -> 38.3), 4096 x 4096 top-2 25.4 -> 25.2 (20.4 ->
+// 20.2), 4096 x 7168 top-8 86.0 -> 86.0 (82.1 -> 81.7), 6000 x 2048 49.5 -> 48.2 (43.1 -> 42.9), 12000 x 4096 top-2 59.2 -> 58.7 (55.1 -> 54.3);
+// 2 MiB: 8192 x 2048 top-8 62.1 -> 61.6 (level), 16384 x 4096 top-2 75.9 -> 75.5 (64.8 -> 64.5), 28000 x 512 top-8 54.7 -> 54.5 (48.1 -> 47.9); with
+// 4 MiB there 8192 x 4096 top-2 44.5 -> 45.0, 16384 x 4096 top-2 76.9, 16384 x 2048 top-4 67.2 -> 67.4; with 4 MiB beside 235 to 251 workgroups
+// 30000 x 512 58.9 -> 60.9 (49.7 -> 50.4), 32000 x 512 62.2 -> 65.3 (55.3 -> 56.1), 16000 x 1024 59.3 -> 60.3 (51.9 -> 52.2).
+// 8 MiB beside the histogram rows: 32768 x 512 top-8 61.1 -> 61.2 (55.0 -> 54.3), 32768 x 1024 105.8 -> 105.9
 // (95.9 -> 94.9), 65536 x 512 top-4 77.8 -> 77.5 (63.3 -> 62.6).  Both, 8 + 4 MiB, gains another percent with resident sources and loses up
 // to 3 with sources from HBM (4096 x 4096 top-2 26.1, 16384 x 2048 68.4, 32768 x 1024 108.2).
 constexpr int64_t kHistogramAheadBytes = int64_t{8} << 20;
@@ -232,9 +236,9 @@ struct LayoutArgs {
 // to them in contiguous shares, so an XCD's L2 then holds the first rows of its first window before the dispatch is launched, and the
 // last-level cache what does not fit.  Of fewer windows, or of the one of up to 256 tokens, every XCD copies rows from all of the batch:
 // those find them in the last-level cache.  (The walk's own prefetch is off for a batch of one window, where it stands in front of
-// one XCD's copies; these reads are ahead of all copies.)  Layout and dispatch, launch period, sources from HBM, nothing -> read ahead:
-// 128 x 7168 top-8 10.6 -> 9.5 us, 200 x 5120 top-6 10.5 -> 9.7, 256 x 4096 10.9 -> 9.8, 256 x 7168 13.7 -> 12.7, top-2 8.8 -> 7.8; up to 64
-// tokens, and with sources in the caches, within 0.1.  Nothing depends on these reads.
+// one XCD's copies; these reads are ahead of all copies.)  Layout and dispatch, launch period, no row used again within 768 MiB, nothing ->
+// read ahead: 128 x 7168 top-8 10.4 -> 9.6 us, 200 x 5120 top-6 10.3 -> 9.8, 256 x 4096 10.5 -> 9.7, 256 x 7168 13.2 -> 12.8, top-2 9.6 -> 9.4;
+// with one x, in the caches, all within 0.1.  Nothing depends on these reads.
 struct SourceAhead {
     const u32x4* x;        // [T][row vectors], or null
     uint32_t work_blocks;  // workgroups of the launch's own
@@ -1117,8 +1121,13 @@ LayoutPlan plan_layout(int64_t num_tokens, int num_topk, int64_t num_local_exper
     const int64_t row_vectors = hidden / 8, xcds = make_xcd_map(knobs.xcds).count;
     if (plan.source != kDirect && pairs >= kOneChunkWaves * kWave)
         plan.beside_rows = plan_ahead(num_tokens, row_vectors, plan.window, xcds, plan.row_waves, kHistogramAheadBytes);
-    else if (plan.source == kDirect || plan.assign_blocks <= static_cast<unsigned>(knobs.cus))
+    else
         plan.beside_assignment = plan_ahead(num_tokens, row_vectors, plan.window, xcds, plan.waves, kAssignAheadBytes);
+    const auto launched = [&] { return static_cast<int64_t>(plan.assign_blocks) + plan.beside_assignment.blocks; };
+    if (launched() * 4 > knobs.cus * int64_t{3})
+        plan.beside_assignment = plan_ahead(num_tokens, row_vectors, plan.window, xcds, plan.waves, kAssignAheadBytes / 2);
+    if (launched() > knobs.cus)
+        plan.beside_assignment = {0, 0, 0};
     return plan;
 }
 

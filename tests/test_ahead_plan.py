@@ -75,8 +75,8 @@ def bytes_ahead(tokens, topk, experts, hidden):
 def test_how_much_a_layout_reads_ahead():
     with cabi.forced_tuning({"XCDS": 8}):
         assert bytes_ahead(16, 2, 2, 256) == 16 * 512  # all of a small batch
-        assert 0 < bytes_ahead(1537, 6, 60, 2816) <= 4 * MIB
-        assert 0 < bytes_ahead(4096, 8, 256, 7168) <= 4 * MIB
+        assert 3 * MIB < bytes_ahead(1537, 6, 60, 2816) <= 4 * MIB
+        assert 3 * MIB < bytes_ahead(4096, 8, 256, 7168) <= 4 * MIB
         assert 4 * MIB < bytes_ahead(32768, 8, 64, 512) <= 8 * MIB
         for refused in ((0, 2, 2, 256), (16, 0, 2, 256), (16, 33, 64, 256), (16, 2, 0, 256), (16, 2, 3840, 256), (16, 2, 2, 0), (16, 2, 2, 252)):
             assert bytes_ahead(*refused) == 0
@@ -92,3 +92,14 @@ def test_nothing_is_read_ahead_where_no_list_is_walked():
                     assert bytes_ahead(*batch) == 0
         with cabi.forced_tuning({"DISPATCH_PREFETCH": 1}):
             assert bytes_ahead(256, 8, 64, 4096) > 0
+
+
+# 4 MiB are 64 workgroups of eight wavefronts or 32 of sixteen: with 128 or 160 of the assignment's own three quarters of the compute units
+# have one.  2 MiB are half as many: with 224 or 240 all have one.
+@pytest.mark.parametrize("topk,hidden,most,some", [(8, 2048, 8128, 14272), (8, 512, 20352, 30592)])
+def test_less_is_read_beside_an_assignment_that_leaves_less_room(topk, hidden, most, some):
+    with cabi.forced_tuning({"XCDS": 8}):
+        assert cabi.device_topology()[0] == 256
+        assert bytes_ahead(most, topk, 64, hidden) == 4 * MIB and bytes_ahead(most + 1, topk, 64, hidden) == 2 * MIB
+        assert bytes_ahead(some, topk, 64, hidden) == 2 * MIB and bytes_ahead(some + 1, topk, 64, hidden) == 0
+        assert bytes_ahead(32767, topk, 64, hidden) == 0
