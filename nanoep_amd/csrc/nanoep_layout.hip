@@ -133,8 +133,8 @@ int layout_histogram_tokens(int64_t tokens_total, int window, int block_tokens, 
 
 // Source rows that a layout which knows of them reads ahead for the dispatch behind it (read_source_ahead): up to 4 MiB beside the
 // assignment while that launch then has a workgroup for no more than three quarters of the compute units, up to 2 MiB until it has one for
-// each, nothing beyond (what waits for a place holds the launch up); 8 MiB beside the histogram rows of batches whose pairs are 4096
-// wavefronts' (2^18) and more.  Both launches wait for round trips, not for bytes, until the reads go on longer than they do.
+// each, nothing beyond (what waits for a place holds the launch up); up to 8 MiB beside the histogram rows of batches of 2^18 pairs and more,
+// whose assignment never has the room.  Both launches wait for round trips, not for bytes, until the reads go on longer than they do.
 // Layout and dispatch, launch period, no row used again within 768 MiB (one x, in the caches), nothing -> this rule:
 // 4 MiB: 800 x 7168 top-8 25.0 -> 24.1 us (21.9 -> 22.0), 1024 x 2048 top-4 11.6 -> 10.4 (10.6 -> 10.6), 1537 x 2816 top-6 22.9 -> 21.4
 // (17.9 -> 17.9), 2048 x 5120 top-8 34.4 -> 34.0 (31.6 -> 31.6), 3000 x 4096 43.9 -> 43.0 (38.5 -> 38.3), 4096 x 4096 top-2 25.4 -> 25.2 (20.4 ->
@@ -142,9 +142,13 @@ int layout_histogram_tokens(int64_t tokens_total, int window, int block_tokens, 
 // 2 MiB: 8192 x 2048 top-8 62.1 -> 61.6 (level), 16384 x 4096 top-2 75.9 -> 75.5 (64.8 -> 64.5), 28000 x 512 top-8 54.7 -> 54.5 (48.1 -> 47.9); with
 // 4 MiB there 8192 x 4096 top-2 44.5 -> 45.0, 16384 x 4096 top-2 76.9, 16384 x 2048 top-4 67.2 -> 67.4; with 4 MiB beside 235 to 251 workgroups
 // 30000 x 512 58.9 -> 60.9 (49.7 -> 50.4), 32000 x 512 62.2 -> 65.3 (55.3 -> 56.1), 16000 x 1024 59.3 -> 60.3 (51.9 -> 52.2).
-// 8 MiB beside the histogram rows: 32768 x 512 top-8 61.1 -> 61.2 (55.0 -> 54.3), 32768 x 1024 105.8 -> 105.9
-// (95.9 -> 94.9), 65536 x 512 top-4 77.8 -> 77.5 (63.3 -> 62.6).  Both, 8 + 4 MiB, gains another percent with resident sources and loses up
-// to 3 with sources from HBM (4096 x 4096 top-2 26.1, 16384 x 2048 68.4, 32768 x 1024 108.2).
+// 8 MiB, no row used again within 768 MiB it is level, one x in the caches it gains: 2^18 pairs 32768 x 512 top-8 61.3 -> 61.2 (55.4 -> 54.6), 32768 x
+// 1024 106.7 -> 106.7 (96.5 -> 95.4), 32768 x 2048 202.3 -> 201.3 (179.8 -> 178.6), 65536 x 512 top-4 77.7 -> 77.9 (63.7 -> 63.1); more: 44000 x
+// 1024 top-6 121.9 -> 121.0 (106.2 -> 105.4), 40000 x 1024 top-8 130.9 -> 131.4 (121.6 -> 120.6), 65536 x 512 114.4 -> 113.7 (101.5 -> 101.2), 65536 x 1024
+// 198.1 -> 197.2 (178.4 -> 178.3), 131072 x 256 143.5 -> 141.8 (118.2 -> 118.5).  At 2^17 pairs it is a trade: 16384 x 1024 top-8 55.9 -> 56.2
+// (51.1 -> 50.8), 16384 x 4096 191.6 -> 192.4 (169.8 -> 169.1), 32768 x 1024 top-4 68.2 -> 69.3 (59.1 -> 58.3).  From about 160000 pairs on it would
+// gain already where the assignment has no room (31000 x 512 top-8 59.4 -> 58.8 (51.7 -> 50.5), 48000 x 512 top-4 58.0 -> 58.0 (49.9 -> 48.8)).
+constexpr int64_t kHistogramAheadPairs = int64_t{1} << 18;
 constexpr int64_t kHistogramAheadBytes = int64_t{8} << 20;
 constexpr int64_t kAssignAheadBytes = int64_t{4} << 20;
 
@@ -1119,7 +1123,7 @@ LayoutPlan plan_layout(int64_t num_tokens, int num_topk, int64_t num_local_exper
     plan.assign_blocks = static_cast<uint32_t>(plan.blocks + (plan.source == kScanned ? 0 : 1));
 
     const int64_t row_vectors = hidden / 8, xcds = make_xcd_map(knobs.xcds).count;
-    if (plan.source != kDirect && pairs >= kOneChunkWaves * kWave)
+    if (plan.source != kDirect && pairs >= kHistogramAheadPairs)
         plan.beside_rows = plan_ahead(num_tokens, row_vectors, plan.window, xcds, plan.row_waves, kHistogramAheadBytes);
     else
         plan.beside_assignment = plan_ahead(num_tokens, row_vectors, plan.window, xcds, plan.waves, kAssignAheadBytes);
