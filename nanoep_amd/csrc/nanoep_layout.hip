@@ -345,18 +345,11 @@ __device__ __forceinline__ void clear_lds(uint32_t* lds, uint32_t words, uint32_
         reinterpret_cast<u32x4*>(lds)[i] = zero;
 }
 
-// A workgroup barrier for what passes through LDS alone: loads from and stores to global memory stay on their way
-// across it.  Nothing in these kernels passes between threads through global memory; a __syncthreads() here waits for
-// the ids' and rows' loads at the first barrier and for the snapshot's stores at the next one.
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // Names a word of every cache line of the arguments: they arrive with the first batch of scalar loads, and what is
 // asked for later is in the scalar cache.  Left where it is first used, a line is a round trip to memory of its own on the
-// way of every wavefront, 0.2 to 0.4 us each.
+// way of every wavefront.  Launch period, without -> with: one launch 256 x 8, 64 experts 4.51 -> 4.37 us, 1537 x 4, 60 experts 6.28 -> 6.13; two
+// launches 1537 x 6 7.90 -> 7.54, 4096 x 8, 64 experts 8.01 -> 7.61, 8192 x 8, 128 experts 9.08 -> 8.67, 32768 x 8 12.5 -> 12.1.  (Barriers that
+// wait for LDS alone, in place of __syncthreads(), give nothing: 0.00 +- 0.05 us over the same batches.)
 __device__ __forceinline__ void fetch_layout_arguments(const LayoutArgs& a) {
     static_assert(sizeof(LayoutArgs) <= 4 * 64, "one word of every line");
     NANOEP_FETCH_ARGS_4(a.topk_idx, a.per_thread, a.alignment, a.dst_slots);
@@ -398,10 +391,10 @@ __global__ void __launch_bounds__(kLayoutThreads) layout_histogram_kernel(const 
             if (threadIdx.x == 0)
                 info = RowInfo{0, 0, 0, 0};
         } else {
-            lds_barrier();
+            __syncthreads();
             clear_lds(bits, a.experts * words, waves * kWave);
         }
-        lds_barrier();
+        __syncthreads();
         while (chunk < end) {
 #pragma unroll
             for (int j = 0; j < kChunks; ++j) {
@@ -434,7 +427,7 @@ __global__ void __launch_bounds__(kLayoutThreads) layout_histogram_kernel(const 
         atomicAdd(&info.assigned, assigned);
         atomicOr(&info.status, bad);
     }
-    lds_barrier();
+    __syncthreads();
     int32_t* row = a.histograms + static_cast<uint64_t>(blockIdx.x) * a.experts;
     for (uint32_t i = threadIdx.x; i < a.experts; i += waves * kWave)
         row[i] = static_cast<int32_t>(counts[i]);
@@ -618,7 +611,7 @@ __device__ __forceinline__ void publish_layout(const LayoutArgs& a, uint32_t* ld
     clear_lds(lds, (a.experts + 3) / 4 * 4 + a.experts * words, a.waves * kWave);
     if (tid == 0)
         all = RowInfo{0, 0, 0, 0};
-    lds_barrier();
+    __syncthreads();
     uint32_t received = 0, assigned = 0;
     int bad = 0;
     if (kSource == kDirect) {
@@ -672,7 +665,7 @@ __device__ __forceinline__ void publish_layout(const LayoutArgs& a, uint32_t* ld
         atomicAdd(&all.assigned, assigned);
         atomicOr(&all.status, bad);
     }
-    lds_barrier();
+    __syncthreads();
     const uint32_t first = tid * a.per_thread < a.experts ? tid * a.per_thread : a.experts;
     const uint32_t last = first + a.per_thread < a.experts ? first + a.per_thread : a.experts;
     uint64_t padded_sum = 0, padded_scan = 0;
@@ -683,7 +676,7 @@ __device__ __forceinline__ void publish_layout(const LayoutArgs& a, uint32_t* ld
         if (at.lane == kWave - 1)
             wave_padded[wave] = padded_scan;
     }
-    lds_barrier();
+    __syncthreads();
     if (wave >= a.expert_waves)
         return;
     uint64_t running = padded_scan - padded_sum, capacity = 0;
@@ -792,7 +785,7 @@ __global__ void __launch_bounds__(kLayoutThreads) layout_assign_kernel(const Lay
         any_bits[tid] = 0;
     if (tid == 0)
         sums = {0, 0, 0, 0, 0};
-    lds_barrier();
+    __syncthreads();
     uint32_t own = 0;
 #pragma unroll
     for (int o = 0; o < kOwn; ++o) {
@@ -894,7 +887,7 @@ __global__ void __launch_bounds__(kLayoutThreads) layout_assign_kernel(const Lay
             }
         }
     }
-    lds_barrier();
+    __syncthreads();
     // Experts: a thread takes a run of them (one each up to the workgroup's threads), the wavefronts
     // without any go on to the last barrier.
     const uint32_t first = tid * a.per_thread < a.experts ? tid * a.per_thread : a.experts;
@@ -955,7 +948,7 @@ __global__ void __launch_bounds__(kLayoutThreads) layout_assign_kernel(const Lay
         }
     }
     if (a.expert_waves > 1)
-        lds_barrier();
+        __syncthreads();
     else
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the sums stay within the one wavefront
     if (wave < a.expert_waves) {
@@ -973,14 +966,14 @@ __global__ void __launch_bounds__(kLayoutThreads) layout_assign_kernel(const Lay
             running_window += window & 0xffffu;
         }
     }
-    lds_barrier();
+    __syncthreads();
     if (kSource == kScanned && tid == 0) {
         sums.assigned_before = sums.assigned;
         sums.assigned = static_cast<uint32_t>(a.totals[0]);
         sums.received_before += a.rows[own_row].received;
     }
     if (kSource == kScanned)
-        lds_barrier();
+        __syncthreads();
 
 #pragma unroll
     for (int o = 0; o < kOwn; ++o) {
