@@ -616,15 +616,19 @@ int nanoep_combine(const void* y, const float* weights, const void* bias, const 
         // 44.7 -> 43.5, 32768 x 1024 84.2 -> 83.7; within half a percent at 2048 x 7168, 3000 x 7168,
         // 4096 x 4096 top-16).  Launches of several rounds lose with it (16384 x 7168: 311 -> 323 us).
         const bool strided = held_groups * chunks <= held_resident;
-        // ... and, with the rows of a token fetched at once and all sixteen tokens a wavefront, every XCD a run of neighbouring
-        // groups: the rows its wavefronts read in an expert's segment at any moment are neighbours too.  Dealt one by one -> in
-        // runs, top-8: 4600 x 7168 83.7 -> 80.9 us, 8192 x 4096 84.1 -> 82.4, 16384 x 2048 83.3 -> 82.2, 32768 x 1024 83.4 -> 82.0, 60000 x
-        // 512 78.4 -> 76.5; top-7 8192 x 4096 78.0 -> 74.5, 32768 x 1024 76.7 -> 76.0.  Nine to fifteen tokens a wavefront are within a
-        // percent of level either way (4096 x 7168 72.9 -> 72.4, with segments padded to 128 level; 3600 x 7168 68.2 -> 67.9, 2800 x 7168 53.4 ->
-        // 53.9, 3300 x 7168 61.8 -> 62.2).  Fewer tokens, more rows a token, several rounds or one token a wavefront: level or
-        // slower (8192 x 2048 45.1 -> 45.4, 4000 x 5120 top-10 70.1 -> 71.0, 12000 x 2816 top-7 80.7 -> 81.4, 16384 x 2048 top-4 47.5 -> 50.0).
+        // ... and, with the rows of a token fetched at once and more than eight tokens a wavefront, every XCD a run of neighbouring
+        // groups.  A line of the slot table is four neighbouring tokens' slots, which are four neighbouring groups': dealt one by one, all
+        // XCDs fetch all of the table (32768 x 1024 top-8 reads 480.7 MB into the L2s dealt and 473.6 in runs, 8192 x 4096 474.4 and 472.7,
+        // 4096 x 7168 415.0 and 414.3), so it is short rows that gain.  Dealt -> in runs, bursts of 12 launches, top-8, rows from HBM: sixteen tokens
+        // a wavefront 32768 x 1024 83.8 -> 82.0 us, 65536 x 512 83.9 -> 82.2, 8192 x 4096 84.0 -> 82.9, 16384 x 2048 83.9 -> 83.1, 4600 x 7168 82.9 -> 82.9,
+        // top-7 8192 x 4096 77.9 -> 74.9; fifteen 30000 x 1024 78.1 -> 76.7, 60000 x 512 78.3 -> 76.9, 4096 x 7168 73.7 -> 73.4; fourteen 28000 x 1024
+        // 72.7 -> 72.1, 7000 x 4096 75.0 -> 72.5; thirteen 50000 x 512 65.9 -> 64.7, 3600 x 7168 66.7 -> 66.2; nine to twelve 24000 x 1024 64.1 ->
+        // 63.9, 20000 x 1024 52.9 -> 52.7, 3000 x 7168 56.3 -> 55.4, 4096 x 5120 56.2 -> 56.5.  In a loop that goes on until the part throttles
+        // all of them are within a percent of level, 32768 x 1024 at sixteen 2 % better.  Fewer tokens, more rows a token, several rounds or one
+        // token a wavefront: level or slower (8192 x 2048 with weights 45.3 -> 46.0, 4000 x 5120 top-10 70.1 -> 71.0, 12000 x 2816 top-7 80.7 -> 81.4,
+        // 16384 x 2048 top-4 47.5 -> 50.0).  At 256 compute units these are launches of 32769 to 65536 wavefronts of one token each.
         const XcdMap xcds = make_xcd_map(topology.xcds);
-        const bool in_runs = strided && held_units == 16 && num_topk <= kHeldRows;
+        const bool in_runs = strided && held_units > 8 && num_topk <= kHeldRows;
         const int64_t per_xcd = in_runs ? (held_groups * chunks + xcds.count - 1) / xcds.count : 0;
         const int64_t held_blocks = held_side_blocks + (in_runs ? per_xcd * xcds.count : held_groups * chunks);
         if (held_blocks >= (int64_t{1} << 31))

@@ -141,6 +141,23 @@ def test_sixteen_held_tokens_in_runs_of_groups(device, tuning, tokens, hidden, t
     assert_same_bits(got_w, want_w)
 
 
+# The same with nine to fifteen tokens a wavefront: a last group of fewer tokens, shares cut short and empty, side workgroups in front.
+@pytest.mark.parametrize("xcds", [0, 3])
+@pytest.mark.parametrize("units", [8, 9, 12, 15])
+@pytest.mark.parametrize("tokens,hidden,topk", [(9, 256, 8), (121, 1536, 6), (400, 2816, 8), (1009, 520, 7)])
+def test_nine_to_fifteen_held_tokens_in_runs_of_groups(device, tuning, tokens, hidden, topk, units, xcds):
+    tuning("XCDS", xcds)
+    idx = cases.routing("dropout", tokens, 24, topk, seed=hidden)
+    lay = oracle.layout(idx, 24, 16)
+    y = cases.payload(lay.expanded_capacity, hidden, seed=tokens)
+    w = cases.gate_weights(lay.expanded_capacity, 1, seed=tokens).reshape(-1)
+    want, want_w = oracle.combine(y, lay.recv_metadata(True), lay.dst_slots, weights=w, do_expand=True)
+    metadata, counts = cabi.layout(idx.to(device), 24, 16, True, hidden=hidden)
+    got, got_w = cabi.combine(y.to(device), w.to(device), None, metadata, counts, True, poison=0xA5, units=units)
+    assert_same_bits(got, want)
+    assert_same_bits(got_w, want_w)
+
+
 def small_case(device, seed, tokens=96, hidden=512, experts=12, topk=4):
     idx = cases.routing("dropout", tokens, experts, topk, seed=seed)
     x, w = cases.payload(tokens, hidden, seed=seed), cases.gate_weights(tokens, topk, seed=seed)
