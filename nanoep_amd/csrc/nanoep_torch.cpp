@@ -13,6 +13,7 @@
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/core/Event.h>
+#include <cxxabi.h>
 #include <hip/hip_runtime_api.h>
 #include <torch/extension.h>
 
@@ -20,6 +21,7 @@
 #include <atomic>
 #include <cstdlib>
 #include <deque>
+#include <exception>
 #include <initializer_list>
 #include <limits>
 #include <memory>
@@ -27,6 +29,7 @@
 #include <optional>
 #include <string>
 #include <tuple>
+#include <utility>
 #include <vector>
 
 #include "nanoep_hip.h"
@@ -1457,12 +1460,11 @@ class Arguments {
     bool fits() const { return fits_; }
 
     PeerRuntime* runtime() {
-        py::detail::type_caster<PeerRuntime> caster;
-        if (!caster.load(py::handle(*next_++), /*convert=*/false) || py::detail::cast_op<PeerRuntime*>(caster) == nullptr) {
-            fits_ = false;
-            return nullptr;
-        }
-        return py::detail::cast_op<PeerRuntime*>(caster);
+        const py::handle object(*next_++);
+        if (py::isinstance<PeerRuntime>(object))
+            return object.cast<PeerRuntime*>();
+        fits_ = false;
+        return nullptr;
     }
     torch::Tensor tensor() {
         PyObject* object = *next_++;
@@ -1533,17 +1535,21 @@ py::list wrapped(std::vector<torch::Tensor>& tensors) {
 
 py::object wrapped(const std::shared_ptr<CompletionEvent>& event) { return event ? py::cast(event) : py::none(); }
 
-// Runs `call` and makes its exceptions Python's, as the bound functions do.
+PyObject* g_rethrow = nullptr;                  // a bound function that throws this thread's exception
+thread_local std::exception_ptr g_exception;
+
+// Runs `call`; the binding makes its exceptions Python's, as it does those of the bound functions.  A thread that is ended inside
+// the call unwinds on.
 template <class Call>
 PyObject* guarded(const Call& call) {
     try {
         return call();
-    } catch (py::error_already_set& error) {
-        error.restore();
+    } catch (abi::__forced_unwind&) {
+        throw;
     } catch (...) {
-        py::detail::try_translate_exceptions();
+        g_exception = std::current_exception();
     }
-    return nullptr;
+    return PyObject_CallNoArgs(g_rethrow);
 }
 
 constexpr Py_ssize_t kDispatchArguments = 16, kCombineArguments = 12;
@@ -1655,4 +1661,5 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, module) {
     static PyMethodDef dispatch_definition, combine_definition;
     nanoep::call_ahead_of(module, dispatch_definition, "dispatch", &nanoep::call_dispatch, nanoep::g_bound_dispatch);
     nanoep::call_ahead_of(module, combine_definition, "combine", &nanoep::call_combine, nanoep::g_bound_combine);
+    nanoep::g_rethrow = py::cpp_function([] { std::rethrow_exception(std::exchange(nanoep::g_exception, nullptr)); }).release().ptr();
 }

@@ -327,3 +327,35 @@ def test_operator_call_forms_agree(device):
             native.combine(*arguments[:8], -1, *arguments[9:])
     finally:
         buffer.close()
+
+
+# What goes wrong inside a call by position reaches Python as it does from a bound one: type, text, and nothing left behind.
+def test_operator_call_forms_raise_the_same(device):
+    native = load_extension()
+    tokens, experts, topk, hidden = 9, 8, 3, 512
+    idx = cases.routing("dropout", tokens, experts, topk, seed=5).to(device)
+    x = cases.payload(tokens, hidden, seed=5).to(device)
+    buffer = ReferenceShapedBuffer(native, device, experts, topk, hidden, tokens)
+    try:
+        stream = buffer.comm_stream.cuda_stream
+        good = [buffer.runtime, x, idx, None, experts, tokens, 4, [], 0, False, True, True, 0, stream, -1, False]
+        names = ("runtime", "x", "indices", "weights", "num_experts", "max_tokens", "alignment", "cached_metadata", "cached_expanded_capacity",
+                 "allow_multiple_reduction", "expand", "zero_padding", "num_sms", "comm_stream", "previous_event", "async_op")
+        bad_idx = idx.clone()
+        bad_idx[3, 0] = experts + 2
+        for position, wrong in ((1, x.float()), (1, x[:, :-1]), (2, bad_idx), (6, 0), (12, -1)):
+            arguments = [*good[:position], wrong, *good[position + 1 :]]
+            raised = []
+            for call in (lambda: native.dispatch(*arguments), lambda: native.dispatch(**dict(zip(names, arguments)))):
+                with pytest.raises(Exception) as info:
+                    call()
+                raised.append((info.type, str(info.value).splitlines()[0]))
+            assert raised[0] == raised[1]
+        outputs, metadata, counts, _ = native.dispatch(*good)
+        arguments = [buffer.runtime, outputs[0], metadata, None, None, tokens, True, False, -1, stream, -1, False]
+        for call in (lambda: native.combine(*arguments), lambda: native.combine(*arguments[:11], async_op=False)):
+            with pytest.raises(RuntimeError, match="num_sms must be between 0"):
+                call()
+        assert native.combine(*arguments[:8], 0, *arguments[9:])[1] is None
+    finally:
+        buffer.close()
