@@ -1610,12 +1610,20 @@ PyObject* call_combine(PyObject*, PyObject* const* args, Py_ssize_t count, PyObj
     });
 }
 
-// Puts `call` in the place of the module's bound function of that name, and keeps that one for the calls it passes on.
+// Puts `call` in the place of the module's bound function of that name, with its docstring, and keeps that one for the calls it
+// passes on.
+struct CallAhead {
+    PyMethodDef definition;
+    std::string doc;
+};
+
 template <class Function>
-void call_ahead_of(py::module_& module, PyMethodDef& definition, const char* name, Function call, PyObject*& bound) {
-    bound = py::object(module.attr(name)).release().ptr();
-    definition = {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(call)), METH_FASTCALL | METH_KEYWORDS, nullptr};
-    module.attr(name) = py::reinterpret_steal<py::object>(PyCFunction_NewEx(&definition, nullptr, module.attr("__name__").ptr()));
+void call_ahead_of(py::module_& module, CallAhead& ahead, const char* name, Function call, PyObject*& bound) {
+    const py::object function = module.attr(name);
+    ahead.doc = py::str(function.attr("__doc__"));
+    bound = py::object(function).release().ptr();
+    ahead.definition = {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(call)), METH_FASTCALL | METH_KEYWORDS, ahead.doc.c_str()};
+    module.attr(name) = py::reinterpret_steal<py::object>(PyCFunction_NewEx(&ahead.definition, nullptr, module.attr("__name__").ptr()));
 }
 
 }  // namespace
@@ -1658,8 +1666,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, module) {
         .def("close", &nanoep::PeerRuntime::close);
     py::class_<nanoep::CompletionEvent, std::shared_ptr<nanoep::CompletionEvent>>(module, "CompletionEvent")
         .def("current_stream_wait", &nanoep::CompletionEvent::current_stream_wait);
-    static PyMethodDef dispatch_definition, combine_definition;
-    nanoep::call_ahead_of(module, dispatch_definition, "dispatch", &nanoep::call_dispatch, nanoep::g_bound_dispatch);
-    nanoep::call_ahead_of(module, combine_definition, "combine", &nanoep::call_combine, nanoep::g_bound_combine);
+    static nanoep::CallAhead dispatch_ahead, combine_ahead;
+    nanoep::call_ahead_of(module, dispatch_ahead, "dispatch", &nanoep::call_dispatch, nanoep::g_bound_dispatch);
+    nanoep::call_ahead_of(module, combine_ahead, "combine", &nanoep::call_combine, nanoep::g_bound_combine);
     nanoep::g_rethrow = py::cpp_function([] { std::rethrow_exception(std::exchange(nanoep::g_exception, nullptr)); }).release().ptr();
 }

@@ -232,3 +232,19 @@ def test_plain_c_client_compiles_links_and_runs(tmp_path):
     assert out[0] == "abi 4 status 0 window 0 96 160 160 9888"
     assert out[1].startswith("invalid 1 '") and "invalid" in out[1].lower()
     assert out[2] == "sizes 32769 256 1"
+
+
+def test_the_operators_have_their_docstrings():
+    from nanoep_amd._native import load_extension
+
+    native = load_extension()
+    for name, arguments in (
+        ("dispatch", "runtime x indices weights num_experts max_tokens alignment cached_metadata cached_expanded_capacity "
+                     "allow_multiple_reduction expand zero_padding num_sms comm_stream previous_event async_op"),
+        ("combine", "runtime x metadata weights bias max_tokens expand allow_multiple_reduction num_sms comm_stream previous_event async_op"),
+    ):
+        text = getattr(native, name).__doc__
+        assert text.startswith(name + "(") and [text.index(f"{argument}: ") for argument in arguments.split()] == sorted(
+            text.index(f"{argument}: ") for argument in arguments.split()
+        )
+        assert getattr(native, name).__name__ == name and getattr(native, name).__module__ == native.__name__
