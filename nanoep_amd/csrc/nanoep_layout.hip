@@ -142,6 +142,10 @@ int layout_histogram_tokens(int64_t tokens_total, int window, int block_tokens, 
 // 2 MiB: 8192 x 2048 top-8 62.1 -> 61.6 (level), 16384 x 4096 top-2 75.9 -> 75.5 (64.8 -> 64.5), 28000 x 512 top-8 54.7 -> 54.5 (48.1 -> 47.9); with
 // 4 MiB there 8192 x 4096 top-2 44.5 -> 45.0, 16384 x 4096 top-2 76.9, 16384 x 2048 top-4 67.2 -> 67.4; with 4 MiB beside 235 to 251 workgroups
 // 30000 x 512 58.9 -> 60.9 (49.7 -> 50.4), 32000 x 512 62.2 -> 65.3 (55.3 -> 56.1), 16000 x 1024 59.3 -> 60.3 (51.9 -> 52.2).
+// The device's compute units count also where a stream's mask (a compute-unit budget) leaves fewer: the workgroups that wait there hold up a layout
+// that is a smaller part of the pass.  32 of 256: 256 x 4096 top-8 24.1 -> 23.1 (18.6 -> 18.7), 800 x 7168 105.5 -> 103.7 (91.1 -> 92.1), 1537 x 2816
+// 73.7 -> 69.2 (55.6 -> 55.8), 4096 x 4096 top-2 75.3 -> 74.6 (63.9 -> 64.1), 4096 x 7168, 8192 x 2048 and 8192 x 4096 top-2 level; 64: 1537 x 2816 46.3
+// -> 42.8, 4096 x 4096 top-2 45.2 -> 45.5 (38.4 -> 38.5); 128: 1537 x 2816 32.4 -> 29.7, 8192 x 2048 84.2 -> 84.4 (78.4 -> 78.5).
 // 8 MiB, no row used again within 768 MiB it is level, one x in the caches it gains: 2^18 pairs 32768 x 512 top-8 61.3 -> 61.2 (55.4 -> 54.6), 32768 x
 // 1024 106.7 -> 106.7 (96.5 -> 95.4), 32768 x 2048 202.3 -> 201.3 (179.8 -> 178.6), 65536 x 512 top-4 77.7 -> 77.9 (63.7 -> 63.1); more: 44000 x
 // 1024 top-6 121.9 -> 121.0 (106.2 -> 105.4), 40000 x 1024 top-8 130.9 -> 131.4 (121.6 -> 120.6), 65536 x 512 114.4 -> 113.7 (101.5 -> 101.2), 65536 x 1024

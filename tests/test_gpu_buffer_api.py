@@ -12,6 +12,7 @@ import pytest
 import torch
 from torch.utils import deterministic
 
+import cabi
 import cases
 from nanoep_amd import Buffer, CudaBuffer, EPConfig
 from nanoep_amd._native import load_extension
@@ -572,6 +573,25 @@ def test_a_compute_unit_budget_confines_the_kernels_and_changes_no_result(device
 
         whole, confined = kernel_us(cus), kernel_us(quarter)
         assert confined > 1.5 * whole, (whole, confined)
+
+
+# A fresh dispatch under a budget: what the layout reads ahead goes by the whole device, and the stream's mask leaves its workgroups
+# fewer places than there are of them.
+@pytest.mark.parametrize("asynchronous", [False, True])
+@pytest.mark.parametrize("tokens,hidden,topk,alignment", [(200, 2048, 6, 1), (1537, 768, 6, 16), (4500, 512, 8, 1)])
+def test_fresh_dispatch_under_a_compute_unit_budget(device, tokens, hidden, topk, alignment, asynchronous):
+    experts = 24
+    assert cabi.lib().nanoep_layout_ahead_bytes(tokens, topk, experts, hidden) > 0
+    idx = cases.routing("dropout", tokens, experts, topk, seed=hidden)
+    x, w = cases.payload(tokens, hidden, seed=tokens), cases.gate_weights(tokens, topk)
+    budget = torch.cuda.get_device_properties(device).multi_processor_count // 8
+    with Buffer(None, EPConfig(experts, topk, hidden, tokens)) as buffer:
+        for scale in (1, 2):
+            result = buffer.dispatch((x * scale).to(device), topk_idx=idx.to(device), weights=w.to(device), do_expand=True, alignment=alignment,
+                                     zero_padding=True, num_sms=budget, async_op=asynchronous)
+            if asynchronous:
+                result.event.current_stream_wait()
+            assert_dispatch_result(result, x * scale, idx, w, experts, True, alignment, True)
 
 
 @pytest.mark.parametrize("expand", [False, True], ids=["compact", "expanded"])
