@@ -1444,9 +1444,10 @@ std::vector<int64_t> window_layout(int ranks, int64_t tokens, int hidden, int to
 
 // The module's dispatch and combine as plain CPython functions.  A call whose arguments are all positional and of the types
 // that the operators take is unpacked here; any other call (keywords, defaults, other types) goes to the bound functions
-// below, which say what is wrong with it.  Results and exceptions are theirs.  A small batch's pass is bound by the host, and a
-// good part of that was the binding: with these and two records made by position, 16 x 256 top-2, replay and combine 14.7 -> 13.0 us,
-// asynchronous 40.7 -> 36.2; fresh and combine 19.6 -> 18.5, 256 x 4096 top-8 21.4 -> 20.4 (the fastest of thirty blocks of passes).
+// below, which say what is wrong with it.  Results and exceptions are theirs.  A small batch's pass is bound by the host, and the
+// binding was a part of that: bound -> these, dispatch and combine, the fastest of sixty blocks of passes, ten processes of each (a process
+// is in one of two modes): 16 x 256 top-2 replay 14.1 -> 13.7 us (the faster mode 13.3 -> 12.8), 256 x 4096 top-8 14.5 -> 13.9 (13.3 -> 12.8), fresh 21.7 ->
+// 21.0 (19.6 -> 19.0) and 22.5 -> 22.1 (21.0 -> 20.5), asynchronous 39.3 -> 39.0 (36.1 -> 35.5).
 namespace nanoep {
 namespace {
 
