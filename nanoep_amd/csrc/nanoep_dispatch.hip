@@ -698,8 +698,9 @@ int nanoep_dispatch(const void* x, const float* weights, const int32_t* recv_met
         // with sources that sit in the last-level cache it costs 0 to 4 %: on unless
         // NANOEP_DISPATCH_PREFETCH=0.  A batch of one window (up to 256 tokens) goes without on a device of several XCDs: every XCD
         // copies a part of that window, and the prefetch would bring its rows to the first one only, ahead of that XCD's copies.
-        // On -> off, sources from HBM (in the caches): 256 x 4096 top-8 5.4 -> 4.9 us (level), 256 x 7168 8.0 -> 7.6 (5.6 -> 5.3), 200 x 5120
-        // top-6 6.3 -> 5.9 (5.1 -> 4.8), 256 x 7168 top-2 5.1 -> 4.4; count on the device 256 x 7168 8.7 -> 7.7; handle in HBM 8.3 -> 7.9.
+        // On -> off, no row used again within 768 MiB (one x, in the caches): 256 x 7168 top-8 8.4 -> 7.8 us (5.6 -> 5.3), 200 x 5120 top-6 5.4 ->
+        // 5.2 (level), 256 x 7168 top-2 5.0 -> 4.4, 256 x 4096 top-8 5.4 -> 5.6 (level); count on the device 256 x 7168 9.4 -> 8.0 (6.5 -> 5.4),
+        // 256 x 4096 6.0 -> 5.7 (4.5 -> 4.4); up to 128 tokens, and rows of up to 2048 elements, level.
         // (NANOEP_DISPATCH_PREFETCH=1 asks for it there too.)  With five to seven windows it depends: 257 x 7168 6.9 -> 6.3, but 384 x 4096 top-6 5.6 -> 5.8 (5.1 -> 5.5).
         const int window_tokens = nanoep_layout_block_tokens(num_tokens, num_local_experts, hidden);
         const bool prefetch = window_tokens > 0 && copy_blocks > 0 &&
