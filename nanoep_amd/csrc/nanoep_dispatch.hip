@@ -701,7 +701,8 @@ int nanoep_dispatch(const void* x, const float* weights, const int32_t* recv_met
         // On -> off, no row used again within 768 MiB (one x, in the caches): 256 x 7168 top-8 8.4 -> 7.8 us (5.6 -> 5.3), 200 x 5120 top-6 5.4 ->
         // 5.2 (level), 256 x 7168 top-2 5.0 -> 4.4, 256 x 4096 top-8 5.4 -> 5.6 (level); count on the device 256 x 7168 9.4 -> 8.0 (6.5 -> 5.4),
         // 256 x 4096 6.0 -> 5.7 (4.5 -> 4.4); up to 128 tokens, and rows of up to 2048 elements, level.
-        // (NANOEP_DISPATCH_PREFETCH=1 asks for it there too.)  With five to seven windows it depends: 257 x 7168 6.9 -> 6.3, but 384 x 4096 top-6 5.6 -> 5.8 (5.1 -> 5.5).
+        // (NANOEP_DISPATCH_PREFETCH=1 asks for it there too.)  With five to seven windows it depends: 257 x 7168 level, 384 x 4096 top-6 6.0 -> 5.7 (level),
+        // 448 x 7168 10.9 -> 10.4 (8.9 -> 9.0, count on the device 8.9 -> 9.3); eight gain with it (512 x 4096 6.9 on, 7.3 off).
         const int window_tokens = nanoep_layout_block_tokens(num_tokens, num_local_experts, hidden);
         const bool prefetch = window_tokens > 0 && copy_blocks > 0 &&
                               (tuning.dispatch_prefetch > 0 || (tuning.dispatch_prefetch != 0 && (num_tokens > window_tokens || xcds.count == 1)));

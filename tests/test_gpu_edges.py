@@ -90,9 +90,9 @@ def test_every_layout_plan_reports_bad_routing(device, tuning, launches, token, 
     assert counts[3] == status
 
 
-# A layout that is told of the rows reads the first of them beside its own work: rows fewer than a wavefront reads, XCD shares
-# that end inside one, as many rows as are read and one more, one launch and three, 2^18 pairs and a few
-# less.  The layout is the same, and so are the rows.
+# A layout that is told of the rows gives the same results (which rows it reads, and that they are there, test_ahead_plan.py
+# shows): rows fewer than a wavefront reads, XCD shares that end inside one, as many rows as are read and one more, one launch and
+# three, 2^18 pairs and a few less.
 @pytest.mark.parametrize("xcds", [0, 3, 16])
 @pytest.mark.parametrize(
     "tokens,hidden,topk,launches",
